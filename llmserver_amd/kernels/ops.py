@@ -171,10 +171,16 @@ class HipOps(KernelNamespace):
 
     def _few_rows_float32(self, x, weight, out):
         """Whether the 32-bit stream over the weights takes this product: few rows (by the kernel's own rule), whole tensors in their natural
-        order at multiples of 16 bytes; anything else is the library's."""
-        return x.dtype == torch.float32 and weight.dtype == torch.float32 and x.is_cuda and x.is_contiguous() and weight.is_contiguous() \
-            and (x.data_ptr() | weight.data_ptr()) % 16 == 0 \
-            and (out is None or (out.dtype == torch.float32 and out.is_contiguous() and tuple(out.shape) == (x.shape[0], weight.shape[0]))) \
+        order at multiples of 16 bytes, all on one GPU, nothing for autograd to follow; anything else is the library's, which refuses what
+        does not fit together."""
+        if not (x.dtype == weight.dtype == torch.float32 and x.is_cuda and x.dim() == weight.dim() == 2 and x.device == weight.device):
+            return False
+        if out is not None and not (out.dtype == torch.float32 and out.device == x.device and out.is_contiguous()
+                                    and tuple(out.shape) == (x.shape[0], weight.shape[0])):
+            return False
+        if torch.is_grad_enabled() and any(tensor is not None and tensor.requires_grad for tensor in (x, weight, out)):
+            return False
+        return x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 \
             and bool(self._gemm.lsa_gemm_few_f32_fits(x.shape[0], weight.shape[0], x.shape[1]))
 
     LIBRARY_MARGIN = 0.93       # the library replaces a few-row kernel only if it takes less than this share of its time

@@ -37,3 +37,22 @@ def test_what_goes_to_the_library_as_before(ops):
         assert not ops._few_rows_float32(x, w, None)
         exact = x.double() @ w.double().T
         assert float((ops.linear(x, w) - exact).norm()) <= 1e-5 * float(exact.norm())
+
+
+def test_operands_that_do_not_fit_together_are_refused(ops):
+    """What the kernel would read by address alone: a matrix or a result in host memory, matrices in a stack.  The library refuses them."""
+    x, w = torch.randn(2, 512, device="cuda"), torch.randn(8, 512, device="cuda")
+    assert ops._few_rows_float32(x, w, None)
+    for weight, out in ((w.cpu(), None), (w, torch.empty(2, 8)), (torch.randn(8, 512, 3, device="cuda"), None)):
+        assert not ops._few_rows_float32(x, weight, out)
+        with pytest.raises((RuntimeError, ValueError)):
+            ops.linear(x, weight, out=out)
+
+
+def test_gradients_pass_through_the_32_bit_product(ops):
+    x, w = torch.randn(2, 512, device="cuda", requires_grad=True), torch.randn(8, 512, device="cuda", requires_grad=True)
+    ops.linear(x, w).sum().backward()
+    exact = w.detach().double().sum(dim=0).expand(2, -1)
+    assert float((x.grad - exact).norm()) <= 1e-6 * float(exact.norm())
+    with torch.no_grad():
+        assert ops._few_rows_float32(x, w, None)
