@@ -21,6 +21,7 @@
 // Keys are stored [page][kv_head][slot][dim], values transposed [page][kv_head][dim][slot], so
 // both A operands are contiguous vector loads straight from the pages.
 #include "common.hpp"
+#include "lds_loads.hpp"
 
 #ifndef LSA_ND
 #error "compile with -DLSA_ND=<head_dim / 16>"
@@ -734,27 +735,6 @@ constexpr int MAX_HALVES = LSA_ND <= 8 ? 2 : 1;
 struct FullStep { static constexpr bool value = true; };        // every key of the step is seen by every pair
 struct MaskedStep { static constexpr bool value = false; };
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) unsigned char* lds_ptr_t;
-
-// One load of a wavefront straight into LDS: lane i's 16 bytes go to `lds_address` + 16 i (a byte address in LDS, the
-// same for all lanes).  Written out rather than called as a builtin: the compiler makes every later LDS read wait for
-// all loads it knows to write LDS, and these are meant to stay in flight while the steps before them are read.
-__device__ __forceinline__ void load_16_bytes_a_lane_to_lds(const void* source, unsigned lds_address) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(source), "s"(lds_address) : "memory", "m0");
-}
-// The same with one base for all lanes and a byte offset per lane.
-__device__ __forceinline__ void load_16_bytes_a_lane_to_lds(const void* base, unsigned offset, unsigned lds_address) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_address) : "memory", "m0");
-}
-
-// Waits until at most PENDING of this wavefront's loads are still under way (they land in the order they were
-// issued), then for the workgroup.  Written out because __syncthreads() would wait for every load, also for those
-// of the steps ahead, which are meant to stay in flight across the barrier.
-template <int PENDING>
-__device__ __forceinline__ void loads_landed_then_barrier() {
-    static_assert(PENDING >= 0 && PENDING < 64, "the counter of loads in flight has six bits");
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PENDING) : "memory");
-}
 
 // HALVES = 2: the workgroup has eight wavefronts; wavefronts 4 .. 7 take the same tiles as wavefronts 0 .. 3 and the
 // second half of the keys' steps, through LDS buffers of their own, and leave their running maximum, sum and

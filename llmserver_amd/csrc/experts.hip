@@ -10,6 +10,7 @@
 // row itself.  And there may be a shared expert that every token uses, possibly weighted by a gate of one number a token: its
 // products are made inside the same two kernels (steps of few tokens), or its output comes ready made.
 #include "common.hpp"
+#include "lds_loads.hpp"
 
 using namespace lsa;
 
@@ -713,17 +714,6 @@ __global__ __launch_bounds__(256) void experts_tile_kernel(const bf16_t* __restr
 // 16-byte reads are served together (0-3, 12-15, 20-23, 24-27 and so on) meet all 64 banks.
 constexpr int WIDE_N = 256, WIDE_ROWS = WIDE_M + WIDE_N, WIDE_SLAB = 64, WIDE_STEP = WIDE_ROWS * WIDE_SLAB * 2;      // bytes a buffer
 constexpr int WIDE_LOADS = WIDE_ROWS / 8 / 16;                  // of a wavefront a slab
-typedef __attribute__((address_space(3))) unsigned char* lds_ptr_t;
-
-// (written out: the compiler would make every LDS read wait for all loads it knows to write LDS)
-__device__ __forceinline__ void load_16_bytes_a_lane_to_lds(const void* base, unsigned offset, unsigned lds_address) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_address) : "memory", "m0");
-}
-// At most PENDING of the wavefront's loads still under way, then the workgroup's barrier.
-template <int PENDING>
-__device__ __forceinline__ void loads_landed_then_barrier() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PENDING) : "memory");
-}
 
 // The workgroup's barrier behind the LDS reads issued so far; loads stay under way.
 __device__ __forceinline__ void everybody_has_read() {

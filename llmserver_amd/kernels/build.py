@@ -11,6 +11,7 @@ from __future__ import annotations
 import concurrent.futures
 import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -62,10 +63,8 @@ def _hash(name: str) -> str:
     source, extra = module_recipe(name)
     digest = hashlib.sha256()
     own_header = os.path.join(CSRC, os.path.splitext(source)[0] + ".h")          # its entry points' declarations, if it has any
-    shared = [os.path.join(CSRC, "common.hpp")]
     with open(os.path.join(CSRC, source)) as handle:
-        if '#include "chunks.hpp"' in handle.read():
-            shared.append(os.path.join(CSRC, "chunks.hpp"))
+        shared = [os.path.join(CSRC, header) for header in re.findall(r'#include "(\w+\.hpp)"', handle.read())]
     paths = [os.path.join(CSRC, source), *shared] + ([own_header] if os.path.isfile(own_header) else [])
     for path in paths:
         with open(path, "rb") as handle:
