@@ -587,6 +587,24 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
     auto own_columns = [&](auto keys_side) {
         constexpr bool KEYS = decltype(keys_side)::value;
         auto token_of = [&](int e) { return KEYS ? 4 * g + e : 4 * e + g; };     // a block's row that a lane's number e belongs to
+        // The matrix instructions multiply the zeros above a block's diagonal too.  Where a token's column is no number, the blocks on the
+        // diagonal are multiplied without them, so that the tokens in front of it keep theirs: of a block's lower half `lower` (rows of
+        // `pitch`) and its 16 x 16 numbers y (as x below), row `t`, column `column`.
+        auto numbers = [&](const auto& of) {
+            float zero = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) zero = __builtin_fmaf((float)of[e], 0.f, zero);
+            return !__any(zero != 0.f);
+        };
+        auto row_of_lower = [&](const float* lower, int pitch, const auto& y, int t, int column) {
+            double sum = 0.0;
+#pragma unroll
+            for (int j = 0; j < BC; ++j) {
+                const double there = __shfl((double)y[KEYS ? j % 4 : j / 4], 16 * (KEYS ? j / 4 : j % 4) + column, 64);
+                if (j <= t) sum += (double)lower[t * pitch + j] * there;
+            }
+            return sum;
+        };
         mc_f4 x[2][MC / BC];
 #pragma unroll
         for (int i = 0; i < MC / BC; ++i) {
@@ -611,6 +629,10 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
                         sum[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], right[e], sum[e], 0, 0, 0);
                     }
                     x[m][i] = together(sum);
+                    if (!numbers(x[m][i])) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) x[m][i][e] = (float)row_of_lower(s.inverse[i], 20, right, 4 * g + e, r);
+                    }
                 }
             } else {
                 mc_d4 right[2] = {};
@@ -630,13 +652,19 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
 #pragma unroll
                     for (int m = 0; m < 2; ++m) {
                         const bool there = t < n && (tile0 + m - KT) * 16 + r < value_dim;
-                        sum[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, there ? right[m][e] + beta * (double)values[m][4 * i + e] : 0.0, sum[m], 0, 0, 0);
+                        right[m][e] = there ? right[m][e] + beta * (double)values[m][4 * i + e] : 0.0;
+                        sum[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, right[m][e], sum[m], 0, 0, 0);
                     }
                 }
 #pragma unroll
-                for (int m = 0; m < 2; ++m)
+                for (int m = 0; m < 2; ++m) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) x[m][i][e] = (float)sum[m][e];
+                    if (!numbers(x[m][i])) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) x[m][i][e] = (float)row_of_lower(s.inverse[i], 20, right[m], 4 * e + g, r);
+                    }
+                }
             }
         }
         const size_t cell = (size_t)blockIdx.x * heads + head;
@@ -675,28 +703,42 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
                 for (int i = 0; i <= block; ++i) {
                     const mc_f4 a = *reinterpret_cast<const mc_f4*>(&s.qk[(block * BC + r) * MC_A + i * BC + 4 * g]);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
+                    for (int m = 0; m < 2; ++m) {
+                        if (i == block && !numbers(x[m][i])) continue;
 #pragma unroll
-                        for (int m = 0; m < 2; ++m) part[m][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[m][i][e], a[e], part[m][e], 0, 0, 0);
+                        for (int e = 0; e < 4; ++e) part[m][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[m][i][e], a[e], part[m][e], 0, 0, 0);
+                    }
                 }
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {                            // a token per lane, four of its channels
-                    const mc_f4 own = *reinterpret_cast<const mc_f4*>(&s.q[(block * BC + r) * A + (tile0 + m) * 16 + 4 * g]);
-                    queries[((cell * (MC / BC) + block) * KT + tile0 + m) * 64 + lane] = own - together(part[m]);
+                    mc_f4 own = *reinterpret_cast<const mc_f4*>(&s.q[(block * BC + r) * A + (tile0 + m) * 16 + 4 * g]);
+                    own -= together(part[m]);
+                    if (!numbers(x[m][block])) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) own[e] -= (float)row_of_lower(&s.qk[block * BC * MC_A + block * BC], MC_A, x[m][block], r, 4 * g + e);
+                    }
+                    queries[((cell * (MC / BC) + block) * KT + tile0 + m) * 64 + lane] = own;
                 }
             } else {
                 mc_d4 sum[2] = {};
 #pragma unroll
                 for (int i = 0; i <= block; ++i)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const double a = (double)s.qk[(block * BC + r) * MC_A + i * BC + 4 * e + g];
+                    for (int m = 0; m < 2; ++m) {
+                        if (i == block && !numbers(x[m][i])) continue;
 #pragma unroll
-                        for (int m = 0; m < 2; ++m) sum[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)x[m][i][e], sum[m], 0, 0, 0);
+                        for (int e = 0; e < 4; ++e) {
+                            const double a = (double)s.qk[(block * BC + r) * MC_A + i * BC + 4 * e + g];
+                            sum[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)x[m][i][e], sum[m], 0, 0, 0);
+                        }
                     }
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {
                     const int column = (tile0 + m - KT) * 16 + r;
+                    if (!numbers(x[m][block])) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) sum[m][e] += row_of_lower(&s.qk[block * BC * MC_A + block * BC], MC_A, x[m][block], 4 * e + g, r);
+                    }
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int t = block * BC + 4 * e + g;

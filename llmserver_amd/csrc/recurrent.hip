@@ -1159,17 +1159,34 @@ __global__ __launch_bounds__(512) void channel_chunk_kernel(const T* __restrict_
             values[e] = v[(token0 + t) * v_stride + (size_t)head * value_dim + c];
         }
         __syncthreads();                                 // the keys are in place; the columns before have been read
+        float no_number = 0.f;                           // NaN once a value is no number
 #pragma unroll
         for (int e = 0; e < MC * 64 / 512; ++e) {
             const int t = 8 * e + (tid >> 6);
-            s_v[t * MC_B + (tid & 63)] = t < n && column0 + (tid & 63) < value_dim ? (float)values[e] : 0.f;
+            const float value = t < n && column0 + (tid & 63) < value_dim ? (float)values[e] : 0.f;
+            s_v[t * MC_B + (tid & 63)] = value;
+            no_number = __builtin_fmaf(value, 0.f, no_number);
         }
-        __syncthreads();
+        const bool all_finite = !__syncthreads_or(no_number != 0.f);
         const int r = lane & 15, g = lane >> 4, half = wave & 1;
         {
             const int block = wave >> 1;
             mc_f4 acc[2] = {};
-            channel_product<2>(acc, &s.score[block * BC * MC_A], MC_A, 1, s_v + 32 * half, MC_B, 1, (block + 1) * BC, lane);
+            if (all_finite) {
+                channel_product<2>(acc, &s.score[block * BC * MC_A], MC_A, 1, s_v + 32 * half, MC_B, 1, (block + 1) * BC, lane);
+            } else {
+                // (the products above the diagonal are of zeros: a later token's infinity or NaN must not meet them)
+#pragma unroll 1
+                for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int t = block * BC + 4 * g + e;
+                        double sum = 0.0;
+                        for (int j = 0; j <= t; ++j) sum += (double)s.score[t * MC_A + j] * (double)s_v[j * MC_B + 32 * half + 16 * ni + r];
+                        if (ni == 0) acc[0][e] = (float)sum;
+                        else acc[1][e] = (float)sum;
+                    }
+            }
 #pragma unroll
             for (int ni = 0; ni < 2; ++ni)
 #pragma unroll

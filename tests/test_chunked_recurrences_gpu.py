@@ -223,3 +223,68 @@ def test_read_outs_of_16_bit_queries_in_chunks(ops, heads, key_heads, dim, vdim)
     print(errors, flush=True)
     for scan, chunked in zip(errors["scan"], errors["chunks"]):
         assert chunked <= 2 * scan + 1e-6
+
+
+NO_NUMBERS = [float("inf"), float("-inf"), float("nan")]
+
+
+@pytest.mark.parametrize("place", [70, 79, 100, 140])
+@pytest.mark.parametrize("what", ["v", "k", "q", "decay"])
+@pytest.mark.parametrize("bonus", [False, True])
+def test_what_is_no_number_reaches_no_earlier_token_of_a_linear_recurrence(ops, place, what, bonus):
+    """A token at the start, at the end and inside a block of 16, of the first chunk of its row and of the next (rows of 20, 130 and 10
+    tokens: the second row's chunks begin at 20 and 84): the chunks leave the same numbers numbers as the walk, and those agree."""
+    heads, dim, vdim, lengths = 2, 64, 80, [20, 130, 10]
+    generator = torch.Generator("cuda").manual_seed(place)
+    draw = lambda *shape: torch.randn(*shape, device="cuda", generator=generator)
+    n = sum(lengths)
+    q, k, v, decay = 0.5 * draw(n, heads * dim), 0.5 * draw(n, heads * dim), draw(n, heads * vdim), draw(n, heads * dim) - 1.0
+    no_number = NO_NUMBERS[place % 3] if what != "decay" else float("nan")
+    {"q": q, "k": k, "v": v, "decay": decay}[what][place, 5] = no_number
+    _, _, row_start, row_len, row_ctx = batch(lengths, [3, 0, 0], "cuda")
+    slots = torch.tensor([1, 2, 0], dtype=torch.int32, device="cuda")
+    start = draw(3, heads * dim * vdim)
+    chunks = n // 64 + len(lengths)
+    scratch = {"sums": torch.empty(chunks, heads, dim, vdim, device="cuda"), "totals": torch.empty(chunks, heads, dim, device="cuda"),
+               "queries": torch.empty(n, heads, dim, device="cuda")}
+    results = []
+    for more in ({}, scratch):
+        state, out = start.clone(), torch.empty(n, heads * vdim, device="cuda")
+        ops.linear_recurrence(q, k, v, decay, None, "double_exp", 1.0, draw(heads, dim) * 0 + 0.3 if bonus else None, 0.3, state, 0, slots, row_start,
+                              row_len, row_ctx, out, heads, dim, vdim, **more)
+        results.append((out, state))
+    for walk, chunked in zip(*results):
+        assert torch.equal(torch.isfinite(walk), torch.isfinite(chunked))
+        keep = torch.isfinite(walk)
+        assert float((walk - chunked)[keep].norm()) <= 1e-5 * float(walk[keep].norm())
+    assert torch.isfinite(results[0][0][:place]).all() and not torch.isfinite(results[0][0][place:]).all()
+
+
+@pytest.mark.parametrize("place", [70, 79, 100, 140])
+@pytest.mark.parametrize("what", ["v", "k", "q", "decay", "strength"])
+@pytest.mark.parametrize("first", [0, 2])
+def test_what_is_no_number_reaches_no_earlier_token_of_a_delta_rule(ops, place, what, first):
+    heads, dim, vdim, lengths = 2, 72, 48, [20, 130, 10]
+    generator = torch.Generator("cuda").manual_seed(place)
+    draw = lambda *shape: torch.randn(*shape, device="cuda", generator=generator)
+    n, size = sum(lengths), heads * dim * vdim
+    q, k = draw(n, heads, dim), draw(n, heads, dim)
+    q, k = q / q.norm(dim=-1, keepdim=True), k / k.norm(dim=-1, keepdim=True)
+    v, strength, decay = draw(n, heads * vdim), torch.sigmoid(draw(n, heads)), torch.exp(-0.2 * torch.rand(n, heads * dim, device="cuda", generator=generator))
+    no_number = NO_NUMBERS[place % 3] if what not in ("decay", "strength") else float("nan")
+    {"q": q.view(n, -1), "k": k.view(n, -1), "v": v, "decay": decay, "strength": strength}[what][place, 1 if what == "strength" else 5] = no_number
+    prepared = torch.cat([q.reshape(n, -1), k.reshape(n, -1), v], dim=1)
+    _, _, row_start, row_len, row_ctx = batch(lengths, [3, first, 0], "cuda")
+    slots = torch.tensor([1, 2, 0], dtype=torch.int32, device="cuda")
+    start = draw(3, size)
+    scratch = torch.empty(ops.delta_rule_scratch(n, len(lengths), 10 ** 6, heads, dim, vdim), device="cuda")
+    results = []
+    for more in ({}, {"scratch": scratch}):
+        state, out = start.clone(), torch.empty(n, heads * vdim, device="cuda")
+        ops.delta_rule(prepared, strength, decay, True, state, 0, slots, row_start, row_len, row_ctx, out, heads, heads, dim, vdim, **more)
+        results.append((out, state))
+    for walk, chunked in zip(*results):
+        assert torch.equal(torch.isfinite(walk), torch.isfinite(chunked))
+        keep = torch.isfinite(walk)
+        assert float((walk - chunked)[keep].norm()) <= 1e-5 * float(walk[keep].norm())
+    assert torch.isfinite(results[0][0][:place]).all() and not torch.isfinite(results[0][0][place:]).all()
