@@ -894,33 +894,36 @@ __global__ __launch_bounds__(256) void experts_combine_kernel(const float* __res
     *reinterpret_cast<Floats*>(out + (size_t)t * width + c) = result;
 }
 
-// Whether the wide kernel multiplies a step with so many pairs.  Both ways, all launches of a step, us: 32 pairs an expert (340 tokens, 6 of
-// 64 experts of 1,408, width 2,048) 250 narrow, 242 wide; 66: 302, 271; 96: 323, 286; 141: 444, 328; 192: 473, 409; at width 4,096,
-// 32 experts: 37 pairs 322, 335; 64 pairs 435, 356; 128 pairs 539, 415.
-static bool wide_tiles(int pairs, int experts, int inter, int width) {
-    // (the wide kernel's offsets have 32 bits)
-    return pairs >= 40 * experts && (size_t)pairs * (size_t)(inter > width ? inter : width) * 2 < 0xFFFFFFFFu &&
-           (size_t)2 * inter * width * 2 < 0xFFFFFFFFu;
+// Whether the wide kernel can multiply such a step: its loads straight into LDS are of 16 bytes at multiples of 16 (`aligned`: x, gate_up and down
+// begin at such), from offsets of 32 bits.
+static bool wide_fits(int pairs, int inter, int width, bool aligned) {
+    return aligned && (size_t)pairs * (size_t)(inter > width ? inter : width) * 2 < 0xFFFFFFFFu && (size_t)2 * inter * width * 2 < 0xFFFFFFFFu;
+}
+
+// Pairs a tile that lsa_experts_tiled should take for a step with so many pairs: 256 (the wide kernel) or 64.  Both ways, all launches of a step, us:
+// 32 pairs an expert (340 tokens, 6 of 64 experts of 1,408, width 2,048) 250 narrow, 242 wide; 66: 302, 271; 96: 323, 286; 141: 444, 328;
+// 192: 473, 409; at width 4,096, 32 experts: 37 pairs 322, 335; 64 pairs 435, 356; 128 pairs 539, 415.
+LSA_EXPORT int lsa_experts_tile_rows(int pairs, int experts, int inter, int width, int aligned) {
+    return pairs >= 40 * experts && wide_fits(pairs, inter, width, aligned != 0) ? WIDE_M : TILE_M;
 }
 
 // Ints of scratch memory that lsa_experts_tiled wants: the sorted pairs, then the tiles and their number.
-LSA_EXPORT int lsa_experts_tiled_ints(int pairs, int experts, int inter, int width) {
-    const int rows = wide_tiles(pairs, experts, inter, width) ? WIDE_M : TILE_M;
-    return ((pairs + rows - 1) / rows + experts) * (rows + 3) + 3;
-}
+LSA_EXPORT int lsa_experts_tiled_ints(int pairs, int experts, int tile_rows) { return ((pairs + tile_rows - 1) / tile_rows + experts) * (tile_rows + 3) + 3; }
 
 // Sorted, tiled products for bfloat16: hidden = silu(G x) * (U x) and y = D hidden for all pairs, then the weighted sums.
-// Scratch: lsa_experts_tiled_ints ints, y [pairs, width] floats.
+// Scratch: lsa_experts_tiled_ints ints, y [pairs, width] floats.  tile_rows: 64 or, where the wide kernel can, 256.
 LSA_EXPORT int lsa_experts_tiled(const void* x, const void* gate_up, const void* down, const int* chosen, const float* weights,
-                                 void* hidden, float* y, float* out, int* scratch, int n, int top,
+                                 void* hidden, float* y, float* out, int* scratch, int tile_rows, int n, int top,
                                  int inter, int width, int experts, float limit, int identity, const float* shared_gate, const void* shared_y,
                                  int plain, hipStream_t stream) {
     if (n <= 0) return 0;
     if (shared_gate != nullptr && shared_y == nullptr) return -1;
     const int pairs = n * top;
     if (width % 32 || inter % 32 || (size_t)experts * 8 > 60000) return -1;
-    const bool wide = wide_tiles(pairs, experts, inter, width);
-    const int tile_rows = wide ? WIDE_M : TILE_M, max_tiles = (pairs + tile_rows - 1) / tile_rows + experts;
+    const bool wide = tile_rows == WIDE_M;
+    if (!wide && tile_rows != TILE_M) return -1;
+    if (wide && !wide_fits(pairs, inter, width, ((size_t)x | (size_t)gate_up | (size_t)down | (size_t)hidden) % 16 == 0)) return -1;
+    const int max_tiles = (pairs + tile_rows - 1) / tile_rows + experts;
     int* sorted = scratch;
     Tile* tiles_of = reinterpret_cast<Tile*>(scratch + (size_t)max_tiles * tile_rows);
     experts_sort_kernel<<<1, 1024, (size_t)experts * 2 * sizeof(int), stream>>>(chosen, pairs, experts, tile_rows, sorted, tiles_of, max_tiles);

@@ -1190,11 +1190,11 @@ class HipOps(KernelNamespace):
         return 0 < n_tokens <= self.SHARED_INSIDE_ROWS
 
     def experts_sorted(self, x, gate_up, down, chosen, weights, out, activation="silu", limit=0.0, identity=0, shared_y=None,
-                       shared_gate=None) -> bool:
+                       shared_gate=None, tile_rows=0) -> bool:
         """Offered in bfloat16 for widths and expert sizes in steps of 32, and taken where the step has no fewer (token,
         expert) pairs than there are experts: below that every pair streaming its own expert reads little more, and combines in its second
         product (48 pairs of 64 experts of 1,408 at width 2,048: 139 us pair by pair, 150 sorted; 32 of 32 of 2,048 at 4,096: 246, 222; 72 of
-        64: 186, 158)."""
+        64: 186, 158).  ``tile_rows``: 64 or 256 pairs a tile whatever the sizes; 0 lets them decide."""
         n, width = x.shape
         experts, top, inter = gate_up.shape[0], chosen.shape[1], down.shape[2]
         if x.dtype != torch.bfloat16 or width % 32 or inter % 32 or n * top < experts or experts > 4096:
@@ -1210,9 +1210,11 @@ class HipOps(KernelNamespace):
         lib = self._part_library("experts")
         hidden = torch.empty((n * top, inter), device=x.device, dtype=x.dtype)
         y = torch.empty((n * top, width), device=x.device, dtype=torch.float32)
-        scratch = torch.empty((lib.lsa_experts_tiled_ints(n * top, experts, inter, width),), device=x.device, dtype=torch.int32)
+        aligned = (x.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0
+        tile_rows = tile_rows or lib.lsa_experts_tile_rows(n * top, experts, inter, width, 1 if aligned else 0)
+        scratch = torch.empty((lib.lsa_experts_tiled_ints(n * top, experts, tile_rows),), device=x.device, dtype=torch.int32)
         _launched(lib.lsa_experts_tiled(_ptr(x), _ptr(gate_up), _ptr(down), _ptr(chosen), _ptr(weights), _ptr(hidden), _ptr(y), _ptr(out),
-                                        _ptr(scratch), n, top, inter, width, experts,
+                                        _ptr(scratch), tile_rows, n, top, inter, width, experts,
                                         self._expert_limit(activation, limit), int(identity), _ptr(shared_gate), _ptr(shared_y),
                                         1 if plain else 0, _stream()),
                   "experts_tiled")
