@@ -900,11 +900,17 @@ static bool wide_fits(int pairs, int inter, int width, bool aligned) {
     return aligned && (size_t)pairs * (size_t)(inter > width ? inter : width) * 2 < 0xFFFFFFFFu && (size_t)2 * inter * width * 2 < 0xFFFFFFFFu;
 }
 
-// Pairs a tile that lsa_experts_tiled should take for a step with so many pairs: 256 (the wide kernel) or 64.  Both ways, all launches of a step, us:
-// 32 pairs an expert (340 tokens, 6 of 64 experts of 1,408, width 2,048) 250 narrow, 242 wide; 66: 302, 271; 96: 323, 286; 141: 444, 328;
-// 192: 473, 409; at width 4,096, 32 experts: 37 pairs 322, 335; 64 pairs 435, 356; 128 pairs 539, 415.
-LSA_EXPORT int lsa_experts_tile_rows(int pairs, int experts, int inter, int width, int aligned) {
-    return pairs >= 40 * experts && wide_fits(pairs, inter, width, aligned != 0) ? WIDE_M : TILE_M;
+// Pairs a tile that lsa_experts_tiled should take for a step with so many pairs: 256 (the wide kernel) or 64.  Wide tiles pay from some 40 pairs
+// an expert on, and where the two products make 224 workgroups or more together, not quite one a compute unit for each: with fewer,
+// tiles of 64 pairs spread the same work over units that would stand idle.  All launches of a step, us, narrow and wide: 64 experts of 1,408 at
+// width 2,048, 40 pairs an expert 270, 259; 64: 316, 278; 128: 404, 327; 192: 502, 383; 16 experts of 2,048 at 4,096 (512 workgroups), 128 pairs
+// 354, 246; 8 of them (256) 183, 159; 16 of 768 at 2,048 (224) 90, 76; 4 of 2,048 at 4,096 (128) 111, 129, with 192 pairs 115, 158; 8 of 1,408
+// at 2,048 (152) with 192 pairs 92, 99; 4 (76) 71, 97; 1 of 512 at 1,024 (8) with 256 pairs 40, 55.  Without gates, 16 of 1,024 at 4,096 (320),
+// 96 pairs 133, 128; 8 of 1,408 at 2,048 (112) with 192 pairs 75, 95.
+LSA_EXPORT int lsa_experts_tile_rows(int pairs, int experts, int inter, int width, int plain, int aligned) {
+    if (pairs < 40 * experts || !wide_fits(pairs, inter, width, aligned != 0)) return TILE_M;
+    const long tiles = (long)experts * ((pairs / experts + WIDE_M - 1) / WIDE_M), columns = plain ? WIDE_N : WIDE_N / 2;
+    return tiles * ((inter + columns - 1) / columns) + tiles * ((width + WIDE_N - 1) / WIDE_N) >= 224 ? WIDE_M : TILE_M;
 }
 
 // Ints of scratch memory that lsa_experts_tiled wants: the sorted pairs, then the tiles and their number.

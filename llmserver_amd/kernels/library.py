@@ -83,7 +83,7 @@ _SIGNATURES = {
     "lsa_delta_chunk_floats": [c_int, c_int],
     "lsa_delta_allow_lds": [],
     "lsa_experts_gate_up": [c_int, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P, _P, c_int, c_int, _P],
-    "lsa_experts_tile_rows": [c_int, c_int, c_int, c_int, c_int],
+    "lsa_experts_tile_rows": [c_int, c_int, c_int, c_int, c_int, c_int],
     "lsa_experts_tiled_ints": [c_int, c_int, c_int],
     "lsa_experts_tiled": [_P, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P, _P, c_int, _P],
     "lsa_experts_down": [c_int, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_int, _P],

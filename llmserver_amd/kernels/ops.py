@@ -1211,7 +1211,7 @@ class HipOps(KernelNamespace):
         hidden = torch.empty((n * top, inter), device=x.device, dtype=x.dtype)
         y = torch.empty((n * top, width), device=x.device, dtype=torch.float32)
         aligned = (x.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0
-        tile_rows = tile_rows or lib.lsa_experts_tile_rows(n * top, experts, inter, width, 1 if aligned else 0)
+        tile_rows = tile_rows or lib.lsa_experts_tile_rows(n * top, experts, inter, width, 1 if plain else 0, 1 if aligned else 0)
         scratch = torch.empty((lib.lsa_experts_tiled_ints(n * top, experts, tile_rows),), device=x.device, dtype=torch.int32)
         _launched(lib.lsa_experts_tiled(_ptr(x), _ptr(gate_up), _ptr(down), _ptr(chosen), _ptr(weights), _ptr(hidden), _ptr(y), _ptr(out),
                                         _ptr(scratch), tile_rows, n, top, inter, width, experts,

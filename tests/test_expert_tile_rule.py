@@ -6,7 +6,7 @@ import pytest
 def tile_rows():
     from llmserver_amd.kernels import library
     lib = library.load("experts")
-    return lambda pairs, experts, inter, width, aligned=True: lib.lsa_experts_tile_rows(pairs, experts, inter, width, 1 if aligned else 0)
+    return lambda pairs, experts, inter, width, plain=False, aligned=True: lib.lsa_experts_tile_rows(pairs, experts, inter, width, int(plain), int(aligned))
 
 
 def test_wide_tiles_want_whole_pieces_of_16_bytes(tile_rows):
@@ -20,4 +20,15 @@ def test_wide_tiles_end_where_their_offsets_do(tile_rows):
     most = (2 ** 32 - 1) // (2 * 4096) - 1                      # pairs of rows of 4,096 bfloat16 numbers
     assert tile_rows(most, 64, 1408, 4096) == 256 and tile_rows(most + 2, 64, 1408, 4096) == 64
     assert tile_rows(most, 64, 4096, 1408) == 256 and tile_rows(most + 2, 64, 4096, 1408) == 64
-    assert tile_rows(1000, 8, 32768 - 32, 32768) == 256 and tile_rows(1000, 8, 32768, 32768) == 64
+    assert tile_rows(1000, 3, 32768 - 32, 32768) == 256 and tile_rows(1000, 3, 32768, 32768) == 64
+
+
+def test_wide_tiles_where_they_were_measured_to_be_faster(tile_rows):
+    """Enough pairs an expert and enough tiles to go round the compute units; few experts or small ones keep the narrow tiles."""
+    for experts, each, width, inter in ((64, 40, 2048, 1408), (64, 192, 2048, 1408), (16, 128, 4096, 2048), (8, 128, 4096, 2048), (8, 400, 2048, 1408),
+                                        (64, 96, 1024, 512)):
+        assert tile_rows(experts * each, experts, inter, width) == 256, (experts, each, width, inter)
+    for experts, each, width, inter in ((64, 39, 2048, 1408), (4, 128, 4096, 2048), (4, 192, 4096, 2048), (8, 192, 2048, 1408), (4, 256, 2048, 1408),
+                                        (1, 256, 1024, 512), (16, 192, 1024, 512), (1, 400, 4096, 2048)):
+        assert tile_rows(experts * each, experts, inter, width) == 64, (experts, each, width, inter)
+    assert tile_rows(16 * 100, 16, 1024, 2048) == 256 and tile_rows(16 * 100, 16, 1024, 2048, plain=True) == 64

@@ -41,6 +41,11 @@ def test_sorted_products_at_the_edges_of_their_tiles(ops, experts, counts, width
         y = x[rows].float() @ up[e].float().T
         y = torch.nn.functional.silu(y[:, :inter]) * y[:, inter:] if gated else y.clamp(min=0) ** 2
         want[rows] = weights[rows] * (y.to(torch.bfloat16).float() @ down[e].float().T)
+    forms = []
+    for tile_rows in (64, 256):                                # (whichever the sizes ask for)
+        forms.append(torch.full((n, width), float("nan"), device="cuda"))
+        assert ops.experts_sorted(x, up, down, chosen, weights, forms[-1], tile_rows=tile_rows, **({} if gated else {"activation": "relu2"}))
+    assert torch.equal(forms[0], forms[1]) and (torch.equal(out, forms[0]))       # (both add a sum's products in the same order)
     assert torch.isfinite(out).all()
     assert float((out - want).norm() / want.norm()) < 2.0 ** -9
     assert float(((out - want).norm(dim=1) / want.norm(dim=1)).max()) < 2.0 ** -7
