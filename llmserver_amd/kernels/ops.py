@@ -1191,13 +1191,18 @@ class HipOps(KernelNamespace):
 
     def experts_sorted(self, x, gate_up, down, chosen, weights, out, activation="silu", limit=0.0, identity=0, shared_y=None,
                        shared_gate=None, tile_rows=0) -> bool:
-        """Offered in bfloat16 for widths and expert sizes in steps of 32, and taken where the step has no fewer (token,
-        expert) pairs than there are experts: below that every pair streaming its own expert reads little more, and combines in its second
-        product (48 pairs of 64 experts of 1,408 at width 2,048: 139 us pair by pair, 150 sorted; 32 of 32 of 2,048 at 4,096: 246, 222; 72 of
-        64: 186, 158).  ``tile_rows``: 64 or 256 pairs a tile whatever the sizes; 0 lets them decide."""
+        """Offered in bfloat16 for widths and expert sizes in steps of 32, and taken where the step has more (token, expert) pairs than there are
+        experts: below that every pair streaming its own expert reads little more, and combines in its second product (48 pairs of 64
+        experts of 1,408 at width 2,048: 139 us pair by pair, 150 sorted; 72 of 64: 186, 158).  With as many pairs as experts it depends on what
+        is read: sorting and combining cost 10 us, an expert read twice costs its time.  At 2 of 2 to 16 of 16 experts pairs win (8 of 8 of 512 at
+        512: 10, 21 us; 16 of 768 at 2,048: 31, 39), at 32 of 32 by the experts' size (768 at 2,048, 0.3 GB: 57, 67; 2,048 at 4,096, 1.6 GB: 250,
+        230), from 96 on sorting (96 of 512 at 1,024: 55, 50; 128 of 1,408 at 2,048: 317, 290).  ``tile_rows``: 64 or 256 pairs a tile whatever
+        the sizes; 0 lets them decide."""
         n, width = x.shape
         experts, top, inter = gate_up.shape[0], chosen.shape[1], down.shape[2]
         if x.dtype != torch.bfloat16 or width % 32 or inter % 32 or n * top < experts or experts > 4096:
+            return False
+        if n * top == experts and experts < 96 and x.element_size() * (gate_up.numel() + down.numel()) < 10 ** 9:
             return False
         plain = activation == "relu2"
         _check(x, "x")

@@ -1,5 +1,8 @@
 """Which tiles the sorted products of routed experts take (host code of the kernel library: no GPU needed)."""
 import pytest
+import torch
+
+from llmserver_amd.kernels.ops import HipOps
 
 
 @pytest.fixture(scope="module")
@@ -32,3 +35,22 @@ def test_wide_tiles_where_they_were_measured_to_be_faster(tile_rows):
                                         (1, 256, 1024, 512), (16, 192, 1024, 512), (1, 400, 4096, 2048)):
         assert tile_rows(experts * each, experts, inter, width) == 64, (experts, each, width, inter)
     assert tile_rows(16 * 100, 16, 1024, 2048) == 256 and tile_rows(16 * 100, 16, 1024, 2048, plain=True) == 64
+
+
+def test_sorted_products_where_they_were_measured_to_be_faster():
+    """(Tensors without storage: what is not refused by its sizes is refused for where it lives.)"""
+    def taken(pairs, experts, width, inter, plain=False):
+        make = lambda *shape, dtype=torch.bfloat16: torch.empty(*shape, dtype=dtype, device="meta")
+        try:
+            return HipOps.experts_sorted(HipOps.__new__(HipOps), make(pairs, width), make(experts, (1 if plain else 2) * inter, width),
+                                         make(experts, width, inter), make(pairs, 1, dtype=torch.int32), make(pairs, 1, dtype=torch.float32),
+                                         make(pairs, width, dtype=torch.float32), activation="relu2" if plain else "silu")
+        except ValueError as error:
+            assert "must live on the GPU" in str(error)
+            return True
+    assert taken(72, 64, 2048, 1408) and taken(9, 8, 512, 512) and not taken(48, 64, 2048, 1408) and not taken(127, 128, 4096, 2048)
+    for experts, width, inter in ((2, 512, 512), (8, 2048, 1408), (16, 1024, 512), (32, 2048, 768), (64, 2048, 768), (72, 2048, 768)):
+        assert not taken(experts, experts, width, inter)
+    for experts, width, inter in ((32, 4096, 2048), (64, 2048, 1408), (96, 1024, 512), (128, 2048, 1408)):
+        assert taken(experts, experts, width, inter)
+    assert taken(64, 64, 2048, 1408) and not taken(64, 64, 2048, 1408, plain=True)
