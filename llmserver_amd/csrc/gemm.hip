@@ -818,10 +818,6 @@ LSA_EXPORT int lsa_gemm_split_gated(const void* x, const void* w, void* hidden, 
 // step is 16 inner indices: a lane loads four neighbouring ones of its row (16 bytes), and the four 16x16x4 MFMAs of the step take the
 // lanes' first, second, third and fourth, each into sums of its own (four short chains round less than one long one: 1.2e-7 from
 // the 64-bit product at K = 1,024 where the library's is 2.9e-7).
-//   us against the library, N x K at 2 rows, each replayed from a graph with cold weights: 151,936 x 1,024 110 (5.7 TB/s) against 209;
-// 4,096 x 1,024 5.5, 8.4; 1,024 x 2,048 5.9, 8.4; 6,144 x 1,024 7.8, 8.9; 1,024 x 3,072 7.8, 8.5; 4,096 x 2,048 8.6, 10.8; 2,048 x 6,144 17.4,
-// 19.5; 12,288 x 2,048 22.7, 22.6.  At 16 rows, where X takes as much of the way into a compute unit as W: 6.3 and 8.5, 9.6 and 8.9; 163
-// and 210 for the head, so beyond 8 rows only matrices of a head's size go this way.
 constexpr int F32_STEPS = 8;
 __global__ __launch_bounds__(GEMM_WAVES * 64, 4) void gemm_few_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y,
                                                                           int M, int N, int K, int R, const float* __restrict__ bias) {
@@ -865,11 +861,25 @@ __global__ __launch_bounds__(GEMM_WAVES * 64, 4) void gemm_few_f32_kernel(const 
     y[(size_t)m * N + n] = bias ? total + bias[n] : total;
 }
 
-// Whether the sizes go this way: up to 8 rows, or up to 16 against a matrix of a vocabulary's size; K a multiple of 4, and 512 or more: eight
-// wavefronts need four steps of 16 each to have anything under way together (2 rows, replayed from a graph, us against the library: 4,096 x
-// 1,024 4.7, 5.6; 4,096 x 512 4.5, 4.4; 1,024 x 512 3.7, 4.2; 4,096 x 256 4.4, 3.7; 1,024 x 256 3.9, 3.7; 1,024 x 128 3.8, 3.3).
+// Whether the sizes go this way (K a multiple of 4): where this stream was measured to be no slower than the library's product, which is poor at short
+// rows and at rows of 1,024 and 2,048 numbers, and good between and behind those.  Here eight wavefronts want four steps of 16 each to have anything
+// under way together, a workgroup more than a compute unit's share waits for a second round, and from 5 rows on X takes a noticeable part of
+// the way into a compute unit.  us against the library's, N x K, replayed from a graph with cold weights, at 2 rows unless stated:
+//   up to 2,048 rows of W: 1,024 x 512 4.0, 4.5; 1,024 x 1,024 4.3, 8.0; 2,048 x 2,048 6.2, 8.7 (8 rows 7.4, 8.8); 1,024 x 3,072 8.5, 8.7 (8 rows 9.8,
+// 8.7); 1,024 x 6,144 1.07 times the library's time, 1,024 x 8,192 1.07.
+//   up to 8,192: 4,096 x 1,024 5.7, 8.6; 6,144 x 1,024 8.1, 9.1 (8 rows 8.9, 9.1); 4,096 x 768 0.73 times the library's time (8 rows 0.77, 6,144 x
+// 768 1.07); 6,144 x 512 1.16; 6,144 x 1,536 1.33; 4,096 x 2,048 8.8, 11.1; 2,560 x 2,048 (a round and a quarter) 1.14; 2,560 x 9,728 43, 32.
+//   a vocabulary: 151,936 x 1,024 111, 209 (8 rows 138, 212; 16 rows 163, 210), x 2,048 218, 256 (8 rows 270, 262); x 512 1.77 times the library's time, x 2,560
+// 1.11; 65,536 x 1,024 1.07 (16 rows 1.40), x 2,560 1.27 (16 rows 232, 120); 16,384 x 1,024 at 16 rows 22, 19.
 LSA_EXPORT int lsa_gemm_few_f32_fits(int M, int N, int K) {
-    return M >= 1 && (M <= 8 || (M <= 16 && N >= 16384)) && N >= 1 && K >= 512 && K % 4 == 0 ? 1 : 0;
+    if (M < 1 || M > 16 || N < 1 || K < 512 || K % 4 != 0) return 0;
+    if (N >= 100000) return K >= 768 && K <= (M <= 6 ? 2048 : M <= 8 ? 1536 : 1024) ? 1 : 0;
+    if (M > 8) return 0;
+    if (N <= 2048) return K <= (M <= 2 ? 3072 : 2048) ? 1 : 0;
+    if (N > 8192) return 0;
+    if (K <= 1024) return K >= 768 + 64 * (M > 4 ? M - 4 : 0) ? 1 : 0;
+    const int workgroups = (N + 15) / 16, rounds = (workgroups + 255) / 256;
+    return K == 2048 && M <= 4 && N >= 4096 && 10 * workgroups >= 9 * 256 * rounds ? 1 : 0;
 }
 
 // x [M, K], w [N, K], y [M, N], bias [N] or nullptr, all float32; M <= 16, K a multiple of 4, x and w at multiples of 16 bytes.

@@ -183,6 +183,14 @@ class HipOps(KernelNamespace):
         return x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 \
             and bool(self._gemm.lsa_gemm_few_f32_fits(x.shape[0], weight.shape[0], x.shape[1]))
 
+    def _linear_few_rows_float32(self, x, weight, out=None, bias=None):
+        """Up to 16 rows of float32 through the stream over the weights, whatever its rule says of the sizes."""
+        if out is None:
+            out = torch.empty((x.shape[0], weight.shape[0]), device=x.device, dtype=torch.float32)
+        _launched(self._gemm.lsa_gemm_few_f32(_ptr(x), _ptr(weight), _ptr(out), x.shape[0], weight.shape[0], x.shape[1], _ptr(bias), _stream()),
+                  "gemm_few_f32")
+        return out
+
     LIBRARY_MARGIN = 0.93       # the library replaces a few-row kernel only if it takes less than this share of its time
 
     def _median_time(self, run, repeats=5):
@@ -377,11 +385,7 @@ class HipOps(KernelNamespace):
             # Few rows: the product is a stream over the weights; the hand-written kernel reads them once at HBM rate.
             return self.linear_few_rows(x, weight, out=out, out_float32=out_float32, rows_per_workgroup=rows_per_workgroup, bias=bias)
         if self._few_rows_float32(x, weight, out):
-            if out is None:
-                out = torch.empty((x.shape[0], weight.shape[0]), device=x.device, dtype=torch.float32)
-            _launched(self._gemm.lsa_gemm_few_f32(_ptr(x), _ptr(weight), _ptr(out), x.shape[0], weight.shape[0], x.shape[1], _ptr(bias), _stream()),
-                      "gemm_few_f32")
-            return out
+            return self._linear_few_rows_float32(x, weight, out, bias)
         if out_float32 and x.dtype != torch.float32:
             y = torch.mm(x, weight.t(), out_dtype=torch.float32)
         elif bias is not None and bias_rounded is not None and bias_rounded.dtype == x.dtype and x.dtype != torch.float32:
