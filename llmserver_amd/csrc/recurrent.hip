@@ -1432,8 +1432,14 @@ static int run_decayed(const T* q, long q_stride, const T* k, long k_stride, con
                                                                        heads, dim, value_dim, group, ones);
         run_carry(sums, run, totals, state, state_stride, slots, row_start, row_len, row_ctx, rows, heads, dim, value_dim, ones, 0, stream);
         if constexpr (sizeof(T) == 2) {
-            // (its loads of queries and keys are of eight numbers, at multiples of 16 bytes)
-            if (dim % 32 == 0 && dim <= READ16_MOST && q_stride % 8 == 0 && k_stride % 8 == 0 && ((size_t)q | (size_t)k) % 16 == 0) {
+            // Its loads of queries and keys are of eight numbers, at multiples of 16 bytes.  A workgroup of it takes longer than one of the kernel
+            // below and has 128 columns where that has 64, so it pays once those go more than one round over the compute units (256 of them;
+            // two where half of its wavefronts would have no column).  All launches of a memory, us, the kernel below and this one: 16
+            // heads of 128 x 128 and a column of ones, rows of 64 tokens (96 workgroups below) 36.3, 38.0; 256 (240) 43.1, 44.2; 320 (288) 52.4, 48.4; 1,024
+            // 91, 84; three of 667 139, 110; 32 heads of 64 x 64, 512 tokens (288) 34.2, 36.2; eight rows of 64 (512) 32.1, 34.3; 16 of 16 (640) 42.3, 34.6.
+            const long below_workgroups = (long)items * heads * ((columns + 63) / 64);
+            const bool enough = below_workgroups > (columns > 64 ? 256 : 512);
+            if (enough && dim % 32 == 0 && dim <= READ16_MOST && q_stride % 8 == 0 && k_stride % 8 == 0 && ((size_t)q | (size_t)k) % 16 == 0) {
                 memory_chunk_read16_kernel<V><<<dim3(items, heads, (columns + 127) / 128), 256, 0, stream>>>(
                     q, q_stride, k, k_stride, v, v_stride, weights, run, q_scale, row_start, row_len, row_ctx, rows, sums, out, below, heads, dim, value_dim,
                     group, ones);

@@ -172,9 +172,11 @@ def test_which_steps_run_their_delta_rules_in_chunks(ops):
     assert not shape([160]) and not shape([1] * 32) and not shape([64] * 16) and not shape([2048], dim=129)
 
 
+@pytest.mark.parametrize("spare", [0, 600])
 @pytest.mark.parametrize("heads,key_heads,dim,vdim", [(2, 2, 32, 31), (2, 2, 96, 1), (1, 1, 128, 257), (3, 3, 64, 128), (4, 2, 128, 96), (2, 1, 32, 33)])
-def test_read_outs_of_16_bit_queries_in_chunks(ops, heads, key_heads, dim, vdim):
-    """Heads of whole steps of 32 channels, rows at multiples of 16 bytes: what a chunk's tokens read is made by wavefronts of 32 columns.  As many
+def test_read_outs_of_16_bit_queries_in_chunks(ops, heads, key_heads, dim, vdim, spare):
+    """Heads of whole steps of 32 channels, rows at multiples of 16 bytes: what a chunk's tokens read is made by wavefronts of 32 columns where the
+    scratch memory makes for enough workgroups (``spare`` chunks that the rows do not have).  As many
     heads of keys as heads: the memory with its normaliser; fewer: a decay and a strength a head.  The kept numbers are the kernel's own
     (32-bit), so the float64 walk starts from the same ones."""
     print(f"read-outs in chunks {heads} {key_heads} {dim} {vdim}", flush=True)
@@ -190,7 +192,7 @@ def test_read_outs_of_16_bit_queries_in_chunks(ops, heads, key_heads, dim, vdim)
     assert q.stride(0) % 8 == 0 and (q.data_ptr() | k.data_ptr()) % 16 == 0
     start = draw(5, size + heads * dim + heads)
     start[:, -heads:] = 0.5
-    chunks, ones = n // 64 + len(lengths), 1 if memory else 0
+    chunks, ones = n // 64 + len(lengths) + spare, 1 if memory else 0
     sums = torch.full((chunks, heads, dim, vdim + ones), float("nan"), device="cuda")
     gates = 3 * draw(n, 2 * heads) + 2.0
     log_keep, take = -torch.nn.functional.softplus(2 * draw(n, heads) - 2.0), torch.sigmoid(draw(n, heads))
