@@ -1072,17 +1072,23 @@ class HipOps(KernelNamespace):
 
     SCORINGS = ("softmax", "sigmoid", "softmax_all")       # (the kernel's codes)
 
-    ROUTE_PARTS_WORKGROUPS = 512    # most workgroups of the router's own product of 16 tokens x 16 experts
+    ROUTE_PARTS_WORKGROUPS = 512    # most workgroups of the router's own product of 16 tokens x 16 experts ...
+    ROUTE_PARTS_WORKGROUPS_A_PART = 64      # ... and for rows that are 32-bit already, for each part of the width
 
     def _route_parts(self, x, router) -> int:
         """In how many partial sums over the width the router's own product of these sizes goes, or 0: the library's takes it (after a
         widening of the rows), because the kernel reads a piece of a row again for every 16 experts.  With the choice behind it, 512 workgroups:
         256 rows of 2048, 128 experts 16.6 us against 19.4; 64 rows of 4096, 256 experts 19 against 22.9; 512 rows of 2048, 64 experts
-        14.5 against 18.4; with 1,024: 23.1 against 20.1, 25.5 against 23.8, 20.9 against 21.1."""
+        14.5 against 18.4; with 1,024: 23.1 against 20.1, 25.5 against 23.8, 20.9 against 21.1.  Rows of 32 bits need no widening: 256 rows of 2048,
+        128 experts 13.4 against 12.7, 512 rows and 64 experts 12.4 against 11.9, 4,096 rows of 512 and 8 experts 11.5 against 10.9; 128 rows of 4096
+        and 128 experts (512 workgroups, eight parts) 13.4 against 15.6, 1,024 rows of 2048 and 16 experts (256, four) 10.7 against 11.9."""
         if (x.data_ptr() | router.data_ptr()) % 16:
             return 0
         parts = self._part_library("experts").lsa_route_logits_parts_count(x.shape[1])
-        return parts if -(-x.shape[0] // 16) * -(-router.shape[0] // 16) * parts <= self.ROUTE_PARTS_WORKGROUPS else 0
+        most = self.ROUTE_PARTS_WORKGROUPS
+        if x.dtype == torch.float32:
+            most = min(most, self.ROUTE_PARTS_WORKGROUPS_A_PART * parts)
+        return parts if -(-x.shape[0] // 16) * -(-router.shape[0] // 16) * parts <= most else 0
 
     def route_experts(self, x, router, top, chosen, weights, scoring="softmax", groups=None, bias=None, correction=None, weight_scale=1.0,
                       gate_out=None):
@@ -1103,13 +1109,13 @@ class HipOps(KernelNamespace):
             _check(gate_out, "gate_out", torch.float32, (n,))
         if not 1 <= top <= experts or experts > 3072:
             raise ValueError(f"the router kernel chooses 1 to {min(experts, 3072)} of up to 3072 experts, asked for {top} of {experts}")
-        lib, parts = self._part_library("experts"), 1
-        if n <= self.LATENT_FEW_ROWS:          # few tokens: a kernel of a few microseconds instead of a library call
+        lib, few = self._part_library("experts"), n <= self.LATENT_FEW_ROWS
+        parts = 0 if few else self._route_parts(x, router)
+        if few:          # few tokens: a kernel of a few microseconds instead of a library call
             logits = torch.empty((n, outputs), device=x.device, dtype=torch.float32)
             _launched(lib.lsa_route_logits(_code(x), _ptr(x), _ptr(router), _ptr(logits), n, outputs, width, _stream()),
                       "route_logits")
-        elif self._route_parts(x, router):
-            parts = self._route_parts(x, router)
+        elif parts:
             logits = torch.empty((parts, n, outputs), device=x.device, dtype=torch.float32)
             _launched(lib.lsa_route_logits_parts(_code(x), _ptr(x), _ptr(router), _ptr(logits), n, outputs, width, _stream()), "route_logits_parts")
         else:
@@ -1123,7 +1129,7 @@ class HipOps(KernelNamespace):
             raise ValueError(f"the router kernel takes up to 64 equal groups: {experts} experts in {count} groups, {keep} kept, {top} chosen")
         _launched(lib.lsa_route_top(_ptr(logits), experts, top, _ptr(chosen), _ptr(weights), n,
                                                               self.SCORINGS.index(scoring), int(count), int(keep), _ptr(bias), _ptr(correction),
-                                                              float(weight_scale), outputs, _ptr(gate_out), parts, _stream()), "route_top")
+                                                              float(weight_scale), outputs, _ptr(gate_out), max(parts, 1), _stream()), "route_top")
 
     @staticmethod
     def _expert_limit(activation, limit) -> float:

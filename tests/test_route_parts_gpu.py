@@ -26,7 +26,7 @@ def test_choices_from_partial_sums(ops, dtype, rows, experts, top, width, scorin
     chosen = torch.empty(rows, top, dtype=torch.int32, device="cuda")
     weights, gate = torch.empty(rows, top, device="cuda"), torch.empty(rows, device="cuda")
     taken = ops._route_parts(x, router)
-    assert bool(taken) == (rows < 600)
+    assert bool(taken) == (rows < (600 if dtype == torch.bfloat16 else 300))
     ops.route_experts(x, router, top, chosen, weights, scoring=scoring, gate_out=gate)
     exact = x.double() @ router.double().T
     bound = float((x.double().abs() @ router.double().abs().T).max()) * width * 2.0 ** -24
