@@ -1410,6 +1410,10 @@ class HipOps(KernelNamespace):
                                                                   _ptr(row_start), _ptr(row_len), _ptr(row_ctx), taps - 1, channels, rows, _stream()),
                   "delta_conv_keep")
 
+    # Most scratch memory that a step's recurrences in chunks ask for; the walk needs none.  A step of 8,192 tokens of 16 heads of 128 x 128 wants
+    # 0.2 GB (the linear recurrence) or 0.34 GB (the delta rule), three times that a step of 24,000; a step's activations grow as fast.
+    CHUNK_SCRATCH_BYTES = 1 << 30
+
     def delta_rule_scratch(self, n_tokens, rows, longest, heads, dim, value_dim):
         """The shape of the scratch memory that the delta rule wants for a step of this shape if it is to run in chunks, or None if it
         runs token by token: short rows, and heads that the chunked kernel's LDS does not hold.  Walking the longest row takes 0.36 us a
@@ -1421,7 +1425,8 @@ class HipOps(KernelNamespace):
         workgroups = items * heads * -(-(128 + value_dim) // 256)
         if dim > lib.lsa_delta_chunked_most_dim() or 0.36 * longest <= 60.0 + 0.2 * workgroups:
             return None
-        return items, heads, lib.lsa_delta_chunk_floats(dim, value_dim)
+        floats = lib.lsa_delta_chunk_floats(dim, value_dim)
+        return (items, heads, floats) if 4 * items * heads * floats <= self.CHUNK_SCRATCH_BYTES else None
 
     def delta_rule(self, prepared, strength, decay, per_channel, state, offset, state_slots, row_start, row_len, row_ctx, out,
                    heads, kv_heads, dim, value_dim, scratch=None):
@@ -1514,7 +1519,8 @@ class HipOps(KernelNamespace):
         workgroups = items * heads * -(-value_dim // 128)
         if dim > self._part_library("recurrent").lsa_linear_recurrence_chunked_most_dim() or 0.43 * longest <= 30.0 + 0.19 * workgroups:
             return 0
-        return items
+        bytes_wanted = 4 * heads * dim * (items * (value_dim + 1) + n_tokens)
+        return items if bytes_wanted <= self.CHUNK_SCRATCH_BYTES else 0
 
     def linear_recurrence(self, q, k, v, decay, decay_bias, decay_mode, tau, bonus, q_scale, state, offset, state_slots,
                           row_start, row_len, row_ctx, out, heads, dim, value_dim, sums=None, totals=None, queries=None):

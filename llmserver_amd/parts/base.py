@@ -250,6 +250,15 @@ class Mixer(Part):
         raise NotImplementedError
 
 
+def scratch_memory(ctx, shapes) -> dict:
+    """Float32 scratch tensors by name, or none at all if the device has no room for them: they make a step faster, and a step runs without
+    them as well."""
+    try:
+        return {name: ctx.empty(shape, dtype=torch.float32) for name, shape in shapes.items()}
+    except torch.OutOfMemoryError:
+        return {}
+
+
 class FeedForward(Part):
     accepts_pending_norm = False
     takes_sink = False

@@ -26,7 +26,7 @@ from typing import Optional
 
 import torch
 
-from .base import VECTOR, Mixer, ParamSpec, StateSpec
+from .base import VECTOR, Mixer, ParamSpec, StateSpec, scratch_memory
 from .linear import Linear
 
 UNIT_EPS = 1e-6         # q / sqrt(sum(q^2) + UNIT_EPS)
@@ -186,7 +186,7 @@ class GatedDeltaRule(Mixer):
                                 ctx.row_len, ctx.row_ctx)
         mixed = ctx.empty((n, self.values), dtype=torch.float32)
         shape = ops.delta_rule_scratch(n, ctx.row_len.shape[0], ctx.longest_row(), self.heads, self.dim, self.value_dim)
-        more = {"scratch": ctx.empty(shape, dtype=torch.float32)} if shape else {}
+        more = scratch_memory(ctx, {"scratch": shape}) if shape else {}
         ops.delta_rule(prepared, strengths, decays, self.decay_per_channel, cache.state, 0, ctx.state_slots, ctx.row_start, ctx.row_len,
                        ctx.row_ctx, mixed, self.heads, self.kv_heads, self.dim, self.value_dim, **more)
         gated = ctx.empty((n, self.values))

@@ -26,7 +26,7 @@ from typing import Optional, Sequence
 
 import torch
 
-from .base import VECTOR, Mixer, ParamSpec, Part, StateSpec
+from .base import VECTOR, Mixer, ParamSpec, Part, StateSpec, scratch_memory
 from .linear import Linear
 
 DECAYS = ("sigmoid_root", "double_exp")
@@ -37,8 +37,7 @@ def _chunk_scratch(ctx, n, heads, dim, value_dim):
     chunks = ctx.ops.linear_recurrence_chunks(n, ctx.row_len.shape[0], ctx.longest_row(), heads, dim, value_dim)
     if not chunks:
         return {}
-    return {"sums": ctx.empty((chunks, heads, dim, value_dim), dtype=torch.float32),
-            "totals": ctx.empty((chunks, heads, dim), dtype=torch.float32), "queries": ctx.empty((n, heads, dim), dtype=torch.float32)}
+    return scratch_memory(ctx, {"sums": (chunks, heads, dim, value_dim), "totals": (chunks, heads, dim), "queries": (n, heads, dim)})
 
 
 class TokenShift(Part):
