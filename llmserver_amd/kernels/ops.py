@@ -81,7 +81,6 @@ class HipOps(KernelNamespace):
         self._gemm = library.load("gemm")
         self._attention = {}
         self._parts_libraries = {}
-        self._chunks_refused = {}       # part library -> whether its chunked forms may not have the LDS they want
         self.skinny_rows = SKINNY_GEMM_ROWS
         # Whether projections may fold the residual sum and the norm between two few-row products into their
         # epilogues (see linear_into_stream); off, every such sum and norm is a kernel of its own.
@@ -830,11 +829,10 @@ class HipOps(KernelNamespace):
             loaded = self._parts_libraries[name] = library.load(name)
             if name == "recurrent":
                 # Once, outside any launch (a launch may be recorded into a graph): the recurrence kernel may ask for
-                # more LDS than the default limit.  If that is refused, launches that need more say so themselves, and
-                # what has a form that needs less keeps to that one.
-                self._chunks_refused["recurrent"] = loaded.lsa_recurrent_prepare() != 0
+                # more LDS than the default limit.  If that is refused, launches that need more say so themselves.
+                loaded.lsa_recurrent_prepare()
             elif name == "delta":
-                self._chunks_refused["delta"] = loaded.lsa_delta_allow_lds() != 0
+                loaded.lsa_delta_allow_lds()
         return loaded
 
     def embedding_norm(self, table, token_ids, weight, eps, out):
@@ -1425,7 +1423,7 @@ class HipOps(KernelNamespace):
         lib = self._part_library("delta")
         items = n_tokens // self.MEMORY_CHUNK + rows
         workgroups = items * heads * -(-(128 + value_dim) // 256)
-        if self._chunks_refused.get("delta") or dim > lib.lsa_delta_chunked_most_dim() or 0.36 * longest <= 60.0 + 0.2 * workgroups:
+        if dim > lib.lsa_delta_chunked_most_dim() or 0.36 * longest <= 60.0 + 0.2 * workgroups:
             return None
         floats = lib.lsa_delta_chunk_floats(dim, value_dim)
         return (items, heads, floats) if 4 * items * heads * floats <= self.CHUNK_SCRATCH_BYTES else None
@@ -1519,8 +1517,7 @@ class HipOps(KernelNamespace):
         us walked, 45 / 46 / 48 / 118 in chunks; 512 tokens beside 16 single ones 209 / 94; 16 rows of 64 63 / 83)."""
         items = n_tokens // self.MEMORY_CHUNK + rows
         workgroups = items * heads * -(-value_dim // 128)
-        lib = self._part_library("recurrent")
-        if self._chunks_refused.get("recurrent") or dim > lib.lsa_linear_recurrence_chunked_most_dim() or 0.43 * longest <= 30.0 + 0.19 * workgroups:
+        if dim > self._part_library("recurrent").lsa_linear_recurrence_chunked_most_dim() or 0.43 * longest <= 30.0 + 0.19 * workgroups:
             return 0
         bytes_wanted = 4 * heads * dim * (items * (value_dim + 1) + n_tokens)
         return items if bytes_wanted <= self.CHUNK_SCRATCH_BYTES else 0

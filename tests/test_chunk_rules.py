@@ -13,7 +13,7 @@ from llmserver_amd.parts.recurrent import _chunk_scratch
 @pytest.fixture()
 def ops():
     made = HipOps.__new__(HipOps)
-    made._parts_libraries, made._chunks_refused = {name: library.load(name) for name in ("recurrent", "delta")}, {}
+    made._parts_libraries = {name: library.load(name) for name in ("recurrent", "delta")}
     return made
 
 
@@ -47,18 +47,3 @@ def test_a_step_without_room_for_scratch_memory_walks():
     given = _chunk_scratch(step(lambda shape, dtype: torch.empty(shape, dtype=dtype)), 301, 2, 8, 16)
     assert {name: tuple(tensor.shape) for name, tensor in given.items()} == {"sums": (7, 2, 8, 16), "totals": (7, 2, 8), "queries": (301, 2, 8)}
     assert asked == [(301, 2, 300, 2, 8, 16)] * 2
-
-
-def test_steps_walk_where_the_chunks_may_not_have_their_lds(ops, monkeypatch):
-    class Loaded:
-        def __init__(self, lib, code):
-            self.lib, self.code = lib, code
-
-        def __getattr__(self, name):
-            return (lambda: self.code) if name in ("lsa_recurrent_prepare", "lsa_delta_allow_lds") else getattr(self.lib, name)
-    load = library.load
-    for code in (0, 1):
-        ops._parts_libraries = {}
-        monkeypatch.setattr(library, "load", lambda name: Loaded(load(name), code))
-        chunked = bool(linear_bytes(ops, [2048], 16, 128, 128)), bool(delta_bytes(ops, [2048], 16, 128, 128))
-        assert chunked == ((code == 0),) * 2
