@@ -1414,18 +1414,39 @@ class HipOps(KernelNamespace):
     # 0.2 GB (the linear recurrence) or 0.34 GB (the delta rule), three times that a step of 24,000; a step's activations grow as fast.
     CHUNK_SCRATCH_BYTES = 1 << 30
 
+    @staticmethod
+    def _delta_rule_us(n_tokens, rows, longest, heads, dim, value_dim):
+        """About what a step's delta rules take token by token and in chunks, in us.  Measured, both ways, at 16 heads of 128 x 128: 1 row of 128 /
+        192 / 256 / 512 / 2,048 tokens 40, 66; 56, 70; 74, 74; 142, 87; 767, 203; 4 rows of 256 / 512 112, 137; 214, 164; 16 rows of 64 / 512 76, 145;
+        586, 725; 512 tokens beside 16 single ones 198, 160; 4 heads, 1 row of 192 56, 67; 8 rows of 256 75, 80; 16 heads of 64 x 64, 1 row of 192 /
+        256 / 2,048 38, 42; 49, 43; 481, 100; 16 rows of 512 147, 288.
+
+        The walk: a row's tokens one after another, slower where its workgroups (a head's 16 value columns each) share compute units and where
+        its rows of input leave L2; never less than what all rows' tokens take on 256 compute units.  The chunks: three launches, a share for each
+        (chunk, head, 256 columns of keys and values), and the walk over the longest row's chunks."""
+        wide, columns = dim > 64, -(-value_dim // 16)
+        load = n_tokens / longest * heads * columns
+        token, crowded, far = (0.27, 0.45, 0.4) if wide else (0.17, 0.3, 0.25)
+        middle = crowded if load >= 256 or rows * heads * columns >= 1024 else token
+        walk = 5.0 + token * min(longest, 256) + middle * min(max(longest - 256, 0), 256) + far * max(longest - 512, 0)
+        walk = max(walk, (0.14 if wide else 0.072) * longest * load / 256)
+        blocks = ((128 if wide else 64) + 16 * columns) / 256
+        workgroups = (n_tokens // HipOps.MEMORY_CHUNK + rows) * heads
+        if wide:
+            chunks = max(64.0 + 0.2 * workgroups * max(1.0, blocks), 0.31 * workgroups * -(-blocks // 1)) + longest / 64
+        else:
+            chunks = 36.0 + 0.12 * workgroups * max(1.0, blocks) + longest / 128
+        return walk, chunks
+
     def delta_rule_scratch(self, n_tokens, rows, longest, heads, dim, value_dim):
         """The shape of the scratch memory that the delta rule wants for a step of this shape if it is to run in chunks, or None if it
-        runs token by token: short rows, and heads that the chunked kernel's LDS does not hold.  Walking the longest row takes 0.36 us a
-        token; the chunks' three launches 60 us and 0.2 us a (chunk, head, 256 columns of keys and values), rows of one token
-        having a chunk of their own (measured at 16 heads of 128 x 128: 1 row of 130 / 256 / 512 / 1,900 / 8,192 tokens 39 / 71 / 137 / 713 /
-        3,714 us walked, 65 / 69 / 82 / 189 / 803 in chunks; 512 tokens beside 16 single ones 191 / 131; 16 rows of 64 71 / 91)."""
+        runs token by token: where that is estimated to be faster (:meth:`_delta_rule_us`), heads that the chunked kernel's LDS does not
+        hold, and steps that would want too much."""
         lib = self._part_library("delta")
-        items = n_tokens // self.MEMORY_CHUNK + rows
-        workgroups = items * heads * -(-(128 + value_dim) // 256)
-        if dim > lib.lsa_delta_chunked_most_dim() or 0.36 * longest <= 60.0 + 0.2 * workgroups:
+        walk, chunks = self._delta_rule_us(n_tokens, rows, max(longest, 1), heads, dim, value_dim)
+        if dim > lib.lsa_delta_chunked_most_dim() or walk <= chunks:
             return None
-        floats = lib.lsa_delta_chunk_floats(dim, value_dim)
+        items, floats = n_tokens // self.MEMORY_CHUNK + rows, lib.lsa_delta_chunk_floats(dim, value_dim)
         return (items, heads, floats) if 4 * items * heads * floats <= self.CHUNK_SCRATCH_BYTES else None
 
     def delta_rule(self, prepared, strength, decay, per_channel, state, offset, state_slots, row_start, row_len, row_ctx, out,
@@ -1509,18 +1530,34 @@ class HipOps(KernelNamespace):
 
     DECAY_MODES = ("sigmoid_root", "double_exp")
 
+    @staticmethod
+    def _linear_recurrence_us(n_tokens, rows, longest, heads, dim, value_dim):
+        """About what a step's recurrences take token by token and in chunks, in us.  Measured, both ways, at 16 heads of 128 x 128: 1 row of 64 / 100 /
+        128 / 256 / 2,048 tokens 30, 47; 45, 48; 54, 48; 103, 51; 919, 122; 4 rows of 128 / 512 58, 60; 237, 116; 16 rows of 64 / 256 / 512 71, 110;
+        241, 220; 471, 473; 512 tokens beside 16 single ones 214, 107; 16 heads of 64 x 64, 1 row of 64 / 128 / 2,048 21, 30; 37, 30; 508, 58; 8 rows of
+        512 157, 90; 16 rows of 512 157, 158.
+
+        The walk: a row's tokens one after another, as many rounds of them as its workgroups (a head's 64 value columns each) go round 256
+        compute units.  The chunks: three launches and a share for each (chunk, head, 128 value columns)."""
+        wide = dim > 64
+        load = n_tokens / longest * heads * -(-value_dim // 64)
+        if wide:
+            walk = 6.0 + (0.39 if load < 128 else 0.46) * longest
+        else:
+            walk = 5.0 + (0.25 if load < 128 else 0.3) * longest
+        walk = max(walk, (0.455 if wide else 0.31) * longest * -(-load // 256))
+        workgroups = (n_tokens // HipOps.MEMORY_CHUNK + rows) * heads * max(1.0, value_dim / 128)
+        return walk, max(48.0, 30.0 + 0.19 * workgroups) if wide else max(31.0, 24.0 + 0.065 * workgroups)
+
     def linear_recurrence_chunks(self, n_tokens, rows, longest, heads, dim, value_dim):
         """How many chunks of scratch memory the recurrence wants for a step of this shape if it is to run in chunks, or 0 if it
-        runs token by token: short rows, and heads that the chunked kernel's LDS does not hold.  Walking the longest row takes 0.43 us a
-        token; the chunks' three launches 30 us and 0.19 us a (chunk, head, 128 value columns), rows of one token
-        having a chunk of their own (measured at heads of 128 x 128 and 128 x 256: 1 row of 66 / 100 / 130 / 2,048 tokens 31 / 44 / 55 / 916
-        us walked, 45 / 46 / 48 / 118 in chunks; 512 tokens beside 16 single ones 209 / 94; 16 rows of 64 63 / 83)."""
-        items = n_tokens // self.MEMORY_CHUNK + rows
-        workgroups = items * heads * -(-value_dim // 128)
-        if dim > self._part_library("recurrent").lsa_linear_recurrence_chunked_most_dim() or 0.43 * longest <= 30.0 + 0.19 * workgroups:
+        runs token by token: where that is estimated to be faster (:meth:`_linear_recurrence_us`), heads that the chunked kernel's LDS does not
+        hold, and steps that would want too much."""
+        walk, chunks = self._linear_recurrence_us(n_tokens, rows, max(longest, 1), heads, dim, value_dim)
+        if dim > self._part_library("recurrent").lsa_linear_recurrence_chunked_most_dim() or walk <= chunks:
             return 0
-        bytes_wanted = 4 * heads * dim * (items * (value_dim + 1) + n_tokens)
-        return items if bytes_wanted <= self.CHUNK_SCRATCH_BYTES else 0
+        items = n_tokens // self.MEMORY_CHUNK + rows
+        return items if 4 * heads * dim * (items * (value_dim + 1) + n_tokens) <= self.CHUNK_SCRATCH_BYTES else 0
 
     def linear_recurrence(self, q, k, v, decay, decay_bias, decay_mode, tau, bonus, q_scale, state, offset, state_slots,
                           row_start, row_len, row_ctx, out, heads, dim, value_dim, sums=None, totals=None, queries=None):

@@ -47,3 +47,25 @@ def test_a_step_without_room_for_scratch_memory_walks():
     given = _chunk_scratch(step(lambda shape, dtype: torch.empty(shape, dtype=dtype)), 301, 2, 8, 16)
     assert {name: tuple(tensor.shape) for name, tensor in given.items()} == {"sums": (7, 2, 8, 16), "totals": (7, 2, 8), "queries": (301, 2, 8)}
     assert asked == [(301, 2, 300, 2, 8, 16)] * 2
+
+
+# (rows' lengths, heads, key channels, value channels): where the chunks were measured to be faster than the walk, and where they were not
+CHUNKS_OF_LINEAR = [([128], 16, 128, 128), ([2048], 8, 128, 256), ([256] * 2, 16, 128, 128), ([512] * 4, 16, 128, 128), ([512] + [1] * 16, 16, 128, 128),
+                    ([128] * 4, 16, 64, 64), ([512] * 8, 16, 64, 64), ([512] * 4, 32, 64, 64), ([512] * 8, 8, 96, 192), ([256] * 16, 8, 96, 192)]
+WALKS_OF_LINEAR = [([100], 16, 128, 128), ([100], 32, 128, 128), ([64], 16, 64, 64), ([64] * 16, 16, 128, 128), ([32] * 32, 16, 64, 64), ([128] * 8, 16, 128, 128),
+                   ([256] * 16, 16, 64, 64), ([1] * 40, 16, 128, 128), ([112] + [1] * 64, 16, 128, 128), ([128] + [1] * 8, 16, 128, 128), ([512] * 16, 16, 128, 128)]
+CHUNKS_OF_DELTA = [([512], 16, 128, 128), ([1900], 16, 128, 128), ([512] * 4, 16, 128, 128), ([512] + [1] * 16, 16, 128, 128), ([256], 16, 64, 64),
+                   ([2048], 32, 64, 64), ([1024] + [64] * 8, 32, 128, 128), ([512] * 4, 8, 96, 192)]
+WALKS_OF_DELTA = [([192], 4, 128, 128), ([160], 16, 128, 128), ([256], 32, 128, 128), ([256] * 8, 4, 128, 128), ([256] * 4, 16, 128, 128), ([64] * 16, 16, 128, 128),
+                  ([512] * 16, 16, 128, 128), ([512] * 16, 8, 128, 256), ([512] * 16, 16, 64, 64), ([256] + [1] * 16, 16, 128, 128), ([1] * 40, 16, 128, 128)]
+
+
+def test_steps_run_the_way_that_was_measured_to_be_faster(ops):
+    for case in CHUNKS_OF_LINEAR:
+        assert linear_bytes(ops, *case), case
+    for case in WALKS_OF_LINEAR:
+        assert not linear_bytes(ops, *case), case
+    for case in CHUNKS_OF_DELTA:
+        assert delta_bytes(ops, *case), case
+    for case in WALKS_OF_DELTA:
+        assert not delta_bytes(ops, *case), case
