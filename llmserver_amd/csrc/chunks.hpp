@@ -24,6 +24,7 @@ __device__ __forceinline__ bool chunk_item(int item, int rows, const int* __rest
 constexpr int BC = 16;                   // tokens a block, where chunks are cut further
 
 typedef float mc_f4 __attribute__((ext_vector_type(4)));
+typedef double mc_d4 __attribute__((ext_vector_type(4)));
 
 // What the four partial sums of a product make together, rounded once.
 __device__ __forceinline__ mc_f4 together(const mc_f4 (&part)[4]) {

@@ -366,8 +366,6 @@ __global__ __launch_bounds__(256) void delta_rule_kernel(const float* __restrict
 constexpr int CHUNKED_MOST_DIM = 128;
 constexpr int CHUNK_TILES = 16;          // blocks of 16 columns (of K or U) a workgroup: two a wavefront
 
-typedef double mc_d4 __attribute__((ext_vector_type(4)));
-
 template <int P>                         // P: key channels filled up to 64 or 128
 struct DeltaChunkLds {
     static constexpr int A = P + 4;

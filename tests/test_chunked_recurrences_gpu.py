@@ -1,8 +1,9 @@
 """The recurrences that run long portions in chunks, against the same recurrence token by token in float64.
 
-What a result may be off by is what the kernel that walks the tokens one by one is off by on the same numbers: both form
-sums of as many float32 products, in another order, so twice its error (2-norm over a step) and a few units in the last
-place (1e-6) bound the chunked form's."""
+What a result may be off by is what the kernel that walks the tokens one by one is off by on the same numbers (2-norm over a step): both
+form sums of as many float32 products, the chunks in short partial sums that meet in 64 bits.  A quarter more, and half a unit in the
+last place (HALF_UNIT) for results of a few numbers, of which the norm is a chance matter, bound the chunked form's; read-outs of the
+kernel of 64 columns, which adds scores' and state's products in one long 32-bit sum, are allowed twice the walk's."""
 import pytest
 import torch
 
@@ -10,6 +11,7 @@ from test_latent_experts_kernels_gpu import batch
 
 pytestmark = pytest.mark.gpu
 DTYPES = [torch.float32, torch.bfloat16]
+HALF_UNIT = 2.0 ** -25
 
 
 @pytest.fixture(scope="module")
@@ -85,7 +87,7 @@ def test_linear_recurrence_in_chunks(ops, dtype, heads, dim, vdim, mode, spread)
         errors = {form: (off(outs[form], exact.reshape(n, -1)), off(states[form], exact_states)) for form in outs}
         print(errors, flush=True)
         for scan, chunked in zip(errors["scan"], errors["chunks"]):
-            assert chunked <= 2 * scan + 1e-6
+            assert chunked <= 1.25 * scan + HALF_UNIT
         assert torch.equal(states["chunks"][3], start[3]) and torch.equal(states["chunks"][:, :offset], start[:, :offset])
         firsts = [first + length for first, length in zip(firsts, lengths)]
 
@@ -158,7 +160,7 @@ def test_delta_rule_in_chunks(ops, per_channel, heads, kv_heads, dim, vdim, spre
         errors = {form: (off(outs[form], exact.reshape(n, -1)), off(turned(states[form]), exact_states)) for form in outs}
         print(errors, flush=True)
         for scan, chunked in zip(errors["scan"], errors["chunks"]):
-            assert chunked <= 2 * scan + 1e-6
+            assert chunked <= 1.25 * scan + HALF_UNIT
         assert torch.equal(states["chunks"][3], start[3]) and torch.equal(states["chunks"][:, size:], start[:, size:])
         padding = states["chunks"][:, :size].view(6, heads, columns // 16, dim, 16)[:, :, -1, :, vdim - columns + 16:]
         assert not padding.any()
@@ -224,7 +226,7 @@ def test_read_outs_of_16_bit_queries_in_chunks(ops, heads, key_heads, dim, vdim,
               for form, (out, below, _) in results.items()}
     print(errors, flush=True)
     for scan, chunked in zip(errors["scan"], errors["chunks"]):
-        assert chunked <= 2 * scan + 1e-6
+        assert chunked <= (1.25 if spare else 2.0) * scan + HALF_UNIT
 
 
 NO_NUMBERS = [float("inf"), float("-inf"), float("nan")]
@@ -290,3 +292,105 @@ def test_what_is_no_number_reaches_no_earlier_token_of_a_delta_rule(ops, place, 
         keep = torch.isfinite(walk)
         assert float((walk - chunked)[keep].norm()) <= 1e-5 * float(walk[keep].norm())
     assert torch.isfinite(results[0][0][:place]).all() and not torch.isfinite(results[0][0][place:]).all()
+
+
+LONG = 2000
+
+
+@pytest.mark.parametrize("kept", [0.9995, 0.99, 0.6])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_a_long_row_of_a_linear_recurrence(ops, dtype, kept):
+    """32 chunks of one row from a kept state, decays around ``kept`` a token: the walk over the chunks rounds no more than the walk over the tokens."""
+    heads, dim, vdim = 2, 128, 128
+    generator = torch.Generator("cuda").manual_seed(int(1e4 * kept))
+    draw = lambda *shape: torch.randn(*shape, device="cuda", generator=generator)
+    proj = (0.5 * draw(LONG, 2 * heads * dim + heads * vdim)).to(dtype)
+    q, k, v = proj[:, :heads * dim], proj[:, heads * dim:2 * heads * dim], proj[:, 2 * heads * dim:]
+    z = torch.log(-torch.log(torch.tensor(kept))).item() + 0.5 * draw(LONG, heads * dim)
+    _, _, row_start, row_len, row_ctx = batch([LONG], [50], "cuda")
+    slots, start = torch.zeros(1, dtype=torch.int32, device="cuda"), draw(1, heads * dim * vdim)
+    chunks = ops.linear_recurrence_chunks(LONG, 1, LONG, 16, dim, vdim)
+    scratch = {"sums": torch.empty(chunks, heads, dim, vdim, device="cuda"), "totals": torch.empty(chunks, heads, dim, device="cuda"),
+               "queries": torch.empty(LONG, heads, dim, device="cuda")}
+    wide = lambda x: x.double().reshape(LONG, heads, -1)
+    exact, after = plain_recurrence(0.3 * wide(q), wide(k), wide(v), torch.exp(-torch.exp(wide(z))), None, start.view(heads, dim, vdim).double())
+    errors = []
+    for more in ({}, scratch):
+        state, out = start.clone(), torch.empty(LONG, heads * vdim, device="cuda")
+        ops.linear_recurrence(q, k, v, z, None, "double_exp", 1.0, None, 0.3, state, 0, slots, row_start, row_len, row_ctx, out, heads, dim, vdim, **more)
+        errors.append((off(out, exact.reshape(LONG, -1)), off(state, after.reshape(1, -1))))
+    print("long linear", dtype, kept, errors, flush=True)
+    for walk, chunked in zip(*errors):
+        assert chunked <= 1.1 * walk
+
+
+@pytest.mark.parametrize("kept", [0.9995, 0.99, 0.6])
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_a_long_row_of_a_delta_rule(ops, per_channel, kept):
+    """The same with keys of which every second repeats one of eight directions, so that writes keep taking back what stands there."""
+    heads, dim, vdim = 2, 128, 128
+    generator = torch.Generator("cuda").manual_seed(int(1e4 * kept) + per_channel)
+    draw = lambda *shape: torch.randn(*shape, device="cuda", generator=generator)
+    q, k, v = draw(LONG, heads, dim), draw(LONG, heads, dim), draw(LONG, heads, vdim)
+    k[::2] = draw(8, heads, dim).repeat(LONG // 16, 1, 1) + 0.05 * k[::2]
+    q, k = q / q.norm(dim=-1, keepdim=True) * dim ** -0.5, k / k.norm(dim=-1, keepdim=True)
+    strength = torch.sigmoid(2 * draw(LONG, heads))
+    decay = torch.exp(torch.log(torch.tensor(kept)).item() * torch.exp(0.5 * draw(LONG, heads * dim if per_channel else heads)))
+    prepared = torch.cat([x.reshape(LONG, -1) for x in (q, k, v)], dim=1)
+    _, _, row_start, row_len, row_ctx = batch([LONG], [50], "cuda")
+    slots, start = torch.zeros(1, dtype=torch.int32, device="cuda"), draw(1, heads * dim * vdim)
+    turned = lambda flat: flat.view(heads, vdim // 16, dim, 16).permute(0, 2, 1, 3).reshape(heads, dim, vdim)
+    scratch = torch.empty(LONG // 64 + 1, heads, ops._part_library("delta").lsa_delta_chunk_floats(dim, vdim), device="cuda")
+    exact, after = plain_delta(q.double(), k.double(), v.double(), decay.double().view(LONG, heads, -1).expand(LONG, heads, dim), strength.double(),
+                               turned(start).double())
+    errors = []
+    for more in ({}, {"scratch": scratch}):
+        state, out = start.clone(), torch.empty(LONG, heads * vdim, device="cuda")
+        ops.delta_rule(prepared, strength, decay, per_channel, state, 0, slots, row_start, row_len, row_ctx, out, heads, heads, dim, vdim, **more)
+        errors.append((off(out, exact.reshape(LONG, -1)), off(turned(state), after)))
+    print("long delta", per_channel, kept, errors, flush=True)
+    for walk, chunked in zip(*errors):
+        assert chunked <= 1.1 * walk
+
+
+@pytest.mark.parametrize("rule", ["linear", "delta"])
+def test_chunks_recorded_in_a_graph_for_rows_of_other_lengths(ops, rule):
+    """256 tokens in three rows, recorded once and replayed with the rows cut elsewhere, one of them empty or new: the numbers of an eager call."""
+    heads, dim, vdim, n = 2, 64, 48, 256
+    generator = torch.Generator("cuda").manual_seed(9)
+    draw = lambda *shape: torch.randn(*shape, device="cuda", generator=generator)
+    slots, start = torch.tensor([2, 0, 1], dtype=torch.int32, device="cuda"), draw(3, heads * dim * vdim)
+    out, state, items = torch.empty(n, heads * vdim, device="cuda"), start.clone(), n // 64 + 3
+    rows = [torch.zeros(3, dtype=torch.int32, device="cuda") for _ in range(3)]
+
+    def cut(lengths, firsts):
+        for kept, value in zip(rows, batch(lengths, firsts, "cuda")[2:]):
+            kept.copy_(value)
+    if rule == "linear":
+        q, k, v, decay = (0.5 * draw(n, heads * width) for width in (dim, dim, vdim, dim))
+        scratch = {"sums": torch.empty(items, heads, dim, vdim, device="cuda"), "totals": torch.empty(items, heads, dim, device="cuda"),
+                   "queries": torch.empty(n, heads, dim, device="cuda")}
+        run = lambda: ops.linear_recurrence(q, k, v, decay, None, "double_exp", 1.0, None, 0.3, state, 0, slots, *rows, out, heads, dim, vdim, **scratch)
+    else:
+        q, k = (torch.nn.functional.normalize(draw(n, heads, dim), dim=-1).reshape(n, -1) for _ in range(2))
+        prepared, strength = torch.cat([q, k, draw(n, heads * vdim)], dim=1), torch.sigmoid(draw(n, heads))
+        decay = torch.exp(-0.1 * torch.rand(n, heads, device="cuda", generator=generator))
+        scratch = torch.empty(items, heads, ops._part_library("delta").lsa_delta_chunk_floats(dim, vdim), device="cuda")
+        run = lambda: ops.delta_rule(prepared, strength, decay, False, state, 0, slots, *rows, out, heads, heads, dim, vdim, scratch=scratch)
+    cut([200, 55, 1], [4, 0, 9])
+    run()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for lengths, firsts in (([200, 55, 1], [4, 0, 9]), ([1, 1, 254], [7, 0, 0]), ([0, 128, 128], [3, 5, 0]), ([85, 85, 86], [0, 64, 2]), ([200, 55, 1], [4, 0, 9])):
+        cut(lengths, firsts)
+        results = []
+        for call in (run, graph.replay):
+            state.copy_(start)
+            out.fill_(float("nan"))
+            call()
+            torch.cuda.synchronize()
+            results.append((out.clone(), state.clone()))
+        assert torch.isfinite(results[0][0]).all()
+        for eager, replayed in zip(*results):
+            assert torch.equal(eager, replayed)
