@@ -134,11 +134,9 @@ class StepContext:
         return torch.empty(shape, device=self.device, dtype=dtype or self.dtype)
 
     def longest_row(self) -> int:
-        """About how many tokens the step's longest row brings, for choices between kernels: the number itself, or, where the step's
-        shapes must be fixed (a captured step is replayed for rows of other lengths), twice the average as far as the rows can reach it."""
-        if self.static_max_keys is None:
-            return int(self.h_row_len.max())
-        return min(self.n_tokens - self.n_rows + 1, 2 * self.n_tokens // self.n_rows)
+        """How many tokens the step's longest row brings, for choices between kernels.  A captured step is replayed for rows of other lengths:
+        what a mixer chooses by this number, it names in its ``length_rules``."""
+        return int(self.h_row_len.max())
 
     def block_table(self, group: int) -> torch.Tensor:
         return self._tables[group]

@@ -85,6 +85,7 @@ class ModelRunner:
         self._flip = 0
         self.vocab = model.head.out_features
         self._mixers = list({id(block.mixer): block.mixer for block in model.blocks}.values())
+        self._length_rules = tuple(dict.fromkeys(rule for mixer in self._mixers for rule in mixer.length_rules()))
         # (rows of nobody's, which fill a captured step up, keep their state in a slot behind the requests')
         graph_safe = all(mixer.graph_safe for mixer in self._mixers)
         if use_graphs is None:
@@ -238,25 +239,28 @@ class ModelRunner:
         pages.  Its wanted places are every row's last token, or none."""
         if not self.capture_portions or len(entries) > PORTION_ROWS:
             return None
-        tokens, longest = 0, 1
+        tokens, longest, longest_row = 0, 1, 0
         for entry in entries:
             record = self.cache.requests.get(entry.request_id)
             want = list(entry.want)
             if record is None or (want and want != [len(entry.tokens) - 1]):
                 return None
             tokens += len(entry.tokens)
+            longest_row = max(longest_row, len(entry.tokens))
             longest = max(longest, record.num_computed + len(entry.tokens))
         rows = padded_rows(len(entries)) + 1
         size = padded_tokens(tokens + rows - 1 - len(entries))          # the rows of one token that fill the rows up bring a token each
         if size is None:
             return None
-        longest = max(longest, size - tokens - (rows - 1 - len(entries)))
+        filler_tokens = size - tokens - (rows - 1 - len(entries))
+        longest, longest_row = max(longest, filler_tokens), max(longest_row, filler_tokens)
         blocks = -(-longest // self.cache.page_size)
         width = -(-blocks // TABLE_WIDTH_STEP) * TABLE_WIDTH_STEP
         if not self._host_bounds_a_step(size, width * self.cache.page_size):
             return None
         wanted = rows if any(entry.want for entry in entries) else 0
-        shapes = tuple(dict.fromkeys(mixer.graph_shape(rows, longest) for mixer in self._mixers))
+        shapes = tuple(dict.fromkeys(mixer.graph_shape(rows, longest) for mixer in self._mixers)) \
+            + tuple(bool(getattr(self.ops, name)(size, rows, longest_row, *sizes)) for name, *sizes in self._length_rules)
         key = ("portions", rows, size, width, wanted, shapes)
         if key not in self._graphs:
             met = self._met[key] = self._met.get(key, 0) + 1

@@ -239,6 +239,11 @@ class Mixer(Part):
         """Contexts at which :meth:`graph_shape` changes its answer (a warm-up captures a graph on either side)."""
         return ()
 
+    def length_rules(self):
+        """``(name, *sizes)`` of the kernel namespace's methods ``name(n_tokens, rows, longest row, *sizes)`` by whose answer (something or
+        nothing) ``forward`` chooses between kernels: steps with portions of prompts share a graph only where the answers are the same."""
+        return ()
+
     def mixing_flops(self, new_tokens: int, context: int) -> float:
         """Floating-point operations between the mixer's projections for a row of ``new_tokens`` tokens that ends at a
         context of ``context`` tokens (attention: scores and weighted values); the projections are counted from

@@ -156,6 +156,9 @@ class GatedDeltaRule(Mixer):
         self.proj.finalize()
         self.o.finalize()
 
+    def length_rules(self):
+        return (("delta_rule_scratch", self.heads, self.dim, self.value_dim),)
+
     def mixing_flops(self, new_tokens: int, context: int) -> float:
         """Per token, head and state element: the decay, what the state returns for the key, the write and the read-out."""
         return 7.0 * new_tokens * self.heads * self.dim * self.value_dim

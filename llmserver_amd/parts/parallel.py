@@ -65,6 +65,9 @@ class ParallelMixers(Mixer):
     def graph_shape_edges(self):
         return tuple(self.left.graph_shape_edges()) + tuple(self.right.graph_shape_edges())
 
+    def length_rules(self):
+        return tuple(self.left.length_rules()) + tuple(self.right.length_rules())
+
     def mixing_flops(self, new_tokens, context):
         return self.left.mixing_flops(new_tokens, context) + self.right.mixing_flops(new_tokens, context)
 

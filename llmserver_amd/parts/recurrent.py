@@ -153,6 +153,9 @@ class GatedLinearAttention(Mixer):
         if self.decay_up.weight.shape[1] != self.low:
             raise ValueError(f"the decay's two matrices disagree about their inner size: {self.low} and {self.decay_up.weight.shape[1]}")
 
+    def length_rules(self):
+        return (("linear_recurrence_chunks", self.heads, self.dim, self.value_dim),)
+
     def mixing_flops(self, new_tokens: int, context: int) -> float:
         """Per token, head and state element: the decay, the outer product's sum and the read-out."""
         return 6.0 * new_tokens * self.heads * self.dim * self.value_dim
@@ -261,6 +264,9 @@ class TimeMixing(Mixer):
             part.finalize()
         if self.decay_up.weight.shape[1] != self.low:
             raise ValueError(f"the decay's two matrices disagree about their inner size: {self.low} and {self.decay_up.weight.shape[1]}")
+
+    def length_rules(self):
+        return (("linear_recurrence_chunks", self.heads, self.dim, self.dim),)
 
     def mixing_flops(self, new_tokens: int, context: int) -> float:
         return 8.0 * new_tokens * self.heads * self.dim * self.dim

@@ -4,10 +4,13 @@ import types
 import pytest
 import torch
 
+from llmserver_amd.engine.batch import StepEntry
+from llmserver_amd.engine.replay import make_runner
 from llmserver_amd.kernels import library
 from llmserver_amd.kernels.ops import HipOps
 from llmserver_amd.parts.base import scratch_memory
 from llmserver_amd.parts.recurrent import _chunk_scratch
+from torch_ops import TorchOps
 
 
 @pytest.fixture()
@@ -69,3 +72,31 @@ def test_steps_run_the_way_that_was_measured_to_be_faster(ops):
         assert delta_bytes(ops, *case), case
     for case in WALKS_OF_DELTA:
         assert not delta_bytes(ops, *case), case
+
+
+# rows' lengths of steps that would be filled up to the same number of tokens and rows: (in chunks, token by token) by the rule of 16 heads of 128 x 128
+@pytest.mark.parametrize("design,rule,in_chunks,walked", [
+    ("barotar", "linear_recurrence_chunks", [[490] + [1] * 15, [300] + [12] * 15], [[32] * 16, [60] + [30] * 15]),
+    ("gogalix", "delta_rule_scratch", [[490] + [1] * 15], [[32] * 16]), ("gogalix", "delta_rule_scratch", [[478, 1, 1]], [[160] * 3])])
+def test_captured_steps_choose_by_their_longest_row(ops, design, rule, in_chunks, walked):
+    """A graph is shared by steps that choose alike only, and each step chooses as it would if it were not captured."""
+    import tiny_barotar, tiny_gogalix
+    tiny = {"barotar": tiny_barotar, "gogalix": tiny_gogalix}[design]
+    twins = TorchOps()
+    setattr(twins, rule, lambda n_tokens, rows, longest, *sizes: getattr(ops, rule)(n_tokens, rows, longest, 16, 128, 128))
+    name = next(iter(tiny.CASES))
+    runner = make_runner(tiny.model_folder(name), "float32", 4096, tiny.CASES[name][2], device="cpu", ops=twins, max_live=16)
+    runner.use_graphs, runner._host_bounds_a_step = True, lambda tokens, keys: True         # (only the keys are asked for)
+    for row in range(16):
+        runner.cache.open(row)
+    keys = {}
+    for lengths in in_chunks + walked:
+        entries = [StepEntry(row, [1] * length, [length - 1]) for row, length in enumerate(lengths)]
+        runner._graph_key(entries)
+        keys[tuple(lengths)] = key = runner._graph_key(entries)
+        step = runner.build_context(entries, filler_rows=key[1] - 1 - len(entries), filler_tokens=key[2] - sum(lengths) - (key[1] - 1 - len(entries)))
+        step.static_max_keys = 4096
+        assert step.n_tokens == key[2] and step.longest_row() == max(int(length) for length in step.h_row_len)
+        eager = bool(getattr(ops, rule)(step.n_tokens, step.n_rows, step.longest_row(), 16, 128, 128))
+        assert eager == (lengths in in_chunks) == key[5][-1], lengths
+    assert len({key[:3] for key in keys.values()}) == 1 and len(set(keys.values())) == 2
