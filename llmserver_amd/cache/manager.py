@@ -264,8 +264,16 @@ class CacheManager:
             raise
 
     def advance(self, request_id, num_computed: int) -> None:
-        """Tokens ``< num_computed`` are in the cache; give back pages that a window has passed or whose chunks have ended."""
+        """Tokens ``< num_computed`` are in the cache; give back pages that a window has passed or whose chunks have ended.  A request
+        cannot go back to where it would see keys on such pages again: the kernels would read in front of the pool."""
         record = self.record(request_id)
+        if num_computed < record.num_computed:
+            for group in self.groups:
+                table = record.tables[group.index]
+                first = group.first_needed_block(num_computed) if group.spec.bounded else len(table)
+                if first < len(table) and table[first] < 0:
+                    raise CacheStateError(f"request {request_id!r} cannot go back from {record.num_computed} to {num_computed} tokens: "
+                                          f"pages that it would see again have been given back")
         record.num_computed = num_computed
         for group in self.groups:
             if not group.spec.bounded:

@@ -120,6 +120,30 @@ def test_window_gives_pages_back_once_every_query_has_passed_them():
     assert m.available_pages() == [5]
 
 
+@pytest.mark.parametrize("spec", [WINDOW, PagedKVSpec(2, 16, chunk=12)])
+def test_no_way_back_to_pages_that_were_given_back(spec):
+    """A step behind such a place would take its keys from page -1."""
+    for back in range(40):
+        m = manager({0: spec, 1: FULL}, page_size=4, pages=16)
+        m.open("a")
+        m.ensure("a", 40)
+        m.advance("a", 40)
+        held = list(m.record("a").tables[0])
+        if all(page >= 0 for page in held[spec.first_key(back) // 4:]):
+            m.advance("a", back)
+            assert m.record("a").num_computed == back
+        else:
+            with pytest.raises(CacheStateError, match="cannot go back from 40"):
+                m.advance("a", back)
+            assert m.record("a").num_computed == 40 and m.record("a").tables[0] == held
+        m.check_invariants()
+    m = manager({0: FULL}, page_size=4, pages=16)
+    m.open("a")
+    m.ensure("a", 40)
+    m.advance("a", 40)
+    m.advance("a", 1)                                              # (nothing is given back without a bound)
+
+
 def test_ensure_is_all_or_nothing():
     m = manager({0: FULL, 1: WINDOW}, pages=[8, 2])
     m.open("a")
