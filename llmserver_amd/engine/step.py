@@ -260,7 +260,7 @@ class ModelRunner:
             return None
         wanted = rows if any(entry.want for entry in entries) else 0
         shapes = tuple(dict.fromkeys(mixer.graph_shape(rows, longest) for mixer in self._mixers)) \
-            + tuple(bool(getattr(self.ops, name)(size, rows, longest_row, *sizes)) for name, *sizes in self._length_rules)
+            + tuple(rule(self.ops, size, rows, longest_row, *sizes) for rule, *sizes in self._length_rules)
         key = ("portions", rows, size, width, wanted, shapes)
         if key not in self._graphs:
             met = self._met[key] = self._met.get(key, 0) + 1

@@ -240,8 +240,8 @@ class Mixer(Part):
         return ()
 
     def length_rules(self):
-        """``(name, *sizes)`` of the kernel namespace's methods ``name(n_tokens, rows, longest row, *sizes)`` by whose answer (something or
-        nothing) ``forward`` chooses between kernels: steps with portions of prompts share a graph only where the answers are the same."""
+        """``(rule, *sizes)`` for every ``rule(ops, n_tokens, rows, longest row, *sizes)`` by whose answer, true or false, ``forward`` chooses
+        between kernels: steps with portions of prompts share a graph only where the answers are the same."""
         return ()
 
     def mixing_flops(self, new_tokens: int, context: int) -> float:

@@ -38,6 +38,10 @@ def matrix_floats(heads: int, dim: int, value_dim: int) -> int:
     return heads * dim * (-(-value_dim // STATE_COLUMNS) * STATE_COLUMNS)
 
 
+def _in_chunks(ops, n_tokens, rows, longest, heads, dim, value_dim) -> bool:
+    return ops.delta_rule_scratch(n_tokens, rows, longest, heads, dim, value_dim) is not None
+
+
 @dataclasses.dataclass(frozen=True)
 class GatedDeltaNames:
     q: str = "q"
@@ -157,7 +161,7 @@ class GatedDeltaRule(Mixer):
         self.o.finalize()
 
     def length_rules(self):
-        return (("delta_rule_scratch", self.heads, self.dim, self.value_dim),)
+        return ((_in_chunks, self.heads, self.dim, self.value_dim),)
 
     def mixing_flops(self, new_tokens: int, context: int) -> float:
         """Per token, head and state element: the decay, what the state returns for the key, the write and the read-out."""

@@ -32,6 +32,10 @@ from .linear import Linear
 DECAYS = ("sigmoid_root", "double_exp")
 
 
+def _in_chunks(ops, n_tokens, rows, longest, heads, dim, value_dim) -> bool:
+    return ops.linear_recurrence_chunks(n_tokens, rows, longest, heads, dim, value_dim) > 0
+
+
 def _chunk_scratch(ctx, n, heads, dim, value_dim):
     """The scratch tensors of ``ops.linear_recurrence`` for a step that runs it in chunks; none for one that does not."""
     chunks = ctx.ops.linear_recurrence_chunks(n, ctx.row_len.shape[0], ctx.longest_row(), heads, dim, value_dim)
@@ -154,7 +158,7 @@ class GatedLinearAttention(Mixer):
             raise ValueError(f"the decay's two matrices disagree about their inner size: {self.low} and {self.decay_up.weight.shape[1]}")
 
     def length_rules(self):
-        return (("linear_recurrence_chunks", self.heads, self.dim, self.value_dim),)
+        return ((_in_chunks, self.heads, self.dim, self.value_dim),)
 
     def mixing_flops(self, new_tokens: int, context: int) -> float:
         """Per token, head and state element: the decay, the outer product's sum and the read-out."""
@@ -266,7 +270,7 @@ class TimeMixing(Mixer):
             raise ValueError(f"the decay's two matrices disagree about their inner size: {self.low} and {self.decay_up.weight.shape[1]}")
 
     def length_rules(self):
-        return (("linear_recurrence_chunks", self.heads, self.dim, self.dim),)
+        return ((_in_chunks, self.heads, self.dim, self.dim),)
 
     def mixing_flops(self, new_tokens: int, context: int) -> float:
         return 8.0 * new_tokens * self.heads * self.dim * self.dim
