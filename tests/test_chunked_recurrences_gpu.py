@@ -394,3 +394,42 @@ def test_chunks_recorded_in_a_graph_for_rows_of_other_lengths(ops, rule):
         assert torch.isfinite(results[0][0]).all()
         for eager, replayed in zip(*results):
             assert torch.equal(eager, replayed)
+
+
+@pytest.mark.parametrize("design,case", [("barotar", "BD"), ("gogalix", "GC")])
+def test_captured_steps_with_portions_in_chunks_and_walked(design, case):
+    """256 tokens of three requests in turns, one long portion beside two short ones (in chunks) and three alike (walked): a graph each, and every
+    replay's logits are those of the same step run eagerly."""
+    import importlib
+    from helpers import random_tokens
+    from llmserver_amd.engine import StepEntry
+    from llmserver_amd.engine.replay import make_runner
+    tiny = importlib.import_module(f"tiny_{design}")
+    vocab, page = tiny.CASES[case][0]["vocab"], tiny.CASES[case][2]
+    print(f"captured portions in chunks {design} {case}", flush=True)
+    runners = [make_runner(tiny.model_folder(case), "float32", 4096, page, max_live=4) for _ in range(2)]
+    runners[1].use_graphs = False
+    forms, worst = {}, 0.0
+    for turn in range(10):
+        lengths = [250, 3, 3] if turn % 2 else [85, 85, 86]
+        logits = []
+        for runner in runners:
+            entries = [StepEntry(f"{turn} {row}", random_tokens(vocab, length, 10 * turn + row), [length - 1]) for row, length in enumerate(lengths)]
+            for entry in entries:
+                runner.cache.open(entry.request_id)
+            logits.append(runner.step(entries).clone())
+            follow = [StepEntry(entry.request_id, [turn], [0]) for entry in entries]              # (the state behind them)
+            logits.append(runner.step(follow).clone())
+            if runner.use_graphs:
+                key = runner._portion_key(entries)
+                if key is not None:
+                    forms.setdefault(turn % 2, set()).add(key)
+            for entry in entries:
+                runner.cache.close(entry.request_id)
+        torch.cuda.synchronize()
+        for replayed, eager in zip(logits[:2], logits[2:]):
+            worst = max(worst, float((replayed - eager).norm() / eager.norm()))
+    print("worst", worst, "replays", runners[0].graph_replays, flush=True)
+    assert len(forms[0]) == len(forms[1]) == 1 and forms[0] != forms[1]
+    assert any(next(iter(forms[1]))[5][1:]) and runners[0].graph_replays >= 6
+    assert worst < 1e-5
