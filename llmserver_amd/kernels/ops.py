@@ -1532,22 +1532,27 @@ class HipOps(KernelNamespace):
 
     @staticmethod
     def _linear_recurrence_us(n_tokens, rows, longest, heads, dim, value_dim):
-        """About what a step's recurrences take token by token and in chunks, in us.  Measured, both ways, at 16 heads of 128 x 128: 1 row of 64 / 100 /
-        128 / 256 / 2,048 tokens 30, 47; 45, 48; 54, 48; 103, 51; 919, 122; 4 rows of 128 / 512 58, 60; 237, 116; 16 rows of 64 / 256 / 512 71, 110;
-        241, 220; 471, 473; 512 tokens beside 16 single ones 214, 107; 16 heads of 64 x 64, 1 row of 64 / 128 / 2,048 21, 30; 37, 30; 508, 58; 8 rows of
-        512 157, 90; 16 rows of 512 157, 158.
+        """About what a step's recurrences take token by token and in chunks, in us.  Measured, both ways, at 16 heads of 128 x 128: 1 row of 64 / 112 /
+        128 / 256 / 2,048 tokens 28, 51; 46, 51; 52, 52; 99, 54; 904, 129; 4 rows of 128 / 160 / 256 / 512 53, 62; 65, 64; 101, 109; 231, 124; 16 rows of
+        64 / 256 / 512 66, 118; 239, 240; 462, 508; 8 rows of 2,048 1,039, 1,000; 512 tokens beside 16 single ones 207, 113; 16 heads of 64 x 64, 1 row of
+        64 / 112 / 128 / 2,048 18, 30; 30, 30; 33, 31; 479, 68; 4 rows of 128 34, 33; 8 rows of 512 148, 111; 16 rows of 512 149, 211.
 
         The walk: a row's tokens one after another, as many rounds of them as its workgroups (a head's 64 value columns each) go round 256
-        compute units.  The chunks: three launches and a share for each (chunk, head, 128 value columns)."""
+        compute units, a token slower where these share what leaves L2 and behind the first thousand.  The chunks: three launches, of which the
+        first has a workgroup a (chunk, head, 128 value columns), and a compute unit holds one of them at a time (two where the head is
+        narrow); rows other than the longest are taken to be of one length."""
         wide = dim > 64
         load = n_tokens / longest * heads * -(-value_dim // 64)
-        if wide:
-            walk = 6.0 + (0.39 if load < 128 else 0.46) * longest
-        else:
-            walk = 5.0 + (0.25 if load < 128 else 0.3) * longest
-        walk = max(walk, (0.455 if wide else 0.31) * longest * -(-load // 256))
-        workgroups = (n_tokens // HipOps.MEMORY_CHUNK + rows) * heads * max(1.0, value_dim / 128)
-        return walk, max(48.0, 30.0 + 0.19 * workgroups) if wide else max(31.0, 24.0 + 0.065 * workgroups)
+        first, alone, crowded, far = (4.5, 0.375, 0.46, 0.07) if wide else (3.0, 0.235, 0.29, 0.04)
+        rounds = -(-load // 256)
+        walk = first + longest * (alone if load <= 128 else crowded * rounds) + far * rounds * max(longest - 1024, 0)
+        chunk, others = HipOps.MEMORY_CHUNK, rows - 1
+        count = -(-longest // chunk) + (others * -(-(n_tokens - longest) // (others * chunk)) if others else 0)
+        workgroups = count * heads * max(1.0, value_dim / 128)
+        if workgroups < 240:
+            return walk, 48.0 + 0.08 * workgroups if wide else 29.3 + 0.027 * workgroups
+        middle, many = min(workgroups, 512) - 256, max(workgroups - 512, 0)
+        return walk, 106.0 + 0.075 * middle + 0.24 * many if wide else 54.0 + 0.04 * middle + 0.095 * many
 
     def linear_recurrence_chunks(self, n_tokens, rows, longest, heads, dim, value_dim):
         """How many chunks of scratch memory the recurrence wants for a step of this shape if it is to run in chunks, or 0 if it

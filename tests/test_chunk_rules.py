@@ -53,10 +53,12 @@ def test_a_step_without_room_for_scratch_memory_walks():
 
 
 # (rows' lengths, heads, key channels, value channels): where the chunks were measured to be faster than the walk, and where they were not
-CHUNKS_OF_LINEAR = [([128], 16, 128, 128), ([2048], 8, 128, 256), ([256] * 2, 16, 128, 128), ([512] * 4, 16, 128, 128), ([512] + [1] * 16, 16, 128, 128),
+CHUNKS_OF_LINEAR = [([144], 16, 128, 128), ([160] * 4, 16, 128, 128), ([2048], 8, 128, 256), ([2048] * 8, 16, 128, 128), ([256] * 2, 16, 128, 128), ([512] * 4, 16, 128, 128), ([512] + [1] * 16, 16, 128, 128),
                     ([128] * 4, 16, 64, 64), ([512] * 8, 16, 64, 64), ([512] * 4, 32, 64, 64), ([512] * 8, 8, 96, 192), ([256] * 16, 8, 96, 192)]
-WALKS_OF_LINEAR = [([100], 16, 128, 128), ([100], 32, 128, 128), ([64], 16, 64, 64), ([64] * 16, 16, 128, 128), ([32] * 32, 16, 64, 64), ([128] * 8, 16, 128, 128),
-                   ([256] * 16, 16, 64, 64), ([1] * 40, 16, 128, 128), ([112] + [1] * 64, 16, 128, 128), ([128] + [1] * 8, 16, 128, 128), ([512] * 16, 16, 128, 128)]
+WALKS_OF_LINEAR = [([100], 16, 128, 128), ([112], 16, 128, 128), ([256] * 4, 16, 128, 128), ([96], 16, 64, 64), ([8] * 4 + [0], 16, 64, 64),
+                   ([100], 32, 128, 128), ([64], 16, 64, 64), ([64] * 16, 16, 128, 128), ([32] * 32, 16, 64, 64), ([128] * 8, 16, 128, 128),
+                   ([256] * 16, 16, 64, 64), ([1] * 40, 16, 128, 128), ([112] + [1] * 64, 16, 128, 128), ([128] + [1] * 8, 16, 128, 128), ([512] * 16, 16, 128, 128),
+                   ([1024] * 8, 16, 128, 128), ([2048] * 16, 16, 64, 64)]
 CHUNKS_OF_DELTA = [([512], 16, 128, 128), ([1900], 16, 128, 128), ([512] * 4, 16, 128, 128), ([512] + [1] * 16, 16, 128, 128), ([256], 16, 64, 64),
                    ([2048], 32, 64, 64), ([1024] + [64] * 8, 32, 128, 128), ([512] * 4, 8, 96, 192)]
 WALKS_OF_DELTA = [([192], 4, 128, 128), ([160], 16, 128, 128), ([256], 32, 128, 128), ([256] * 8, 4, 128, 128), ([256] * 4, 16, 128, 128), ([64] * 16, 16, 128, 128),
