@@ -674,6 +674,10 @@ __global__ __launch_bounds__(256, LSA_MIN_WAVES) void paged_attention_kernel(
     }
 }
 
+#if !LSA_BF16 || LSA_ND % 2 == 0      // (whole 32-wide steps of the score product)
+#include "attention_single.hpp"
+#endif
+
 #if LSA_BF16
 // ------------------------------------------------------------------------------------------------
 // Portions of prompts: the four wavefronts of a workgroup take 4 * SUB consecutive tiles of 16 pairs
@@ -1439,6 +1443,67 @@ __global__ __launch_bounds__(MERGE_WAVES * 64) void merge_kernel(
     }
 }
 
+static Geometry geometry_of(int n_q, int n_kv, int gheads, int tokens_per_tile, int gtiles, int page_size, int window, float scale, const float* sinks,
+                            float softcap, int chunk, const float* slopes, const void* gates, long gate_stride) {
+    Geometry g;
+    g.n_q = n_q; g.n_kv = n_kv; g.group = n_q / n_kv; g.gheads = gheads; g.tokens_per_tile = tokens_per_tile;
+    g.gtiles = gtiles; g.page_size = page_size; g.window = window; g.scale = scale; g.sinks = sinks;
+    g.cap = softcap; g.cap_inverse = softcap > 0.f ? 1.f / softcap : 0.f; g.scale_inverse = scale != 0.f ? 1.f / scale : 0.f;
+    g.chunk = chunk; g.slopes = slopes; g.gates = (const elem_t*)gates; g.gate_stride = gate_stride;
+    g.page_magic = (unsigned)(((1ull << 32) + page_size - 1) / page_size);
+    return g;
+}
+
+// Whether attention_single_kernel takes pages of `page_size` keys, and, if `fused`, norm, rotation and the new token's way into the cache with them.
+LSA_EXPORT int lsa_attention_single_fits(int page_size, int fused) {
+    return page_size > 0 && page_size % 16 == 0 && (!LSA_BF16 || D % 32 == 0) && (!fused || D % (LSA_BF16 ? 64 : 32) == 0) ? 1 : 0;
+}
+
+// A step of `rows` rows of one token each, row i's at place i, in one launch (see attention_single.hpp).
+LSA_EXPORT int lsa_attention_single(
+    const void* q, long q_token_stride, void* out, const void* keys, const void* values, const int* table, int table_stride, const int* row_ctx,
+    int rows, float scale, int window, int page_size, int n_q, int n_kv, int gheads, int gtiles, int decode_fusion, const float* q_weight,
+    const float* k_weight, float norm_eps, const float* cos_sin, const float* sinks, float softcap, int chunk, const float* slopes,
+    const void* gates, long gate_stride, hipStream_t stream) {
+#if LSA_BF16 && LSA_ND % 2
+    return -1;
+#else
+    if (rows <= 0) return 0;
+    if (!lsa_attention_single_fits(page_size, decode_fusion) || table_stride < 1 || n_kv < 1 || n_q % n_kv || gheads < 1 || gheads > 16
+        || gtiles < 1 || (gtiles - 1) * gheads >= n_q / n_kv || gtiles * gheads < n_q / n_kv) return -1;
+    if (softcap < 0.f || chunk < 0 || (gates != nullptr && gate_stride < n_q) || (slopes != nullptr && (decode_fusion || !(scale > 0.f)))) return -1;
+    if (decode_fusion != 0 && decode_fusion != 1 && decode_fusion != 3) return -1;
+    if (decode_fusion && (q_weight == nullptr || k_weight == nullptr || cos_sin == nullptr)) return -1;
+    const Geometry g = geometry_of(n_q, n_kv, gheads, 1, gtiles, page_size, window, scale, sinks, softcap, chunk, slopes, gates, gate_stride);
+    const DecodeFusion fusion = {q_weight, k_weight, cos_sin, norm_eps, decode_fusion};
+    constexpr int CHUNK = ND < 8 ? ND : 8;
+    const dim3 grid(rows, n_kv * gtiles);
+#define LSA_SINGLE(MODE, WAVES, HEADS) attention_single_kernel<MODE, WAVES, HEADS><<<grid, 64 * WAVES, \
+        (size_t)WAVES * CHUNK * (HEADS ? 16 * HEADS : 4 * gheads) * 16, stream>>>( \
+        (const elem_t*)q, q_token_stride, (elem_t*)out, (const elem_t*)keys, (const elem_t*)values, table, table_stride, row_ctx, g, fusion)
+#if LSA_BF16 ? LSA_ND % 4 == 0 : LSA_ND % 2 == 0
+#define LSA_SINGLE_MODES(WAVES, HEADS) do { if (decode_fusion == 3) LSA_SINGLE(3, WAVES, HEADS); else if (decode_fusion == 1) LSA_SINGLE(1, WAVES, HEADS); \
+        else LSA_SINGLE(0, WAVES, HEADS); } while (0)
+#else
+#define LSA_SINGLE_MODES(WAVES, HEADS) LSA_SINGLE(0, WAVES, HEADS)
+#endif
+#if !LSA_BF16 && LSA_ND <= 8
+    const bool vector = slopes == nullptr && softcap == 0.f && gtiles == 1;
+    if (vector && n_q == n_kv) LSA_SINGLE_MODES(8, 1);
+    else if (vector && n_q == 2 * n_kv) LSA_SINGLE_MODES(8, 2);
+    else
+#endif
+#if LSA_ND <= 8
+    if (gheads <= 8) LSA_SINGLE_MODES(8, 0);
+    else
+#endif
+    LSA_SINGLE_MODES(4, 0);
+#undef LSA_SINGLE_MODES
+#undef LSA_SINGLE
+    LSA_LAUNCH_CHECK();
+#endif
+}
+
 LSA_EXPORT int lsa_paged_attention(
     const void* q, long q_token_stride, void* out, const void* keys, const void* values, const int* table, int table_stride,
     const int* row_start, const int* row_len, const int* row_ctx, const void* items, const int* item_slot, int n_items,
@@ -1455,12 +1520,7 @@ LSA_EXPORT int lsa_paged_attention(
     DecodeFusion fusion = {q_weight, k_weight, cos_sin, norm_eps, decode_fusion};
     if (decode_fusion != 0 && decode_fusion != 1 && decode_fusion != 3) return -1;
     if (decode_fusion && (!LSA_BF16 || D % 64 != 0 || n_tiles > 0 || (q_weight == nullptr) != (k_weight == nullptr))) return -1;
-    Geometry g;
-    g.n_q = n_q; g.n_kv = n_kv; g.group = n_q / n_kv; g.gheads = gheads; g.tokens_per_tile = tokens_per_tile;
-    g.gtiles = gtiles; g.page_size = page_size; g.window = window; g.scale = scale; g.sinks = sinks;
-    g.cap = softcap; g.cap_inverse = softcap > 0.f ? 1.f / softcap : 0.f; g.scale_inverse = scale != 0.f ? 1.f / scale : 0.f;
-    g.chunk = chunk; g.slopes = slopes; g.gates = (const elem_t*)gates; g.gate_stride = gate_stride;
-    g.page_magic = (unsigned)(((1ull << 32) + page_size - 1) / page_size);
+    const Geometry g = geometry_of(n_q, n_kv, gheads, tokens_per_tile, gtiles, page_size, window, scale, sinks, softcap, chunk, slopes, gates, gate_stride);
     if (n_tiles > 0) {
 #if LSA_BF16
         // The plan's entries of `tiles` span what a workgroup takes: 4 or 8 tiles.  A load brings 8 keys of a value row.

@@ -87,6 +87,9 @@ _SIGNATURES = {
     "lsa_experts_tiled_ints": [c_int, c_int, c_int],
     "lsa_experts_tiled": [_P, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P, _P, c_int, _P],
     "lsa_experts_down": [c_int, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_int, _P],
+    "lsa_attention_single": [_P, c_long, _P, _P, _P, _P, c_int, _P, c_int, c_float, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P, _P, c_float, _P, _P,
+                             c_float, c_int, _P, _P, c_long, _P],
+    "lsa_attention_single_fits": [c_int, c_int],
     "lsa_attention_workgroup_tiles": [],
     "lsa_attention_tile_page_multiple": [],
     "lsa_attention_tile_halves": [],

@@ -719,6 +719,10 @@ class HipOps(KernelNamespace):
         on itself in a step in which every row brings one token."""
         return dtype == torch.bfloat16 and head_dim % 64 == 0
 
+    def single_token_fusion_fits(self, dtype, head_dim, page_size) -> bool:
+        """The same for steps whose plan says ``rows_in_order`` (one token a row, short contexts): there is a kernel of its own for them."""
+        return bool(self._attention_library(dtype, head_dim).lsa_attention_single_fits(int(page_size), 1))
+
     def paged_attention(self, qkv, out, keys, values, table, row_start, row_len, row_ctx, plan, scale, window, page_size,
                         n_q, n_kv, head_dim, ctx, decode_fusion=None, sinks=None, softcap=None, chunk=None, slopes=None, gates=None):
         """Attention of the step's tokens over their requests' pages.
@@ -792,7 +796,8 @@ class HipOps(KernelNamespace):
         fusion_mode, q_weight, k_weight, norm_eps, cos_sin = 0, None, None, 0.0, None
         if decode_fusion is not None:
             q_weight, k_weight, norm_eps, cos_sin, write_cache = decode_fusion
-            if not self.decode_fusion_fits(qkv.dtype, head_dim) or n_tiles or n != rows:
+            if not (self.decode_fusion_fits(qkv.dtype, head_dim) or plan.get("rows_in_order") and
+                    self.single_token_fusion_fits(qkv.dtype, head_dim, page_size)) or n_tiles or n != rows:
                 raise ValueError("decode fusion takes bfloat16, head sizes in steps of 64 and steps of one token per row")
             for name, w in (("q_weight", q_weight), ("k_weight", k_weight)):
                 if w is not None:
@@ -808,6 +813,14 @@ class HipOps(KernelNamespace):
             raise ValueError("merging in the workgroup takes a plan that gives every tile four key ranges (or, in steps of one token "
                              "per row, two, with tiles in pairs) and no slots, and, with decode fusion, both norm weights and a rotation")
         lib = self._attention_library(qkv.dtype, head_dim)
+        if plan.get("rows_in_order") and merge_in_workgroup and n == rows and lib.lsa_attention_single_fits(page_size, int(fusion_mode > 0)):
+            # one token a row, row i's at place i, behind short contexts: a kernel that finds its work without the plan
+            _launched(lib.lsa_attention_single(
+                _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(keys), _ptr(values), _ptr(table), table.shape[1], _ptr(row_ctx), rows, float(scale),
+                int(window) if window else 0, page_size, n_q, n_kv, gheads, gtiles, fusion_mode, _ptr(q_weight), _ptr(k_weight), float(norm_eps),
+                _ptr(cos_sin), _ptr(sinks), float(softcap) if softcap else 0.0, int(chunk) if chunk else 0, _ptr(slopes), _ptr(gates),
+                gates.stride(0) if gates is not None else 0, _stream()), "attention_single")
+            return
         if n_tiles and int(plan.get("tile_halves", 1)) not in (1, lib.lsa_attention_tile_halves()):
             raise ValueError(f"the plan splits a workgroup's keys into {plan['tile_halves']} halves, this kernel takes 1 or {lib.lsa_attention_tile_halves()}")
         if plan.get("most_splits", 0) > lib.lsa_attention_most_splits():

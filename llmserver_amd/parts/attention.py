@@ -512,10 +512,12 @@ def stage_attention_plan(ctx, key, group_size: int, n_kv_heads: int, head_dim: i
     #  * so many rows that a tile gets four ranges anyway;
     #  * two ranges a tile: two tiles to a workgroup, if the rows come in pairs.  (Two or three ranges in a workgroup
     #    of one tile leave wavefronts idle through the others' walk: a tenth slower at 64 rows behind 4,096 tokens.)
-    in_workgroup = 0
+    in_workgroup, in_order = 0, False
     if single_tokens:
         if ctx.static_max_keys is not None and graph_shape(ctx.n_rows, int(np.max(ctx.h_row_ctx))) is not None:
             in_workgroup = fixed = WORKGROUP_RANGES
+            # (rows of one token each, row i's at place i: a kernel may find its row by its place in the launch)
+            in_order = bool((ctx.h_row_len == 1).all()) and bool((ctx.h_row_start == np.arange(ctx.n_rows)).all())
         elif fixed == WORKGROUP_RANGES or (fixed == 2 and ctx.n_rows % 2 == 0):
             in_workgroup = fixed
     elif ctx.static_max_keys is not None and graph_shape(ctx.n_rows, int(np.max(ctx.h_row_ctx))) is not None:
@@ -540,7 +542,7 @@ def stage_attention_plan(ctx, key, group_size: int, n_kv_heads: int, head_dim: i
         "items": plan.items, "item_slot": plan.item_slot, "merges": plan.merges, "tiles": plan.tiles,
         "n_tiles": len(plan.tiles), "n_items": len(plan.items), "n_merges": len(plan.merges),
         "n_slots": plan.n_slots, "tiles_per_workgroup": plan.tiles_per_workgroup, "tile_halves": int(plan.tile_halves),
-        "merge_in_workgroup": int(plan.merge_in_workgroup),
+        "merge_in_workgroup": int(plan.merge_in_workgroup), "rows_in_order": in_order,
         "most_splits": int(plan.merges[:, 3].max()) if len(plan.merges) else 0,
     })
 
@@ -804,8 +806,10 @@ class GQAttention(Mixer):
         fusion = None
         # (the kernel that merges a tile's key ranges in its workgroup fuses only the whole of norm and rotation)
         whole = self.q_norm_weight is not None and cos_sin is not None
-        if ctx.n_tokens == ctx.n_rows and ctx.ops.decode_fusion_fits(qkv.dtype, self.head_dim) \
-                and (whole or not ctx.get_plan(self.plan_key()).get("merge_in_workgroup")):
+        plan = ctx.get_plan(self.plan_key())
+        if ctx.n_tokens == ctx.n_rows and (
+                ctx.ops.decode_fusion_fits(qkv.dtype, self.head_dim) and (whole or not plan.get("merge_in_workgroup"))
+                or whole and plan.get("rows_in_order") and ctx.ops.single_token_fusion_fits(qkv.dtype, self.head_dim, cache.page_size)):
             fusion = (self.q_norm_weight, self.k_norm_weight, eps, cos_sin, cache.writable)
         else:
             ctx.ops.qk_norm_rope_kv_write(
@@ -820,6 +824,6 @@ class GQAttention(Mixer):
         extra.update(self._seen())
         ctx.ops.paged_attention(
             qkv, out, cache.keys, cache.values, table, ctx.row_start, ctx.row_len, ctx.row_ctx,
-            ctx.get_plan(self.plan_key()), self.scale, self.window, cache.page_size,
+            plan, self.scale, self.window, cache.page_size,
             self.n_heads, self.n_kv_heads, self.head_dim, ctx, **extra)
         return self.o.forward(out, ctx, sink=sink)

@@ -410,6 +410,10 @@ class KernelNamespace:
         """Whether ``paged_attention`` takes q/k norm, rotation and the cache write on itself in single-token steps."""
         return False
 
+    def single_token_fusion_fits(self, dtype, head_dim, page_size) -> bool:
+        """The same for steps whose plan says ``rows_in_order``: one token a row, row i's at place i, all contexts short."""
+        return False
+
     def measuring(self):
         """A context in which unknown shapes may be timed and entered into a table of choices; here: nothing happens."""
         return contextlib.nullcontext(None)
