@@ -37,7 +37,7 @@ struct Fusion {
     const float* square_sums;            // [M, n_parts]
     int n_parts;
     float eps;
-    // Stream update (resid null: none); bfloat16 results only.
+    // Stream update (resid null: none); bfloat16 results only (in the 32-bit kernel the three tensors are float32).
     const bf16_t* resid;                 // [M, N]
     const float* norm_weight;            // [N]
     bf16_t* resid_out;                   // [M, N]
@@ -818,19 +818,29 @@ LSA_EXPORT int lsa_gemm_split_gated(const void* x, const void* w, void* hidden, 
 // step is 16 inner indices: a lane loads four neighbouring ones of its row (16 bytes), and the four 16x16x4 MFMAs of the step take the
 // lanes' first, second, third and fourth, each into sums of its own (four short chains round less than one long one: 1.2e-7 from
 // the 64-bit product at K = 1,024 where the library's is 2.9e-7).
-constexpr int F32_STEPS = 8;
+//
+// What stands around the product in a step can be folded in as in the bfloat16 kernels (the row scale, the stream update, the bias; GATED: silu(gate) *
+// up of 8 gate rows and their 8 up rows), for up to 8 rows (each wavefront finds the scale of one): every norm, activation and sum that is a kernel of its
+// own costs such a step 2 to 3 us (two rows of a 0.6B-sized model: 24 launches fewer a step, a prompt of 333 tokens and 8 steps 6.22 -> 5.85 ms).
+// In 32 bits the stream update has no roundings of its own: s' = resid + y, and the next product takes s' * weight with 1 / rms(s') on its sums.
+constexpr int F32_STEPS = 8, F32_FUSED_ROWS = GEMM_WAVES;
+template <bool GATED>
 __global__ __launch_bounds__(GEMM_WAVES * 64, 4) void gemm_few_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y,
-                                                                          int M, int N, int K, int R, const float* __restrict__ bias) {
+                                                                          int M, int N, int K, int R, Fusion fusion) {
     __shared__ float partial[GEMM_WAVES][256];
+    __shared__ float row_scale[F32_FUSED_ROWS];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), col = lane & 15, quad = lane >> 4;
-    const int n0 = blockIdx.x * R;
+    const int n0 = blockIdx.x * R;                                 // GATED: R <= 8 pairs, the up rows in the tile's second half
     const int steps = (K + 15) / 16, share = (steps + GEMM_WAVES - 1) / GEMM_WAVES;
     const int begin = min(steps, wave * share), end = min(steps, begin + share);
-    const float* wp = w + (size_t)min(n0 + min(col, R - 1), N - 1) * K;
+    const int w_row = GATED ? (col < 8 ? 0 : N / 2) + min(n0 + min(col & 7, R - 1), N / 2 - 1) : min(n0 + min(col, R - 1), N - 1);
+    const float* wp = w + (size_t)w_row * K;
     const float* xp = x + (size_t)min(col, M - 1) * K;
+    RowScaleLoads scale_loads;
     f32x4 acc[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (fusion.square_sums) row_scale_issue(scale_loads, fusion, x, M, wave, lane);        // (there by the time the last products are through)
     for (int step = begin; step < end; step += F32_STEPS) {
         f32x4 ws[F32_STEPS], xs[F32_STEPS];
 #pragma unroll
@@ -851,14 +861,38 @@ __global__ __launch_bounds__(GEMM_WAVES * 64, 4) void gemm_few_f32_kernel(const 
     const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) partial[wave][16 * col + 4 * quad + r] = sum[r];          // [row of X][row of W]
+    row_scale_finish(scale_loads, fusion, M, K, wave, lane, row_scale);
     __syncthreads();
     const int m = threadIdx.x >> 4, j = threadIdx.x & 15, n = n0 + j;
-    if (m >= M || j >= R || n >= N) return;                        // (the second half of the threads has no row)
-    float p[GEMM_WAVES];
+    if (m >= 16) return;                                           // (the second half of the threads has no row; whole wavefronts)
+    auto total_of = [&](int at) {
+        float p[GEMM_WAVES];
 #pragma unroll
-    for (int v = 0; v < GEMM_WAVES; ++v) p[v] = partial[v][threadIdx.x];
-    const float total = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-    y[(size_t)m * N + n] = bias ? total + bias[n] : total;
+        for (int v = 0; v < GEMM_WAVES; ++v) p[v] = partial[v][at];
+        const float total = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+        return fusion.square_sums ? total * row_scale[min(m, F32_FUSED_ROWS - 1)] : total;
+    };
+    const float total = total_of(threadIdx.x);
+    if (GATED) {
+        if (j < R && m < M && n < N / 2) y[(size_t)m * (N / 2) + n] = total / (1.f + expf(-total)) * total_of(threadIdx.x + 8);
+        return;
+    }
+    const bool own = m < M && j < R && n < N;
+    if (fusion.resid) {
+        float s = 0.f;
+        if (own) {
+            const size_t at = (size_t)m * N + n;
+            s = reinterpret_cast<const float*>(fusion.resid)[at] + total;
+            reinterpret_cast<float*>(fusion.resid_out)[at] = s;
+            reinterpret_cast<float*>(fusion.weighted_out)[at] = s * fusion.norm_weight[n];
+        }
+        float sq = s * s;                                          // the 16 lanes of a row are neighbours
+#pragma unroll
+        for (int offset = 1; offset < 16; offset *= 2) sq += __shfl_xor(sq, offset, 64);
+        if (j == 0 && m < M) fusion.square_sums_out[(size_t)m * gridDim.x + blockIdx.x] = sq;
+        return;
+    }
+    if (own) y[(size_t)m * N + n] = fusion.bias ? total + fusion.bias[n] : total;
 }
 
 // Whether the sizes go this way (K a multiple of 4): where this stream was measured to be no slower than the library's product, which is poor at short
@@ -882,12 +916,49 @@ LSA_EXPORT int lsa_gemm_few_f32_fits(int M, int N, int K) {
     return K == 2048 && M <= 4 && N >= 4096 && 10 * workgroups >= 9 * 256 * rounds ? 1 : 0;
 }
 
-// x [M, K], w [N, K], y [M, N], bias [N] or nullptr, all float32; M <= 16, K a multiple of 4, x and w at multiples of 16 bytes.
-LSA_EXPORT int lsa_gemm_few_f32(const float* x, const float* w, float* y, int M, int N, int K, const float* bias, hipStream_t stream) {
+// rows of W a workgroup: 16 where every compute unit gets them, else 8 or 4 (1,024 x 2,048: 7.3, 5.9 and 5.7 us; 4,096 x 1,024: 5.5, 5.9, 9.2)
+static int few_f32_rows(int N) { return N >= 4096 ? 16 : N >= 1024 ? 8 : 4; }
+static bool few_f32_takes(const float* x, const float* w, int M, int K, const float* square_sums, int n_parts, const void* resid) {
+    if (M > 16 || K < 4 || K % 4 != 0 || ((reinterpret_cast<size_t>(x) | reinterpret_cast<size_t>(w)) & 15)) return false;
+    return M <= F32_FUSED_ROWS ? fusion_fits(M, square_sums, n_parts, resid) : !square_sums && !resid;
+}
+
+// x [M, K], w [N, K], y [M, N], bias [N] or nullptr, all float32; M <= 16, K a multiple of 4, x and w at multiples of 16 bytes.  square_sums [M, n_parts]
+// (or nullptr): the row scale, as lsa_gemm_skinny takes it, for M <= 8.
+LSA_EXPORT int lsa_gemm_few_f32(const float* x, const float* w, float* y, int M, int N, int K, const float* bias, const float* square_sums, int n_parts,
+                                float eps, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K < 4 || K % 4 != 0 || ((reinterpret_cast<size_t>(x) | reinterpret_cast<size_t>(w)) & 15)) return -1;
-    // rows of W a workgroup: 16 where every compute unit gets them, else 8 or 4 (1,024 x 2,048: 7.3, 5.9 and 5.7 us; 4,096 x 1,024: 5.5, 5.9, 9.2)
-    const int rows = N >= 4096 ? 16 : N >= 1024 ? 8 : 4;
-    gemm_few_f32_kernel<<<(N + rows - 1) / rows, GEMM_WAVES * 64, 0, stream>>>(x, w, y, M, N, K, rows, bias);
+    if (!few_f32_takes(x, w, M, K, square_sums, n_parts, nullptr)) return -1;
+    const Fusion fusion = {square_sums, n_parts, eps, nullptr, nullptr, nullptr, nullptr, nullptr, bias, 0};
+    const int rows = few_f32_rows(N);
+    gemm_few_f32_kernel<false><<<(N + rows - 1) / rows, GEMM_WAVES * 64, 0, stream>>>(x, w, y, M, N, K, rows, fusion);
+    LSA_LAUNCH_CHECK();
+}
+
+// hidden [M, I] = silu(x . gate^T) * (x . up^T), w [2 I, K] with the gate rows first; M <= 8.
+LSA_EXPORT int lsa_gemm_few_f32_gated(const float* x, const float* w, float* hidden, int M, int I, int K, const float* square_sums, int n_parts, float eps,
+                                      hipStream_t stream) {
+    if (M <= 0 || I <= 0) return 0;
+    if (M > F32_FUSED_ROWS || !few_f32_takes(x, w, M, K, square_sums, n_parts, nullptr)) return -1;
+    const Fusion fusion = {square_sums, n_parts, eps, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
+    const int pairs = few_f32_rows(2 * I) / 2;
+    gemm_few_f32_kernel<true><<<(I + pairs - 1) / pairs, GEMM_WAVES * 64, 0, stream>>>(x, w, hidden, M, 2 * I, K, pairs, fusion);
+    LSA_LAUNCH_CHECK();
+}
+
+// Partial sums per row that lsa_gemm_few_f32_stream writes (the second dimension of square_sums_out).
+LSA_EXPORT int lsa_gemm_few_f32_parts(int N) { return N <= 0 ? -1 : (N + few_f32_rows(N) - 1) / few_f32_rows(N); }
+
+// resid_out = resid + x . w^T [/ rms, if square_sums], weighted_out = resid_out * norm_weight, square_sums_out [M, lsa_gemm_few_f32_parts(N)] = sums of
+// resid_out^2 over the columns of each workgroup; M <= 8.  resid_out may be resid itself.
+LSA_EXPORT int lsa_gemm_few_f32_stream(const float* x, const float* w, int M, int N, int K, const float* square_sums, int n_parts, float eps,
+                                       const float* resid, const float* norm_weight, float* resid_out, float* weighted_out, float* square_sums_out,
+                                       hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (M > F32_FUSED_ROWS || !resid || !norm_weight || !resid_out || !weighted_out || !square_sums_out
+        || !few_f32_takes(x, w, M, K, square_sums, n_parts, resid)) return -1;
+    const Fusion fusion = {square_sums, n_parts, eps, (const bf16_t*)resid, norm_weight, (bf16_t*)resid_out, (bf16_t*)weighted_out, square_sums_out, nullptr, 0};
+    const int rows = few_f32_rows(N);
+    gemm_few_f32_kernel<false><<<(N + rows - 1) / rows, GEMM_WAVES * 64, 0, stream>>>(x, w, nullptr, M, N, K, rows, fusion);
     LSA_LAUNCH_CHECK();
 }

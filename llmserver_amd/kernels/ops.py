@@ -183,13 +183,20 @@ class HipOps(KernelNamespace):
         return x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 \
             and bool(self._gemm.lsa_gemm_few_f32_fits(x.shape[0], weight.shape[0], x.shape[1]))
 
-    def _linear_few_rows_float32(self, x, weight, out=None, bias=None):
+    def _linear_few_rows_float32(self, x, weight, out=None, bias=None, row_scale=None):
         """Up to 16 rows of float32 through the stream over the weights, whatever its rule says of the sizes."""
         if out is None:
             out = torch.empty((x.shape[0], weight.shape[0]), device=x.device, dtype=torch.float32)
-        _launched(self._gemm.lsa_gemm_few_f32(_ptr(x), _ptr(weight), _ptr(out), x.shape[0], weight.shape[0], x.shape[1], _ptr(bias), _stream()),
+        sums, parts, eps = self._row_scale_args(row_scale, x.shape[0])
+        _launched(self._gemm.lsa_gemm_few_f32(_ptr(x), _ptr(weight), _ptr(out), x.shape[0], weight.shape[0], x.shape[1], _ptr(bias), sums, parts, eps, _stream()),
                   "gemm_few_f32")
         return out
+
+    FUSED_ROWS_FLOAT32 = 8      # most rows for which the 32-bit stream folds in what stands around a product
+
+    def _fuses_float32(self, x, weight, row_scale):
+        """Whether the 32-bit stream takes the product with a row scale (if there is one), a stream update or a gate in its epilogue."""
+        return x.shape[0] <= self.FUSED_ROWS_FLOAT32 and self._few_rows_float32(x, weight, None) and self._row_scale_fits(row_scale, x.shape[0])
 
     LIBRARY_MARGIN = 0.93       # the library replaces a few-row kernel only if it takes less than this share of its time
 
@@ -244,7 +251,7 @@ class HipOps(KernelNamespace):
         activation kernel after it if ``kind`` is "gated") beats the kernel of this repository that does it all;
         ``kind`` "partial": the product in partial sums and the norm kernel that adds them up, against the library's
         product and the plain norm kernel.  Looked up in the table of choices; measured only inside ``measuring()``."""
-        if not self.consult_choices:
+        if not self.consult_choices or x.dtype == torch.float32:      # (the table speaks of bfloat16)
             return False
         rows, width = x.shape
         # Beyond the few-row kernels one entry stands for eight neighbouring numbers of rows (portions of prompts
@@ -366,6 +373,8 @@ class HipOps(KernelNamespace):
 
     def row_scale_fits(self, x, weight, row_scale) -> bool:
         """Whether the few-row products take ``x`` with this ``row_scale`` (then they do not return None for it)."""
+        if x.dtype == torch.float32:
+            return x.shape[1] == weight.shape[1] and self._fuses_float32(x, weight, row_scale)
         return x.shape[1] == weight.shape[1] and self._few_rows(x, weight) and self._row_scale_fits(row_scale, x.shape[0])
 
     fuses_bias = True       # linear() and linear_few_rows() take the bias themselves
@@ -417,6 +426,13 @@ class HipOps(KernelNamespace):
         rows, width = x.shape
         if activation is not None and activation not in self.PLAIN_ACTIVATIONS:
             raise ValueError(f"the product's epilogue computes {', '.join(self.PLAIN_ACTIVATIONS)}; {activation!r} is not built")
+        if x.dtype == torch.float32 and row_scale is not None and activation is None and not rows_per_workgroup \
+                and x.shape[1] == weight.shape[1] and self._fuses_float32(x, weight, row_scale):
+            if out is not None:
+                _check(out, "out", torch.float32, (rows, weight.shape[0]))
+            if bias is not None:
+                _check(bias, "bias", torch.float32, (weight.shape[0],))
+            return self._linear_few_rows_float32(x, weight, out, bias, row_scale)
         if x.shape[1] != weight.shape[1] or not self._few_rows(x, weight) or not self._row_scale_fits(row_scale, rows) \
                 or (rows_per_workgroup > 16 and rows > 16):
             return None
@@ -530,6 +546,9 @@ class HipOps(KernelNamespace):
         ``row_scale`` of the next product takes.  None if this is no case for it (more than 16 rows, other types)."""
         rows, width = x.shape
         n = weight.shape[0]
+        if x.dtype == torch.float32 == resid.dtype and not rows_per_workgroup and x.shape[1] == weight.shape[1] \
+                and self._gemm.lsa_gemm_few_f32_parts(n) <= self.SCALE_PARTS and self._fuses_float32(x, weight, row_scale):
+            return self._linear_into_stream_float32(x, weight, resid, norm_weight, row_scale)
         if x.shape[1] != weight.shape[1] or not self._few_rows(x, weight) or rows > self.FUSED_ROWS \
                 or not self._row_scale_fits(row_scale, rows) or resid.dtype != torch.bfloat16:
             return None
@@ -549,6 +568,17 @@ class HipOps(KernelNamespace):
                   "gemm_skinny_stream")
         return stream, weighted, square_sums
 
+    def _linear_into_stream_float32(self, x, weight, resid, norm_weight, row_scale):
+        rows, n = resid.shape[0], weight.shape[0]
+        _check(resid, "resid", torch.float32, (x.shape[0], n))
+        _check(norm_weight, "norm_weight", torch.float32, (n,))
+        stream, weighted = torch.empty_like(resid), torch.empty_like(resid)
+        square_sums = torch.empty((rows, self._gemm.lsa_gemm_few_f32_parts(n)), device=x.device, dtype=torch.float32)
+        sums, parts, eps = self._row_scale_args(row_scale, rows)
+        _launched(self._gemm.lsa_gemm_few_f32_stream(_ptr(x), _ptr(weight), rows, n, x.shape[1], sums, parts, eps, _ptr(resid), _ptr(norm_weight),
+                                                     _ptr(stream), _ptr(weighted), _ptr(square_sums), _stream()), "gemm_few_f32_stream")
+        return stream, weighted, square_sums
+
     ACTIVATIONS = ("silu", "gelu_tanh")       # what the activation kernel computes (its codes are the places in this list)
     FUSED_ACTIVATIONS = ("silu",)             # ... and what the gated products' epilogues compute
 
@@ -561,6 +591,14 @@ class HipOps(KernelNamespace):
         inter = gate_up_weight.shape[0] // 2
         if activation not in self.FUSED_ACTIVATIONS:
             return None
+        if x.dtype == torch.float32:
+            if pairs_per_workgroup or gate_up_weight.shape[1] != width or gate_up_weight.shape[0] % 2 or not self._fuses_float32(x, gate_up_weight, row_scale):
+                return None
+            out = torch.empty((rows, inter), device=x.device, dtype=torch.float32)
+            sums, parts, eps = self._row_scale_args(row_scale, rows)
+            _launched(self._gemm.lsa_gemm_few_f32_gated(_ptr(x), _ptr(gate_up_weight), _ptr(out), rows, inter, width, sums, parts, eps, _stream()),
+                      "gemm_few_f32_gated")
+            return out
         if rows > self.skinny_rows:
             return self._linear_gated_beyond_few_rows(x, gate_up_weight) if row_scale is None and pairs_per_workgroup == 0 else None
         if not self._few_rows(x, gate_up_weight) or inter % 8 or gate_up_weight.shape[1] != width or rows > 16 \
