@@ -247,6 +247,40 @@ SHORT_CONTEXT = 512     # captured steps whose contexts all stay within this are
                         # a tile's four key ranges itself (no partial results in memory, no launch that merges them)
 
 
+def _shared_ranges(lengths: np.ndarray, splits: int, key_align: int, most_splits: int):
+    """Keys a range and ranges a row where rows of ``lengths`` keys share ``splits`` ranges a row, so that the longest range, which a launch of
+    about as many wavefronts as the chip holds waits for, is as short as can be; what the rows do not need goes round as empty
+    ranges, the same number in all whatever the lengths are.  33 rows of 667 to 2,000 keys (and 7 that fill them up to a captured step's 40) with
+    three ranges a row: ranges of 480 keys instead of 672, 38.0 us instead of 43.3 with the merge."""
+    total = len(lengths) * splits
+    aligned = lambda keys: -(-int(keys) // key_align) * key_align
+    shortest, longest = max(aligned(-(-lengths.sum() // total)), key_align), max(aligned(-(-lengths.max() // splits)), key_align)
+    keys = np.append(np.arange(shortest, longest, max(aligned((longest - shortest) // 32), key_align)), longest)
+    counts = np.maximum(-(-lengths[None, :] // keys[:, None]), 1)
+    fits = (counts.sum(axis=1) <= total) & (counts.max(axis=1) + splits <= most_splits)
+    best = int(np.argmax(fits))              # (the longest range of the even cut always fits)
+    counts = counts[best]
+    spare = total - int(counts.sum())
+    return int(keys[best]), counts + spare // len(lengths) + (np.arange(len(lengths)) < spare % len(lengths))
+
+
+def _shared_single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, key_align: int, most_splits: int,
+                              chunk: Optional[int]) -> AttentionPlan:
+    """As :func:`_single_token_plan` without merging in the workgroup, the ranges cut by :func:`_shared_ranges`."""
+    rows = np.arange(len(row_ctx), dtype=np.int64)
+    k_begin = first_keys(row_ctx - 1, window, chunk)
+    start = (k_begin // key_align) * key_align
+    keys, counts = _shared_ranges(row_ctx - start, splits, key_align, most_splits)
+    of_row = np.repeat(rows, counts)
+    first_slot = np.cumsum(counts) - counts
+    begin = start[of_row] + (np.arange(len(of_row)) - first_slot[of_row]) * keys
+    end = row_ctx[of_row]
+    lo = np.minimum(np.maximum(begin, k_begin[of_row]), end)
+    items = np.stack([of_row, np.zeros_like(of_row), lo, np.maximum(lo, np.minimum(begin + keys, end))], axis=1).astype(np.int32)
+    merges = np.stack([rows, np.zeros_like(rows), first_slot, counts], axis=1).astype(np.int32)
+    return AttentionPlan(items, np.arange(len(items), dtype=np.int32), merges, len(items))
+
+
 def _single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, merge_in_workgroup: int = 0,
                        key_align: int = KEY_ALIGN, chunk: Optional[int] = None) -> AttentionPlan:
     """The plan of a step in which every row brings one token and every tile gets ``splits`` key ranges: what the
@@ -335,7 +369,8 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
                          target_waves: int = TARGET_WAVES, fixed_splits: Optional[int] = None,
                          workgroup_tiles: int = 0, single_token_shortcut: bool = True, merge_in_workgroup: int = 0,
                          tuning: AttentionTuning = DEFAULT_TUNING, tile_halves: int = 1, tile_min_workgroups: int = 0,
-                         tile_key_ranges: int = 1, fixed_tiles: Optional[int] = None, chunk: Optional[int] = None) -> AttentionPlan:
+                         tile_key_ranges: int = 1, fixed_tiles: Optional[int] = None, chunk: Optional[int] = None,
+                         share_ranges: bool = False) -> AttentionPlan:
     """Cut the step's rows into tiles of tokens and, where that pays, ranges of keys.  ``window`` / ``chunk``: which keys a
     query sees (see :func:`first_keys`); a tile's keys begin at the first one that its first token sees.
 
@@ -352,7 +387,8 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
     ``fixed_tiles`` is at least the number of tiles any rows of the step's shape can have), with repetitions of the
     first tile's entries, which compute and write the same numbers once more.  ``merge_in_workgroup`` (4, or 2 in steps
     of one token per row with an even number of rows): every tile gets that many ranges, the items of a workgroup, which
-    merges them itself: no slots, no merges, no workgroups of tiles."""
+    merges them itself: no slots, no merges, no workgroups of tiles.  ``share_ranges`` (with ``fixed_splits``, in steps of one token per
+    row): the rows share that many ranges a row among them by their lengths (:func:`_shared_ranges`)."""
     _, tokens_per_tile, group_tiles = group_tiling(group_size, tuning.tile_rows)
     key_align, key_step, most_splits = tuning.key_align, tuning.key_step, tuning.most_splits
     row_len = np.asarray(row_len, dtype=np.int64)
@@ -363,6 +399,8 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
         raise ValueError("two key ranges of each of two tiles are merged in a workgroup only in steps of one token per row")
     if merge_in_workgroup not in (0, 2, WORKGROUP_RANGES) or (merge_in_workgroup == 2 and len(row_len) % 2):
         raise ValueError("a workgroup merges four key ranges of one tile, or two ranges of each of two tiles (an even number of rows)")
+    if share_ranges and single_tokens and not merge_in_workgroup and len(row_len) > 1 and 1 < int(fixed_splits or 0) <= most_splits // 2:
+        return _shared_single_token_plan(row_ctx, window, int(fixed_splits), key_align, most_splits, chunk)
     if (merge_in_workgroup or (single_token_shortcut and fixed_splits is not None)) and single_tokens:
         return _single_token_plan(row_ctx, window, int(fixed_splits or merge_in_workgroup or 1), merge_in_workgroup, key_align, chunk)
     if merge_in_workgroup:
@@ -536,7 +574,7 @@ def stage_attention_plan(ctx, key, group_size: int, n_kv_heads: int, head_dim: i
         plan = build_attention_plan(ctx.h_row_len, ctx.h_row_ctx, group_size, n_kv_heads, window,
                                     target_waves=tuning.target_waves, fixed_splits=fixed, workgroup_tiles=per_workgroup,
                                     merge_in_workgroup=in_workgroup, tuning=tuning, tile_halves=halves, tile_min_workgroups=fewest,
-                                    tile_key_ranges=key_ranges, fixed_tiles=fixed_tiles, chunk=chunk)
+                                    tile_key_ranges=key_ranges, fixed_tiles=fixed_tiles, chunk=chunk, share_ranges=True)
     ctx.set_plan(key, {
         **({"tile_slots": plan.tile_slots} if plan.tile_slots is not None else {}),
         "items": plan.items, "item_slot": plan.item_slot, "merges": plan.merges, "tiles": plan.tiles,
