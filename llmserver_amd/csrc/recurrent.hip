@@ -4,15 +4,17 @@
 // per-head norm and gate behind them.  Decays, their exponentials and logarithms, the state, the sums and the norm are float32; projections
 // arrive in the activations' type and are widened where they are read; a result for a 16-bit consumer is rounded once.
 #include "common.hpp"
+#include <type_traits>
 #include "chunks.hpp"
 
 using namespace lsa;
 
 // out[m][t] = h[t] + (before[t] - h[t]) * mu[m], before[t] = the row of the token before t in its request: a row of this
-// step, the request's state for a row's first token, zeros at position 0.  grid (tokens, blocks of 256 columns): a thread
-// has one column of one token, so its two loads are the only ones it waits for.  keep (only in steps of one token per
-// row, where a column of a row's state is one thread's): the state becomes this token's row.
-template <typename T>
+// step, the request's state for a row's first token, zeros at position 0.  grid (tokens, blocks of 256 V columns): a thread
+// has V neighbouring columns of one token (one where the width or an address is no multiple of 16 bytes), so its two loads are the only ones it waits for.  keep (only in steps of one token per
+// row, where a column of a row's state is one thread's): the state becomes this token's row.  2,048 tokens of 2,048 columns in five mixes, us: a column a
+// thread 28.9, eight 13.2.
+template <typename T, int V>
 __global__ __launch_bounds__(256) void token_shift_kernel(const T* __restrict__ h, const float* __restrict__ mu, int mixes,
                                                           float* state, long state_stride, const int* __restrict__ slots,
                                                           const int* __restrict__ token_row, const int* __restrict__ positions,
@@ -22,14 +24,36 @@ __global__ __launch_bounds__(256) void token_shift_kernel(const T* __restrict__ 
     const int row = token_row[t];
     const bool first_of_sequence = positions[t] == 0, first_of_row = t == row_start[row];
     float* mine = state + (size_t)slots[row] * state_stride;
-    for (int c = blockIdx.y * blockDim.x + threadIdx.x; c < width; c += gridDim.y * blockDim.x) {
-        const float own = (float)h[(size_t)t * width + c];
-        float before = 0.f;
-        if (!first_of_sequence) before = first_of_row ? mine[c] : (float)h[(size_t)(t - 1) * width + c];
-        const float difference = before - own;
-        for (int m = 0; m < mixes; ++m)
-            out[((size_t)m * n_tokens + t) * width + c] = (T)(own + difference * mu[(size_t)m * width + c]);
-        if (keep) mine[c] = own;
+    const int c = (blockIdx.y * blockDim.x + threadIdx.x) * V;
+    if (c >= width) return;
+    struct alignas(V * sizeof(T) >= 16 ? 16 : sizeof(T)) Few { T v[V]; };
+    struct alignas(V * sizeof(float) >= 16 ? 16 : sizeof(float)) Floats { float v[V]; };
+    const Few here = *reinterpret_cast<const Few*>(h + (size_t)t * width + c);
+    float own[V], difference[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) own[k] = (float)here.v[k];
+    if (first_of_sequence) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) difference[k] = 0.f - own[k];
+    } else if (first_of_row) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) difference[k] = mine[c + k] - own[k];
+    } else {
+        const Few last = *reinterpret_cast<const Few*>(h + (size_t)(t - 1) * width + c);
+#pragma unroll
+        for (int k = 0; k < V; ++k) difference[k] = (float)last.v[k] - own[k];
+    }
+#pragma unroll 5
+    for (int m = 0; m < mixes; ++m) {
+        const Floats share = *reinterpret_cast<const Floats*>(mu + (size_t)m * width + c);
+        Few mixed;
+#pragma unroll
+        for (int k = 0; k < V; ++k) mixed.v[k] = (T)(own[k] + difference[k] * share.v[k]);
+        *reinterpret_cast<Few*>(out + ((size_t)m * n_tokens + t) * width + c) = mixed;
+    }
+    if (keep) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) mine[c + k] = own[k];
     }
 }
 
@@ -221,6 +245,69 @@ __global__ __launch_bounds__(64) void heads_norm_gate_kernel(const float* __rest
         const float sigmoid = 1.f / (1.f + expf(-gv));
         const float xv = below ? row[j] / under : row[j];
         o[j] = (T)(xv * inv * (w ? w[j] : 1.f) * (gate_kind ? sigmoid : gv * sigmoid));
+    }
+}
+
+// The same for long steps whose rows lie at multiples of 16 bytes, heads of up to 128 C numbers: sixteen lanes a (token, head), eight neighbouring
+// numbers a lane, sixteen heads a workgroup.  With two numbers a lane what is around them takes longer than they do: 2,048 tokens of 16 heads of
+// 128 16.6 us, 10.3 so; with the read-out's denominators (2,001 tokens of 16 heads of 256) 29.7, 19.2.
+template <typename T, int C>
+__global__ __launch_bounds__(256) void heads_norm_gate_long_kernel(const float* __restrict__ x, const float* __restrict__ weight, int weight_stride,
+                                                                   float eps, const T* __restrict__ gate, long gate_stride, T* __restrict__ out,
+                                                                   int heads, int value_dim, int gate_kind, const float* __restrict__ below,
+                                                                   float floor, int pairs) {
+    const int index = (int)blockIdx.x * 16 + (threadIdx.x >> 4), first = 8 * (threadIdx.x & 15);
+    const int pair = min(index, pairs - 1), t = pair / heads, head = pair - t * heads;
+    struct alignas(16) Eight { float4 low, high; };
+    struct alignas(16) Gates { T v[8]; };
+    const float* row = x + (size_t)pair * value_dim;
+    const T* g = gate + (size_t)t * gate_stride + (size_t)head * value_dim;
+    float v[C][8];
+    Gates gates[C];
+    float sq = 0.f, under = 1.f;
+    if (below) under = fmaxf(fabsf(below[(size_t)pair * 2]), below[(size_t)pair * 2 + 1]) + floor;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int j = first + 128 * c;
+        if (j < value_dim) {
+            const Eight here = *reinterpret_cast<const Eight*>(row + j);
+            gates[c] = *reinterpret_cast<const Gates*>(g + j);
+            const float eight[8] = {here.low.x, here.low.y, here.low.z, here.low.w, here.high.x, here.high.y, here.high.z, here.high.w};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                v[c][k] = below ? eight[k] / under : eight[k];
+                sq += v[c][k] * v[c][k];
+            }
+        }
+    }
+    const auto across = [](float value, auto control) {
+        return value + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(value), decltype(control)::value, 0xf, 0xf, true));
+    };
+    sq = across(sq, std::integral_constant<int, 0xB1>());          // quad_perm [1, 0, 3, 2]
+    sq = across(sq, std::integral_constant<int, 0x4E>());          // quad_perm [2, 3, 0, 1]
+    sq = across(sq, std::integral_constant<int, 0x141>());         // row_half_mirror
+    sq = across(sq, std::integral_constant<int, 0x140>());         // row_mirror
+    if (index >= pairs) return;
+    const float inv = rsqrtf(sq / (float)value_dim + eps);
+    const float* w = weight ? weight + (size_t)head * weight_stride : nullptr;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int j = first + 128 * c;
+        if (j < value_dim) {
+            float scale[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
+            if (w) {
+                const Eight here = *reinterpret_cast<const Eight*>(w + j);
+                scale[0] = here.low.x; scale[1] = here.low.y; scale[2] = here.low.z; scale[3] = here.low.w;
+                scale[4] = here.high.x; scale[5] = here.high.y; scale[6] = here.high.z; scale[7] = here.high.w;
+            }
+            Gates result;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float gv = (float)gates[c].v[k], sigmoid = 1.f / (1.f + expf(-gv));
+                result.v[k] = (T)(v[c][k] * inv * scale[k] * (gate_kind ? sigmoid : gv * sigmoid));
+            }
+            *reinterpret_cast<Gates*>(out + (size_t)pair * value_dim + j) = result;
+        }
     }
 }
 
@@ -1304,10 +1391,14 @@ LSA_EXPORT int lsa_token_shift(int code, const void* h, const float* mu, int mix
                                int keep, hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (mixes < 1 || state == nullptr || slots == nullptr) return -1;
-    const dim3 grid(n_tokens, (width + 255) / 256);
-#define LSA_LAUNCH(T) token_shift_kernel<T><<<grid, 256, 0, stream>>>((const T*)h, mu, mixes, state, state_stride, slots, token_row, positions, \
+    const bool wide = width % 8 == 0 && ((size_t)h | (size_t)mu | (size_t)out) % 16 == 0 && (long)n_tokens * width >= 1 << 18;
+    const int columns = 256 * (!wide ? 1 : code ? 8 : 4);
+    const dim3 grid(n_tokens, (width + columns - 1) / columns);
+#define LSA_LAUNCH(T) do { if (wide) LSA_LAUNCH_OF(T, Elem<T>::kVec); else LSA_LAUNCH_OF(T, 1); } while (0)
+#define LSA_LAUNCH_OF(T, V) token_shift_kernel<T, V><<<grid, 256, 0, stream>>>((const T*)h, mu, mixes, state, state_stride, slots, token_row, positions, \
         row_start, (T*)out, n_tokens, width, keep)
     if (code) LSA_LAUNCH(bf16_t); else LSA_LAUNCH(float);
+#undef LSA_LAUNCH_OF
 #undef LSA_LAUNCH
     LSA_LAUNCH_CHECK();
 }
@@ -1442,6 +1533,17 @@ LSA_EXPORT int lsa_heads_norm_gate(int code, const float* x, const float* weight
     if (gate_kind != 0 && gate_kind != 1) return -1;
     dim3 grid(n_tokens, heads);
     const int weight_stride = weight_per_channel ? value_dim : 0;
+    const long pairs = (long)n_tokens * heads;
+    if (pairs >= 4096 && pairs < 0x7fffffffL && value_dim % 8 == 0 && value_dim <= 256 && gate_stride % 8 == 0
+        && ((size_t)x | (size_t)weight | (size_t)gate | (size_t)out) % 16 == 0) {
+        const unsigned blocks = (unsigned)((pairs + 15) / 16);
+#define LSA_LONG(T, C) heads_norm_gate_long_kernel<T, C><<<blocks, 256, 0, stream>>>(x, weight, weight_stride, eps, (const T*)gate, gate_stride, (T*)out, heads, \
+        value_dim, gate_kind, below, floor, (int)pairs)
+        if (value_dim <= 128) { if (code) LSA_LONG(bf16_t, 1); else LSA_LONG(float, 1); }
+        else { if (code) LSA_LONG(bf16_t, 2); else LSA_LONG(float, 2); }
+#undef LSA_LONG
+        LSA_LAUNCH_CHECK();
+    }
     if (code) heads_norm_gate_kernel<bf16_t><<<grid, 64, 0, stream>>>(x, weight, weight_stride, eps, (const bf16_t*)gate, gate_stride, (bf16_t*)out, heads, value_dim, gate_kind, below, floor);
     else heads_norm_gate_kernel<float><<<grid, 64, 0, stream>>>(x, weight, weight_stride, eps, (const float*)gate, gate_stride, (float*)out, heads, value_dim, gate_kind, below, floor);
     LSA_LAUNCH_CHECK();

@@ -12,6 +12,7 @@
 //   neighbouring tokens (neighbouring slots of a page) coalesce: further workgroups of the same launch.
 // Norm sums, angles, cos/sin and the rotation are 32-bit; results are rounded once.
 #include "common.hpp"
+#include <type_traits>
 
 using namespace lsa;
 
@@ -283,6 +284,100 @@ __global__ __launch_bounds__(64) void qkv_prepare_kernel(const T* __restrict__ q
     }
 }
 
+// The same for long steps of heads of up to 128 numbers whose rows lie at multiples of 16 bytes: sixteen lanes a (token, head), eight neighbouring
+// dimensions a lane, and the values through LDS in tiles of 64 tokens (further workgroups of the launch).  What bounds the kernel above in such steps is instructions:
+// a wavefront finds its place and one inverse root for two numbers a lane, and every value goes out alone.  2,048 tokens of 16 heads
+// on 4 of 128, us: 29.6, 13.6 so.
+constexpr int LONG_STEP = 4 * VT_TOKENS;
+__device__ __forceinline__ float sum_of_16_lanes(float v) {
+    const auto across = [](float x, auto control) {
+        return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(control)::value, 0xf, 0xf, true));
+    };
+    v = across(v, std::integral_constant<int, 0xB1>());        // quad_perm [1, 0, 3, 2]
+    v = across(v, std::integral_constant<int, 0x4E>());        // quad_perm [2, 3, 0, 1]
+    v = across(v, std::integral_constant<int, 0x141>());       // row_half_mirror
+    return across(v, std::integral_constant<int, 0x140>());    // row_mirror
+}
+template <typename T>
+__global__ __launch_bounds__(256) void qkv_prepare_long_kernel(const T* __restrict__ qkv, long stride, T* __restrict__ keys, T* __restrict__ values,
+                                                               const int* __restrict__ table, int table_stride, const int* __restrict__ token_row,
+                                                               const int* __restrict__ positions, const float* __restrict__ q_weight,
+                                                               const float* __restrict__ k_weight, float eps, const float* __restrict__ cos_sin,
+                                                               int pairs, int page_size, int n_q, int n_kv, int dim, int value_dim, int D,
+                                                               T* __restrict__ out_q, int heads, int halves, int value_share, int n_tokens, int row_blocks) {
+    extern __shared__ unsigned char tile_bytes[];
+    if ((int)blockIdx.x >= row_blocks) {
+        constexpr int VEC = Elem<T>::kVec;
+        const int index = (int)blockIdx.x - row_blocks, token0 = index / n_kv * VT_TOKENS, kv = index % n_kv;
+        T* tile = reinterpret_cast<T*>(tile_bytes);
+        const int pitch = value_dim + VEC, pieces = value_dim / VEC;
+        const T* v = qkv + (size_t)(n_q + n_kv) * dim + (size_t)(kv / value_share) * value_dim;
+        for (int e = threadIdx.x; e < VT_TOKENS * pieces; e += 256) {
+            const int t = e / pieces, piece = e - t * pieces;
+            if (token0 + t < n_tokens) store_vec16(tile + t * pitch + piece * VEC, load_vec16(v + (size_t)(token0 + t) * stride + piece * VEC));
+        }
+        store_value_tile(tile, pitch, token0, kv, value_dim, values, table, table_stride, token_row, positions, page_size, n_kv, D, n_tokens);
+        return;
+    }
+    const int pair_index = (int)blockIdx.x * 16 + (threadIdx.x >> 4), e0 = 8 * (threadIdx.x & 15);
+    const bool active = pair_index < n_tokens * heads;
+    const int t = active ? pair_index / heads : 0, head = active ? pair_index - t * heads : 0;
+    const bool is_query = head < n_q;
+    const T* src = qkv + (size_t)t * stride + (size_t)head * dim;
+    const float* weight = is_query ? q_weight : k_weight;
+    Eight<T> own = {}, partner = {};
+    const bool mine = e0 < dim, turns = cos_sin != nullptr && e0 < 2 * pairs;
+    const int other = e0 < pairs ? e0 + pairs : e0 - pairs;               // (halves: pairs is a multiple of eight)
+    if (mine) own = load8(src + e0);
+    if (turns && halves) partner = load8(src + other);
+    float inv = 1.f;
+    if (weight) {
+        float sq = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sq += own.v[k] * own.v[k];
+        inv = rsqrtf(sum_of_16_lanes(sq) / (float)dim + eps);
+        if (mine) {
+            const Eight<float> w = load8(weight + e0);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) own.v[k] = own.v[k] * inv * w.v[k];
+        }
+        if (turns && halves) {
+            const Eight<float> w = load8(weight + other);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) partner.v[k] = partner.v[k] * inv * w.v[k];
+        }
+    }
+    if (!active) return;
+    float result[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) result[k] = own.v[k];
+    if (turns) {
+        const float* cs = cos_sin + (size_t)t * 2 * pairs;
+        if (halves) {
+            const int first = e0 < pairs ? e0 : other;
+            const Eight<float> c = load8(cs + first), s = load8(cs + pairs + first);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) result[k] = e0 < pairs ? own.v[k] * c.v[k] - partner.v[k] * s.v[k] : own.v[k] * c.v[k] + partner.v[k] * s.v[k];
+        } else {
+            const Vec16<float> c = load_vec16(cs + e0 / 2), s = load_vec16(cs + pairs + e0 / 2);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float u = own.v[2 * k], w = own.v[2 * k + 1];
+                result[2 * k] = u * c.v[k] - w * s.v[k];
+                result[2 * k + 1] = w * c.v[k] + u * s.v[k];
+            }
+        }
+    }
+    if (e0 >= D) return;
+    if (is_query) {
+        store8(out_q + ((size_t)t * n_q + head) * D + e0, result);
+        return;
+    }
+    const int position = positions[t], block = position / page_size;
+    const int page = table[(size_t)token_row[t] * table_stride + block];
+    if (page >= 0) store8(keys + (((size_t)page * n_kv + (head - n_q)) * page_size + (position - block * page_size)) * D + e0, result);
+}
+
 LSA_EXPORT int lsa_qkv_prepare(int dtype, const void* qkv, long stride, void* keys, void* values, const int* table, int table_stride,
                                const int* token_row, const int* positions, const float* q_weight, const float* k_weight, float eps,
                                const float* cos_sin, int pairs, int page_size, int n_q, int n_kv, int dim, int value_dim, int D,
@@ -290,6 +385,20 @@ LSA_EXPORT int lsa_qkv_prepare(int dtype, const void* qkv, long stride, void* ke
     if (n_tokens <= 0) return 0;
     if (value_share < 1 || n_kv % value_share) return -1;
     if (dim > D || value_dim > D || 2 * pairs > dim || page_size <= 0 || (q_weight == nullptr) != (k_weight == nullptr)) return -1;
+    // (every piece of eight numbers lies whole in a head, in what turns and in what does not, at a multiple of 16 bytes)
+    const bool pieces = dim % 8 == 0 && value_dim % 8 == 0 && D <= 128 && D % 8 == 0 && (cos_sin == nullptr || pairs % (halves ? 8 : 4) == 0) && stride % 8 == 0
+        && ((size_t)qkv | (size_t)keys | (size_t)values | (size_t)out_q | (size_t)q_weight | (size_t)k_weight | (size_t)cos_sin) % 16 == 0;
+    const int heads = write_cache ? n_q + n_kv : n_q;
+    if (pieces && n_tokens >= LONG_STEP && (long)n_tokens * heads < 0x7fffffffL && page_size % 4 == 0) {
+        const int row_blocks = (int)(((long)n_tokens * heads + 15) / 16), value_blocks = write_cache ? (n_tokens + VT_TOKENS - 1) / VT_TOKENS * n_kv : 0;
+        const size_t element = dtype ? 2 : 4, lds = write_cache ? VT_TOKENS * (value_dim + 16 / element) * element : 0;
+#define LSA_LAUNCH(T) qkv_prepare_long_kernel<T><<<row_blocks + value_blocks, 256, lds, stream>>>((const T*)qkv, stride, (T*)keys, (T*)values, table, \
+        table_stride, token_row, positions, q_weight, k_weight, eps, cos_sin, pairs, page_size, n_q, n_kv, dim, value_dim, D, (T*)out_q, heads, halves, \
+        value_share, n_tokens, row_blocks)
+        if (dtype) LSA_LAUNCH(bf16_t); else LSA_LAUNCH(float);
+#undef LSA_LAUNCH
+        LSA_LAUNCH_CHECK();
+    }
     dim3 grid(n_tokens, n_q + n_kv);
 #define LSA_LAUNCH(T) qkv_prepare_kernel<T><<<grid, 64, 0, stream>>>((const T*)qkv, stride, (T*)keys, (T*)values, table, table_stride, token_row, \
         positions, q_weight, k_weight, eps, cos_sin, pairs, page_size, n_q, n_kv, dim, value_dim, D, (T*)out_q, write_cache, halves, value_share)
