@@ -8,41 +8,86 @@
 
 using namespace lsa;
 
-template <typename T>
-__device__ inline float row_square_sum(const T* __restrict__ row, int width, float* scratch) {
-    float sq = 0.f;
-    for (int i = threadIdx.x; i < width; i += blockDim.x) {
-        const float v = (float)row[i];
-        sq += v * v;
+// V (1 or 4) neighbouring numbers as float32, in one load where they are four.
+template <int V, typename T>
+__device__ __forceinline__ void load_few(const T* p, float (&v)[V]) {
+    struct alignas(V * sizeof(T)) Few { T v[V]; };
+    const Few few = *reinterpret_cast<const Few*>(p);
+#pragma unroll
+    for (int k = 0; k < V; ++k) v[k] = (float)few.v[k];
+}
+template <int V, typename T>
+__device__ __forceinline__ void store_few(T* p, const float (&v)[V]) {
+    struct alignas(V * sizeof(T)) Few { T v[V]; } few;
+#pragma unroll
+    for (int k = 0; k < V; ++k) few.v[k] = (T)v[k];
+    *reinterpret_cast<Few*>(p) = few;
+}
+// Whether rows of `width` numbers may be taken four at a time: they and everything else that is read or written so lie at multiples of 16 bytes
+// (8 where the numbers are of 16 bits: the caller passes those addresses doubled).
+static bool in_fours(int width, size_t addresses) { return width % 4 == 0 && width >= 4 && addresses % 16 == 0; }
+static size_t place_of(const void* p, int code) { return (size_t)p * (code ? 2 : 1); }
+
+// A row times one over its root mean square times weights: a thread's first ROW_CACHE pieces of V numbers and their weights are asked for
+// together (of places that are there, so that no load stands under a condition) and stay in registers between the two passes.  In steps of a few rows these
+// trips to memory are all there is: one row of 2,048 3.9 us, one number a load and the row read twice, 2.3 so.
+constexpr int ROW_CACHE = 4;
+template <int V, typename T, typename O>
+__device__ __forceinline__ void normed_row(const T* __restrict__ row, bool there, const float* __restrict__ weight, float eps, O* __restrict__ out, int width) {
+    __shared__ float scratch[16];
+    const int stride = 256 * V;
+    float kept[ROW_CACHE][V], weights[ROW_CACHE][V], sq = 0.f;
+#pragma unroll
+    for (int k = 0; k < ROW_CACHE; ++k) {
+        const int at = min((int)threadIdx.x * V + k * stride, width - V);
+        load_few(row + at, kept[k]);
+        load_few(weight + at, weights[k]);
     }
-    return block_sum(sq, scratch);
+#pragma unroll
+    for (int k = 0; k < ROW_CACHE; ++k)
+#pragma unroll
+        for (int v = 0; v < V; ++v) sq += (int)threadIdx.x * V + k * stride < width ? kept[k][v] * kept[k][v] : 0.f;
+    for (int i = threadIdx.x * V + ROW_CACHE * stride; i < width; i += stride) {
+        float more[V];
+        load_few(row + i, more);
+#pragma unroll
+        for (int v = 0; v < V; ++v) sq += more[v] * more[v];
+    }
+    const float total = block_sum(sq, scratch), inv = there ? rsqrtf(total / (float)width + eps) : 0.f;
+#pragma unroll
+    for (int k = 0; k < ROW_CACHE; ++k) {
+        const int i = threadIdx.x * V + k * stride;
+        if (i >= width) continue;
+#pragma unroll
+        for (int v = 0; v < V; ++v) kept[k][v] = kept[k][v] * inv * weights[k][v];
+        store_few(out + i, kept[k]);
+    }
+    for (int i = threadIdx.x * V + ROW_CACHE * stride; i < width; i += stride) {
+        float more[V], w[V];
+        load_few(row + i, more);
+        load_few(weight + i, w);
+#pragma unroll
+        for (int v = 0; v < V; ++v) more[v] = more[v] * inv * w[v];
+        store_few(out + i, more);
+    }
 }
 
 // out[t] = table[ids[t]] * rsqrt(mean(.^2) + eps) * weight.  An id outside the table gives a zero row (the host
 // refuses such ids before the launch).
-template <typename T>
+template <typename T, int V>
 __global__ __launch_bounds__(256) void embedding_norm_kernel(const T* __restrict__ table, const int* __restrict__ ids,
                                                              const float* __restrict__ weight, float eps, float* __restrict__ out,
                                                              int width, int vocab) {
-    __shared__ float scratch[16];
     const int id = ids[blockIdx.x];
     const bool ok = id >= 0 && id < vocab;
-    const T* row = table + (size_t)(ok ? id : 0) * width;
-    const float sq = row_square_sum(row, width, scratch);
-    const float inv = ok ? rsqrtf(sq / (float)width + eps) : 0.f;
-    float* o = out + (size_t)blockIdx.x * width;
-    for (int i = threadIdx.x; i < width; i += blockDim.x) o[i] = (float)row[i] * inv * weight[i];
+    normed_row<V>(table + (size_t)(ok ? id : 0) * width, ok, weight, eps, out + (size_t)blockIdx.x * width, width);
 }
 
 // out[i] = x[rows[i]] * rsqrt(mean(.^2) + eps) * weight (rows == nullptr: every row).
-template <typename O>
+template <typename O, int V>
 __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                                                         const float* __restrict__ weight, float eps, O* __restrict__ out, int width) {
-    __shared__ float scratch[16];
-    const float* row = x + (size_t)(rows ? rows[blockIdx.x] : blockIdx.x) * width;
-    const float inv = rsqrtf(row_square_sum(row, width, scratch) / (float)width + eps);
-    O* o = out + (size_t)blockIdx.x * width;
-    for (int i = threadIdx.x; i < width; i += blockDim.x) o[i] = (O)(row[i] * inv * weight[i]);
+    normed_row<V>(x + (size_t)(rows ? rows[blockIdx.x] : blockIdx.x) * width, true, weight, eps, out + (size_t)blockIdx.x * width, width);
 }
 
 // out[t] = x[t] + sum_j w[:, j] * h(position - (taps - 1 - j)), where h(p) is the input at position p of the token's
@@ -85,6 +130,51 @@ __global__ __launch_bounds__(256) void short_conv_kernel(const float* __restrict
 #pragma unroll
             for (int v = 0; v < V; ++v) mine[(size_t)(kept - 1) * width + c + v] = own[v];
         }
+    }
+}
+
+// The same for TAPS taps known when the kernel is compiled, four channels a thread, grid (tokens, blocks of 1,024 channels): what a tap reads is a row of the
+// step, a row of the state, or (before the sequence) the token's own row, which then does not count, so that all loads are asked for together;
+// with `keep` the rows that have been read are the state's new ones.  Tap by tap, each waited for and the state read again, eight tokens of 2,048
+// channels and four taps took 6.9 us, 3.2 so.
+template <typename O, int TAPS>
+__global__ __launch_bounds__(256) void short_conv_taps_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                              float* state, const int* __restrict__ slots,
+                                                              const int* __restrict__ token_row, const int* __restrict__ positions,
+                                                              const int* __restrict__ row_start, O* __restrict__ out, int width, int keep) {
+    constexpr int KEPT = TAPS - 1;
+    const int t = blockIdx.x, c = 4 * (blockIdx.y * 256 + threadIdx.x);
+    if (c >= width) return;
+    const int row = token_row[t], position = positions[t];
+    const int first = position - (t - row_start[row]);
+    float* mine = state + (size_t)slots[row] * KEPT * width + c;
+    const float* here = x + (size_t)t * width + c;
+    float own[4], before[KEPT][4], taps[4][TAPS], acc[4];
+    load_few(here, own);
+#pragma unroll
+    for (int j = 0; j < KEPT; ++j) {
+        const int place = position - (KEPT - j);
+        const float* src = place >= first ? here - (size_t)(KEPT - j) * width : place >= 0 || keep ? mine + (size_t)max(KEPT - (first - place), 0) * width : here;
+        load_few(src, before[j]);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) taps[v][j] = w[(size_t)(c + v) * TAPS + j];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = own[v];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (j == KEPT) acc[v] += taps[v][j] * own[v];
+            else if (position - (KEPT - j) >= 0) acc[v] += taps[v][j] * before[j][v];
+        }
+    store_few(out + (size_t)t * width + c, acc);
+    if (keep) {                                            // (steps of one token a row: every tap in front of the token was the state's)
+#pragma unroll
+        for (int k = 0; k + 1 < KEPT; ++k) store_few(mine + (size_t)k * width, before[k + 1]);
+        store_few(mine + (size_t)(KEPT - 1) * width, own);
     }
 }
 
@@ -140,21 +230,41 @@ __global__ __launch_bounds__(256) void scaled_norm_add_kernel(const float* __res
     for (int i = threadIdx.x * V + CACHE * stride; i < width; i += stride)
 #pragma unroll
         for (int v = 0; v < V; ++v) sq += (float)yr[i + v] * (float)yr[i + v];
-    const float inv = rsqrtf(block_sum(sq, scratch) / (float)width + eps);
-    auto finish = [&](int i, const float (&yv)[V]) {
-        float s[V], total[V];
+    // What else a piece takes, asked for before the sum of squares is waited for: the stream, the weights, the results of the layers so far.
+    struct Beside { float x[V], weight[V], scale[V], total[V]; };
+    auto beside = [&](int i) {
+        Beside b;
+        load_few(x + base + i, b.x);
+        load_few(weight + i, b.weight);
+        load_few((scale ? scale : weight) + i, b.scale);
 #pragma unroll
-        for (int v = 0; v < V; ++v) {
-            s[v] = x[base + i + v] + yv[v] * inv * weight[i + v] * (scale ? scale[i + v] : 1.f);
-            total[v] = 0.f;
-        }
+        for (int v = 0; v < V; ++v) b.total[v] = 0.f;
         if (history) {
             for (int j = 0; j < before; ++j) {
                 const float m = mix[j];
-                const float* h = history + (size_t)j * state_stride + base + i;
+                float h[V];
+                load_few(history + (size_t)j * state_stride + base + i, h);
 #pragma unroll
-                for (int v = 0; v < V; ++v) total[v] += m * h[v];
+                for (int v = 0; v < V; ++v) b.total[v] += m * h[v];
             }
+        }
+        return b;
+    };
+    Beside with[CACHE];
+#pragma unroll
+    for (int k = 0; k < CACHE; ++k) {
+        const int i = threadIdx.x * V + k * stride;
+        if (i < width) with[k] = beside(i);
+    }
+    const float inv = rsqrtf(block_sum(sq, scratch) / (float)width + eps);
+    auto finish = [&](int i, const float (&yv)[V], const Beside& b) {
+        float s[V], total[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            s[v] = b.x[v] + yv[v] * inv * b.weight[v] * (scale ? b.scale[v] : 1.f);
+            total[v] = b.total[v];
+        }
+        if (history) {
             const float m = mix[before];
 #pragma unroll
             for (int v = 0; v < V; ++v) {
@@ -171,13 +281,13 @@ __global__ __launch_bounds__(256) void scaled_norm_add_kernel(const float* __res
 #pragma unroll
     for (int k = 0; k < CACHE; ++k) {
         const int i = threadIdx.x * V + k * stride;
-        if (i < width) finish(i, kept[k]);
+        if (i < width) finish(i, kept[k], with[k]);
     }
     for (int i = threadIdx.x * V + CACHE * stride; i < width; i += stride) {
         float yv[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) yv[v] = (float)yr[i + v];
-        finish(i, yv);
+        finish(i, yv, beside(i));
     }
 }
 
@@ -313,57 +423,80 @@ __global__ __launch_bounds__(256) void stream_inject_kernel(float* __restrict__ 
 constexpr int MOST_STREAMS = 8;
 constexpr int STREAM_CACHE = 8;           // elements of a row a thread keeps between the two passes (rows of up to 2,048 are read once; sixteen gained nothing at 4,096 and cost a prompt a little)
 
+constexpr int FEW_STREAM_ROWS = 256;      // up to this many rows a row gets 1,024 threads (a workgroup a compute unit)
+
 // The kernels below take the number of streams as a template parameter: the small per-stream arrays then live in registers
 // (indexed by a run-time count they would go to scratch memory, and a row of one token would wait for that).
+// V (1 or 4) neighbouring columns a load, THREADS a row: 1,024 where the rows are few, so that a row of 4,096 columns is one piece a thread and a kernel of few
+// instructions (one number a load and 256 threads: sixteen times the instructions, which a decoding step brings in cold).  Three rows of two streams of
+// 4,096, us behind cold caches: the update 6.3, 3.7 so; the read-out 4.7, 2.9.
 // out[i] = rmsnorm(sum_s read[s] * x[s][rows[i]]) * weight (rows == nullptr: every row).
-template <typename O, int S>
-__global__ __launch_bounds__(256) void streams_read_kernel(const float* __restrict__ x, size_t stream_stride,
-                                                           const float* __restrict__ read, const int* __restrict__ rows,
-                                                           const float* __restrict__ weight, float eps, O* __restrict__ out, int width) {
+template <typename O, int S, int V, int THREADS>
+__global__ __launch_bounds__(THREADS) void streams_read_kernel(const float* __restrict__ x, size_t stream_stride,
+                                                               const float* __restrict__ read, const int* __restrict__ rows,
+                                                               const float* __restrict__ weight, float eps, O* __restrict__ out, int width) {
+    constexpr int FIT = STREAM_CACHE * 256 / (V * THREADS), PIECES = FIT > 0 ? FIT : 1, STRIDE = V * THREADS;
     __shared__ float scratch[16];
     const float* row = x + (size_t)(rows ? rows[blockIdx.x] : blockIdx.x) * width;
     float r[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) r[s] = read[s];
-    auto summed = [&](int i) {
-        float u = 0.f;
+    auto summed = [&](int i, float (&u)[V]) {
+        float from[S][V];
 #pragma unroll
-        for (int s = 0; s < S; ++s) u += r[s] * row[(size_t)s * stream_stride + i];
-        return u;
+        for (int s = 0; s < S; ++s) load_few(row + (size_t)s * stream_stride + i, from[s]);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            u[v] = 0.f;
+#pragma unroll
+            for (int s = 0; s < S; ++s) u[v] += r[s] * from[s][v];
+        }
     };
-    float kept[STREAM_CACHE], weights[STREAM_CACHE];
-    float sq = 0.f;
+    float kept[PIECES][V], weights[PIECES][V], sq = 0.f;
 #pragma unroll
-    for (int k = 0; k < STREAM_CACHE; ++k) {
-        const int i = threadIdx.x + k * 256;
-        const float u = summed(min(i, width - 1));       // (a load of a place that is there stands under no condition)
-        weights[k] = weight[min(i, width - 1)];          // (asked for now: behind the sum of squares nothing waits for memory)
-        kept[k] = i < width ? u : 0.f;
-        sq += kept[k] * kept[k];
+    for (int k = 0; k < PIECES; ++k) {
+        const int i = threadIdx.x * V + k * STRIDE, at = min(i, width - V);      // (a load of a place that is there stands under no condition)
+        summed(at, kept[k]);
+        load_few(weight + at, weights[k]);               // (asked for now: behind the sum of squares nothing waits for memory)
+#pragma unroll
+        for (int v = 0; v < V; ++v) sq += i < width ? kept[k][v] * kept[k][v] : 0.f;
     }
-    for (int i = threadIdx.x + STREAM_CACHE * 256; i < width; i += 256) {
-        const float u = summed(i);
-        sq += u * u;
+    for (int i = threadIdx.x * V + PIECES * STRIDE; i < width; i += STRIDE) {
+        float u[V];
+        summed(i, u);
+#pragma unroll
+        for (int v = 0; v < V; ++v) sq += u[v] * u[v];
     }
     const float inv = rsqrtf(block_sum(sq, scratch) / (float)width + eps);
     O* o = out + (size_t)blockIdx.x * width;
+    auto normed = [&](int i, float (&u)[V], const float (&w)[V]) {
 #pragma unroll
-    for (int k = 0; k < STREAM_CACHE; ++k) {
-        const int i = threadIdx.x + k * 256;
-        if (i < width) o[i] = (O)(kept[k] * inv * weights[k]);
+        for (int v = 0; v < V; ++v) u[v] = u[v] * inv * w[v];
+        store_few(o + i, u);
+    };
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) {
+        const int i = threadIdx.x * V + k * STRIDE;
+        if (i < width) normed(i, kept[k], weights[k]);
     }
-    for (int i = threadIdx.x + STREAM_CACHE * 256; i < width; i += 256) o[i] = (O)(summed(i) * inv * weight[i]);
+    for (int i = threadIdx.x * V + PIECES * STRIDE; i < width; i += STRIDE) {
+        float u[V], w[V];
+        summed(i, u);
+        load_few(weight + i, w);
+        normed(i, u, w);
+    }
 }
 
 // Every new stream from the streams as they stood before the update, stored where they lie: x[t] <- sum_s mix[s][t] * x[s] + write[t] * y, and, where next_read
 // is given, normed = rmsnorm(sum_t next_read[t] * x[t]) * next_weight: what the next sublayer reads, in the same pass (the
 // row of sums stays in registers between the two passes; wider rows are formed again from the streams just written, by the
 // thread that wrote them).  One workgroup a token row.
-template <typename Y, typename R, int S>
-__global__ __launch_bounds__(256) void streams_update_kernel(float* __restrict__ x, size_t stream_stride, const Y* __restrict__ y,
-                                                             const float* __restrict__ mix, const float* __restrict__ write,
-                                                             const float* __restrict__ next_read, const float* __restrict__ next_weight,
-                                                             float next_eps, R* __restrict__ normed, int width) {
+template <typename Y, typename R, int S, int V, int THREADS>
+__global__ __launch_bounds__(THREADS) void streams_update_kernel(float* __restrict__ x, size_t stream_stride, const Y* __restrict__ y,
+                                                                 const float* __restrict__ mix, const float* __restrict__ write,
+                                                                 const float* __restrict__ next_read, const float* __restrict__ next_weight,
+                                                                 float next_eps, R* __restrict__ normed, int width) {
+    constexpr int FIT = STREAM_CACHE * 256 / (V * THREADS), PIECES = FIT > 0 ? FIT : 1, STRIDE = V * THREADS;
     __shared__ float scratch[16];
     float m[S][S], w[S], r[S];
 #pragma unroll
@@ -375,72 +508,80 @@ __global__ __launch_bounds__(256) void streams_update_kernel(float* __restrict__
     }
     float* row = x + (size_t)blockIdx.x * width;
     const Y* yr = y + (size_t)blockIdx.x * width;
-    // one column of all streams: the new streams are written, what the next sublayer reads of them is returned
-    auto updated = [&](int i) {
-        float old[S];
+    struct Columns { float old[S][V], update[V]; };
+    auto load = [&](int i) {
+        Columns c;
 #pragma unroll
-        for (int s = 0; s < S; ++s) old[s] = row[(size_t)s * stream_stride + i];
-        const float update = (float)yr[i];
-        float u = 0.f;
+        for (int s = 0; s < S; ++s) load_few(row + (size_t)s * stream_stride + i, c.old[s]);
+        load_few(yr + i, c.update);
+        return c;
+    };
+    // the new streams are written, what the next sublayer reads of them is returned
+    auto updated = [&](int i, const Columns& c, float (&u)[V]) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) u[v] = 0.f;
 #pragma unroll
         for (int t = 0; t < S; ++t) {
-            float fresh = 0.f;
+            float fresh[V];
 #pragma unroll
-            for (int s = 0; s < S; ++s) fresh += m[s][t] * old[s];
-            fresh += w[t] * update;
-            row[(size_t)t * stream_stride + i] = fresh;
-            u += r[t] * fresh;
+            for (int v = 0; v < V; ++v) {
+                fresh[v] = 0.f;
+#pragma unroll
+                for (int s = 0; s < S; ++s) fresh[v] += m[s][t] * c.old[s][v];
+                fresh[v] += w[t] * c.update[v];
+                u[v] += r[t] * fresh[v];
+            }
+            store_few(row + (size_t)t * stream_stride + i, fresh);
         }
-        return u;
     };
-    // the first STREAM_CACHE columns of a thread: every load is issued before the first store (a store to the streams would
+    // the first PIECES of a thread: every load is issued before the first store (a store to the streams would
     // otherwise hold back the loads behind it, and a row of one token would wait for memory once a column), and every load
     // is of a place that is there, so that none stands under a condition
-    float kept[STREAM_CACHE], olds[STREAM_CACHE][S], updates[STREAM_CACHE], weights[STREAM_CACHE];
-    float sq = 0.f;
+    float kept[PIECES][V], weights[PIECES][V], sq = 0.f;
+    Columns columns[PIECES];
 #pragma unroll
-    for (int k = 0; k < STREAM_CACHE; ++k) {
-        const int i = min((int)threadIdx.x + k * 256, width - 1);
-#pragma unroll
-        for (int s = 0; s < S; ++s) olds[k][s] = row[(size_t)s * stream_stride + i];
-        updates[k] = (float)yr[i];
-        weights[k] = next_read ? next_weight[i] : 0.f;    // (asked for now: behind the sum of squares nothing waits for memory)
+    for (int k = 0; k < PIECES; ++k) {
+        const int at = min((int)threadIdx.x * V + k * STRIDE, width - V);
+        columns[k] = load(at);
+        load_few((next_read ? next_weight : row) + at, weights[k]);    // (asked for now: behind the sum of squares nothing waits for memory)
     }
 #pragma unroll
-    for (int k = 0; k < STREAM_CACHE; ++k) {
-        const int i = threadIdx.x + k * 256;
-        float u = 0.f;
-        if (i < width) {
+    for (int k = 0; k < PIECES; ++k) {
+        const int i = threadIdx.x * V + k * STRIDE;
+        if (i >= width) continue;
+        updated(i, columns[k], kept[k]);
 #pragma unroll
-            for (int t = 0; t < S; ++t) {
-                float fresh = 0.f;
-#pragma unroll
-                for (int s = 0; s < S; ++s) fresh += m[s][t] * olds[k][s];
-                fresh += w[t] * updates[k];
-                row[(size_t)t * stream_stride + i] = fresh;
-                u += r[t] * fresh;
-            }
-        }
-        kept[k] = u;
-        sq += u * u;
+        for (int v = 0; v < V; ++v) sq += kept[k][v] * kept[k][v];
     }
-    for (int i = threadIdx.x + STREAM_CACHE * 256; i < width; i += 256) {
-        const float u = updated(i);
-        sq += u * u;
+    for (int i = threadIdx.x * V + PIECES * STRIDE; i < width; i += STRIDE) {
+        float u[V];
+        updated(i, load(i), u);
+#pragma unroll
+        for (int v = 0; v < V; ++v) sq += u[v] * u[v];
     }
     if (!next_read) return;                              // (the whole workgroup)
     const float inv = rsqrtf(block_sum(sq, scratch) / (float)width + next_eps);
     R* o = normed + (size_t)blockIdx.x * width;
 #pragma unroll
-    for (int k = 0; k < STREAM_CACHE; ++k) {
-        const int i = threadIdx.x + k * 256;
-        if (i < width) o[i] = (R)(kept[k] * inv * weights[k]);
-    }
-    for (int i = threadIdx.x + STREAM_CACHE * 256; i < width; i += 256) {
-        float u = 0.f;
+    for (int k = 0; k < PIECES; ++k) {
+        const int i = threadIdx.x * V + k * STRIDE;
+        if (i >= width) continue;
 #pragma unroll
-        for (int t = 0; t < S; ++t) u += r[t] * row[(size_t)t * stream_stride + i];
-        o[i] = (R)(u * inv * next_weight[i]);
+        for (int v = 0; v < V; ++v) kept[k][v] = kept[k][v] * inv * weights[k][v];
+        store_few(o + i, kept[k]);
+    }
+    for (int i = threadIdx.x * V + PIECES * STRIDE; i < width; i += STRIDE) {
+        const Columns c = load(i);                       // (the new streams)
+        float u[V], w_next[V];
+        load_few(next_weight + i, w_next);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            u[v] = 0.f;
+#pragma unroll
+            for (int s = 0; s < S; ++s) u[v] += r[s] * c.old[s][v];
+            u[v] = u[v] * inv * w_next[v];
+        }
+        store_few(o + i, u);
     }
 }
 
@@ -550,12 +691,15 @@ LSA_EXPORT int lsa_streams_read(const float* x, int streams, int n_tokens, const
     if (n_out <= 0) return 0;
     if (streams < 1 || streams > MOST_STREAMS) return -1;
     const size_t stream_stride = (size_t)n_tokens * width;
-#define LSA_LAUNCH(O, S) streams_read_kernel<O, S><<<n_out, 256, 0, stream>>>(x, stream_stride, read, rows, weight, eps, (O*)out, width)
+    const bool fours = in_fours(width, (size_t)x | (size_t)weight | place_of(out, out_code)), few = n_out <= FEW_STREAM_ROWS && width > 1024;
+#define LSA_LAUNCH(O, S) do { if (fours && few) LSA_LAUNCH_V(O, S, 4, 1024); else if (fours) LSA_LAUNCH_V(O, S, 4, 256); else LSA_LAUNCH_V(O, S, 1, 256); } while (0)
+#define LSA_LAUNCH_V(O, S, V, T) streams_read_kernel<O, S, V, T><<<n_out, T, 0, stream>>>(x, stream_stride, read, rows, weight, eps, (O*)out, width)
 #define LSA_BY_STREAMS(O) switch (streams) { case 1: LSA_LAUNCH(O, 1); break; case 2: LSA_LAUNCH(O, 2); break; case 3: LSA_LAUNCH(O, 3); break; \
         case 4: LSA_LAUNCH(O, 4); break; case 5: LSA_LAUNCH(O, 5); break; case 6: LSA_LAUNCH(O, 6); break; case 7: LSA_LAUNCH(O, 7); break; \
         default: LSA_LAUNCH(O, 8); }
     if (out_code) LSA_BY_STREAMS(bf16_t) else LSA_BY_STREAMS(float)
 #undef LSA_BY_STREAMS
+#undef LSA_LAUNCH_V
 #undef LSA_LAUNCH
     LSA_LAUNCH_CHECK();
 }
@@ -566,7 +710,11 @@ LSA_EXPORT int lsa_streams_update(float* x, int streams, int n_tokens, const voi
     if (n_tokens <= 0) return 0;
     if (streams < 1 || streams > MOST_STREAMS || (next_read != nullptr && (normed == nullptr || next_weight == nullptr))) return -1;
     const size_t stream_stride = (size_t)n_tokens * width;
-#define LSA_LAUNCH_S(Y, R, S) streams_update_kernel<Y, R, S><<<n_tokens, 256, 0, stream>>>(x, stream_stride, (const Y*)y, mix, write, next_read, \
+    const bool fours = in_fours(width, (size_t)x | (size_t)next_weight | place_of(y, y_code) | place_of(normed, normed_code));
+    const bool few = n_tokens <= FEW_STREAM_ROWS && width > 1024;
+#define LSA_LAUNCH_S(Y, R, S) do { if (fours && few) LSA_LAUNCH_V(Y, R, S, 4, 1024); else if (fours) LSA_LAUNCH_V(Y, R, S, 4, 256); \
+        else LSA_LAUNCH_V(Y, R, S, 1, 256); } while (0)
+#define LSA_LAUNCH_V(Y, R, S, V, T) streams_update_kernel<Y, R, S, V, T><<<n_tokens, T, 0, stream>>>(x, stream_stride, (const Y*)y, mix, write, next_read, \
                                                                                           next_weight, next_eps, (R*)normed, width)
 #define LSA_LAUNCH(Y, R) switch (streams) { case 1: LSA_LAUNCH_S(Y, R, 1); break; case 2: LSA_LAUNCH_S(Y, R, 2); break; case 3: LSA_LAUNCH_S(Y, R, 3); break; \
         case 4: LSA_LAUNCH_S(Y, R, 4); break; case 5: LSA_LAUNCH_S(Y, R, 5); break; case 6: LSA_LAUNCH_S(Y, R, 6); break; \
@@ -576,6 +724,7 @@ LSA_EXPORT int lsa_streams_update(float* x, int streams, int n_tokens, const voi
     else if (normed_code) LSA_LAUNCH(float, bf16_t)
     else LSA_LAUNCH(float, float)
 #undef LSA_LAUNCH
+#undef LSA_LAUNCH_V
 #undef LSA_LAUNCH_S
     LSA_LAUNCH_CHECK();
 }
@@ -600,16 +749,24 @@ LSA_EXPORT int lsa_norm_add_norm(const float* x, const void* y, const void* y2, 
 LSA_EXPORT int lsa_embedding_norm(int table_code, const void* table, const int* ids, const float* weight, float eps, float* out,
                                   int n, int width, int vocab, hipStream_t stream) {
     if (n <= 0) return 0;
-    if (table_code) embedding_norm_kernel<bf16_t><<<n, 256, 0, stream>>>((const bf16_t*)table, ids, weight, eps, out, width, vocab);
-    else embedding_norm_kernel<float><<<n, 256, 0, stream>>>((const float*)table, ids, weight, eps, out, width, vocab);
+    const bool fours = in_fours(width, place_of(table, table_code) | (size_t)weight | (size_t)out);
+#define LSA_LAUNCH(T) do { if (fours) LSA_LAUNCH_V(T, 4); else LSA_LAUNCH_V(T, 1); } while (0)
+#define LSA_LAUNCH_V(T, V) embedding_norm_kernel<T, V><<<n, 256, 0, stream>>>((const T*)table, ids, weight, eps, out, width, vocab)
+    if (table_code) LSA_LAUNCH(bf16_t); else LSA_LAUNCH(float);
+#undef LSA_LAUNCH_V
+#undef LSA_LAUNCH
     LSA_LAUNCH_CHECK();
 }
 
 LSA_EXPORT int lsa_norm_rows(const float* x, const int* rows, const float* weight, float eps, void* out, int out_code, int n_out,
                              int width, hipStream_t stream) {
     if (n_out <= 0) return 0;
-    if (out_code) norm_rows_kernel<bf16_t><<<n_out, 256, 0, stream>>>(x, rows, weight, eps, (bf16_t*)out, width);
-    else norm_rows_kernel<float><<<n_out, 256, 0, stream>>>(x, rows, weight, eps, (float*)out, width);
+    const bool fours = in_fours(width, (size_t)x | (size_t)weight | place_of(out, out_code));
+#define LSA_LAUNCH(O) do { if (fours) LSA_LAUNCH_V(O, 4); else LSA_LAUNCH_V(O, 1); } while (0)
+#define LSA_LAUNCH_V(O, V) norm_rows_kernel<O, V><<<n_out, 256, 0, stream>>>(x, rows, weight, eps, (O*)out, width)
+    if (out_code) LSA_LAUNCH(bf16_t); else LSA_LAUNCH(float);
+#undef LSA_LAUNCH_V
+#undef LSA_LAUNCH
     LSA_LAUNCH_CHECK();
 }
 
@@ -619,6 +776,16 @@ LSA_EXPORT int lsa_short_conv(const float* x, const float* w, int taps, float* s
     if (n <= 0) return 0;
     if (taps < 1 || (taps > 1 && (state == nullptr || slots == nullptr))) return -1;
 #define LSA_LAUNCH(O, V) short_conv_kernel<O, V><<<n, 256, 0, stream>>>(x, w, taps, state, slots, token_row, positions, row_start, (O*)out, width, keep)
+    const bool fours = in_fours(width, (size_t)x | (size_t)state | place_of(out, out_code));
+    if (fours && taps >= 2 && taps <= 4) {
+        const dim3 grid(n, (width + 1023) / 1024);
+#define LSA_TAPS(O, TAPS) short_conv_taps_kernel<O, TAPS><<<grid, 256, 0, stream>>>(x, w, state, slots, token_row, positions, row_start, (O*)out, width, keep)
+        if (taps == 2) { if (out_code) LSA_TAPS(bf16_t, 2); else LSA_TAPS(float, 2); }
+        else if (taps == 3) { if (out_code) LSA_TAPS(bf16_t, 3); else LSA_TAPS(float, 3); }
+        else { if (out_code) LSA_TAPS(bf16_t, 4); else LSA_TAPS(float, 4); }
+#undef LSA_TAPS
+        LSA_LAUNCH_CHECK();
+    }
     if (width % 4 == 0) { if (out_code) LSA_LAUNCH(bf16_t, 4); else LSA_LAUNCH(float, 4); }
     else { if (out_code) LSA_LAUNCH(bf16_t, 1); else LSA_LAUNCH(float, 1); }
 #undef LSA_LAUNCH
@@ -651,9 +818,11 @@ LSA_EXPORT int lsa_scaled_norm_add(const float* x, const void* y, int y_code, co
                                    const float* mix, int n, int width, hipStream_t stream) {
     if (n <= 0) return 0;
     if (history != nullptr && (mix == nullptr || before < 0)) return -1;
+    const bool fours = in_fours(width, (size_t)x | place_of(y, y_code) | (size_t)weight | (size_t)scale | (size_t)out | place_of(rounded, rounded_code)
+                                | (size_t)history | (history != nullptr ? (size_t)state_stride * 4 : 0));
 #define LSA_LAUNCH_V(Y, R, V) scaled_norm_add_kernel<Y, R, V><<<n, 256, 0, stream>>>(x, (const Y*)y, weight, scale, eps, out, (R*)rounded, history, \
                                                                                   (size_t)state_stride, before, mix, width)
-#define LSA_LAUNCH(Y, R) do { if (width % 4 == 0) LSA_LAUNCH_V(Y, R, 4); else LSA_LAUNCH_V(Y, R, 1); } while (0)
+#define LSA_LAUNCH(Y, R) do { if (fours) LSA_LAUNCH_V(Y, R, 4); else LSA_LAUNCH_V(Y, R, 1); } while (0)
     if (y_code && rounded_code) LSA_LAUNCH(bf16_t, bf16_t);
     else if (y_code) LSA_LAUNCH(bf16_t, float);
     else if (rounded_code) LSA_LAUNCH(float, bf16_t);
