@@ -103,6 +103,19 @@ __global__ __launch_bounds__(64) void differential_heads_kernel(const T* __restr
     for (int j = lane; j < value_dim; j += 64) o[j] = (T)(((float)a1[j] - lam * (float)a2[j]) * inv);
 }
 
+template <int CTRL>
+__device__ inline float add_across(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+// the sum over the 16 lanes of a row of lanes; every lane gets it
+__device__ inline float sum_of_16(float v) {
+    v = add_across<0xB1>(v);        // quad_perm [1, 0, 3, 2]
+    v = add_across<0x4E>(v);        // quad_perm [2, 3, 0, 1]
+    v = add_across<0x141>(v);       // row_half_mirror
+    v = add_across<0x140>(v);       // row_mirror
+    return v;
+}
+
 // ---- the delta rule's inputs ----------------------------------------------------------------------------------------------
 // grid (tokens, 2 kv_heads + 2 heads), one wavefront.  Blocks 0 .. 2 kv_heads - 1: a query or key head: causal convolution over
 // the request's tokens per channel, silu, the head divided by sqrt(sum of squares + unit_eps), queries times q_scale.  The next
@@ -179,6 +192,114 @@ __global__ __launch_bounds__(64) void delta_prepare_kernel(const T* __restrict__
     for (int e = lane; e < size; e += 64, ++n) out[(size_t)t * channels + base + e] = held[n] * inv;
 }
 
+// The same for TAPS taps known when the kernel is compiled and heads of up to 128 channels whose rows lie at multiples of 16 bytes: sixteen lanes a (token, block),
+// eight neighbouring channels a lane.  A token whose predecessors are all rows of the step asks for those alone; any other asks for both places that
+// a tap's input can come from, all at once, and with `keep` puts the state's rows that it has read back one place on.  us, the kernel above and this one: 1,900
+// tokens of 16 + 16 + 16 heads of 128 57, 32; one token 6.4, 4.3.
+template <typename T>
+__device__ __forceinline__ void load_eight(const T* p, float (&v)[8]) {
+    constexpr int V = Elem<T>::kVec;
+#pragma unroll
+    for (int at = 0; at < 8; at += V) {
+        const Vec16<T> piece = load_vec16(p + at);
+#pragma unroll
+        for (int k = 0; k < V; ++k) v[at + k] = (float)piece.v[k];
+    }
+}
+__device__ __forceinline__ void store_eight(float* p, const float (&v)[8]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+template <typename T, int TAPS>
+__global__ __launch_bounds__(256) void delta_prepare_wide_kernel(const T* __restrict__ proj, long stride, const float* __restrict__ w,
+                                                                 float* state, long state_stride, const int* __restrict__ slots,
+                                                                 const int* __restrict__ token_row, const int* __restrict__ positions,
+                                                                 const int* __restrict__ row_start, float* __restrict__ out,
+                                                                 int kv_heads, int heads, int dim, int value_dim, float q_scale, float unit_eps, int keep,
+                                                                 const T* __restrict__ strength, long strength_stride, const void* __restrict__ decay,
+                                                                 long decay_stride, int per_channel, const float* __restrict__ decay_scale,
+                                                                 const float* __restrict__ decay_bias, float* __restrict__ out_strength,
+                                                                 float* __restrict__ out_decay, int n_tokens) {
+    constexpr int KEPT = TAPS - 1;
+    const int blocks = 2 * kv_heads + 2 * heads, index = (int)blockIdx.x * 16 + (threadIdx.x >> 4), e = 8 * (threadIdx.x & 15);
+    const bool there = index < n_tokens * blocks;
+    const int t = there ? index / blocks : 0, block = there ? index - t * blocks : 0;
+    const int keys = kv_heads * dim, channels = 2 * keys + heads * value_dim;
+    if (there && block >= 2 * kv_heads + heads) {
+        const int head = block - 2 * kv_heads - heads;
+        const float rate = expf(decay_scale[head]);
+        if (per_channel) {
+            if (e < dim) {
+                float z[8], bias[8];
+                load_eight(reinterpret_cast<const float*>(decay) + (size_t)t * decay_stride + (size_t)head * dim + e, z);
+                load_eight(decay_bias + (size_t)head * dim + e, bias);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) z[k] = expf(-rate * softplus_of(z[k] + bias[k]));
+                store_eight(out_decay + ((size_t)t * heads + head) * dim + e, z);
+            }
+        } else if (e == 0) {
+            const float z = (float)reinterpret_cast<const T*>(decay)[(size_t)t * decay_stride + head];
+            out_decay[(size_t)t * heads + head] = expf(-rate * softplus_of(z + decay_bias[head]));
+        }
+        if (e == 0) out_strength[(size_t)t * heads + head] = sigmoid_of((float)strength[(size_t)t * strength_stride + head]);
+    }
+    const bool convolves = there && block < 2 * kv_heads + heads, unit = block < 2 * kv_heads;
+    const int size = unit ? dim : value_dim;
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const int c = (unit ? block * dim : 2 * keys + (block - 2 * kv_heads) * value_dim) + e;
+    if (convolves && e < size) {
+        const int row = token_row[t], position = positions[t];
+        const int first = position - (t - row_start[row]);
+        const T* here = proj + (size_t)t * stride + c;
+        float own[8], before[KEPT][8], taps[8 * TAPS];
+        load_eight(here, own);
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k) load_eight(w + (size_t)c * TAPS + 8 * k, *reinterpret_cast<float (*)[8]>(taps + 8 * k));
+        if (position - KEPT >= first) {
+#pragma unroll
+            for (int j = 0; j < KEPT; ++j) load_eight(here - (size_t)(KEPT - j) * stride, before[j]);
+        } else {
+            float* mine = state + (size_t)slots[row] * state_stride + c;
+            float of_step[KEPT][8];
+#pragma unroll
+            for (int j = 0; j < KEPT; ++j) {
+                const int place = position - (KEPT - j);
+                load_eight(place >= first ? here - (size_t)(KEPT - j) * stride : here, of_step[j]);
+                load_eight(mine + (size_t)max(place >= first ? 0 : KEPT - (first - place), 0) * channels, before[j]);
+            }
+            if (keep) {                                    // (steps of one token a row: every tap in front of the token is the state's)
+#pragma unroll
+                for (int k = 0; k + 1 < KEPT; ++k) store_eight(mine + (size_t)k * channels, before[k + 1]);
+                store_eight(mine + (size_t)(KEPT - 1) * channels, own);
+            }
+#pragma unroll
+            for (int j = 0; j < KEPT; ++j) {
+                const int place = position - (KEPT - j);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) before[j][k] = place >= first ? of_step[j][k] : place >= 0 ? before[j][k] : 0.f;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+#pragma unroll
+            for (int j = 0; j < KEPT; ++j) acc[k] += taps[k * TAPS + j] * before[j][k];
+            acc[k] += taps[k * TAPS + KEPT] * own[k];
+            acc[k] *= sigmoid_of(acc[k]);
+        }
+    }
+    float sq = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) sq += acc[k] * acc[k];
+    sq = sum_of_16(sq);                                    // (every lane takes part)
+    if (!convolves || e >= size) return;
+    if (unit) {
+        const float inv = rsqrtf(sq + unit_eps) * (block < kv_heads ? q_scale : 1.f);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] *= inv;
+    }
+    store_eight(out + (size_t)t * channels + c, acc);
+}
+
 // After the step: state[slot][k] = input at position end - kept + k, from the step's rows where it brought that position, from
 // the old state where it did not (k + count then indexes it), zero before the sequence.  A thread owns a channel of a row
 // and goes through k upwards, so what it still has to read lies above what it has written.
@@ -215,18 +336,6 @@ constexpr int PARTS = 16;           // lanes that share a column's key channels
 constexpr int CHUNK = 16;           // tokens staged at a time
 constexpr int BLOCK_COLUMNS = 16;   // value columns a workgroup
 
-template <int CTRL>
-__device__ inline float add_across(float v) {
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
-}
-// the sum over the 16 lanes of a row of lanes; every lane gets it
-__device__ inline float sum_of_16(float v) {
-    v = add_across<0xB1>(v);        // quad_perm [1, 0, 3, 2]
-    v = add_across<0x4E>(v);        // quad_perm [2, 3, 0, 1]
-    v = add_across<0x141>(v);       // row_half_mirror
-    v = add_across<0x140>(v);       // row_mirror
-    return v;
-}
 
 // One token of a column's walk: `S` the lane's key channels of the column, `kp`, `qp`, `gp` the token's key, query and
 // decays as the lane's part reads them, `g` the head's decay where there is one a head.
@@ -921,7 +1030,22 @@ LSA_EXPORT int lsa_delta_prepare(int code, const void* proj, long stride, const 
                                  hipStream_t stream) {
     if (n <= 0) return 0;
     if (taps < 1 || dim < 1 || dim > MOST_DIM || heads < 1 || kv_heads < 1 || heads % kv_heads || (taps > 1 && (!state || !slots))) return -1;
-    dim3 grid(n, 2 * kv_heads + 2 * heads);
+    const int blocks = 2 * kv_heads + 2 * heads;
+    const bool pieces = dim % 8 == 0 && value_dim % 8 == 0 && dim <= 128 && value_dim <= 128 && stride % 8 == 0 && state_stride % 4 == 0
+        && (!per_channel || decay_stride % 4 == 0) && (long)n * blocks < 0x7fffffffL
+        && ((size_t)proj | (size_t)w | (size_t)state | (size_t)out | (per_channel ? (size_t)decay | (size_t)decay_bias | (size_t)out_decay : 0)) % 16 == 0;
+    if (pieces && taps >= 2 && taps <= 4) {
+        const unsigned workgroups = (unsigned)(((long)n * blocks + 15) / 16);
+#define LSA_LAUNCH(T, TAPS) delta_prepare_wide_kernel<T, TAPS><<<workgroups, 256, 0, stream>>>((const T*)proj, stride, w, state, state_stride, slots, token_row, \
+        positions, row_start, out, kv_heads, heads, dim, value_dim, q_scale, unit_eps, keep, (const T*)strength, strength_stride, decay, decay_stride, per_channel, \
+        decay_scale, decay_bias, out_strength, out_decay, n)
+        if (taps == 2) { if (code) LSA_LAUNCH(bf16_t, 2); else LSA_LAUNCH(float, 2); }
+        else if (taps == 3) { if (code) LSA_LAUNCH(bf16_t, 3); else LSA_LAUNCH(float, 3); }
+        else { if (code) LSA_LAUNCH(bf16_t, 4); else LSA_LAUNCH(float, 4); }
+#undef LSA_LAUNCH
+        LSA_LAUNCH_CHECK();
+    }
+    dim3 grid(n, blocks);
 #define LSA_LAUNCH(T) delta_prepare_kernel<T><<<grid, 64, 0, stream>>>((const T*)proj, stride, w, taps, state, state_stride, slots, token_row, positions, \
         row_start, out, kv_heads, heads, dim, value_dim, q_scale, unit_eps, keep, (const T*)strength, strength_stride, decay, decay_stride, \
         per_channel, decay_scale, decay_bias, out_strength, out_decay)

@@ -248,11 +248,11 @@ __global__ __launch_bounds__(64) void heads_norm_gate_kernel(const float* __rest
     }
 }
 
-// The same for long steps whose rows lie at multiples of 16 bytes, heads of up to 128 C numbers: sixteen lanes a (token, head), eight neighbouring
+// The same for rows at multiples of 16 bytes and heads of up to 128 C numbers: sixteen lanes a (token, head), eight neighbouring
 // numbers a lane, sixteen heads a workgroup.  With two numbers a lane what is around them takes longer than they do: 2,048 tokens of 16 heads of
-// 128 16.6 us, 10.3 so; with the read-out's denominators (2,001 tokens of 16 heads of 256) 29.7, 19.2.
+// 128 16.6 us, 10.3 so; with the read-out's denominators (2,001 tokens of 16 heads of 256) 29.7, 19.2; one token of 16 heads 2.9, 2.5; 32 tokens of 8 of 256 4.9, 4.0.
 template <typename T, int C>
-__global__ __launch_bounds__(256) void heads_norm_gate_long_kernel(const float* __restrict__ x, const float* __restrict__ weight, int weight_stride,
+__global__ __launch_bounds__(256) void heads_norm_gate_eights_kernel(const float* __restrict__ x, const float* __restrict__ weight, int weight_stride,
                                                                    float eps, const T* __restrict__ gate, long gate_stride, T* __restrict__ out,
                                                                    int heads, int value_dim, int gate_kind, const float* __restrict__ below,
                                                                    float floor, int pairs) {
@@ -1534,10 +1534,10 @@ LSA_EXPORT int lsa_heads_norm_gate(int code, const float* x, const float* weight
     dim3 grid(n_tokens, heads);
     const int weight_stride = weight_per_channel ? value_dim : 0;
     const long pairs = (long)n_tokens * heads;
-    if (pairs >= 4096 && pairs < 0x7fffffffL && value_dim % 8 == 0 && value_dim <= 256 && gate_stride % 8 == 0
+    if (pairs < 0x7fffffffL && value_dim % 8 == 0 && value_dim <= 256 && gate_stride % 8 == 0
         && ((size_t)x | (size_t)weight | (size_t)gate | (size_t)out) % 16 == 0) {
         const unsigned blocks = (unsigned)((pairs + 15) / 16);
-#define LSA_LONG(T, C) heads_norm_gate_long_kernel<T, C><<<blocks, 256, 0, stream>>>(x, weight, weight_stride, eps, (const T*)gate, gate_stride, (T*)out, heads, \
+#define LSA_LONG(T, C) heads_norm_gate_eights_kernel<T, C><<<blocks, 256, 0, stream>>>(x, weight, weight_stride, eps, (const T*)gate, gate_stride, (T*)out, heads, \
         value_dim, gate_kind, below, floor, (int)pairs)
         if (value_dim <= 128) { if (code) LSA_LONG(bf16_t, 1); else LSA_LONG(float, 1); }
         else { if (code) LSA_LONG(bf16_t, 2); else LSA_LONG(float, 2); }

@@ -127,3 +127,39 @@ def test_long_norm_and_gate_of_heads(ops, dtype, tokens, heads, value_dim, per_c
     for a in range(0, tokens, 100):
         run(few, a, min(a + 100, tokens))
     torch.testing.assert_close(out, few, **CLOSE[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kv_heads, heads, dim, value_dim, taps, per_channel", [(2, 4, 128, 128, 4, 0), (1, 1, 8, 16, 2, 1), (3, 3, 40, 24, 3, 1), (2, 2, 64, 128, 4, 1)])
+@pytest.mark.parametrize("rows", [[(1, 0), (1, 1), (1, 2), (1, 3), (1, 50)], [(70, 0), (1, 2), (2, 1), (5, 7)]])
+def test_inputs_of_the_delta_rule(ops, dtype, kv_heads, heads, dim, value_dim, taps, per_channel, rows):
+    """Rows at multiples of 16 bytes against the same rows elsewhere, which another kernel takes: read-outs, decays, strengths and the state."""
+    print(f"delta inputs {dtype} {kv_heads} {heads} {dim} {value_dim} {taps} {per_channel} {len(rows)}", flush=True)
+    torch.manual_seed(dim + taps)
+    tokens, keep = sum(c for c, _ in rows), int(all(c == 1 for c, _ in rows))
+    channels = 2 * kv_heads * dim + heads * value_dim
+    stride = -(-(channels + 2 * heads) // 8) * 8
+    numbers = torch.randn(tokens * stride, device="cuda").to(dtype)
+    w, old = torch.randn(channels, taps, device="cuda"), torch.randn(len(rows), (taps - 1) * channels + 4, device="cuda")
+    slots = torch.randperm(len(rows)).int().cuda()
+    start = torch.tensor([sum(c for c, _ in rows[:r]) for r in range(len(rows))], dtype=torch.int32, device="cuda")
+    token_row = torch.cat([torch.full((c,), r) for r, (c, _) in enumerate(rows)]).int().cuda()
+    positions = torch.cat([torch.arange(b, b + c) for c, b in rows]).int().cuda()
+    wide = heads * dim if per_channel else heads
+    z = torch.randn(tokens, wide, device="cuda")
+    scale, bias = torch.randn(heads, device="cuda"), torch.randn(wide, device="cuda")
+    lib, p = ops._part_library("delta"), lambda tensor: tensor.data_ptr()
+    def run(offset):
+        proj = torch.cat([numbers.new_zeros(offset), numbers])[offset:].view(tokens, stride)
+        state, out = old.clone(), torch.full((tokens, channels), float("nan"), device="cuda")
+        strengths, decays = torch.full((tokens, heads), float("nan"), device="cuda"), torch.full((tokens, wide), float("nan"), device="cuda")
+        strength = proj[:, channels:]
+        decay = z if per_channel else proj[:, channels + heads:]
+        assert lib.lsa_delta_prepare(0 if dtype == torch.float32 else 1, p(proj), stride, p(w), taps, p(state), state.stride(0), p(slots), p(token_row), p(positions), p(start),
+                                     p(out), kv_heads, heads, dim, value_dim, dim ** -0.5, 1e-6, keep, p(strength), stride, p(decay), wide if per_channel else stride,
+                                     per_channel, p(scale), p(bias), p(strengths), p(decays), tokens, torch.cuda.current_stream().cuda_stream) == 0
+        return out, strengths, decays, state
+    got, want = run(0), run(1)
+    torch.testing.assert_close(got[0], want[0], rtol=1e-5, atol=1e-5)
+    assert all(torch.equal(a, b) for a, b in zip(got[1:], want[1:])) and not torch.isnan(got[0]).any()
+    assert keep or torch.equal(got[3], old)
