@@ -395,6 +395,13 @@ class HipOps(KernelNamespace):
             return self.linear_few_rows(x, weight, out=out, out_float32=out_float32, rows_per_workgroup=rows_per_workgroup, bias=bias)
         if self._few_rows_float32(x, weight, out):
             return self._linear_few_rows_float32(x, weight, out, bias)
+        if not out_float32 and bias is None and not rows_per_workgroup and (out is None or (out.dtype == torch.bfloat16 and out.is_contiguous() and
+                out.device == x.device and tuple(out.shape) == (x.shape[0], weight.shape[0]) and not out.requires_grad and out.data_ptr() % 8 == 0)):
+            sums = self._partial_sums_to_add(x, weight)
+            if sums is not None:
+                out = torch.empty((x.shape[0], weight.shape[0]), device=x.device, dtype=torch.bfloat16) if out is None else out
+                _launched(self._elementwise.lsa_sum_parts(_ptr(sums), sums.shape[0], _ptr(out), x.shape[0], weight.shape[0], _stream()), "sum_parts")
+                return out
         if out_float32 and x.dtype != torch.float32:
             y = torch.mm(x, weight.t(), out_dtype=torch.float32)
         elif bias is not None and bias_rounded is not None and bias_rounded.dtype == x.dtype and x.dtype != torch.float32:
@@ -600,7 +607,15 @@ class HipOps(KernelNamespace):
                       "gemm_few_f32_gated")
             return out
         if rows > self.skinny_rows:
-            return self._linear_gated_beyond_few_rows(x, gate_up_weight) if row_scale is None and pairs_per_workgroup == 0 else None
+            if row_scale is not None or pairs_per_workgroup:
+                return None
+            sums = self._partial_sums_to_add(x, gate_up_weight, gated=True)
+            if sums is None:
+                return self._linear_gated_beyond_few_rows(x, gate_up_weight)
+            out = torch.empty((rows, inter), device=x.device, dtype=torch.bfloat16)
+            _launched(self._elementwise.lsa_gated_parts(_ptr(sums), sums.shape[0], _ptr(out), rows, inter, self.ACTIVATIONS.index(activation), _stream()),
+                      "gated_parts")
+            return out
         if not self._few_rows(x, gate_up_weight) or inter % 8 or gate_up_weight.shape[1] != width or rows > 16 \
                 or not self._row_scale_fits(row_scale, rows):
             return None
@@ -613,6 +628,30 @@ class HipOps(KernelNamespace):
         _launched(self._gemm.lsa_gemm_skinny_gated(_ptr(x), _ptr(gate_up_weight), _ptr(out), rows, inter, width, int(pairs_per_workgroup), sums, parts,
                                                    eps, _stream()), "gemm_skinny_gated")
         return out
+
+    SUMMED_ROWS, SUMMED_GATED_ROWS = 32, 64             # most rows, and the sizes of the weight in numbers, for which the product in partial
+    SUMMED_WEIGHT, SUMMED_GATED_WEIGHT = (1 << 22, 1 << 23), (1 << 20, 9 << 20)       # sums and the kernel that adds them up replace the library's
+
+    def _partial_sums_to_add(self, x, weight, gated=False):
+        """The product's partial sums where adding them up in a kernel behind it (with the gate's activation, which would be one anyway) is faster than
+        the library's product: 17 rows and more of a small weight, whose tiles fill a part of the chip there; else None.  us at 17, 32, 48, 64
+        rows, library and here, each with the activation's kernel where gated: 2,816 x 2,048 8.8, 8.8, 8.8, 9.2 and 7.5, 7.6, 8.6, 9.6, gated 10.9,
+        11.1, 11.2, 11.6 and 8.1, 8.1, 9.1, 9.8; 4,096 x 1,024 8.5, 8.3, 8.4, 8.8 and 7.0, 7.3, 8.0, 8.6; 4,096 x 2,048 9.0, 8.9, 9.0, 9.4 and 8.2, 8.6,
+        9.7, 10.7, gated 11.1, 11.2, 11.4, 11.8 and 8.7, 9.1, 10.1, 11.0.  Smaller ones tie (2,048 x 1,408 6.8, 7.1 and 6.9, 7.2) unless gated (9.1, 9.5
+        and 7.4, 7.8); larger ones are the library's (6,144 x 2,048 9.0, 9.1 and 9.7, 10.1, gated at 64 rows 12.2 and 12.8)."""
+        rows, width = x.shape
+        low, high = self.SUMMED_GATED_WEIGHT if gated else self.SUMMED_WEIGHT
+        if not self.skinny_rows < rows <= (self.SUMMED_GATED_ROWS if gated else self.SUMMED_ROWS) or not self.split_products or not low <= weight.numel() <= high \
+                or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or width < 1024 or width % 8 or weight.dim() != 2 or weight.shape[1] != width \
+                or weight.shape[0] % (8 if gated else 4) or x.device != weight.device or not x.is_cuda or not x.is_contiguous() or not weight.is_contiguous() \
+                or (x.data_ptr() | weight.data_ptr()) % 16 or torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+            return None
+        parts = self._gemm.lsa_gemm_split_parts(rows, weight.shape[0], width)
+        if parts < 2:
+            return None
+        sums = torch.empty((parts, rows, weight.shape[0]), device=x.device, dtype=torch.float32)
+        _launched(self._gemm.lsa_gemm_split(_ptr(x), _ptr(weight), _ptr(sums), rows, weight.shape[0], width, _stream()), "gemm_split")
+        return sums
 
     def _linear_gated_beyond_few_rows(self, x, gate_up_weight):
         """The same for 17 to 32 rows where the weight has so many rows that one workgroup can take the whole inner
