@@ -559,6 +559,102 @@ __global__ __launch_bounds__(512) void matrix_memory_kernel(const T* __restrict_
         if ((is_value || is_normaliser) && channel0 + i < dim) mine[(size_t)i * channel_stride] = S[i];
 }
 
+// The same for steps of about a token a row, where the state's way through the chip is what there is to do: sixteen lanes have 64 columns, four
+// each (16-byte loads and stores of the state), and DK channels as a wavefront above has; a token's queries, keys and values come straight into
+// registers behind the state's loads, and the read-outs' partial sums alone go through LDS.  The same sums in the same order as above.  It wants
+// value columns in fours, channels in whole DKs and 16-byte pieces at multiples of 16 bytes.
+//   us, the walk above and this, cold caches: 64 heads of 128 x 64 in bfloat16, 1 row 6.5, 5.7; 8 rows 12.2, 10.4; 32 rows (134 MB both ways) 37.1, 23.4 (5.7
+// TB/s); 128 rows 140, 100; 8 heads of 128 x 256, 32 rows 21.4, 14.8; 32 heads of 64 x 64, 3 rows 5.8, 5.0, 32 rows 12.0, 9.4; 16 of 128 x 128 in
+// float32 at 32 rows 21.6, 13.8.  The walk's workgroups hold 53 KB of LDS for tokens that are not there, three a compute unit.
+template <typename T, typename V, int DK>
+__global__ __launch_bounds__(128) void matrix_memory_single_kernel(const T* __restrict__ q, long q_stride, const T* __restrict__ k, long k_stride,
+                                         const V* __restrict__ v, long v_stride, DecayWeights weights, float q_scale,
+                                         float* state, long state_stride, const int* __restrict__ slots,
+                                         const int* __restrict__ row_start, const int* __restrict__ row_len, const int* __restrict__ row_ctx,
+                                         float* __restrict__ out, float* __restrict__ below, int heads, int dim, int value_dim, int group, int ones) {
+    struct alignas(sizeof(T) * 8 < 16 ? sizeof(T) * 8 : 16) Eight { T v[8]; };
+    struct alignas(sizeof(V) * 4) Four { V v[4]; };
+    __shared__ __align__(16) float s_o[8 * 64];
+    const int row = blockIdx.x, head = blockIdx.y, column0 = blockIdx.z * 64;
+    const int count = row_len[row], start = row_start[row], context = row_ctx[row];
+    const size_t place = (size_t)slots[row] * state_stride;
+    if (count <= 0) return;                              // (the whole workgroup)
+    const int part = threadIdx.x >> 4, parts = dim / DK, channel0 = part * DK;
+    const int column = column0 + 4 * (threadIdx.x & 15);
+    const bool is_value = column < value_dim, is_normaliser = ones && column == value_dim;
+    const bool active = part < parts && (is_value || is_normaliser);
+    float* mine = is_value ? state + place + ((size_t)head * dim + channel0) * value_dim + column
+                           : state + place + (size_t)heads * dim * value_dim + (size_t)head * dim + channel0;
+    float S[DK][4];
+#pragma unroll
+    for (int i = 0; i < DK; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) S[i][c] = 0.f;
+    if (active && context > count) {
+        if (is_value) {
+#pragma unroll
+            for (int i = 0; i < DK; ++i) {
+                const float4 s4 = *reinterpret_cast<const float4*>(mine + (size_t)i * value_dim);
+                S[i][0] = s4.x; S[i][1] = s4.y; S[i][2] = s4.z; S[i][3] = s4.w;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < DK; ++i) S[i][0] = mine[i];
+        }
+    }
+    const size_t key_column = (size_t)(head / group) * dim + channel0;
+    for (int t = 0; t < count; ++t) {
+        const size_t token = (size_t)(start + t);
+        float sums[4] = {0.f, 0.f, 0.f, 0.f};
+        if (active) {
+            Eight q8[DK / 8], k8[DK / 8];
+#pragma unroll
+            for (int i = 0; i < DK / 8; ++i) {
+                q8[i] = *reinterpret_cast<const Eight*>(q + token * q_stride + key_column + 8 * i);
+                k8[i] = *reinterpret_cast<const Eight*>(k + token * k_stride + key_column + 8 * i);
+            }
+            const float take = weights.take_of(token, head, heads), keep = weights.keep_of(token, head, heads);
+            float value[4] = {take, 0.f, 0.f, 0.f};      // (the column behind the values is one of ones)
+            if (is_value) {
+                const Four v4 = *reinterpret_cast<const Four*>(v + token * v_stride + (size_t)head * value_dim + column);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) value[c] = take * (float)v4.v[c];
+            }
+            float o[4][4] = {};
+#pragma unroll
+            for (int i = 0; i < DK; ++i) {
+                const float ki = (float)k8[i / 8].v[i % 8], qi = (float)q8[i / 8].v[i % 8] * q_scale;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    S[i][c] = __builtin_fmaf(keep, S[i][c], ki * value[c]);
+                    o[i % 4][c] = __builtin_fmaf(S[i][c], qi, o[i % 4][c]);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sums[c] = (o[0][c] + o[1][c]) + (o[2][c] + o[3][c]);
+        }
+        if (t > 0) __syncthreads();                      // the token before has been read out of LDS
+        if (part < parts) *reinterpret_cast<float4*>(s_o + part * 64 + 4 * (threadIdx.x & 15)) = make_float4(sums[0], sums[1], sums[2], sums[3]);
+        if (t + 1 == count && active) {
+            if (is_value) {
+#pragma unroll
+                for (int i = 0; i < DK; ++i) *reinterpret_cast<float4*>(mine + (size_t)i * value_dim) = make_float4(S[i][0], S[i][1], S[i][2], S[i][3]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < DK; ++i) mine[i] = S[i][0];
+            }
+        }
+        __syncthreads();
+        const int c = column0 + (int)threadIdx.x;
+        if (threadIdx.x < 64 && c < value_dim + ones) {
+            float total = 0.f;
+            for (int w = 0; w < parts; ++w) total += s_o[w * 64 + threadIdx.x];
+            if (c < value_dim) out[token * heads * value_dim + (size_t)head * value_dim + c] = total;
+            else below[(token * heads + head) * 2] = total;
+        }
+    }
+}
+
 // ---- the same recurrences in chunks -------------------------------------------------------------------------------------
 // A row's tokens of a step in chunks of 64, counted from the row's first token of the step.  With L_t the sum of log keep
 // from the chunk's first token to t, the state behind token t is e^(L_t) S_0 + sum_(j <= t) e^(L_t - L_j) take_j k_j v_j^T
@@ -1588,6 +1684,19 @@ static int run_decayed(const T* q, long q_stride, const T* k, long k_stride, con
     const size_t lds = sizeof(float) * ((size_t)2 * CHUNK * waves * dk + (size_t)CHUNK * 64 + CHUNK + (size_t)waves * CHUNK * 64);
     if (lds > (size_t)MOST_LDS) return -1;
     dim3 grid(rows, heads, (columns + 63) / 64);
+    // (items: without sums, how many tokens the step has; 0 if that is not known.)  About a token a row: see the kernel for both sides.  More
+    // tokens are what the walk stages in LDS sixteen at a time.
+    if (items > 0 && items <= rows && dk <= 16 && dim % dk == 0 && value_dim % 4 == 0 && state_stride % 4 == 0
+        && q_stride * sizeof(T) % 16 == 0 && k_stride * sizeof(T) % 16 == 0 && v_stride % 4 == 0
+        && ((size_t)state | (size_t)q | (size_t)k) % 16 == 0 && (size_t)v % (4 * sizeof(V)) == 0) {
+        const int threads = (dim / dk * 16 + 63) / 64 * 64;
+#define LSA_SINGLE(DK) \
+        matrix_memory_single_kernel<T, V, DK><<<grid, threads, 0, stream>>>(q, q_stride, k, k_stride, v, v_stride, weights, q_scale, state, state_stride, \
+            slots, row_start, row_len, row_ctx, out, below, heads, dim, value_dim, group, ones)
+        if (dk == 8) LSA_SINGLE(8); else LSA_SINGLE(16);
+#undef LSA_SINGLE
+        LSA_LAUNCH_CHECK();
+    }
 #define LSA_LAUNCH(DK) \
         matrix_memory_kernel<T, V, DK><<<grid, waves * 64, lds, stream>>>(q, q_stride, k, k_stride, v, v_stride, weights, q_scale, state, state_stride, \
             slots, row_start, row_len, row_ctx, out, below, heads, dim, value_dim, group, ones)

@@ -1714,7 +1714,7 @@ class HipOps(KernelNamespace):
         chunked form, both or neither; ``chunks`` is what :meth:`matrix_memory_chunks` said."""
         n = out.shape[0]
         rows = row_len.shape[0]
-        items = 0
+        items = n                   # (token by token: how many tokens there are)
         if (run is None) != (sums is None):
             raise ValueError("the chunked memory takes both of its scratch tensors")
         if run is not None:
@@ -1778,7 +1778,7 @@ class HipOps(KernelNamespace):
             _check(tensor, name, torch.int32, (rows,))
         if (sums is None) != (totals is None):
             raise ValueError("the chunked recurrence takes both of its scratch tensors")
-        items = 0
+        items = n                   # (token by token: how many tokens there are)
         if sums is not None:
             items = sums.shape[0]
             if items < n // self.MEMORY_CHUNK + rows:
