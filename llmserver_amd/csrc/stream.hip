@@ -31,7 +31,10 @@ static size_t place_of(const void* p, int code) { return (size_t)p * (code ? 2 :
 // A row times one over its root mean square times weights: a thread's first ROW_CACHE pieces of V numbers and their weights are asked for
 // together (of places that are there, so that no load stands under a condition) and stay in registers between the two passes.  In steps of a few rows these
 // trips to memory are all there is: one row of 2,048 3.9 us, one number a load and the row read twice, 2.3 so.
+// V is 4 for rows that one number a load would not keep whole (and where addresses allow it): us for 1 and 2,048 rows, one number and four, 256 wide
+// 2.1, 3.5 and 2.3, 4.7; 512 2.4, 4.1 and 2.3, 5.1; 1,024 2.4, 5.0 and 2.4, 5.8; 2,048 4.6, 7.9 and 2.3, 7.0; 4,096 7.9, 15.8 and 2.6, 11.0.
 constexpr int ROW_CACHE = 4;
+static bool row_in_fours(int width, size_t addresses) { return width > 256 * ROW_CACHE && in_fours(width, addresses); }
 template <int V, typename T, typename O>
 __device__ __forceinline__ void normed_row(const T* __restrict__ row, bool there, const float* __restrict__ weight, float eps, O* __restrict__ out, int width) {
     __shared__ float scratch[16];
@@ -749,7 +752,7 @@ LSA_EXPORT int lsa_norm_add_norm(const float* x, const void* y, const void* y2, 
 LSA_EXPORT int lsa_embedding_norm(int table_code, const void* table, const int* ids, const float* weight, float eps, float* out,
                                   int n, int width, int vocab, hipStream_t stream) {
     if (n <= 0) return 0;
-    const bool fours = in_fours(width, place_of(table, table_code) | (size_t)weight | (size_t)out);
+    const bool fours = row_in_fours(width, place_of(table, table_code) | (size_t)weight | (size_t)out);
 #define LSA_LAUNCH(T) do { if (fours) LSA_LAUNCH_V(T, 4); else LSA_LAUNCH_V(T, 1); } while (0)
 #define LSA_LAUNCH_V(T, V) embedding_norm_kernel<T, V><<<n, 256, 0, stream>>>((const T*)table, ids, weight, eps, out, width, vocab)
     if (table_code) LSA_LAUNCH(bf16_t); else LSA_LAUNCH(float);
@@ -761,7 +764,7 @@ LSA_EXPORT int lsa_embedding_norm(int table_code, const void* table, const int* 
 LSA_EXPORT int lsa_norm_rows(const float* x, const int* rows, const float* weight, float eps, void* out, int out_code, int n_out,
                              int width, hipStream_t stream) {
     if (n_out <= 0) return 0;
-    const bool fours = in_fours(width, (size_t)x | (size_t)weight | place_of(out, out_code));
+    const bool fours = row_in_fours(width, (size_t)x | (size_t)weight | place_of(out, out_code));
 #define LSA_LAUNCH(O) do { if (fours) LSA_LAUNCH_V(O, 4); else LSA_LAUNCH_V(O, 1); } while (0)
 #define LSA_LAUNCH_V(O, V) norm_rows_kernel<O, V><<<n_out, 256, 0, stream>>>(x, rows, weight, eps, (O*)out, width)
     if (out_code) LSA_LAUNCH(bf16_t); else LSA_LAUNCH(float);
