@@ -82,11 +82,11 @@ __device__ __forceinline__ void store_value_tile(const T* tile, int pitch, int t
             const int p = table[(size_t)token_row[token] * table_stride + block];
             if (p >= 0) place = (((long)p * n_kv + kv_head) * d) * page_size + (pos - block * page_size);
         }
-        place_of[t] = place;
-        // (a slot's number modulo four is its offset's: pages are a multiple of four slots)
-        bool first = place >= 0 && (place & 3) == 0 && t + 3 < VT_TOKENS;
-#pragma unroll
-        for (int r = 1; r < 4; ++r) first = first && place_of[min(t + r, VT_TOKENS - 1)] == place + r;
+        place_of[t] = place;                               // (read behind the barrier)
+        // The token behind this one lies behind it in its page: told from lane to lane, not through LDS, where nothing would order another lane's
+        // write in front of the read.  (A slot's number modulo four is its offset's: pages are a multiple of four slots.)
+        const unsigned long long next_behind = __ballot(__shfl_down((long long)place, 1) == place + 1 && t + 1 < VT_TOKENS);
+        const bool first = place >= 0 && (place & 3) == 0 && (next_behind >> t & 7) == 7;
         const unsigned long long firsts = __ballot(first), together = firsts | firsts << 1 | firsts << 2 | firsts << 3;
         const unsigned long long alone = __ballot(place >= 0) & ~together, below = (1ull << t) - 1;
         if (first) fours[__popcll(firsts & below)] = (unsigned char)t;
