@@ -13,6 +13,8 @@
 //   bfloat16, 16 heads on 8 of 128 dimensions, 1 row 8.5, 8.7, 13.3 against 6.3, 7.5, 12.2; 32 rows 8.4, 9.8, 17.3 against 6.3, 8.7, 15.6
 //   bfloat16, 16 heads on 1 of 256, 8 rows 9.3, 9.2, 20.8 against 6.4, 8.4, 18.4
 //   float32, 16 heads on 8 of 128, 1 row 9.6, 12.1, 21.9 against 6.4, 9.5, 19.8; 32 rows 10.4, 14.5, 30.0 against 6.9, 11.1, 26.1
+// (The host takes this kernel as long as every workgroup has a compute unit of its own, and beyond that where it stays the faster one.  float32, 16 heads
+// on 1 of 256, 16, 128, 256 and 512 keys: 11.7, 18.3, 27.2, 43.9 against 9.8, 17.0, 27.2, 48.4: the last of these contexts are a little slower.)
 // Eight wavefronts where registers and LDS allow it (up to 256 keys in one round), else four.  A thread computes one head's outputs at the end, so
 // that few of them work out the wavefronts' weights (all of them doing so: 6.9 us instead of 6.2 at 40 keys).
 #pragma once

@@ -796,9 +796,26 @@ class HipOps(KernelNamespace):
         on itself in a step in which every row brings one token."""
         return dtype == torch.bfloat16 and head_dim % 64 == 0
 
-    def single_token_fusion_fits(self, dtype, head_dim, page_size) -> bool:
-        """The same for steps whose plan says ``rows_in_order`` (one token a row, short contexts): there is a kernel of its own for them."""
-        return bool(self._attention_library(dtype, head_dim).lsa_attention_single_fits(int(page_size), 1))
+    def single_tokens_pay(self, dtype, head_dim, rows, n_q, n_kv, plain=True) -> bool:
+        """Whether steps of one token a row behind short contexts are faster in the kernel of their own (attention_single.hpp) than in the kernel for all
+        steps.  Its workgroups have eight wavefronts and a row's keys of one KV head each: as long as every one has a compute unit of its own, yes.
+        Beyond that the other kernel's smaller workgroups fill the chip better.  us, the other kernel and this one, contexts of 16, 128 and 512: bfloat16, 16
+        heads on 8 of 128, 32 rows (256 workgroups) 8.8, 10.6, 18.0 and 6.7, 9.3, 16.0; 64 rows 11.1, 13.8, 27.8 and 11.4, 16.4, 28.4; 128 rows 19.1, 23.7, 56
+        and 20.6, 29.5, 64; 64 on 8 of 64, 64 rows 7.9, 9.1, 16.9 and 8.4, 10.2, 18.2; float32, 16 on 8 of 128, 64 rows 12.6, 20.4, 53 and 12.7, 20.9, 58.
+        Forms of four wavefronts stay the better ones at heads above 128 dimensions (bfloat16, 16 on 4 of 256, 128 rows: 28, 33, 67 and 16, 24, 60)
+        and up to 96 with more than eight heads a KV head (40 on 2 of 96, 256 rows: 22.7, 24.1, 42 and 19.7, 22.9, 40), not at 128 (64 on 4, 128 rows: 11.9,
+        14.4, 28.1 and 11.1, 16.5, 29.6); so does float32 with a KV head for every head of up to 64 dimensions and ``plain`` scores (no cap, no bias by
+        distance; 8 of 64, 128 rows: 13.7, 20.8, 54 and 10.8, 17.2, 50; with a cap 13.9, 21.4, 54 and 15.0, 25.6, 62)."""
+        heads, _, tiles = group_tiling(n_q // n_kv)
+        if rows * n_kv * tiles <= self.attention_tuning_for(dtype, head_dim).target_waves // 4:
+            return True
+        return head_dim > 128 or (heads > 8 and head_dim <= 96) or (dtype == torch.float32 and plain and n_q == n_kv and head_dim <= 64)
+
+    def single_token_fusion_fits(self, dtype, head_dim, page_size, rows=1, n_q=1, n_kv=1, plain=True) -> bool:
+        """The same for steps whose plan says ``rows_in_order`` (one token a row, short contexts): there is a kernel of its own for them,
+        where that is the faster one (see :meth:`single_tokens_pay`)."""
+        return bool(self._attention_library(dtype, head_dim).lsa_attention_single_fits(int(page_size), 1)) \
+            and self.single_tokens_pay(dtype, head_dim, rows, n_q, n_kv, plain)
 
     def paged_attention(self, qkv, out, keys, values, table, row_start, row_len, row_ctx, plan, scale, window, page_size,
                         n_q, n_kv, head_dim, ctx, decode_fusion=None, sinks=None, softcap=None, chunk=None, slopes=None, gates=None):
@@ -890,7 +907,9 @@ class HipOps(KernelNamespace):
             raise ValueError("merging in the workgroup takes a plan that gives every tile four key ranges (or, in steps of one token "
                              "per row, two, with tiles in pairs) and no slots, and, with decode fusion, both norm weights and a rotation")
         lib = self._attention_library(qkv.dtype, head_dim)
-        if plan.get("rows_in_order") and merge_in_workgroup and n == rows and lib.lsa_attention_single_fits(page_size, int(fusion_mode > 0)):
+        if plan.get("rows_in_order") and merge_in_workgroup and n == rows and lib.lsa_attention_single_fits(page_size, int(fusion_mode > 0)) \
+                and (self.single_tokens_pay(qkv.dtype, head_dim, rows, n_q, n_kv, not softcap and slopes is None)
+                     or fusion_mode > 0 and not self.decode_fusion_fits(qkv.dtype, head_dim)):
             # one token a row, row i's at place i, behind short contexts: a kernel that finds its work without the plan
             _launched(lib.lsa_attention_single(
                 _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(keys), _ptr(values), _ptr(table), table.shape[1], _ptr(row_ctx), rows, float(scale),

@@ -847,7 +847,8 @@ class GQAttention(Mixer):
         plan = ctx.get_plan(self.plan_key())
         if ctx.n_tokens == ctx.n_rows and (
                 ctx.ops.decode_fusion_fits(qkv.dtype, self.head_dim) and (whole or not plan.get("merge_in_workgroup"))
-                or whole and plan.get("rows_in_order") and ctx.ops.single_token_fusion_fits(qkv.dtype, self.head_dim, cache.page_size)):
+                or whole and plan.get("rows_in_order") and ctx.ops.single_token_fusion_fits(
+                    qkv.dtype, self.head_dim, cache.page_size, ctx.n_rows, self.n_heads, self.n_kv_heads, self.softcap is None and self.slopes is None)):
             fusion = (self.q_norm_weight, self.k_norm_weight, eps, cos_sin, cache.writable)
         else:
             ctx.ops.qk_norm_rope_kv_write(

@@ -410,8 +410,9 @@ class KernelNamespace:
         """Whether ``paged_attention`` takes q/k norm, rotation and the cache write on itself in single-token steps."""
         return False
 
-    def single_token_fusion_fits(self, dtype, head_dim, page_size) -> bool:
-        """The same for steps whose plan says ``rows_in_order``: one token a row, row i's at place i, all contexts short."""
+    def single_token_fusion_fits(self, dtype, head_dim, page_size, rows=1, n_q=1, n_kv=1, plain=True) -> bool:
+        """The same for steps whose plan says ``rows_in_order``: one token a row, row i's at place i, all contexts short.  ``plain``: scores without a
+        cap or a bias by distance."""
         return False
 
     def measuring(self):
