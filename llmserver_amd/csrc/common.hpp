@@ -60,7 +60,7 @@ __device__ inline float block_sum(float v, float* scratch) {
 }
 
 // Puts 64 consecutive tokens of one KV head, staged in LDS as [VT_TOKENS][pitch] with `filled` numbers a token, into their
-// pages values[page][kv_head][:][slot], zeros for the dimensions from `filled` to d.  Four slots of one dimension go out at
+// pages values[page][kv_head][0 .. dims)[slot] (of d dimensions), zeros for the dimensions from `filled` to `dims`.  Four slots of one dimension go out at
 // a time (8 or 16 bytes) wherever four tokens are neighbours in one page from a slot that is a multiple of four on, which is the rule inside a portion; a page's
 // [d][page_size] block is contiguous, so these stores coalesce.  At least 64 threads; whoever wrote the tile need not have waited.
 // Every token's place is found once, by a thread of its own, and only then are the tokens sorted into fours and singles: a tile in which portions meet
@@ -70,7 +70,7 @@ constexpr int VT_TOKENS = 64;
 template <typename T>
 __device__ __forceinline__ void store_value_tile(const T* tile, int pitch, int token0, int kv_head, int filled, T* __restrict__ values,
                                                  const int* __restrict__ table, int table_stride, const int* __restrict__ token_row,
-                                                 const int* __restrict__ positions, int page_size, int n_kv, int d, int n_tokens) {
+                                                 const int* __restrict__ positions, int page_size, int n_kv, int d, int n_tokens, int dims) {
     __shared__ long place_of[VT_TOKENS];                   // element offset of the token's slot in `values`, or -1
     __shared__ unsigned char fours[VT_TOKENS / 4], singles[VT_TOKENS];       // first tokens of fours; tokens that go alone
     __shared__ int n_fours, n_singles;
@@ -98,7 +98,7 @@ __device__ __forceinline__ void store_value_tile(const T* tile, int pitch, int t
     }
     __syncthreads();
     const int groups = n_fours, rest = n_singles;
-    for (int e = threadIdx.x; e < (VT_TOKENS / 4) * d; e += blockDim.x) {
+    for (int e = threadIdx.x; e < (VT_TOKENS / 4) * dims; e += blockDim.x) {
         const int g = e & (VT_TOKENS / 4 - 1), i = e / (VT_TOKENS / 4);      // neighbouring threads: neighbouring groups of slots
         if (g >= groups) continue;
         const int first = fours[g];
@@ -109,10 +109,9 @@ __device__ __forceinline__ void store_value_tile(const T* tile, int pitch, int t
         if (sizeof(T) == 2) *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(four);
         else *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(four);
     }
-    for (int g = 0; g < rest; ++g) {                       // (a handful where portions meet, all of them where a page's slots are in no order)
-        const int t = singles[g];
-        T* dst = values + place_of[t];
-        for (int i = threadIdx.x; i < d; i += blockDim.x) dst[(size_t)i * page_size] = i < filled ? tile[t * pitch + i] : (T)0.f;
+    for (int e = threadIdx.x; e < rest * dims; e += blockDim.x) {        // (a handful where portions meet, all of them where a page's slots are in no order)
+        const int g = e / dims, i = e - g * dims, t = singles[g];
+        values[place_of[t] + (long)i * page_size] = i < filled ? tile[t * pitch + i] : (T)0.f;
     }
 }
 

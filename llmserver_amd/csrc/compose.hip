@@ -168,7 +168,7 @@ __device__ __forceinline__ void values_block(int index, int tiled, const Taps& c
         *reinterpret_cast<Piece<T, V>*>(tile + i * pitch + c) = piece;
     }
     store_value_tile(tile, pitch, token0, head, h.value_dim, rows.values, h.table, h.table_stride, conv.token_row, conv.positions, h.page_size, h.n_kv,
-                     h.D, rows.n_tokens);
+                     h.D, rows.n_tokens, h.D);
 }
 
 // Where a token's queries or keys go: its row of out_q, or its slot in its page (heads then lie page_size * D apart), or nullptr.

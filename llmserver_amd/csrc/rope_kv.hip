@@ -165,7 +165,7 @@ __device__ __forceinline__ void value_tiles_block(
             store_vec16(tile + t * pitch + part * VEC,
                         load_vec16(qkv + (size_t)(token0 + t) * width + (size_t)(n_q + n_kv + kv_head) * d + part * VEC));
     }
-    store_value_tile(tile, pitch, token0, kv_head, d, values, table, table_stride, token_row, positions, page_size, n_kv, d, n_tokens);
+    store_value_tile(tile, pitch, token0, kv_head, d, values, table, table_stride, token_row, positions, page_size, n_kv, d, n_tokens, d);
 }
 
 // One launch for both: the first `qk_blocks` workgroups take the (token, head) pairs of the q and k heads (and of the v
@@ -286,8 +286,10 @@ __global__ __launch_bounds__(64) void qkv_prepare_kernel(const T* __restrict__ q
 
 // The same for long steps of heads of up to 128 numbers whose rows lie at multiples of 16 bytes: sixteen lanes a (token, head), eight neighbouring
 // dimensions a lane, and the values through LDS in tiles of 64 tokens (further workgroups of the launch).  What bounds the kernel above in such steps is instructions:
-// a wavefront finds its place and one inverse root for two numbers a lane, and every value goes out alone.  2,048 tokens of 16 heads
-// on 4 of 128, us: 29.6, 13.6 so.
+// a wavefront finds its place and one inverse root for two numbers a lane, and every value goes out alone.  us, that kernel and this one, 16 heads on 4 of
+// 128 in bfloat16: 2,048 tokens of one row 24.1, 9.5; 256 6.4, 4.0; 256 rows of one token 6.8, 5.4; float32 24.8, 13.3; 6.8, 4.2; 7.1, 6.2.
+// A tile's dimensions are shared by so many workgroups that every compute unit has one: a compute unit puts a value that goes alone (all of them, in
+// rows of one token) away in 0.4 ns or so, and with a tile to a workgroup, 16 of them, the 256 rows of one token took 14.6 us, 17.0 in float32.
 constexpr int LONG_STEP = 4 * VT_TOKENS;
 __device__ __forceinline__ float sum_of_16_lanes(float v) {
     const auto across = [](float x, auto control) {
@@ -304,19 +306,23 @@ __global__ __launch_bounds__(256) void qkv_prepare_long_kernel(const T* __restri
                                                                const int* __restrict__ positions, const float* __restrict__ q_weight,
                                                                const float* __restrict__ k_weight, float eps, const float* __restrict__ cos_sin,
                                                                int pairs, int page_size, int n_q, int n_kv, int dim, int value_dim, int D,
-                                                               T* __restrict__ out_q, int heads, int halves, int value_share, int n_tokens, int row_blocks) {
+                                                               T* __restrict__ out_q, int heads, int halves, int value_share, int n_tokens, int row_blocks, int value_parts,
+                                                               int part_dims) {
     extern __shared__ unsigned char tile_bytes[];
     if ((int)blockIdx.x >= row_blocks) {
         constexpr int VEC = Elem<T>::kVec;
-        const int index = (int)blockIdx.x - row_blocks, token0 = index / n_kv * VT_TOKENS, kv = index % n_kv;
+        const int index = (int)blockIdx.x - row_blocks, part = index % value_parts, tile_of = index / value_parts;
+        const int token0 = tile_of / n_kv * VT_TOKENS, kv = tile_of % n_kv;
+        const int from = part * part_dims, dims = min(part_dims, D - from), filled = max(min(dims, value_dim - from), 0);     // (multiples of eight)
         T* tile = reinterpret_cast<T*>(tile_bytes);
-        const int pitch = value_dim + VEC, pieces = value_dim / VEC;
-        const T* v = qkv + (size_t)(n_q + n_kv) * dim + (size_t)(kv / value_share) * value_dim;
+        const int pitch = part_dims + VEC, pieces = filled / VEC;
+        const T* v = qkv + (size_t)(n_q + n_kv) * dim + (size_t)(kv / value_share) * value_dim + from;
         for (int e = threadIdx.x; e < VT_TOKENS * pieces; e += 256) {
             const int t = e / pieces, piece = e - t * pieces;
             if (token0 + t < n_tokens) store_vec16(tile + t * pitch + piece * VEC, load_vec16(v + (size_t)(token0 + t) * stride + piece * VEC));
         }
-        store_value_tile(tile, pitch, token0, kv, value_dim, values, table, table_stride, token_row, positions, page_size, n_kv, D, n_tokens);
+        store_value_tile(tile, pitch, token0, kv, filled, values + (size_t)from * page_size, table, table_stride, token_row, positions, page_size, n_kv, D,
+                         n_tokens, dims);
         return;
     }
     const int pair_index = (int)blockIdx.x * 16 + (threadIdx.x >> 4), e0 = 8 * (threadIdx.x & 15);
@@ -390,11 +396,14 @@ LSA_EXPORT int lsa_qkv_prepare(int dtype, const void* qkv, long stride, void* ke
         && ((size_t)qkv | (size_t)keys | (size_t)values | (size_t)out_q | (size_t)q_weight | (size_t)k_weight | (size_t)cos_sin) % 16 == 0;
     const int heads = write_cache ? n_q + n_kv : n_q;
     if (pieces && n_tokens >= LONG_STEP && (long)n_tokens * heads < 0x7fffffffL && page_size % 4 == 0) {
-        const int row_blocks = (int)(((long)n_tokens * heads + 15) / 16), value_blocks = write_cache ? (n_tokens + VT_TOKENS - 1) / VT_TOKENS * n_kv : 0;
-        const size_t element = dtype ? 2 : 4, lds = write_cache ? VT_TOKENS * (value_dim + 16 / element) * element : 0;
-#define LSA_LAUNCH(T) qkv_prepare_long_kernel<T><<<row_blocks + value_blocks, 256, lds, stream>>>((const T*)qkv, stride, (T*)keys, (T*)values, table, \
+        const int row_blocks = (int)(((long)n_tokens * heads + 15) / 16), tiles = write_cache ? (n_tokens + VT_TOKENS - 1) / VT_TOKENS * n_kv : 0;
+        // The dimensions of a tile of values are shared by as many workgroups as give every compute unit one.
+        const int wanted = tiles > 0 ? (256 + tiles - 1) / tiles : 1, part_dims = (D / wanted > 16 ? (D / wanted + 7) / 8 * 8 : D < 16 ? D : 16);
+        const int value_parts = (D + part_dims - 1) / part_dims;
+        const size_t element = dtype ? 2 : 4, lds = write_cache ? VT_TOKENS * (part_dims + 16 / element) * element : 0;
+#define LSA_LAUNCH(T) qkv_prepare_long_kernel<T><<<row_blocks + tiles * value_parts, 256, lds, stream>>>((const T*)qkv, stride, (T*)keys, (T*)values, table, \
         table_stride, token_row, positions, q_weight, k_weight, eps, cos_sin, pairs, page_size, n_q, n_kv, dim, value_dim, D, (T*)out_q, heads, halves, \
-        value_share, n_tokens, row_blocks)
+        value_share, n_tokens, row_blocks, value_parts, part_dims)
         if (dtype) LSA_LAUNCH(bf16_t); else LSA_LAUNCH(float);
 #undef LSA_LAUNCH
         LSA_LAUNCH_CHECK();
