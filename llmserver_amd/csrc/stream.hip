@@ -426,13 +426,15 @@ __global__ __launch_bounds__(256) void stream_inject_kernel(float* __restrict__ 
 constexpr int MOST_STREAMS = 8;
 constexpr int STREAM_CACHE = 8;           // elements of a row a thread keeps between the two passes (rows of up to 2,048 are read once; sixteen gained nothing at 4,096 and cost a prompt a little)
 
-constexpr int FEW_STREAM_ROWS = 256;      // up to this many rows a row gets 1,024 threads (a workgroup a compute unit)
+constexpr int FEW_STREAM_ROWS = 256, FEW_UPDATED_ROWS = 512;      // up to so many rows a row gets 1,024 threads: of a read-out, of an update
 
 // The kernels below take the number of streams as a template parameter: the small per-stream arrays then live in registers
 // (indexed by a run-time count they would go to scratch memory, and a row of one token would wait for that).
 // V (1 or 4) neighbouring columns a load, THREADS a row: 1,024 where the rows are few, so that a row of 4,096 columns is one piece a thread and a kernel of few
 // instructions (one number a load and 256 threads: sixteen times the instructions, which a decoding step brings in cold).  Three rows of two streams of
-// 4,096, us behind cold caches: the update 6.3, 3.7 so; the read-out 4.7, 2.9.
+// 4,096, us behind cold caches: the update 6.3, 3.7 so; the read-out 4.7, 2.9.  Where the lines lie, 256 threads and 1,024, bfloat16: read-outs of two streams of
+// 2,048, 256 rows 3.6, 3.4, 257 rows 3.3, 3.6, 1,024 rows 5.2, 6.7 (of 4,096 they are no slower at any number: 257 rows 4.8, 4.3, 1,024 rows 8.7, 8.8); updates of four streams of 2,048, 320
+// rows 7.2, 7.0, 512 rows 9.1, 8.3, 768 rows 10.5, 11.2; of two 6.1, 6.1 and 7.6, 8.1; of two of 4,096, 512 rows 9.0, 8.6, 1,024 rows 13.4, 14.6.
 // out[i] = rmsnorm(sum_s read[s] * x[s][rows[i]]) * weight (rows == nullptr: every row).
 template <typename O, int S, int V, int THREADS>
 __global__ __launch_bounds__(THREADS) void streams_read_kernel(const float* __restrict__ x, size_t stream_stride,
@@ -713,8 +715,11 @@ LSA_EXPORT int lsa_streams_update(float* x, int streams, int n_tokens, const voi
     if (n_tokens <= 0) return 0;
     if (streams < 1 || streams > MOST_STREAMS || (next_read != nullptr && (normed == nullptr || next_weight == nullptr))) return -1;
     const size_t stream_stride = (size_t)n_tokens * width;
-    const bool fours = in_fours(width, (size_t)x | (size_t)next_weight | place_of(y, y_code) | place_of(normed, normed_code));
-    const bool few = n_tokens <= FEW_STREAM_ROWS && width > 1024;
+    const bool few = n_tokens <= FEW_UPDATED_ROWS && width > 1024;
+    // (more rows that one column a load keeps whole in registers are no slower so: four streams of 2,048, us, one column and four, 1,024 rows 12.8, 13.2,
+    // 2,048 rows 23.2, 24.5; in float32 25.0, 26.6; two streams 14.0, 14.0; rows of 1,024 within 3 % either way)
+    const bool fours = in_fours(width, (size_t)x | (size_t)next_weight | place_of(y, y_code) | place_of(normed, normed_code))
+        && (few || width <= 1024 || width > 256 * STREAM_CACHE);
 #define LSA_LAUNCH_S(Y, R, S) do { if (fours && few) LSA_LAUNCH_V(Y, R, S, 4, 1024); else if (fours) LSA_LAUNCH_V(Y, R, S, 4, 256); \
         else LSA_LAUNCH_V(Y, R, S, 1, 256); } while (0)
 #define LSA_LAUNCH_V(Y, R, S, V, T) streams_update_kernel<Y, R, S, V, T><<<n_tokens, T, 0, stream>>>(x, stream_stride, (const Y*)y, mix, write, next_read, \
