@@ -206,7 +206,7 @@ __global__ __launch_bounds__(256) void short_conv_keep_kernel(const float* __res
 
 // s = x + y * rsqrt(mean(y^2) + eps) * weight * scale.  Without history: out = s.  With history [states][T][W]:
 // history[before] = s and out = sum_{j <= before} mix[j] * history[j].  `rounded` (may be null) gets out as well.
-template <typename Y, typename R, int V>
+template <typename Y, typename R, int V, bool HISTORY>
 __global__ __launch_bounds__(256) void scaled_norm_add_kernel(const float* __restrict__ x, const Y* __restrict__ y,
                                                               const float* __restrict__ weight, const float* __restrict__ scale, float eps,
                                                               float* __restrict__ out, R* __restrict__ rounded, float* history,
@@ -233,7 +233,10 @@ __global__ __launch_bounds__(256) void scaled_norm_add_kernel(const float* __res
     for (int i = threadIdx.x * V + CACHE * stride; i < width; i += stride)
 #pragma unroll
         for (int v = 0; v < V; ++v) sq += (float)yr[i + v] * (float)yr[i + v];
-    // What else a piece takes, asked for before the sum of squares is waited for: the stream, the weights, the results of the layers so far.
+    // What else a piece takes: the stream, the weights, the results of the layers so far.  Without those it is asked for before the sum of squares is
+    // waited for.  With them it would take the registers of the next workgroups: 2,048 rows of 2,048 and four results, us, all of it one number a load
+    // behind the sum 22.2 (float32 24.8), ahead of it 24.4 (30.4), behind it in fours 20.5 (22.7); 32 rows 7.1, 6.1, 6.1.
+    constexpr bool AHEAD = !HISTORY;
     struct Beside { float x[V], weight[V], scale[V], total[V]; };
     auto beside = [&](int i) {
         Beside b;
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(256) void scaled_norm_add_kernel(const float* __res
         load_few((scale ? scale : weight) + i, b.scale);
 #pragma unroll
         for (int v = 0; v < V; ++v) b.total[v] = 0.f;
-        if (history) {
+        if constexpr (HISTORY) {
             for (int j = 0; j < before; ++j) {
                 const float m = mix[j];
                 float h[V];
@@ -253,11 +256,13 @@ __global__ __launch_bounds__(256) void scaled_norm_add_kernel(const float* __res
         }
         return b;
     };
-    Beside with[CACHE];
+    Beside with[AHEAD ? CACHE : 1];
+    if constexpr (AHEAD) {
 #pragma unroll
-    for (int k = 0; k < CACHE; ++k) {
-        const int i = threadIdx.x * V + k * stride;
-        if (i < width) with[k] = beside(i);
+        for (int k = 0; k < CACHE; ++k) {
+            const int i = threadIdx.x * V + k * stride;
+            if (i < width) with[k] = beside(i);
+        }
     }
     const float inv = rsqrtf(block_sum(sq, scratch) / (float)width + eps);
     auto finish = [&](int i, const float (&yv)[V], const Beside& b) {
@@ -267,7 +272,7 @@ __global__ __launch_bounds__(256) void scaled_norm_add_kernel(const float* __res
             s[v] = b.x[v] + yv[v] * inv * b.weight[v] * (scale ? b.scale[v] : 1.f);
             total[v] = b.total[v];
         }
-        if (history) {
+        if constexpr (HISTORY) {
             const float m = mix[before];
 #pragma unroll
             for (int v = 0; v < V; ++v) {
@@ -284,7 +289,7 @@ __global__ __launch_bounds__(256) void scaled_norm_add_kernel(const float* __res
 #pragma unroll
     for (int k = 0; k < CACHE; ++k) {
         const int i = threadIdx.x * V + k * stride;
-        if (i < width) finish(i, kept[k], with[k]);
+        if (i < width) finish(i, kept[k], AHEAD ? with[AHEAD ? k : 0] : beside(i));
     }
     for (int i = threadIdx.x * V + CACHE * stride; i < width; i += stride) {
         float yv[V];
@@ -828,9 +833,10 @@ LSA_EXPORT int lsa_scaled_norm_add(const float* x, const void* y, int y_code, co
     if (history != nullptr && (mix == nullptr || before < 0)) return -1;
     const bool fours = in_fours(width, (size_t)x | place_of(y, y_code) | (size_t)weight | (size_t)scale | (size_t)out | place_of(rounded, rounded_code)
                                 | (size_t)history | (history != nullptr ? (size_t)state_stride * 4 : 0));
-#define LSA_LAUNCH_V(Y, R, V) scaled_norm_add_kernel<Y, R, V><<<n, 256, 0, stream>>>(x, (const Y*)y, weight, scale, eps, out, (R*)rounded, history, \
-                                                                                  (size_t)state_stride, before, mix, width)
-#define LSA_LAUNCH(Y, R) do { if (fours) LSA_LAUNCH_V(Y, R, 4); else LSA_LAUNCH_V(Y, R, 1); } while (0)
+#define LSA_LAUNCH_V(Y, R, V, H) scaled_norm_add_kernel<Y, R, V, H><<<n, 256, 0, stream>>>(x, (const Y*)y, weight, scale, eps, out, (R*)rounded, history, \
+                                                                                     (size_t)state_stride, before, mix, width)
+#define LSA_LAUNCH(Y, R) do { if (history != nullptr) { if (fours) LSA_LAUNCH_V(Y, R, 4, true); else LSA_LAUNCH_V(Y, R, 1, true); } \
+        else if (fours) LSA_LAUNCH_V(Y, R, 4, false); else LSA_LAUNCH_V(Y, R, 1, false); } while (0)
     if (y_code && rounded_code) LSA_LAUNCH(bf16_t, bf16_t);
     else if (y_code) LSA_LAUNCH(bf16_t, float);
     else if (rounded_code) LSA_LAUNCH(float, bf16_t);
