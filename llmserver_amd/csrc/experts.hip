@@ -283,9 +283,10 @@ __global__ __launch_bounds__(256) void route_top_kernel(const float* __restrict_
 
 // The same for up to 64 * E experts in one group and up to 64 choices, which is what decoding steps of most models have: a lane keeps its experts'
 // values in registers and its choice of its own number until the end, so that a round is two exchanges between lanes without LDS or memory, and a
-// round's stores wait for nothing.  The same numbers bit by bit.  us a launch in a decoding step, that kernel and this one:
-// 32 tokens, 6 of 72 9.0 and 6.7; one token, 6 of 64 6.6 and 3.8.
-template <int E>
+// round's stores wait for nothing.  The same numbers bit by bit.  us a launch behind 64 MB of other reads, that kernel and this one: 6 of 64 of one token 4.9 and
+// 3.1, 6 of 72 of 32 tokens in eight partial sums 6.5 and 3.9, of 8,192 tokens 11.5 and 8.3.  (PARTS: with the loads of partial sums under a condition on their number
+// those of 32 tokens took 6.9, for the compiler then waits for them one by one.)
+template <int E, bool PARTS>
 __global__ __launch_bounds__(64) void route_top_registers_kernel(const float* __restrict__ all_logits, int experts, int top,
                                                                  int* __restrict__ chosen, float* __restrict__ weights, int n_tokens,
                                                                  int scoring, const float* __restrict__ bias, const float* __restrict__ correction,
@@ -294,23 +295,27 @@ __global__ __launch_bounds__(64) void route_top_registers_kernel(const float* __
     // Everything is asked for at once: lane's experts, the gate's logit (its partial sums in lanes of their own), bias and correction.
     const float* first = all_logits + (size_t)t * stride;
     const size_t part_stride = (size_t)n_tokens * stride;
-    float piece[E][ROUTE_PARTS], add[E], gate_piece = 0.f;
+    constexpr int MOST = PARTS ? ROUTE_PARTS : 1;                 // (partial sums behind the last are the last one's again: no load under a condition)
+    float piece[E][MOST], add[E], gate_piece = 0.f;
     const float* added = bias ? bias : correction ? correction : first;
 #pragma unroll
     for (int j = 0; j < E; ++j) {
         const int e = min(lane + 64 * j, experts - 1);
 #pragma unroll
-        for (int part = 0; part < ROUTE_PARTS; ++part) piece[j][part] = part == 0 || parts > 1 ? first[(size_t)min(part, parts - 1) * part_stride + e] : 0.f;
+        for (int part = 0; part < MOST; ++part) piece[j][part] = first[(PARTS ? (size_t)min(part, parts - 1) * part_stride : 0) + e];
         add[j] = added[e];
     }
     if (gate_out) gate_piece = first[(size_t)min(lane, parts - 1) * part_stride + experts];
     float value[E], score[E], most = NEG_INF;
 #pragma unroll
     for (int j = 0; j < E; ++j) {
-        double sum = 0.0;
+        float v = piece[j][0];
+        if constexpr (PARTS) {
+            double sum = 0.0;
 #pragma unroll
-        for (int part = 0; part < ROUTE_PARTS; ++part) sum += part < parts ? (double)piece[j][part] : 0.0;
-        float v = (float)sum;
+            for (int part = 0; part < MOST; ++part) sum += part < parts ? (double)piece[j][part] : 0.0;
+            v = (float)sum;
+        }
         if (bias) v += add[j];
         const bool there = lane + 64 * j < experts;
         if (there) most = fmaxf(most, v);
@@ -321,7 +326,7 @@ __global__ __launch_bounds__(64) void route_top_registers_kernel(const float* __
     if (gate_out) {
         double sum = 0.0;
 #pragma unroll
-        for (int part = 0; part < ROUTE_PARTS; ++part) {
+        for (int part = 0; part < MOST; ++part) {
             const double one = (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(gate_piece), part));
             sum += part < parts ? one : 0.0;
         }
@@ -586,9 +591,10 @@ LSA_EXPORT int lsa_route_top(const float* logits, int experts, int top, int* cho
     if (top < 1 || top > experts || (size_t)experts * 32 > 60000) return -1;
     if (groups > 1 && (!sigmoid_scores || groups > 64 || experts % groups || keep < 1 || keep > groups || top > keep * (experts / groups))) return -1;
     if (experts <= 128 && top <= 64 && groups <= 1 && !(bias != nullptr && correction != nullptr)) {
-#define LSA_TOP(E) route_top_registers_kernel<E><<<n, 64, 0, stream>>>(logits, experts, top, chosen, weights, n, scoring, bias, correction, weight_scale, stride, gate_out, parts)
-        if (experts <= 64) LSA_TOP(1);
-        else LSA_TOP(2);
+#define LSA_TOP(E, P) route_top_registers_kernel<E, P><<<n, 64, 0, stream>>>(logits, experts, top, chosen, weights, n, scoring, bias, correction, weight_scale, stride, gate_out, parts)
+        if (experts <= 64) { if (parts > 1) LSA_TOP(1, true); else LSA_TOP(1, false); }
+        else if (parts > 1) LSA_TOP(2, true);
+        else LSA_TOP(2, false);
 #undef LSA_TOP
         LSA_LAUNCH_CHECK();
     }
