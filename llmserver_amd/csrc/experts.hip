@@ -387,15 +387,24 @@ __global__ __launch_bounds__(64) void route_top_registers_kernel(const float* __
     weights[(size_t)t * top + lane] = scoring == 1 ? mine : scoring == 0 ? mine / total : mine / (total + 1e-20f) * weight_scale;
 }
 
-// Where a workgroup of the two kernels below stands: the tokens' (or pairs') workgroups of one block of columns follow one another on one XCD
-// (workgroups go round the eight in turn), so that what two of them read of one expert comes out of that XCD's cache the second time.  Before, the
-// eight of a block read it once each on an XCD of its own.  48 pairs of about 35 of 64 experts of 1,408 at width 2,048: 89 -> 81 us for
-// the first product, 43.5 -> 42.9 for the second (behind cold caches; its 35 experts take 73 and 37 at 5.5 TB/s); six pairs of one token are as fast as before.
+// Where a workgroup of the two kernels below stands.  Together (several tokens, which may share experts; grid (XCDS * units, blocks / XCDS)): the tokens' or
+// pairs' workgroups of one block of columns follow one another on one XCD (workgroups go round the eight in turn), so that what two of them read of one expert
+// comes out of that XCD's cache the second time; with a block's workgroups all over the chip each reads it once on an XCD of its own.  48 pairs of about 35 of
+// 64 experts of 1,408 at width 2,048: 86 -> 76 us for the first product, 44.5 -> 40.3 for the second (behind cold caches); 96 pairs 148 -> 120, 83 -> 77.  Two
+// dimensions, because dividing by the number of units costs the workgroups of few tokens 0.4 us (the second product of two tokens, 2 of 8 experts of
+// 1,024 at 1,024: 4.8 -> 5.3), and because one holds 2^24 workgroups only.  The pairs of one token share nothing and go one after another, grid (units,
+// blocks): 8 of 128 experts of 768 at 2,048 14.0 us so, 14.8 in the other order, 6 of 64 of 1,408 15.2, 15.8.
 constexpr int XCDS = 8;
-__device__ __forceinline__ void shared_columns(int units, int& unit, int& block) {
-    const int rounds = (int)blockIdx.x / (XCDS * units), place = (int)blockIdx.x - rounds * XCDS * units;
-    block = rounds * XCDS + (place & (XCDS - 1));
-    unit = place / XCDS;
+__device__ __forceinline__ void shared_columns(bool together, int& unit, int& block) {
+    unit = together ? (int)blockIdx.x / XCDS : (int)blockIdx.x;
+    block = together ? (int)blockIdx.y * XCDS + ((int)blockIdx.x & (XCDS - 1)) : (int)blockIdx.y;
+}
+// The grid, or false where a launch does not hold it.
+static bool shared_grid(bool together, long units, int blocks, dim3& grid) {
+    const long wide = together ? units * XCDS : units, rounds = together ? (blocks + XCDS - 1) / XCDS : blocks;
+    if (wide * 256 > 0xffffffffL || rounds > 65535) return false;
+    grid = dim3((unsigned)wide, (unsigned)rounds);
+    return true;
 }
 
 // workgroups (pairs x blocks of hidden columns, as shared_columns lays them): hidden[pair][f] = silu(G[f] . x) * (U[f] . x) for the pair's expert.  With a shared
@@ -406,11 +415,11 @@ __global__ __launch_bounds__(256) void experts_gate_up_kernel(const T* __restric
                                                               const int* __restrict__ chosen, T* __restrict__ hidden, int top,
                                                               int inter, int width, int experts, int columns_per_block, bool in_lds,
                                                               float limit, int identity, const T* __restrict__ shared_gate_up,
-                                                              T* __restrict__ shared_hidden, int shared_inter, int plain, int n_tokens) {
+                                                              T* __restrict__ shared_hidden, int shared_inter, int plain, bool together) {
     extern __shared__ __align__(16) unsigned char lds_bytes[];
     const int slots = top + (shared_gate_up ? 1 : 0);
     int unit, block;
-    shared_columns(n_tokens * slots, unit, block);
+    shared_columns(together, unit, block);
     const int t = unit / slots, slot = unit - t * slots;
     const bool shared = slot == top;
     const int pair = t * top + slot;
@@ -465,11 +474,11 @@ template <typename T>
 __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__ hidden, const T* __restrict__ down,
                                                            const int* __restrict__ chosen, const float* __restrict__ weights,
                                                            float* __restrict__ out, int top, int inter, int width, int experts,
-                                                           int columns_per_block, bool in_lds, BesideExperts<T> beside, int n_tokens) {
+                                                           int columns_per_block, bool in_lds, BesideExperts<T> beside, bool together) {
     extern __shared__ __align__(16) unsigned char lds_bytes[];
     constexpr int V = Elem<T>::kVec;
     int t, block;
-    shared_columns(n_tokens, t, block);
+    shared_columns(together, t, block);
     if (block * columns_per_block >= width) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const T* h_lds = hidden + (size_t)t * top * inter;
@@ -613,11 +622,10 @@ LSA_EXPORT int lsa_experts_gate_up(int code, const void* x, const void* gate_up,
     const bool in_lds = lds <= 64000;
     if (!in_lds) lds = 0;
     const int columns = 16;
-    const long blocks = ((most_inter + columns - 1) / columns + XCDS - 1) / XCDS * XCDS, workgroups = blocks * n * (top + (shared_gate_up ? 1 : 0));
-    if (workgroups > 0x7fffffffL) return -1;
-    const dim3 grid((unsigned)workgroups);
-    if (code) experts_gate_up_kernel<bf16_t><<<grid, 256, lds, stream>>>((const bf16_t*)x, (const bf16_t*)gate_up, chosen, (bf16_t*)hidden, top, inter, width, experts, columns, in_lds, limit, identity, (const bf16_t*)shared_gate_up, (bf16_t*)shared_hidden, shared_inter, plain, n);
-    else experts_gate_up_kernel<float><<<grid, 256, lds, stream>>>((const float*)x, (const float*)gate_up, chosen, (float*)hidden, top, inter, width, experts, columns, in_lds, limit, identity, (const float*)shared_gate_up, (float*)shared_hidden, shared_inter, plain, n);
+    dim3 grid;
+    if (!shared_grid(n > 1, (long)n * (top + (shared_gate_up ? 1 : 0)), (most_inter + columns - 1) / columns, grid)) return -1;
+    if (code) experts_gate_up_kernel<bf16_t><<<grid, 256, lds, stream>>>((const bf16_t*)x, (const bf16_t*)gate_up, chosen, (bf16_t*)hidden, top, inter, width, experts, columns, in_lds, limit, identity, (const bf16_t*)shared_gate_up, (bf16_t*)shared_hidden, shared_inter, plain, n > 1);
+    else experts_gate_up_kernel<float><<<grid, 256, lds, stream>>>((const float*)x, (const float*)gate_up, chosen, (float*)hidden, top, inter, width, experts, columns, in_lds, limit, identity, (const float*)shared_gate_up, (float*)shared_hidden, shared_inter, plain, n > 1);
     LSA_LAUNCH_CHECK();
 }
 
@@ -630,12 +638,11 @@ LSA_EXPORT int lsa_experts_down(int code, const void* hidden, const void* down, 
     const size_t lds = 0;
     const bool in_lds = false;
     const int columns = 4;
-    const long workgroups = (long)((width + columns - 1) / columns + XCDS - 1) / XCDS * XCDS * n;
-    if (workgroups > 0x7fffffffL) return -1;
-    const dim3 grid((unsigned)workgroups);
+    dim3 grid;
+    if (!shared_grid(n > 1, n, (width + columns - 1) / columns, grid)) return -1;
 #define LSA_BESIDE(T) BesideExperts<T>{(const T*)x, shared_gate, (const T*)shared_y, (const T*)shared_down, (const T*)shared_hidden, shared_inter}
-    if (code) experts_down_kernel<bf16_t><<<grid, 256, lds, stream>>>((const bf16_t*)hidden, (const bf16_t*)down, chosen, weights, out, top, inter, width, experts, columns, in_lds, LSA_BESIDE(bf16_t), n);
-    else experts_down_kernel<float><<<grid, 256, lds, stream>>>((const float*)hidden, (const float*)down, chosen, weights, out, top, inter, width, experts, columns, in_lds, LSA_BESIDE(float), n);
+    if (code) experts_down_kernel<bf16_t><<<grid, 256, lds, stream>>>((const bf16_t*)hidden, (const bf16_t*)down, chosen, weights, out, top, inter, width, experts, columns, in_lds, LSA_BESIDE(bf16_t), n > 1);
+    else experts_down_kernel<float><<<grid, 256, lds, stream>>>((const float*)hidden, (const float*)down, chosen, weights, out, top, inter, width, experts, columns, in_lds, LSA_BESIDE(float), n > 1);
 #undef LSA_BESIDE
     LSA_LAUNCH_CHECK();
 }
