@@ -1630,7 +1630,9 @@ LSA_EXPORT int lsa_heads_norm_gate(int code, const float* x, const float* weight
     dim3 grid(n_tokens, heads);
     const int weight_stride = weight_per_channel ? value_dim : 0;
     const long pairs = (long)n_tokens * heads;
-    if (pairs < 0x7fffffffL && value_dim % 8 == 0 && value_dim <= 256 && gate_stride % 8 == 0
+    // (heads of up to 64 numbers leave half of its lanes idle, which pays for many of them only: 64 heads of 64, us, the kernel above and this one, 8 tokens 2.7, 3.0,
+    // 32 tokens 2.9, 3.1, 64 tokens 3.3, 3.2, 512 tokens 10.2, 7.9; in float32 2.7, 3.2; 2.8, 3.3; 3.3, 3.2; 10.5, 9.0)
+    if (pairs < 0x7fffffffL && value_dim % 8 == 0 && value_dim <= 256 && gate_stride % 8 == 0 && (value_dim > 64 || pairs >= 4096)
         && ((size_t)x | (size_t)weight | (size_t)gate | (size_t)out) % 16 == 0) {
         const unsigned blocks = (unsigned)((pairs + 15) / 16);
 #define LSA_LONG(T, C) heads_norm_gate_eights_kernel<T, C><<<blocks, 256, 0, stream>>>(x, weight, weight_stride, eps, (const T*)gate, gate_stride, (T*)out, heads, \
