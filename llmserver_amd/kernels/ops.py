@@ -12,6 +12,7 @@ from __future__ import annotations
 import dataclasses
 
 import torch
+from torch.autograd import forward_ad
 
 from ..parts.attention import AttentionTuning, TileLaunchCost, group_tiling
 from ..parts.base import paged_part
@@ -61,6 +62,23 @@ def _stream():
 def _launched(code: int, what: str):
     if code != 0:
         raise RuntimeError(f"launch of {what} failed with HIP error {code}")
+
+
+def _followed(*tensors) -> bool:
+    """Whether anybody follows what torch does with these tensors (None: no tensor), so that a kernel that takes their addresses would go behind its
+    back: autograd, a tangent of forward-mode differentiation, ``vmap`` and the other function transforms, tracing, a dispatch mode.  Asked
+    (2 us) where a product that a library call served before goes to a kernel."""
+    if torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None or torch._C._functorch.peek_interpreter_stack() is not None:
+        return True
+    grads = torch.is_grad_enabled()
+    return any(t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or grads and t.requires_grad
+                                  or forward_ad.unpack_dual(t).tangent is not None) for t in tensors)
+
+
+def _on_current_gpu(*tensors) -> bool:
+    """Whether all of them (None: no tensor) are on the GPU that launches go to."""
+    current = torch.cuda.current_device()
+    return all(t is None or t.device.index == current for t in tensors)
 
 
 class HipOps(KernelNamespace):
@@ -171,17 +189,16 @@ class HipOps(KernelNamespace):
 
     def _few_rows_float32(self, x, weight, out):
         """Whether the 32-bit stream over the weights takes this product: few rows (by the kernel's own rule), whole tensors in their natural
-        order at multiples of 16 bytes, all on one GPU, nothing for autograd to follow; anything else is the library's, which refuses what
+        order at multiples of 16 bytes, all on the GPU that launches go to, nobody who follows the call; anything else is the library's, which refuses what
         does not fit together."""
         if not (x.dtype == weight.dtype == torch.float32 and x.is_cuda and x.dim() == weight.dim() == 2 and x.device == weight.device):
             return False
         if out is not None and not (out.dtype == torch.float32 and out.device == x.device and out.is_contiguous()
                                     and tuple(out.shape) == (x.shape[0], weight.shape[0])):
             return False
-        if torch.is_grad_enabled() and any(tensor is not None and tensor.requires_grad for tensor in (x, weight, out)):
+        if not x.is_contiguous() or not weight.is_contiguous() or not self._gemm.lsa_gemm_few_f32_fits(x.shape[0], weight.shape[0], x.shape[1]):
             return False
-        return x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 \
-            and bool(self._gemm.lsa_gemm_few_f32_fits(x.shape[0], weight.shape[0], x.shape[1]))
+        return not _followed(x, weight, out) and _on_current_gpu(x) and (x.data_ptr() | weight.data_ptr()) % 16 == 0
 
     def _linear_few_rows_float32(self, x, weight, out=None, bias=None, row_scale=None):
         """Up to 16 rows of float32 through the stream over the weights, whatever its rule says of the sizes."""
@@ -194,9 +211,10 @@ class HipOps(KernelNamespace):
 
     FUSED_ROWS_FLOAT32 = 8      # most rows for which the 32-bit stream folds in what stands around a product
 
-    def _fuses_float32(self, x, weight, row_scale):
-        """Whether the 32-bit stream takes the product with a row scale (if there is one), a stream update or a gate in its epilogue."""
-        return x.shape[0] <= self.FUSED_ROWS_FLOAT32 and self._few_rows_float32(x, weight, None) and self._row_scale_fits(row_scale, x.shape[0])
+    def _fuses_float32(self, x, weight, row_scale, *beside):
+        """Whether the 32-bit stream takes the product with a row scale (if there is one), a stream update or a gate in its epilogue (``beside``: what joins it there)."""
+        return x.shape[0] <= self.FUSED_ROWS_FLOAT32 and self._few_rows_float32(x, weight, None) and self._row_scale_fits(row_scale, x.shape[0]) \
+            and not _followed(*beside, *(row_scale[:1] if row_scale is not None else ()))
 
     LIBRARY_MARGIN = 0.93       # the library replaces a few-row kernel only if it takes less than this share of its time
 
@@ -554,7 +572,7 @@ class HipOps(KernelNamespace):
         rows, width = x.shape
         n = weight.shape[0]
         if x.dtype == torch.float32 == resid.dtype and not rows_per_workgroup and x.shape[1] == weight.shape[1] \
-                and self._gemm.lsa_gemm_few_f32_parts(n) <= self.SCALE_PARTS and self._fuses_float32(x, weight, row_scale):
+                and self._gemm.lsa_gemm_few_f32_parts(n) <= self.SCALE_PARTS and self._fuses_float32(x, weight, row_scale, resid, norm_weight):
             return self._linear_into_stream_float32(x, weight, resid, norm_weight, row_scale)
         if x.shape[1] != weight.shape[1] or not self._few_rows(x, weight) or rows > self.FUSED_ROWS \
                 or not self._row_scale_fits(row_scale, rows) or resid.dtype != torch.bfloat16:
@@ -644,7 +662,7 @@ class HipOps(KernelNamespace):
         if not self.skinny_rows < rows <= (self.SUMMED_GATED_ROWS if gated else self.SUMMED_ROWS) or not self.split_products or not low <= weight.numel() <= high \
                 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or width < 1024 or width % 8 or weight.dim() != 2 or weight.shape[1] != width \
                 or weight.shape[0] % (8 if gated else 4) or x.device != weight.device or not x.is_cuda or not x.is_contiguous() or not weight.is_contiguous() \
-                or (x.data_ptr() | weight.data_ptr()) % 16 or torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+                or _followed(x, weight) or not _on_current_gpu(x) or (x.data_ptr() | weight.data_ptr()) % 16:
             return None
         parts = self._gemm.lsa_gemm_split_parts(rows, weight.shape[0], width)
         if parts < 2:
