@@ -840,15 +840,15 @@ class GQAttention(Mixer):
         table = ctx.block_table(cache.group)
         eps = self.qk_norm_eps if self.qk_norm_eps is not None else 0.0
         cos_sin = self.position.cos_sin(ctx)
-        # A step of single tokens: the attention kernel does the norm, the rotation and the cache write itself.
+        # A step of single tokens: the attention kernel does the norm, the rotation and the cache write itself, unless scores have a bias by distance.
         fusion = None
         # (the kernel that merges a tile's key ranges in its workgroup fuses only the whole of norm and rotation)
         whole = self.q_norm_weight is not None and cos_sin is not None
         plan = ctx.get_plan(self.plan_key())
-        if ctx.n_tokens == ctx.n_rows and (
+        if ctx.n_tokens == ctx.n_rows and self.slopes is None and (
                 ctx.ops.decode_fusion_fits(qkv.dtype, self.head_dim) and (whole or not plan.get("merge_in_workgroup"))
                 or whole and plan.get("rows_in_order") and ctx.ops.single_token_fusion_fits(
-                    qkv.dtype, self.head_dim, cache.page_size, ctx.n_rows, self.n_heads, self.n_kv_heads, self.softcap is None and self.slopes is None)):
+                    qkv.dtype, self.head_dim, cache.page_size, ctx.n_rows, self.n_heads, self.n_kv_heads, self.softcap is None)):
             fusion = (self.q_norm_weight, self.k_norm_weight, eps, cos_sin, cache.writable)
         else:
             ctx.ops.qk_norm_rope_kv_write(
