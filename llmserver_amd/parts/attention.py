@@ -250,42 +250,37 @@ SHORT_CONTEXT = 512     # captured steps whose contexts all stay within this are
 def _shared_ranges(lengths: np.ndarray, splits: int, key_align: int, most_splits: int):
     """Keys a range and ranges a row where rows of ``lengths`` keys share ``splits`` ranges a row, so that the longest range, which a launch of
     about as many wavefronts as the chip holds waits for, is as short as can be; what the rows do not need goes round as empty
-    ranges, the same number in all whatever the lengths are.  33 rows of 667 to 2,000 keys (and 7 that fill them up to a captured step's 40) with
-    three ranges a row: ranges of 480 keys instead of 672, 38.0 us instead of 43.3 with the merge."""
+    ranges, the same number in all whatever the lengths are.  None where the even cut is the better one: the rows are about equally long, or ranges are so short
+    that the merge of a long row's many counts for more than what its keys do.  us with the merge, the even cut and this one, 32 heads on 8 of 128
+    (profilers' stamps are longer): 33 rows of 667 to 2,000 keys, three ranges a row, of 544 keys instead of 672 44.8, 38.5; one row of 2,000 and 32 of 100 41.4, 18.8; rows of
+    1,600 to 2,000, ranges as long as before 53.1, 53.4.  24 rows, five ranges, of 320 instead of 416 33.7, 31.2; 416 instead of 416 38, 37; 600 keys at the most, 96 instead of
+    128 18.8, 18.4, 128 instead of 128 20.3, 20.7.  16 rows, eight ranges, 384 instead of 576 43.3, 39.7; 192 instead of 256 25.1, 25.7; 96 instead of 128 17.8, 18.5.  8
+    rows, sixteen, 64 instead of 96 17.0, 16.2; 96 instead of 128 17.8, 18.6; 32 instead of 64 13.7, 14.5.  Four rows, 32 ranges, 64 instead of 96 16.6, 17.2."""
     total = len(lengths) * splits
     aligned = lambda keys: -(-int(keys) // key_align) * key_align
     shortest, longest = max(aligned(-(-lengths.sum() // total)), key_align), max(aligned(-(-lengths.max() // splits)), key_align)
+    most = longest                           # the longest range that pays
+    if splits > 3:
+        most = int((0.72 if splits >= 8 else 0.85) * longest) if longest >= 3 * key_align and longest > 3 * splits else 0
+    if shortest > most or shortest >= longest:
+        return None
     keys = np.append(np.arange(shortest, longest, max(aligned((longest - shortest) // 32), key_align)), longest)
     counts = np.maximum(-(-lengths[None, :] // keys[:, None]), 1)
     fits = (counts.sum(axis=1) <= total) & (counts.max(axis=1) + splits <= most_splits)
     best = int(np.argmax(fits))              # (the longest range of the even cut always fits)
+    if keys[best] > most:
+        return None
     counts = counts[best]
     spare = total - int(counts.sum())
     return int(keys[best]), counts + spare // len(lengths) + (np.arange(len(lengths)) < spare % len(lengths))
 
 
-def _shared_single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, key_align: int, most_splits: int,
-                              chunk: Optional[int]) -> AttentionPlan:
-    """As :func:`_single_token_plan` without merging in the workgroup, the ranges cut by :func:`_shared_ranges`."""
-    rows = np.arange(len(row_ctx), dtype=np.int64)
-    k_begin = first_keys(row_ctx - 1, window, chunk)
-    start = (k_begin // key_align) * key_align
-    keys, counts = _shared_ranges(row_ctx - start, splits, key_align, most_splits)
-    of_row = np.repeat(rows, counts)
-    first_slot = np.cumsum(counts) - counts
-    begin = start[of_row] + (np.arange(len(of_row)) - first_slot[of_row]) * keys
-    end = row_ctx[of_row]
-    lo = np.minimum(np.maximum(begin, k_begin[of_row]), end)
-    items = np.stack([of_row, np.zeros_like(of_row), lo, np.maximum(lo, np.minimum(begin + keys, end))], axis=1).astype(np.int32)
-    merges = np.stack([rows, np.zeros_like(rows), first_slot, counts], axis=1).astype(np.int32)
-    return AttentionPlan(items, np.arange(len(items), dtype=np.int32), merges, len(items))
-
-
 def _single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, merge_in_workgroup: int = 0,
-                       key_align: int = KEY_ALIGN, chunk: Optional[int] = None) -> AttentionPlan:
+                       key_align: int = KEY_ALIGN, chunk: Optional[int] = None, share_up_to: int = 0) -> AttentionPlan:
     """The plan of a step in which every row brings one token and every tile gets ``splits`` key ranges: what the
     loop of :func:`build_attention_plan` makes for it, row by row, computed for all rows at once (a decode step of
-    many rows is planned thousands of times a second)."""
+    many rows is planned thousands of times a second).  ``share_up_to`` (ranges that a tile may have): the rows share their ranges
+    where :func:`_shared_ranges` says so."""
     n_rows = len(row_ctx)
     rows = np.arange(n_rows, dtype=np.int64)
     k_end = row_ctx
@@ -297,6 +292,15 @@ def _single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, 
     if merge_in_workgroup:          # four (or two) items a tile; with fewer ranges wanted, the last ones come out empty
         ranges, splits = max(1, min(splits, merge_in_workgroup)), merge_in_workgroup
     start = (k_begin // key_align) * key_align
+    shared = _shared_ranges(k_end - start, splits, key_align, share_up_to) if share_up_to else None
+    if shared is not None:
+        keys, counts = shared
+        of_row, first_slot = np.repeat(rows, counts), np.cumsum(counts) - counts
+        begin, end = start[of_row] + (np.arange(len(of_row)) - first_slot[of_row]) * keys, k_end[of_row]
+        lo = np.minimum(np.maximum(begin, k_begin[of_row]), end)
+        items = np.stack([of_row, np.zeros_like(of_row), lo, np.maximum(lo, np.minimum(begin + keys, end))], axis=1).astype(np.int32)
+        merges = np.stack([rows, zeros, first_slot, counts], axis=1).astype(np.int32)
+        return AttentionPlan(items, np.arange(len(items), dtype=np.int32), merges, len(items))
     per = -(-(k_end - start) // (ranges if merge_in_workgroup else splits))
     per = -(-per // key_align) * key_align
     piece = start[:, None] + np.arange(splits, dtype=np.int64)[None, :] * per[:, None]
@@ -399,10 +403,9 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
         raise ValueError("two key ranges of each of two tiles are merged in a workgroup only in steps of one token per row")
     if merge_in_workgroup not in (0, 2, WORKGROUP_RANGES) or (merge_in_workgroup == 2 and len(row_len) % 2):
         raise ValueError("a workgroup merges four key ranges of one tile, or two ranges of each of two tiles (an even number of rows)")
-    if share_ranges and single_tokens and not merge_in_workgroup and len(row_len) > 1 and 1 < int(fixed_splits or 0) <= most_splits // 2:
-        return _shared_single_token_plan(row_ctx, window, int(fixed_splits), key_align, most_splits, chunk)
-    if (merge_in_workgroup or (single_token_shortcut and fixed_splits is not None)) and single_tokens:
-        return _single_token_plan(row_ctx, window, int(fixed_splits or merge_in_workgroup or 1), merge_in_workgroup, key_align, chunk)
+    share_up_to = most_splits if share_ranges and not merge_in_workgroup and len(row_len) > 1 and 1 < int(fixed_splits or 0) <= most_splits // 2 else 0
+    if (merge_in_workgroup or share_up_to or (single_token_shortcut and fixed_splits is not None)) and single_tokens:
+        return _single_token_plan(row_ctx, window, int(fixed_splits or merge_in_workgroup or 1), merge_in_workgroup, key_align, chunk, share_up_to)
     if merge_in_workgroup:
         # Rows of several tokens: every tile of every row gets exactly four ranges (the last ones may be empty), four
         # neighbouring items, which their workgroup merges: no slots, no merge, and no workgroups of tiles.

@@ -36,3 +36,16 @@ def test_uneven_rows_get_shorter_ranges():
     shared, even = (build_attention_plan([1] * 40, contexts, 4, 8, None, fixed_splits=3, share_ranges=share) for share in (True, False))
     longest = lambda p: int((p.items[:, 3] - p.items[:, 2]).max())
     assert longest(shared) == 480 and longest(even) == 672
+
+
+def test_where_the_even_cut_is_the_better_one():
+    """Rows of one length, and ranges that sharing hardly shortens or that are short already: the very plan of the even cut."""
+    order = random.Random(7)
+    for rows, splits, contexts in ((40, 3, [2000] * 40), (8, 16, [4001] * 8), (2, 32, [1300, 1400]), (4, 32, [2000, 600, 600, 600]), (16, 8, order.sample(range(1700, 2000), 16)),
+                                   (8, 16, [600, 300, 300, 300, 200, 200, 200, 200]), (16, 8, [int(2000 * (15 + 2 * i) / 45) for i in range(16)])):
+        shared, even = (build_attention_plan([1] * rows, contexts, 4, 8, None, fixed_splits=splits, share_ranges=share) for share in (True, False))
+        assert np.array_equal(shared.items, even.items) and np.array_equal(shared.merges, even.merges) and shared.n_slots == even.n_slots
+    for rows, splits, contexts in ((24, 5, [2000] + [100] * 23), (16, 8, [int(4400 * (15 + 2 * i) / 45) for i in range(16)]), (8, 16, [1300] * 4 + [325] * 4)):
+        shared, even = (build_attention_plan([1] * rows, contexts, 4, 8, None, fixed_splits=splits, share_ranges=share) for share in (True, False))
+        longest = lambda p: int((p.items[:, 3] - p.items[:, 2]).max())
+        assert longest(shared) <= 0.72 * longest(even)
