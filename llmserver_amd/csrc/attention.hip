@@ -107,7 +107,8 @@ __device__ __forceinline__ float inverse_of_sum(float total, float top, const fl
 // then reads its queries raw from the projection, and the one whose key range ends at the new
 // token takes that token's key and value from the projection too (normalised, rotated, written to
 // the cache on the side) instead of from the pages.  One launch less between the projection and
-// the attention.  bfloat16 and head sizes in steps of 64 only.
+// the attention.  In the kernel below bfloat16 and head sizes in steps of 64 only; in the one for steps of single tokens in order (attention_single.hpp) float32
+// and head sizes in steps of 32 too, with pages of a multiple of 16 keys.
 struct DecodeFusion {
     const float* q_weight;     // [D] or null: no norm
     const float* k_weight;

@@ -53,7 +53,6 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
     // HEADS > 0 (float32 only): that many query heads share the KV head, and the products are plain multiply-adds of a lane's own
     // numbers: the 32-bit matrix products would do sixteen columns' work for one or two of them (1,024 cycles against 128 a step and head).
     constexpr bool VECTOR = HEADS > 0;
-    constexpr bool AHEAD = ND <= 8 || WAVES == 4;                                // a step's loads are under way while the one before is multiplied
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int col = lane & 15, quad = lane >> 4;
     const int row = blockIdx.x, kv_head = blockIdx.y / g.gtiles, gtile = blockIdx.y % g.gtiles;
@@ -290,8 +289,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
 
     while (kt < hi) {
         const int following = kt + WAVES * KEY_STEP;
-        Step next;
-        if (AHEAD && following < hi) load_step(next, following);
+        Step next;                                                 // its loads are under way while this one is multiplied
+        if (following < hi) load_step(next, following);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (VECTOR) {
 #if !LSA_BF16
@@ -400,10 +399,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
             }
 #endif
         }
-        if (following < hi) {
-            if (AHEAD) now = next;
-            else load_step(now, following);
-        }
+        if (following < hi) now = next;
         kt = following;
     }
 
