@@ -910,7 +910,9 @@ class HipOps(KernelNamespace):
             q_weight, k_weight, norm_eps, cos_sin, write_cache = decode_fusion
             if not (self.decode_fusion_fits(qkv.dtype, head_dim) or plan.get("rows_in_order") and
                     self.single_token_fusion_fits(qkv.dtype, head_dim, page_size)) or n_tiles or n != rows:
-                raise ValueError("decode fusion takes bfloat16, head sizes in steps of 64 and steps of one token per row")
+                raise ValueError("decode fusion takes steps of one token per row: bfloat16 with head sizes in steps of 64, or, with a plan that says rows_in_order, "
+                                 "also float32 with head sizes in steps of 32 and pages of a multiple of 16 keys; "
+                                 f"got {qkv.dtype}, heads of {head_dim}, pages of {page_size}, {n} tokens in {rows} rows")
             for name, w in (("q_weight", q_weight), ("k_weight", k_weight)):
                 if w is not None:
                     _check(w, name, torch.float32, (head_dim,))
