@@ -816,16 +816,19 @@ class HipOps(KernelNamespace):
 
     def single_tokens_pay(self, dtype, head_dim, rows, n_q, n_kv, plain=True) -> bool:
         """Whether steps of one token a row behind short contexts are faster in the kernel of their own (attention_single.hpp) than in the kernel for all
-        steps.  Its workgroups have eight wavefronts and a row's keys of one KV head each: as long as every one has a compute unit of its own, yes.
-        Beyond that the other kernel's smaller workgroups fill the chip better.  us, the other kernel and this one, contexts of 16, 128 and 512: bfloat16, 16
-        heads on 8 of 128, 32 rows (256 workgroups) 8.8, 10.6, 18.0 and 6.7, 9.3, 16.0; 64 rows 11.1, 13.8, 27.8 and 11.4, 16.4, 28.4; 128 rows 19.1, 23.7, 56
-        and 20.6, 29.5, 64; 64 on 8 of 64, 64 rows 7.9, 9.1, 16.9 and 8.4, 10.2, 18.2; float32, 16 on 8 of 128, 64 rows 12.6, 20.4, 53 and 12.7, 20.9, 58.
+        steps.  Its workgroups have eight wavefronts and a row's keys of one KV head each: as long as every one has a compute unit of its own, yes, in
+        float32, where norm and rotation are a launch more otherwise, two on a unit.  Beyond that the other kernel's smaller workgroups fill the chip better.
+        us, the other kernel and this one, contexts of 16, 128 and 512: bfloat16, 16 heads on 8 of 128, 32 rows (256 workgroups) 8.8, 10.6, 18.0 and 6.7, 9.3, 16.0;
+        64 rows 11.1, 13.8, 27.8 and 11.4, 16.4, 28.4; 128 rows 19.1, 23.7, 56 and 20.6, 29.5, 64; 64 on 8 of 64, 64 rows 7.9, 9.1, 16.9 and 8.4, 10.2, 18.2.
+        float32, norm and rotation with either, contexts of 40, 300 and 512: 16 on 8 of 128, 40 rows 14.7, 32.3, 44.0 and 13.5, 29.0, 45.1, 64 rows 15.4, 36.0, 52.3 and
+        14.2, 32.7, 57.1, 80 rows 19.3, 46.4, 75.9 and 19.2, 46.1, 83.7, 128 rows 23.2, 73.5, 112 and 25.8, 78.0, 122.
         Forms of four wavefronts stay the better ones at heads above 128 dimensions (bfloat16, 16 on 4 of 256, 128 rows: 28, 33, 67 and 16, 24, 60)
         and up to 96 with more than eight heads a KV head (40 on 2 of 96, 256 rows: 22.7, 24.1, 42 and 19.7, 22.9, 40), not at 128 (64 on 4, 128 rows: 11.9,
         14.4, 28.1 and 11.1, 16.5, 29.6); so does float32 with a KV head for every head of up to 64 dimensions and ``plain`` scores (no cap, no bias by
         distance; 8 of 64, 128 rows: 13.7, 20.8, 54 and 10.8, 17.2, 50; with a cap 13.9, 21.4, 54 and 15.0, 25.6, 62)."""
         heads, _, tiles = group_tiling(n_q // n_kv)
-        if rows * n_kv * tiles <= self.attention_tuning_for(dtype, head_dim).target_waves // 4:
+        units = self.attention_tuning_for(dtype, head_dim).target_waves // 4
+        if rows * n_kv * tiles <= (2 * units if dtype == torch.float32 else units):
             return True
         return head_dim > 128 or (heads > 8 and head_dim <= 96) or (dtype == torch.float32 and plain and n_q == n_kv and head_dim <= 64)
 

@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows, n_q, n_kv, d", [(70, 16, 8, 128), (40, 32, 8, 64), (17, 32, 16, 32)])
+@pytest.mark.parametrize("rows, n_q, n_kv, d", [(70, 16, 8, 128), (66, 32, 8, 64), (33, 32, 16, 32)])
 @pytest.mark.parametrize("fused", [False, True])
 def test_rows_beyond_the_compute_units(dtype, rows, n_q, n_kv, d, fused):
     from llmserver_amd.kernels import default_ops
