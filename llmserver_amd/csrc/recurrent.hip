@@ -1487,6 +1487,8 @@ LSA_EXPORT int lsa_token_shift(int code, const void* h, const float* mu, int mix
                                int keep, hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (mixes < 1 || state == nullptr || slots == nullptr) return -1;
+    // (16 bytes a load leave too few threads where there are few numbers: five mixes of 2,048 columns in bfloat16, us, one number a load and eight, 32 tokens 3.5, 4.1, 96
+    // tokens 4.1, 4.2, 128 tokens (2^18 numbers) 4.8, 4.3, 512 tokens 8.4, 5.8)
     const bool wide = width % 8 == 0 && ((size_t)h | (size_t)mu | (size_t)out) % 16 == 0 && (long)n_tokens * width >= 1 << 18;
     const int columns = 256 * (!wide ? 1 : code ? 8 : 4);
     const dim3 grid(n_tokens, (width + columns - 1) / columns);

@@ -289,7 +289,8 @@ __global__ __launch_bounds__(64) void qkv_prepare_kernel(const T* __restrict__ q
 // a wavefront finds its place and one inverse root for two numbers a lane, and every value goes out alone.  us, that kernel and this one, 16 heads on 4 of
 // 128 in bfloat16: 2,048 tokens of one row 24.1, 9.5; 256 6.4, 4.0; 256 rows of one token 6.8, 5.4; float32 24.8, 13.3; 6.8, 4.2; 7.1, 6.2.
 // A tile's dimensions are shared by so many workgroups that every compute unit has one: a compute unit puts a value that goes alone (all of them, in
-// rows of one token) away in 0.4 ns or so, and with a tile to a workgroup, 16 of them, the 256 rows of one token took 14.6 us, 17.0 in float32.
+// rows of one token) away in about 1.2 ns, and with a tile to a workgroup, 16 of them, the 256 rows of one token took 14.6 us, 17.0 in float32.
+// LONG_STEP is where this kernel was measured first; it is the faster one below as well, 64 tokens of one row 5.3, 3.8, 64 rows of one token 5.3, 4.5, 32 tokens 5.1, 3.6.
 constexpr int LONG_STEP = 4 * VT_TOKENS;
 __device__ __forceinline__ float sum_of_16_lanes(float v) {
     const auto across = [](float x, auto control) {
