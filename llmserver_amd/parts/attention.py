@@ -247,21 +247,24 @@ SHORT_CONTEXT = 512     # captured steps whose contexts all stay within this are
                         # a tile's four key ranges itself (no partial results in memory, no launch that merges them)
 
 
-def _shared_ranges(lengths: np.ndarray, splits: int, key_align: int, most_splits: int):
+def _shared_ranges(lengths: np.ndarray, splits: int, key_align: int, most_splits: int, fused: bool):
     """Keys a range and ranges a row where rows of ``lengths`` keys share ``splits`` ranges a row, so that the longest range, which a launch of
     about as many wavefronts as the chip holds waits for, is as short as can be; what the rows do not need goes round as empty
-    ranges, the same number in all whatever the lengths are.  None where the even cut is the better one: the rows are about equally long, or ranges are so short
-    that the merge of a long row's many counts for more than what its keys do.  us with the merge, the even cut and this one, 32 heads on 8 of 128
-    (profilers' stamps are longer): 33 rows of 667 to 2,000 keys, three ranges a row, of 544 keys instead of 672 44.8, 38.5; one row of 2,000 and 32 of 100 41.4, 18.8; rows of
-    1,600 to 2,000, ranges as long as before 53.1, 53.4.  24 rows, five ranges, of 320 instead of 416 33.7, 31.2; 416 instead of 416 38, 37; 600 keys at the most, 96 instead of
-    128 18.8, 18.4, 128 instead of 128 20.3, 20.7.  16 rows, eight ranges, 384 instead of 576 43.3, 39.7; 192 instead of 256 25.1, 25.7; 96 instead of 128 17.8, 18.5.  8
-    rows, sixteen, 64 instead of 96 17.0, 16.2; 96 instead of 128 17.8, 18.6; 32 instead of 64 13.7, 14.5.  Four rows, 32 ranges, 64 instead of 96 16.6, 17.2."""
+    ranges, the same number in all whatever the lengths are.  None where the even cut is the better one: where the longest range would not get shorter (the merge of a
+    long row's many ranges costs 2 to 5 %), and, in attention that prepares its queries itself (``fused``), where it hardly would or is short already.
+
+    us with the merge, the even cut and this one (profilers' stamps are longer).  32 heads on 8 of 128, fused: 33 rows of 667 to 2,000 keys, three ranges a row, of 544 keys instead of 672
+    44.8, 38.5; one row of 2,000 and 32 of 100 41.4, 18.8.  24 rows, five ranges, 320 instead of 416 33.7, 31.2; 416 as before 38, 37; 96 instead of 128 18.8, 18.4, 128 as before 20.3, 20.7.
+    16 rows, eight ranges, 384 instead of 576 43.3, 39.7; 192 instead of 256 25.1, 25.7 (lengths in thirds), 24.2, 23.4 (halves); 96 instead of 128 17.8, 18.5.  8 rows, sixteen, 64 instead of 96
+    17.0, 16.2; 96 instead of 128 17.8, 18.6; 32 instead of 64 13.7, 14.5.  Four rows, 32 ranges, 64 instead of 96 16.6, 17.2.  Not fused: 16 heads on 1 of 256, 2 to 64 rows, sixteen ranges, 32
+    instead of 64 18.4, 15.0; 64 as before 18.5, 18.9; 32 on 16 of 128, 8 rows, eight ranges, 96 instead of 128 18.2, 16.9, 416 instead of 576 43.3, 39.1."""
     total = len(lengths) * splits
     aligned = lambda keys: -(-int(keys) // key_align) * key_align
     shortest, longest = max(aligned(-(-lengths.sum() // total)), key_align), max(aligned(-(-lengths.max() // splits)), key_align)
-    most = longest                           # the longest range that pays
-    if splits > 3:
-        most = int((0.72 if splits >= 8 else 0.85) * longest) if longest >= 3 * key_align and longest > 3 * splits else 0
+    most = longest if fused else longest - 1              # the longest range that pays
+    if fused and splits > 3:
+        share = 0.85 if splits < 8 else 0.76 if longest >= 8 * key_align else 0.72
+        most = int(share * longest) if longest >= 3 * key_align and longest > 3 * splits else 0
     if shortest > most or shortest >= longest:
         return None
     keys = np.append(np.arange(shortest, longest, max(aligned((longest - shortest) // 32), key_align)), longest)
@@ -276,7 +279,7 @@ def _shared_ranges(lengths: np.ndarray, splits: int, key_align: int, most_splits
 
 
 def _single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, merge_in_workgroup: int = 0,
-                       key_align: int = KEY_ALIGN, chunk: Optional[int] = None, share_up_to: int = 0) -> AttentionPlan:
+                       key_align: int = KEY_ALIGN, chunk: Optional[int] = None, share_up_to: int = 0, fused: bool = False) -> AttentionPlan:
     """The plan of a step in which every row brings one token and every tile gets ``splits`` key ranges: what the
     loop of :func:`build_attention_plan` makes for it, row by row, computed for all rows at once (a decode step of
     many rows is planned thousands of times a second).  ``share_up_to`` (ranges that a tile may have): the rows share their ranges
@@ -292,7 +295,7 @@ def _single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, 
     if merge_in_workgroup:          # four (or two) items a tile; with fewer ranges wanted, the last ones come out empty
         ranges, splits = max(1, min(splits, merge_in_workgroup)), merge_in_workgroup
     start = (k_begin // key_align) * key_align
-    shared = _shared_ranges(k_end - start, splits, key_align, share_up_to) if share_up_to else None
+    shared = _shared_ranges(k_end - start, splits, key_align, share_up_to, fused) if share_up_to else None
     if shared is not None:
         keys, counts = shared
         of_row, first_slot = np.repeat(rows, counts), np.cumsum(counts) - counts
@@ -374,7 +377,7 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
                          workgroup_tiles: int = 0, single_token_shortcut: bool = True, merge_in_workgroup: int = 0,
                          tuning: AttentionTuning = DEFAULT_TUNING, tile_halves: int = 1, tile_min_workgroups: int = 0,
                          tile_key_ranges: int = 1, fixed_tiles: Optional[int] = None, chunk: Optional[int] = None,
-                         share_ranges: bool = False) -> AttentionPlan:
+                         share_ranges: bool = False, fused: bool = False) -> AttentionPlan:
     """Cut the step's rows into tiles of tokens and, where that pays, ranges of keys.  ``window`` / ``chunk``: which keys a
     query sees (see :func:`first_keys`); a tile's keys begin at the first one that its first token sees.
 
@@ -392,7 +395,8 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
     first tile's entries, which compute and write the same numbers once more.  ``merge_in_workgroup`` (4, or 2 in steps
     of one token per row with an even number of rows): every tile gets that many ranges, the items of a workgroup, which
     merges them itself: no slots, no merges, no workgroups of tiles.  ``share_ranges`` (with ``fixed_splits``, in steps of one token per
-    row): the rows share that many ranges a row among them by their lengths (:func:`_shared_ranges`)."""
+    row): the rows share that many ranges a row among them by their lengths where that pays (:func:`_shared_ranges`); ``fused``: attention prepares
+    its queries itself."""
     _, tokens_per_tile, group_tiles = group_tiling(group_size, tuning.tile_rows)
     key_align, key_step, most_splits = tuning.key_align, tuning.key_step, tuning.most_splits
     row_len = np.asarray(row_len, dtype=np.int64)
@@ -405,7 +409,7 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
         raise ValueError("a workgroup merges four key ranges of one tile, or two ranges of each of two tiles (an even number of rows)")
     share_up_to = most_splits if share_ranges and not merge_in_workgroup and len(row_len) > 1 and 1 < int(fixed_splits or 0) <= most_splits // 2 else 0
     if (merge_in_workgroup or share_up_to or (single_token_shortcut and fixed_splits is not None)) and single_tokens:
-        return _single_token_plan(row_ctx, window, int(fixed_splits or merge_in_workgroup or 1), merge_in_workgroup, key_align, chunk, share_up_to)
+        return _single_token_plan(row_ctx, window, int(fixed_splits or merge_in_workgroup or 1), merge_in_workgroup, key_align, chunk, share_up_to, fused)
     if merge_in_workgroup:
         # Rows of several tokens: every tile of every row gets exactly four ranges (the last ones may be empty), four
         # neighbouring items, which their workgroup merges: no slots, no merge, and no workgroups of tiles.
@@ -531,9 +535,10 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
 
 
 def stage_attention_plan(ctx, key, group_size: int, n_kv_heads: int, head_dim: int, window: Optional[int], graph_shape,
-                         chunk: Optional[int] = None) -> None:
+                         chunk: Optional[int] = None, fused: bool = False) -> None:
     """Make the step's attention work list for a mixer of this geometry and put it among the step's staged arrays under
-    ``key`` (mixers of equal geometry share it).  ``graph_shape``: the mixer's :meth:`Mixer.graph_shape`."""
+    ``key`` (mixers of equal geometry share it).  ``graph_shape``: the mixer's :meth:`Mixer.graph_shape`; ``fused``: in steps of single tokens attention prepares
+    the mixer's queries itself."""
     if ctx.has_plan(key):
         return
     fixed = fixed_tiles = None
@@ -577,7 +582,7 @@ def stage_attention_plan(ctx, key, group_size: int, n_kv_heads: int, head_dim: i
         plan = build_attention_plan(ctx.h_row_len, ctx.h_row_ctx, group_size, n_kv_heads, window,
                                     target_waves=tuning.target_waves, fixed_splits=fixed, workgroup_tiles=per_workgroup,
                                     merge_in_workgroup=in_workgroup, tuning=tuning, tile_halves=halves, tile_min_workgroups=fewest,
-                                    tile_key_ranges=key_ranges, fixed_tiles=fixed_tiles, chunk=chunk, share_ranges=True)
+                                    tile_key_ranges=key_ranges, fixed_tiles=fixed_tiles, chunk=chunk, share_ranges=True, fused=fused)
     ctx.set_plan(key, {
         **({"tile_slots": plan.tile_slots} if plan.tile_slots is not None else {}),
         "items": plan.items, "item_slot": plan.item_slot, "merges": plan.merges, "tiles": plan.tiles,
@@ -773,7 +778,8 @@ class GQAttention(Mixer):
         return 2.0 * self.n_heads * (self.head_dim + self.value_dim) * pairs
 
     def prepare(self, ctx):
-        stage_attention_plan(ctx, self.plan_key(), self.group_size, self.n_kv_heads, self.row, self.window, self.graph_shape, self.chunk)
+        stage_attention_plan(ctx, self.plan_key(), self.group_size, self.n_kv_heads, self.row, self.window, self.graph_shape, self.chunk,
+                             not self.general and self.slopes is None and ctx.ops.decode_fusion_fits(ctx.dtype, self.row))
 
     def _compose(self, qkv, ctx, cache, table, q):
         """Convolution, norm and rotation of queries and keys, convolution and mixing of values, and the cache write."""

@@ -38,14 +38,38 @@ def test_uneven_rows_get_shorter_ranges():
     assert longest(shared) == 480 and longest(even) == 672
 
 
-def test_where_the_even_cut_is_the_better_one():
-    """Rows of one length, and ranges that sharing hardly shortens or that are short already: the very plan of the even cut."""
+@pytest.mark.parametrize("fused", [False, True])
+def test_where_the_even_cut_is_the_better_one(fused):
+    """Rows of one length and ranges that sharing does not shorten: the very plan of the even cut; where attention prepares its queries itself, also ranges
+    that sharing hardly shortens or that are short already."""
     order = random.Random(7)
-    for rows, splits, contexts in ((40, 3, [2000] * 40), (8, 16, [4001] * 8), (2, 32, [1300, 1400]), (4, 32, [2000, 600, 600, 600]), (16, 8, order.sample(range(1700, 2000), 16)),
-                                   (8, 16, [600, 300, 300, 300, 200, 200, 200, 200]), (16, 8, [int(2000 * (15 + 2 * i) / 45) for i in range(16)])):
-        shared, even = (build_attention_plan([1] * rows, contexts, 4, 8, None, fixed_splits=splits, share_ranges=share) for share in (True, False))
+    plans = lambda rows, splits, contexts: [build_attention_plan([1] * rows, contexts, 4, 8, None, fixed_splits=splits, share_ranges=share, fused=fused) for share in (True, False)]
+    longest = lambda p: int((p.items[:, 3] - p.items[:, 2]).max())
+    for rows, splits, contexts in ((40, 3, [2000] * 40), (8, 16, [4001] * 8), (2, 32, [1300, 1400]), (4, 32, [2000, 2000, 500, 500]), (16, 8, order.sample(range(1900, 2000), 16))):
+        shared, even = plans(rows, splits, contexts)
         assert np.array_equal(shared.items, even.items) and np.array_equal(shared.merges, even.merges) and shared.n_slots == even.n_slots
+    for rows, splits, contexts in ((8, 16, [600, 300, 300, 300, 200, 200, 200, 200]), (16, 8, [int(900 * (15 + 2 * i) / 45) for i in range(16)])):
+        shared, even = plans(rows, splits, contexts)
+        assert np.array_equal(shared.items, even.items) == fused and (fused or longest(shared) <= 0.75 * longest(even))
     for rows, splits, contexts in ((24, 5, [2000] + [100] * 23), (16, 8, [int(4400 * (15 + 2 * i) / 45) for i in range(16)]), (8, 16, [1300] * 4 + [325] * 4)):
-        shared, even = (build_attention_plan([1] * rows, contexts, 4, 8, None, fixed_splits=splits, share_ranges=share) for share in (True, False))
-        longest = lambda p: int((p.items[:, 3] - p.items[:, 2]).max())
+        shared, even = plans(rows, splits, contexts)
         assert longest(shared) <= 0.72 * longest(even)
+
+
+def test_who_prepares_its_queries_itself():
+    """Mixers say so to the plan: a plain one in the type and head sizes of the fused start, no other."""
+    import types
+
+    import torch
+
+    from llmserver_amd.parts import attention
+    from llmserver_amd.parts.rope import RotaryPosition
+    asked = []
+    ops = types.SimpleNamespace(decode_fusion_fits=lambda dtype, head_dim: dtype == torch.bfloat16 and head_dim % 64 == 0)
+    stage, attention.stage_attention_plan = attention.stage_attention_plan, lambda *args: asked.append(args[8])
+    try:
+        for head_dim, dtype, general in ((64, torch.bfloat16, {}), (64, torch.float32, {}), (48, torch.bfloat16, {}), (64, torch.bfloat16, {"head_gate": True})):
+            attention.GQAttention(64, 4, 2, head_dim, RotaryPosition(head_dim, 1e4), qk_norm_eps=1e-6, **general).prepare(types.SimpleNamespace(ops=ops, dtype=dtype))
+    finally:
+        attention.stage_attention_plan = stage
+    assert asked == [True, False, False, False]
