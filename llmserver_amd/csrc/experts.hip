@@ -11,6 +11,7 @@
 // products are made inside the same two kernels (steps of few tokens), or its output comes ready made.
 #include "common.hpp"
 #include "lds_loads.hpp"
+#include "wide_product.hpp"
 
 using namespace lsa;
 
@@ -658,7 +659,7 @@ LSA_EXPORT int lsa_experts_down(int code, const void* hidden, const void* down, 
 // give; every pair's row is computed on its own, so the results do not depend on it.  The choices are read four a
 // thread at a time; an expert's first place is a sum over 64 lanes and not a walk by one thread (12,288 pairs of 64 experts: 20.7 -> 11.7
 // us; 32,760 pairs: 43 -> 24 us; 192 pairs: 8.8 -> 4.6 us).
-constexpr int TILE_M = 64, WIDE_M = 256;                        // pairs a tile: see below
+constexpr int TILE_M = 64, WIDE_M = WIDE_TILE;                        // pairs a tile: see below
 struct Tile { int expert, first, count; };
 
 __global__ __launch_bounds__(1024) void experts_sort_kernel(const int* __restrict__ chosen, int n_pairs, int experts, int tile_rows,
@@ -714,8 +715,6 @@ __global__ __launch_bounds__(1024) void experts_sort_kernel(const int* __restric
     }
 }
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // C = A . B^T for one tile of 64 sorted pairs and 128 rows of the expert's matrix (K contiguous in both).
 // FORM 0: the products themselves.  FORM 2: max(product, 0)^2.  FORM 1 is GATED:
@@ -843,36 +842,24 @@ __global__ __launch_bounds__(256) void experts_tile_kernel(const bf16_t* __restr
 }
 
 // ---- many pairs an expert ---------------------------------------------------------------------------------------------------
-// C = A . B^T as above for tiles of 256 sorted pairs and 256 rows of the expert's matrix, sixteen wavefronts of 64 x 64 (4 x 4 MFMA tiles
-// of 16 x 16; GATED: 32 gate columns and their 32 up columns).  k in slabs of 64 through two LDS buffers of 64 KB that loads
-// fill without registers (global_load_lds, 16 bytes a lane).
-//   Why this size: a compute unit took 16 to 21 bytes a cycle from L2 whatever the form (tiles of 64 x 256 staged through registers, 535 us
-// for 32,760 pairs of 64 experts of 2,112 at width 2,048; 128 x 256 in three buffers, slabs of 32 or 64, 467 and 445 us), so what
-// counts is products for a byte: 396 us, 716 TFLOP/s.  Beside that a wavefront's own reads of LDS bound it: with its loads taken out the
-// same loop runs at 1.03 PFLOP/s, eight wavefronts of 128 x 64 with two sets of operands as fast (and slower with the loads).
-// A buffer is rows of 128 bytes, 256 of A and then 256 of B: a load asks for whole lines of 128 bytes.  A load writes 64 lanes x 16 bytes to
-// 1 KB (8 rows) in lane order; the eight 16-byte pieces of row r stand at places piece ^ (r / 2 % 8), so that the sixteen lanes whose
-// 16-byte reads are served together (0-3, 12-15, 20-23, 24-27 and so on) meet all 64 banks.
-constexpr int WIDE_N = 256, WIDE_ROWS = WIDE_M + WIDE_N, WIDE_SLAB = 64, WIDE_STEP = WIDE_ROWS * WIDE_SLAB * 2;      // bytes a buffer
-constexpr int WIDE_LOADS = WIDE_ROWS / 8 / 16;                  // of a wavefront a slab
-
-// The workgroup's barrier behind the LDS reads issued so far; loads stay under way.
-__device__ __forceinline__ void everybody_has_read() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
+// C = A . B^T as above for tiles of 256 sorted pairs and 256 rows of the expert's matrix (GATED: 128 gate rows and their up rows, 128 columns of the result).
+//   What bounds it is what passes between the XCDs' L2 and the memory side: a workgroup's share of an expert's matrix is read once for each 256 of its pairs and
+// half of that comes from the neighbour's read.  12,288 pairs of 64 gated experts of 1,408 at width 2,048, chosen unevenly, us a launch, first and second product, with sixteen
+// wavefronts of 64 x 64 in step and now: 251 + 143, 224 + 138 (191 of them the matrices' loads alone); 32,760 pairs of 2,112 without gates 341 + 341, 307 + 316; with the same
+// number of pairs everywhere and experts of 2,048 230 (1.19 PFLOP/s).  No faster: one workgroup a compute unit that goes from tile to tile with its loads running on;
+// shares of the XCDs by work; slabs in another order for each block of columns; the experts' pairs shared evenly by its tiles; three slabs of the matrix in LDS.
 template <int FORM, typename O>
-__global__ __launch_bounds__(1024) void experts_wide_kernel(const bf16_t* __restrict__ a, int a_stride, int pair_div,
+__global__ __launch_bounds__(WIDE_THREADS) void experts_wide_kernel(const bf16_t* __restrict__ a, int a_stride, int pair_div,
                                                            const bf16_t* __restrict__ b, long expert_stride, int b_up_offset,
                                                            const int* __restrict__ sorted, const Tile* __restrict__ tiles_of, int max_tiles,
                                                            O* __restrict__ out, int out_stride, int n_out, int k, float limit, int blocks) {
     constexpr bool GATED = FORM == 1;
-    constexpr int COLUMNS = GATED ? WIDE_N / 2 : WIDE_N;           // output columns of a workgroup
-    __shared__ __attribute__((aligned(1024))) unsigned char buffers[2 * WIDE_STEP];
-    __shared__ int rows_of[WIDE_M];
+    constexpr int COLUMNS = GATED ? WIDE_TILE / 2 : WIDE_TILE;     // output columns of a workgroup
+    __shared__ __attribute__((aligned(1024))) unsigned char buffers[2 * WIDE_BUFFER];
+    __shared__ int rows_of[WIDE_TILE];
     // Workgroups go to the eight XCDs in turn by their number: an XCD gets an eighth of the tiles and walks one expert's (at most
     // eight) through all blocks of columns, so that their rows stay in its L2 while the expert's matrix comes into it once.  What passes
-    // between L2 and memory: 1.1 GB in the case above, 1.5 with groups of four tiles whatever their experts.
+    // between L2 and memory: 1.1 GB for 32,760 pairs of 64 experts of 2,112 at width 2,048, 1.5 with groups of four tiles whatever their experts.
     const int tiles = tiles_of[max_tiles].expert, share = (tiles + 7) / 8, begin = (int)(blockIdx.x % 8) * share, end = min(begin + share, tiles);
     const int index = blockIdx.x / 8, slot = begin + index / blocks;
     if (slot >= end) return;
@@ -882,112 +869,42 @@ __global__ __launch_bounds__(1024) void experts_wide_kernel(const bf16_t* __rest
     const int in_group = index - (group - begin) * blocks;
     const int block_n = in_group / group_tiles, tile = group + in_group % group_tiles;
     const int expert = of.expert;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), col = lane & 15, quad = lane >> 4;
-    const int wave_m = wave >> 2, wave_n = wave & 3;
-    if (threadIdx.x < WIDE_M) rows_of[threadIdx.x] = sorted[tile * WIDE_M + threadIdx.x];
+    if (threadIdx.x < WIDE_TILE) rows_of[threadIdx.x] = sorted[tile * WIDE_TILE + threadIdx.x];
     __syncthreads();
     const int n0 = block_n * COLUMNS;
-    const bf16_t* bm = b + (size_t)expert * expert_stride;
-    // What a lane fetches in each of its wavefront's loads of a slab: 8 rows of A for the first two, of B for the other two.
-    const unsigned lds_begin = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(lds_ptr_t)buffers);
-    const int piece = (lane & 7) ^ ((lane >> 4) + 4 * (wave & 1));            // (row / 2 % 8: a load's rows are 8 * (wave + 16 u) + lane / 8)
-    unsigned offset[WIDE_LOADS];
-#pragma unroll
-    for (int u = 0; u < WIDE_LOADS; ++u) {
-        const int r = 8 * (wave + 16 * u) + (lane >> 3);
-        if (u < WIDE_M / 128) {
-            const int pair = rows_of[r];
-            offset[u] = 2u * ((unsigned)(pair < 0 ? 0 : pair / pair_div) * (unsigned)a_stride + 8 * piece);
-        } else {
-            const int line = r - WIDE_M;                           // GATED: 128 gate rows, then their up rows; rows behind the matrix repeat its last one
-            const int column = min(n0 + (GATED ? line & (WIDE_N / 2 - 1) : line), n_out - 1);
-            offset[u] = 2u * ((unsigned)(column + (GATED && line >= WIDE_N / 2 ? b_up_offset : 0)) * (unsigned)k + 8 * piece);
-        }
-    }
-    const int slabs = (k + WIDE_SLAB - 1) / WIDE_SLAB;
-    const bool half_slab = k % WIDE_SLAB != 0;                     // (k is a multiple of 32: then the last slab is half a slab)
-    unsigned place = lds_begin + 1024 * wave;                      // of the next slab's first load
-    int fetched = 0;
-    auto fetch = [&]() __attribute__((always_inline)) {
-        const unsigned back = half_slab && fetched == slabs - 1 && piece >= 4 ? 64 : 0;          // (what lies behind the rows' end is not read)
-#pragma unroll
-        for (int u = 0; u < WIDE_LOADS; ++u) {
-            load_16_bytes_a_lane_to_lds(u < WIDE_M / 128 ? (const void*)a : (const void*)bm, offset[u] - back, place + 16384 * u);
-            offset[u] += 2 * WIDE_SLAB;
-        }
-        ++fetched;
-        place += fetched % 2 ? WIDE_STEP : -WIDE_STEP;
+    auto a_offset = [&](int r) __attribute__((always_inline)) {
+        const int pair = rows_of[r];                               // (padding stands behind the expert's last pair)
+        return pair < 0 ? NOWHERE : 2u * ((unsigned)(pair / pair_div) * (unsigned)a_stride);
     };
-    // A wavefront whose rows are all padding, or whose columns lie behind the matrix, fetches and waits with the others only.
-    const bool busy = rows_of[64 * wave_m] >= 0 && n0 + wave_n * (COLUMNS / 4) < n_out;
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // (the count below starts from nothing under way)
-    // (the rows that a lane reads are col and multiples of 16 apart: their pieces stand at the same places)
-    const int first_piece = 16 * (quad ^ (col >> 1)), second_piece = 16 * ((quad + 4) ^ (col >> 1));
-    struct Operands { bf16x8 a[4], b[4]; };
-    auto read = [&](Operands& x, int buffer, int at) __attribute__((always_inline)) {
-        const unsigned char* rows = buffers + buffer + col * 128 + at;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x.a[i] = *reinterpret_cast<const bf16x8*>(rows + (64 * wave_m + 16 * i) * 128);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            // GATED: the first half of a wavefront's tiles are its gate columns, the second half their up columns
-            const int r = GATED ? (j < 2 ? 32 * wave_n + 16 * j : WIDE_N / 2 + 32 * wave_n + 16 * (j - 2)) : 64 * wave_n + 16 * j;
-            x.b[j] = *reinterpret_cast<const bf16x8*>(rows + (WIDE_M + r) * 128);
-        }
-        __builtin_amdgcn_sched_barrier(0);                         // (the reads stay in front of the products that they are to hide behind)
+    auto b_offset = [&](int r) __attribute__((always_inline)) {
+        const int column = n0 + (GATED ? r & (WIDE_TILE / 2 - 1) : r);
+        return column >= n_out ? NOWHERE : 2u * ((unsigned)(column + (GATED && r >= WIDE_TILE / 2 ? b_up_offset : 0)) * (unsigned)k);
     };
-    auto multiply = [&](const Operands& x) __attribute__((always_inline)) {
+    const int row_blocks = 1 + (rows_of[64] >= 0) + (rows_of[128] >= 0) + (rows_of[192] >= 0);
+    WideSums sums;
+    wide_product(sums, buffers, a, a_offset, b + (size_t)expert * expert_stride, b_offset, k, __builtin_amdgcn_readfirstlane(row_blocks),
+                 GATED || n0 + WIDE_TILE / 2 < n_out);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+    for (int half = 0; half < 2; ++half)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.a[i], x.b[j], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    Operands x;
-    fetch();
-    if (slabs > 1) fetch();
-    for (int slab = 0; slab < slabs; ++slab) {
-        if (slab + 1 < slabs) loads_landed_then_barrier<WIDE_LOADS>();
-        else loads_landed_then_barrier<0>();
-        const int buffer = slab % 2 * WIDE_STEP;
-        const bool whole = !half_slab || slab + 1 < slabs;
-        if (busy) {
-            read(x, buffer, first_piece);
-            multiply(x);
-            if (whole) read(x, buffer, second_piece);
-        }
-        if (slab + 2 < slabs) {
-            everybody_has_read();
-            fetch();                                               // into this slab's buffer
-        }
-        if (busy && whole) multiply(x);
-    }
-    if (!busy) return;
-    // lane holds rows 4 * quad + r of each 16 x 16 tile, column col
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int pair = rows_of[64 * wave_m + 16 * i + 4 * quad + r];
+        for (int i = 0; i < 4; ++i) {
+            const int pair = rows_of[wide_row(half, i, wave, lane)];
             if (pair < 0) continue;
-            O* o = out + (size_t)pair * out_stride;
-            if (GATED) {
+            O* o = out + (size_t)pair * out_stride + n0;
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int f = n0 + 32 * wave_n + 16 * j + col;
-                    if (f < n_out) o[f] = (O)gated_activation(acc[i][j][r], acc[i][j + 2][r], limit);
-                }
-            } else {
+            for (int other = 0; other < (GATED ? 1 : 2); ++other) {
+                const int c = wide_column(other, wave, lane);
+                if (n0 + c >= n_out) continue;                     // (n_out is a multiple of 32)
+                struct alignas(16) Eight { O v[8]; } eight;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int c = n0 + 64 * wave_n + 16 * j + col;
-                    if (c < n_out) o[c] = (O)(FORM == 2 ? rectified_square(acc[i][j][r]) : acc[i][j][r]);
-                }
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float z = sums[half][other][i][j][r];
+                        eight.v[4 * j + r] = (O)(GATED ? gated_activation(z, sums[half][1][i][j][r], limit) : FORM == 2 ? rectified_square(z) : z);
+                    }
+                *reinterpret_cast<Eight*>(o + c) = eight;
             }
         }
 }
@@ -1038,7 +955,7 @@ __global__ __launch_bounds__(256) void experts_combine_kernel(const float* __res
 // Whether the wide kernel can multiply such a step: its loads straight into LDS are of 16 bytes at multiples of 16 (`aligned`: x, gate_up and down
 // begin at such), from offsets of 32 bits.
 static bool wide_fits(int pairs, int inter, int width, bool aligned) {
-    return aligned && (size_t)pairs * (size_t)(inter > width ? inter : width) * 2 < 0xFFFFFFFFu && (size_t)2 * inter * width * 2 < 0xFFFFFFFFu;
+    return aligned && (size_t)pairs * (size_t)(inter > width ? inter : width) * 2 < BUFFER_BYTES && (size_t)2 * inter * width * 2 < BUFFER_BYTES;
 }
 
 // Pairs a tile that lsa_experts_tiled should take for a step with so many pairs: 256 (the wide kernel) or 64.  Wide tiles pay from some 40 pairs
@@ -1050,8 +967,8 @@ static bool wide_fits(int pairs, int inter, int width, bool aligned) {
 // 96 pairs 133, 128; 8 of 1,408 at 2,048 (112) with 192 pairs 75, 95.
 LSA_EXPORT int lsa_experts_tile_rows(int pairs, int experts, int inter, int width, int plain, int aligned) {
     if (pairs < 40 * experts || !wide_fits(pairs, inter, width, aligned != 0)) return TILE_M;
-    const long tiles = (long)experts * ((pairs / experts + WIDE_M - 1) / WIDE_M), columns = plain ? WIDE_N : WIDE_N / 2;
-    return tiles * ((inter + columns - 1) / columns) + tiles * ((width + WIDE_N - 1) / WIDE_N) >= 224 ? WIDE_M : TILE_M;
+    const long tiles = (long)experts * ((pairs / experts + WIDE_M - 1) / WIDE_M), columns = plain ? WIDE_TILE : WIDE_TILE / 2;
+    return tiles * ((inter + columns - 1) / columns) + tiles * ((width + WIDE_TILE - 1) / WIDE_TILE) >= 224 ? WIDE_M : TILE_M;
 }
 
 // Ints of scratch memory that lsa_experts_tiled wants: the sorted pairs, then the tiles and their number.
@@ -1079,15 +996,15 @@ LSA_EXPORT int lsa_experts_tiled(const void* x, const void* gate_up, const void*
     const bf16_t* dn = (const bf16_t*)down;
     bf16_t* hb = (bf16_t*)hidden;
     if (wide) {
-        const int gated_blocks = (inter + WIDE_N / 2 - 1) / (WIDE_N / 2), plain_blocks = (inter + WIDE_N - 1) / WIDE_N, down_blocks = (width + WIDE_N - 1) / WIDE_N;
+        const int gated_blocks = (inter + WIDE_TILE / 2 - 1) / (WIDE_TILE / 2), plain_blocks = (inter + WIDE_TILE - 1) / WIDE_TILE, down_blocks = (width + WIDE_TILE - 1) / WIDE_TILE;
         const int numbers = 8 * ((max_tiles + 7) / 8);
         if (plain)
-            experts_wide_kernel<2, bf16_t><<<numbers * plain_blocks, 1024, 0, stream>>>(xb, width, top, gu, (long)inter * width, 0, sorted, tiles_of, max_tiles, hb,
+            experts_wide_kernel<2, bf16_t><<<numbers * plain_blocks, WIDE_THREADS, 0, stream>>>(xb, width, top, gu, (long)inter * width, 0, sorted, tiles_of, max_tiles, hb,
                                                                                        inter, inter, width, 0.f, plain_blocks);
         else
-            experts_wide_kernel<1, bf16_t><<<numbers * gated_blocks, 1024, 0, stream>>>(xb, width, top, gu, (long)2 * inter * width, inter, sorted, tiles_of,
+            experts_wide_kernel<1, bf16_t><<<numbers * gated_blocks, WIDE_THREADS, 0, stream>>>(xb, width, top, gu, (long)2 * inter * width, inter, sorted, tiles_of,
                                                                                        max_tiles, hb, inter, inter, width, limit, gated_blocks);
-        experts_wide_kernel<0, float><<<numbers * down_blocks, 1024, 0, stream>>>(hb, inter, 1, dn, (long)width * inter, 0, sorted, tiles_of, max_tiles, y, width,
+        experts_wide_kernel<0, float><<<numbers * down_blocks, WIDE_THREADS, 0, stream>>>(hb, inter, 1, dn, (long)width * inter, 0, sorted, tiles_of, max_tiles, y, width,
                                                                                  width, inter, 0.f, down_blocks);
     } else {
         const bool many = pairs >= 16 * experts;                // pairs to an expert: wide tiles pay
