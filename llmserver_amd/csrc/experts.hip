@@ -845,8 +845,8 @@ __global__ __launch_bounds__(256) void experts_tile_kernel(const bf16_t* __restr
 // C = A . B^T as above for tiles of 256 sorted pairs and 256 rows of the expert's matrix (GATED: 128 gate rows and their up rows, 128 columns of the result).
 //   What bounds it is what passes between the XCDs' L2 and the memory side: a workgroup's share of an expert's matrix is read once for each 256 of its pairs and
 // half of that comes from the neighbour's read.  12,288 pairs of 64 gated experts of 1,408 at width 2,048, chosen unevenly, us a launch, first and second product, with sixteen
-// wavefronts of 64 x 64 in step and now: 251 + 143, 224 + 138 (191 of them the matrices' loads alone); 32,760 pairs of 2,112 without gates 341 + 341, 307 + 316; with the same
-// number of pairs everywhere and experts of 2,048 230 (1.19 PFLOP/s).  No faster: one workgroup a compute unit that goes from tile to tile with its loads running on;
+// wavefronts of 64 x 64 in step and now: 251 + 143, 224 + 138 (191 of them the matrices' loads alone); 32,760 pairs of 2,112 without gates, all launches 808, 710; with the same
+// number of pairs everywhere and experts of 2,048 230 for the first product (1.19 PFLOP/s).  No faster: one workgroup a compute unit that goes from tile to tile with its loads running on;
 // shares of the XCDs by work; slabs in another order for each block of columns; the experts' pairs shared evenly by its tiles; three slabs of the matrix in LDS.
 template <int FORM, typename O>
 __global__ __launch_bounds__(WIDE_THREADS) void experts_wide_kernel(const bf16_t* __restrict__ a, int a_stride, int pair_div,
