@@ -1,0 +1,272 @@
+// Matrix products of many rows, Y[M, N] = X[M, K] . W[N, K]^T in bfloat16 with 32-bit sums, for prompts and portions of prompts: where the library's tiles leave
+// compute units idle (some hundred rows, small weights), and where what follows the product can go into it:
+//   plain       round(sum)
+//   gated       W stacks a gate matrix on an up matrix ([2N, K], gate first): round(act(gate) * up), [M, N]
+//   activated   round(act(sum))
+//   sums        the sums themselves, of `parts` ranges of K, [parts, M, N] in 32-bit: whoever reads the product adds them up
+//
+// Two kernels.  The one below has small tiles, which a step of a few hundred rows has enough of to go round the compute units; the other one multiplies tiles
+// of 256 x 256 (wide_product.hpp) for prompts of a thousand tokens and more.
+#include "common.hpp"
+#include "lds_loads.hpp"
+#include "wide_product.hpp"
+
+using namespace lsa;
+
+enum Form { PLAIN, GATED, ACTIVATED, SUMS };
+enum Activation { SILU, GELU_TANH, RELU2 };          // (the last one has no gated form)
+
+__device__ __forceinline__ float activation_of(int activation, float z) {
+    if (activation == SILU) return z / (1.f + expf(-z));
+    if (activation == GELU_TANH) return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+    const float r = fmaxf(z, 0.f);
+    return r * r;
+}
+
+constexpr int XCDS = 8;
+// Workgroups go to the eight XCDs in turn by their number: an XCD gets neighbours of an order that walks eight rows of tiles through all columns, so that the
+// rows of X stay in its L2 while every row of W comes into it once.
+__device__ __forceinline__ bool tile_of_workgroup(int rows, int columns, int& row, int& column) {
+    const int tiles = rows * columns, share = (tiles + XCDS - 1) / XCDS, index = blockIdx.x / XCDS, tile = (int)(blockIdx.x % XCDS) * share + index;
+    if (index >= share || tile >= tiles) return false;
+    const int group = tile / (8 * columns), within = tile - group * 8 * columns, group_rows = min(8, rows - 8 * group);
+    row = 8 * group + within % group_rows;
+    column = within / group_rows;
+    return true;
+}
+static int workgroups(int M, int N, int tile_m, int tile_n) {
+    const long tiles = (long)((M + tile_m - 1) / tile_m) * ((N + tile_n - 1) / tile_n);
+    return tiles > (1 << 24) - XCDS ? -1 : (int)((tiles + XCDS - 1) / XCDS * XCDS);
+}
+
+constexpr int SLAB = 64;
+
+// Tiles of 16 MI WAVES_M rows x 32 WAVES_N columns (GATED: half of them gate columns, half their up columns), a wavefront 16 MI x 32.  Slabs of 64 of K go
+// through BUFFERS buffers of LDS that loads fill without registers, BUFFERS - 1 slabs ahead; one barrier a slab.  grid (tiles, parts), a part of K each.
+//   What bounds it: with every tile on a compute unit of its own a slab takes 0.25 us (64 x 64 tiles, 4 wavefronts), 0.31 (128 x 64, 8) and 0.5 (128 x 128, 8), in
+// turn waiting, reading LDS and multiplying, and a launch 3 to 4 us around them; the kernel is for products of one such round, whatever the chip could
+// do with more.  us alone, library and here: 190 rows, 4,096 x 2,048 13.8, 11.9; 2,048 x 2,048 in four parts 12.0, 7.6; 12,288 x 2,048 26.3, 20.6; 2,048 x 6,144 in four
+// parts 22.9, 13.6; 1,000 rows, 4,096 x 2,048 23.9, 20.7; 2,048 rows, 2,048 x 2,048 24.6, 21.9.  No faster: operands of half a slab read while the other half is
+// multiplied; slabs shared by groups of wavefronts that add up in LDS; four wavefronts of 64 x 64.
+template <int WAVES_M, int WAVES_N, int MI, int BUFFERS, int FORM>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void product_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out,
+                                                                         int M, int N, int K, int activation) {
+    constexpr int TILE_M = WAVES_M * MI * 16, TILE_B = WAVES_N * 32, COLUMNS = FORM == GATED ? TILE_B / 2 : TILE_B, WAVES = WAVES_M * WAVES_N;
+    constexpr int BUFFER = (TILE_M + TILE_B) * SLAB * 2, A_LOADS = TILE_M / 8 / WAVES, B_LOADS = TILE_B / 8 / WAVES, LOADS = A_LOADS + B_LOADS;
+    static_assert(TILE_M % (8 * WAVES) == 0 && TILE_B % (8 * WAVES) == 0 && BUFFERS * BUFFER <= 160 * 1024, "a load is 8 rows");
+    __shared__ __attribute__((aligned(1024))) unsigned char buffers[BUFFERS * BUFFER];
+    int tile_m, tile_n;
+    if (!tile_of_workgroup((M + TILE_M - 1) / TILE_M, (N + COLUMNS - 1) / COLUMNS, tile_m, tile_n)) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), col = lane & 15, quad = lane >> 4;
+    const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N, m0 = tile_m * TILE_M, n0 = tile_n * COLUMNS;
+    const int all = K / SLAB, first = (int)((long)all * blockIdx.y / gridDim.y), slabs = (int)((long)all * (blockIdx.y + 1) / gridDim.y) - first;
+    const buffer_t a_buffer = buffer_at(x + (size_t)m0 * K), b_buffer = buffer_at(w + (FORM == GATED ? 0 : (size_t)n0 * K));
+    // The eight 16-byte pieces of row r stand at places piece ^ f(r), so that sixteen lanes whose reads are served together meet all 64 banks.  Rows of W are read in
+    // the order of the columns (GATED: sixteen gate rows and their up rows for each 32), or so that a lane has eight neighbouring columns of the result.
+    unsigned a_at[A_LOADS], b_at[B_LOADS];
+#pragma unroll
+    for (int u = 0; u < A_LOADS; ++u) {
+        const int r = 8 * (wave + WAVES * u) + (lane >> 3);
+        a_at[u] = (unsigned)min(r, M - 1 - m0) * (unsigned)(2 * K) + 16 * ((lane & 7) ^ (r >> 1 & 7));
+    }
+#pragma unroll
+    for (int u = 0; u < B_LOADS; ++u) {
+        const int r = 8 * (wave + WAVES * u) + (lane >> 3);
+        if (FORM == GATED) {
+            const int c = min(n0 + 16 * (r >> 5) + (r & 15), N - 1);
+            b_at[u] = (unsigned)(c + (r & 16 ? N : 0)) * (unsigned)(2 * K) + 16 * ((lane & 7) ^ (r >> 1 & 7));
+        } else {
+            b_at[u] = (unsigned)min(r, N - 1 - n0) * (unsigned)(2 * K) + 16 * ((lane & 7) ^ ((r >> 1 & 1) | (r >> 3 & 3) << 1));
+        }
+    }
+    unsigned place = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(lds_ptr_t)buffers) + 1024 * wave;
+    int asked = 0, slot = 0;
+    auto ask = [&]() __attribute__((always_inline)) {
+        const unsigned from = (first + min(asked, slabs - 1)) * (2 * SLAB);       // (behind the last slab: that once more, into a buffer that nobody reads again)
+#pragma unroll
+        for (int u = 0; u < A_LOADS; ++u) load_16_bytes_a_lane_to_lds(a_buffer, a_at[u], from, place + 1024 * WAVES * u);
+#pragma unroll
+        for (int u = 0; u < B_LOADS; ++u) load_16_bytes_a_lane_to_lds(b_buffer, b_at[u], from, place + TILE_M * 128 + 1024 * WAVES * u);
+        ++asked;
+        slot = slot == BUFFERS - 1 ? 0 : slot + 1;
+        place += slot == 0 ? -(BUFFERS - 1) * BUFFER : BUFFER;
+    };
+    f32x4 sums[MI][2];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) sums[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int pieces[2] = {16 * (quad ^ (col >> 1)), 16 * ((quad + 4) ^ (col >> 1))};
+    const unsigned char* a_rows = buffers + (16 * MI * wave_m + col) * 128;
+    const unsigned char* b_rows = buffers + (TILE_M + 32 * wave_n + (FORM == GATED ? col : 8 * (col >> 2) + (col & 3))) * 128;
+    constexpr int B_STEP = (FORM == GATED ? 16 : 4) * 128;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // (the count below starts from nothing under way)
+#pragma unroll
+    for (int b = 0; b < BUFFERS - 1; ++b) ask();
+    int buffer = 0;
+    for (int slab = 0; slab < slabs; ++slab) {
+        loads_landed_then_barrier<LOADS * (BUFFERS - 2)>();        // and everybody is through with the slab before this one, whose buffer is asked for
+        bf16x8 a[2][MI], b[2][2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) a[s][i] = *reinterpret_cast<const bf16x8*>(a_rows + buffer + 2048 * i + pieces[s]);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) b[s][j] = *reinterpret_cast<const bf16x8*>(b_rows + buffer + B_STEP * j + pieces[s]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        ask();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][j], a[s][i], sums[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        buffer = buffer == (BUFFERS - 1) * BUFFER ? 0 : buffer + BUFFER;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // (no load may land when this LDS is somebody else's)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int m = m0 + 16 * (MI * wave_m + i) + col;
+        if (m >= M) continue;
+        if (FORM == GATED) {
+            const int n = n0 + 16 * wave_n + 4 * quad;             // (N is a multiple of 8 in every form)
+            if (n >= N) continue;
+            struct alignas(8) Four { bf16_t v[4]; } four;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) four.v[r] = (bf16_t)(activation_of(activation, sums[i][0][r]) * sums[i][1][r]);
+            *reinterpret_cast<Four*>((bf16_t*)out + (size_t)m * N + n) = four;
+            continue;
+        }
+        const int n = n0 + 32 * wave_n + 8 * quad;
+        if (n >= N) continue;
+        if (FORM == SUMS) {
+            float* to = (float*)out + ((size_t)blockIdx.y * M + m) * N + n;
+            *reinterpret_cast<f32x4*>(to) = sums[i][0];
+            *reinterpret_cast<f32x4*>(to + 4) = sums[i][1];
+            continue;
+        }
+        bf16x8 eight;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const float z = sums[i][r >> 2][r & 3];
+            eight[r] = (bf16_t)(FORM == ACTIVATED ? activation_of(activation, z) : z);
+        }
+        *reinterpret_cast<bf16x8*>((bf16_t*)out + (size_t)m * N + n) = eight;
+    }
+}
+
+// The gated form on tiles of 256 x 256: 256 rows, 128 columns of the result.
+//   The library's products of such sizes run at what power allows, as this one does; what it saves is the activation's launch and the way of the gate's and the up
+// projection's columns through memory.  us with the activation, library and here: 2,048 rows, 12,288 x 4,096 316, 304; 8,192 x 4,096 210, 203; 4,096 rows 593, 576 and 400, 390.
+// Without a gate there is half as much to save (2,048 rows, 8,192 x 4,096 103, 107): that stays the library's.
+__global__ __launch_bounds__(WIDE_THREADS) void wide_gated_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf16_t* __restrict__ out, int M, int N, int K,
+                                                                  int activation) {
+    constexpr int COLUMNS = WIDE_TILE / 2;
+    __shared__ __attribute__((aligned(1024))) unsigned char buffers[2 * WIDE_BUFFER];
+    int tile_m, tile_n;
+    if (!tile_of_workgroup((M + WIDE_TILE - 1) / WIDE_TILE, (N + COLUMNS - 1) / COLUMNS, tile_m, tile_n)) return;
+    const int m0 = tile_m * WIDE_TILE, n0 = tile_n * COLUMNS;
+    auto a_offset = [&](int r) __attribute__((always_inline)) { return m0 + r < M ? (unsigned)r * (unsigned)(2 * K) : NOWHERE; };
+    auto b_offset = [&](int r) __attribute__((always_inline)) {    // gate rows, then their up rows
+        const int c = r & (COLUMNS - 1);
+        return n0 + c >= N ? NOWHERE : (unsigned)(c + (r >= COLUMNS ? N : 0)) * (unsigned)(2 * K);
+    };
+    WideSums sums;
+    wide_product(sums, buffers, x + (size_t)m0 * K, a_offset, w + (size_t)n0 * K, b_offset, K, min(4, (M - m0 + 63) / 64), true);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = n0 + wide_column(0, wave, lane);
+    if (n >= N) return;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = m0 + wide_row(half, i, wave, lane);
+            if (m >= M) continue;
+            bf16x8 eight;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) eight[r] = (bf16_t)(activation_of(activation, sums[half][0][i][r >> 2][r & 3]) * sums[half][1][i][r >> 2][r & 3]);
+            *reinterpret_cast<bf16x8*>(out + (size_t)m * N + n) = eight;
+        }
+}
+
+// What lsa_product can be asked for: a tile, and for SUMS the parts of K, as 16 parts + tile.
+enum Tile { NONE, SMALL, TALL, LARGE, WIDE };
+struct TileShape { int rows, columns; double start, slab; };       // columns of W; us of a launch with a tile a compute unit, and a slab's
+static const TileShape SHAPES[] = {{0, 0, 0, 0}, {64, 64, 3.0, 0.31}, {128, 64, 3.6, 0.31}, {128, 128, 4.2, 0.50}, {256, 256, 4.5, 0}};
+constexpr int UNITS = 256;                                         // compute units
+constexpr int MOST_PARTS = 8;
+
+static bool fits(int form, long M, long N, long K) {
+    return M >= 1 && N >= 8 && K >= SLAB && K % SLAB == 0 && N % 8 == 0 && (form == GATED ? 2 * N : 256) * K * 2 + K * 2 < (long)BUFFER_BYTES && 256 * K * 2 < (long)BUFFER_BYTES;
+}
+
+// The tile (and parts) for a product of these sizes, or 0 where the library's product is expected to be as fast (with the kernel of the activation behind it).  Both
+// times are lines through what was measured at 17 to 3,000 rows of 31 products of this package's models: a launch's start and a slab's time for the tiles here,
+// for the library (whose own choice of tiles nobody can foretell) a start, K and the operations.  Over 186 of them at random rows, the way taken against the library: gated 1.12
+// times as fast, plain 1.06, activated 1.12, sums with the norm behind them 1.15, the worst 0.94.  A product whose tiles do not go round the compute units in one
+// round stays the library's unless it is gated and large.
+LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
+    if (form < PLAIN || form > SUMS || !fits(form, M, N, K)) return NONE;
+    const double slabs = K / SLAB, weights = (form == GATED ? 2.0 : 1.0) * N, megabytes = weights * K * 2e-6, gigaflops = 2e-9 * M * weights * K;
+    double best = 1e30;
+    int plan = NONE;
+    for (int tile = SMALL; tile <= LARGE; ++tile) {
+        const TileShape& shape = SHAPES[tile];
+        const int columns = form == GATED ? shape.columns / 2 : shape.columns;
+        const long tiles = (long)((M + shape.rows - 1) / shape.rows) * ((N + columns - 1) / columns);
+        for (int parts = 1; parts <= (form == SUMS ? MOST_PARTS : 1); parts *= 2) {
+            if (tiles * parts > UNITS || slabs < 4 * parts) continue;
+            double us = shape.start + shape.slab * ((K / SLAB + parts - 1) / parts) * (tiles * parts > 7 * UNITS / 8 ? 1.15 : 1.0);
+            us = us > megabytes / 5.2 + 3.0 ? us : megabytes / 5.2 + 3.0;
+            if (form == SUMS) us += parts * 8e-6 * M * N / 4.0;    // written and read
+            if (us < best) {
+                best = us;
+                plan = 16 * parts + tile;
+            }
+        }
+    }
+    double library = 10.0 + 0.0016 * K + (gigaflops < 40 ? 0.75 * gigaflops : 30 + 0.69 * (gigaflops - 40));
+    if (M <= 64 && N <= 2048 && form != GATED) library = 4.0 + 0.0022 * K;        // (it cuts K there)
+    library = library > megabytes / 4.3 ? library : megabytes / 4.3;
+    if (form == GATED) library += 3.5 + 6e-6 * M * N / 5.0;
+    if (form == ACTIVATED) library += 3.5 + 4e-6 * M * N / 5.0;
+    if (form == GATED) {
+        const long tiles = (long)((M + WIDE_TILE - 1) / WIDE_TILE) * ((N + WIDE_TILE / 2 - 1) / (WIDE_TILE / 2)), last = tiles % UNITS;
+        // (a slab takes 1.05 us where few compute units work, 1.5 where all do: power)
+        const double us = 3.0 + tiles / UNITS * (4.5 + 1.5 * slabs) + (last ? 4.5 + (1.05 + 0.45 * last / UNITS) * slabs : 0.0);
+        if (us < best && us < 0.97 * library) return 16 + WIDE;
+    }
+    return best < (form == SUMS ? 0.9 : 0.95) * library ? plan : NONE;
+}
+
+template <int FORM>
+static int launch(int tile, int parts, const bf16_t* x, const bf16_t* w, void* out, int M, int N, int K, int activation, hipStream_t stream) {
+    const int columns = FORM == GATED ? SHAPES[tile].columns / 2 : SHAPES[tile].columns, blocks = workgroups(M, N, SHAPES[tile].rows, columns);
+    if (blocks < 0) return -1;
+    const dim3 grid(blocks, parts);
+    if (tile == SMALL) product_kernel<2, 2, 2, 5, FORM><<<grid, 256, 0, stream>>>(x, w, out, M, N, K, activation);
+    else if (tile == TALL) product_kernel<4, 2, 2, 6, FORM><<<grid, 512, 0, stream>>>(x, w, out, M, N, K, activation);
+    else product_kernel<2, 4, 4, 4, FORM><<<grid, 512, 0, stream>>>(x, w, out, M, N, K, activation);
+    LSA_LAUNCH_CHECK();
+}
+
+// plan: what lsa_product_plan gave, or any other tile (1 to 4; with 16 parts, 1 to 8, for SUMS).  x, w and out begin at multiples of 16 bytes.
+LSA_EXPORT int lsa_product(int plan, int form, int activation, const void* x, const void* w, void* out, int M, int N, int K, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    const int tile = plan % 16, parts = plan / 16;
+    if (form < PLAIN || form > SUMS || !fits(form, M, N, K) || tile < SMALL || tile > WIDE || parts < 1 || parts > MOST_PARTS || parts > K / SLAB
+        || (parts > 1 && form != SUMS) || activation < SILU || activation > (form == GATED ? GELU_TANH : RELU2) || (((size_t)x | (size_t)w | (size_t)out) & 15)) return -1;
+    const bf16_t *xb = (const bf16_t*)x, *wb = (const bf16_t*)w;
+    if (tile != WIDE) {
+        if (form == PLAIN) return launch<PLAIN>(tile, parts, xb, wb, out, M, N, K, activation, stream);
+        if (form == GATED) return launch<GATED>(tile, parts, xb, wb, out, M, N, K, activation, stream);
+        if (form == ACTIVATED) return launch<ACTIVATED>(tile, parts, xb, wb, out, M, N, K, activation, stream);
+        return launch<SUMS>(tile, parts, xb, wb, out, M, N, K, activation, stream);
+    }
+    const int blocks = workgroups(M, N, WIDE_TILE, WIDE_TILE / 2);
+    if (blocks < 0 || form != GATED) return -1;
+    wide_gated_kernel<<<blocks, WIDE_THREADS, 0, stream>>>(xb, wb, (bf16_t*)out, M, N, K, activation);
+    LSA_LAUNCH_CHECK();
+}

@@ -26,7 +26,7 @@ ARCH = "gfx950"
 FLAGS = ["-O3", f"--offload-arch={ARCH}", "-shared", "-fPIC", "-std=c++17",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 HEAD_DIMS = tuple(range(16, 257, 16))
-BASE_MODULES = ("elementwise", "rope_kv", "sampling", "gemm")
+BASE_MODULES = ("elementwise", "rope_kv", "sampling", "gemm", "product")
 # Libraries that only some models call (a 32-bit residual stream, attention over a latent, routed experts, mixers with a
 # recurrent state, the delta rule, state-space mixers, attention whose projections are convolved or mixed): loaded, and compiled if need be, when the first such call is made.
 PART_MODULES = ("stream", "latent", "experts", "recurrent", "delta", "statespace", "compose")

@@ -101,6 +101,8 @@ _SIGNATURES = {
     "lsa_attention_is_bf16": [],
     "lsa_gemm_skinny": [c_int, _P, _P, _P, c_int, c_int, c_int, c_int, _P, c_int, c_float, _P, c_int, _P],
     "lsa_gemm_few_f32_fits": [c_int, c_int, c_int],
+    "lsa_product_plan": [c_int, c_int, c_int, c_int],
+    "lsa_product": [c_int, c_int, c_int, _P, _P, _P, c_int, c_int, c_int, _P],
     "lsa_gemm_few_f32": [_P, _P, _P, c_int, c_int, c_int, _P, _P, c_int, c_float, _P],
     "lsa_gemm_few_f32_gated": [_P, _P, _P, c_int, c_int, c_int, _P, c_int, c_float, _P],
     "lsa_gemm_few_f32_parts": [c_int],

@@ -97,6 +97,7 @@ class HipOps(KernelNamespace):
         self._rope_kv = library.load("rope_kv")
         self._sampling = library.load("sampling")
         self._gemm = library.load("gemm")
+        self._product = library.load("product")
         self._attention = {}
         self._parts_libraries = {}
         self.skinny_rows = SKINNY_GEMM_ROWS
@@ -420,6 +421,10 @@ class HipOps(KernelNamespace):
                 out = torch.empty((x.shape[0], weight.shape[0]), device=x.device, dtype=torch.bfloat16) if out is None else out
                 _launched(self._elementwise.lsa_sum_parts(_ptr(sums), sums.shape[0], _ptr(out), x.shape[0], weight.shape[0], _stream()), "sum_parts")
                 return out
+        if bias is None and not rows_per_workgroup and (out is None or not out_float32):
+            done = self._tiled_product("plain", x, weight, out=out, out_float32=out_float32)
+            if done is not None:
+                return done
         if out_float32 and x.dtype != torch.float32:
             y = torch.mm(x, weight.t(), out_dtype=torch.float32)
         elif bias is not None and bias_rounded is not None and bias_rounded.dtype == x.dtype and x.dtype != torch.float32:
@@ -436,6 +441,9 @@ class HipOps(KernelNamespace):
         rounding), behind the library's product otherwise."""
         if self._few_rows(x, weight) and not self.library_is_faster("plain", x, weight, False, False):
             return self.linear_few_rows(x, weight, activation=activation)
+        done = self._tiled_product("activated", x, weight, activation) if activation in self.PLAIN_ACTIVATIONS else None
+        if done is not None:
+            return done
         y = self.linear(x, weight)
         self.activation_(y, activation)
         return y
@@ -472,6 +480,36 @@ class HipOps(KernelNamespace):
         _launched(self._gemm.lsa_gemm_skinny(1 if out_float32 else 0, _ptr(x), _ptr(weight), _ptr(out), rows, weight.shape[0], width,
                                              int(rows_per_workgroup), sums, parts, eps, _ptr(bias) if bias is not None else None,
                                              0 if activation is None else 1 + self.PLAIN_ACTIVATIONS.index(activation), _stream()), "gemm_skinny")
+        return out
+
+    PRODUCT_FORMS = ("plain", "gated", "activated", "sums")           # what lsa_product computes (its codes)
+
+    def _tiled_product(self, form, x, weight, activation="silu", out=None, out_float32=False):
+        """The product of many rows by this package's own tiles where they are expected to be faster than the library's (the rule stands in ``csrc/product.hip``,
+        by sizes alone), else None.  ``form``: "plain"; "gated", ``act(gate) * up`` with ``weight [2I, K]``; "activated"; "sums", float32 partial sums ``[parts, T,
+        out]`` over ranges of the inner dimension, where there are several.  Whole bfloat16 tensors in their natural order at multiples of 16 bytes, all on the GPU that launches go
+        to, and nobody who follows the call; anything else is the library's, which refuses what does not fit together."""
+        if not (x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and x.dim() == weight.dim() == 2 and x.device == weight.device and x.shape[0] > self.skinny_rows
+                and x.shape[1] == weight.shape[1] and x.is_contiguous() and weight.is_contiguous()):
+            return None
+        (rows, width), code = x.shape, self.PRODUCT_FORMS.index(form)
+        columns = weight.shape[0] // 2 if form == "gated" else weight.shape[0]
+        if form == "gated" and weight.shape[0] % 2:
+            return None
+        plan = self._product.lsa_product_plan(code, rows, columns, width)
+        if not plan or (form == "sums" and plan < 32) or _followed(x, weight, out) or not _on_current_gpu(x) or (x.data_ptr() | weight.data_ptr()) % 16:
+            return None
+        if out is not None:
+            if not (out.dtype == torch.bfloat16 and out.device == x.device and out.is_contiguous() and tuple(out.shape) == (rows, columns) and out.data_ptr() % 16 == 0):
+                return None
+        elif form == "sums":
+            out = torch.empty((plan // 16, rows, columns), device=x.device, dtype=torch.float32)
+        else:
+            out = torch.empty((rows, columns), device=x.device, dtype=torch.float32 if out_float32 else torch.bfloat16)
+        if out_float32:
+            code = self.PRODUCT_FORMS.index("sums")                   # of one part
+        activations = self.ACTIVATIONS if form == "gated" else self.PLAIN_ACTIVATIONS
+        _launched(self._product.lsa_product(plan, code, activations.index(activation), _ptr(x), _ptr(weight), _ptr(out), rows, columns, width, _stream()), "product")
         return out
 
     SPLIT_ROWS = 128        # most rows the product that leaves partial sums takes (it starts above the few-row kernels')
@@ -545,7 +583,9 @@ class HipOps(KernelNamespace):
         rows, width = x.shape
         if rows > self.SPLIT_ROWS and x.shape[1] == weight.shape[1]:
             parts = self.library_parts(x, weight)      # beyond this repository's product: the library's, whole or in ranges
-            return self._in_parts(x, weight, parts) if parts else None
+            if parts:
+                return self._in_parts(x, weight, parts)
+            return self._tiled_product("sums", x, weight) if self.split_products else None
         if not ((0 if few_rows_too else self.skinny_rows) < rows <= self.SPLIT_ROWS) or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 \
                 or x.shape[1] != weight.shape[1] or not self.split_products:
             return None
@@ -615,7 +655,7 @@ class HipOps(KernelNamespace):
         rows, width = x.shape
         inter = gate_up_weight.shape[0] // 2
         if activation not in self.FUSED_ACTIVATIONS:
-            return None
+            return None if row_scale is not None or pairs_per_workgroup or activation not in self.ACTIVATIONS else self._tiled_product("gated", x, gate_up_weight, activation)
         if x.dtype == torch.float32:
             if pairs_per_workgroup or gate_up_weight.shape[1] != width or gate_up_weight.shape[0] % 2 or not self._fuses_float32(x, gate_up_weight, row_scale):
                 return None
@@ -629,7 +669,8 @@ class HipOps(KernelNamespace):
                 return None
             sums = self._partial_sums_to_add(x, gate_up_weight, gated=True)
             if sums is None:
-                return self._linear_gated_beyond_few_rows(x, gate_up_weight)
+                done = self._linear_gated_beyond_few_rows(x, gate_up_weight)
+                return done if done is not None else self._tiled_product("gated", x, gate_up_weight, activation)
             out = torch.empty((rows, inter), device=x.device, dtype=torch.bfloat16)
             _launched(self._elementwise.lsa_gated_parts(_ptr(sums), sums.shape[0], _ptr(out), rows, inter, self.ACTIVATIONS.index(activation), _stream()),
                       "gated_parts")

@@ -1,0 +1,142 @@
+"""Products of many rows on this package's own tiles (``csrc/product.hip``) at the edges of the tiles, against 64 bits, and who gets them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+FORMS = ("plain", "gated", "activated", "sums")
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from llmserver_amd.kernels import default_ops
+    return default_ops()
+
+
+def drawn(rows, columns, inner, seed):
+    generator = torch.Generator("cuda").manual_seed(seed)
+    x = torch.randn(rows, inner, device="cuda", generator=generator).to(torch.bfloat16)
+    return x, (torch.randn(columns, inner, device="cuda", generator=generator) * inner ** -0.5).to(torch.bfloat16)
+
+
+def silu(z):
+    return z * torch.sigmoid(z)
+
+
+def gelu(z):
+    return torch.nn.functional.gelu(z, approximate="tanh")
+
+
+# Rows and columns around the edges of tiles of 64, 128 and 256, from one slab of the inner dimension to more than there are buffers for.
+@pytest.mark.parametrize("rows,columns,inner", [(1, 8, 64), (63, 72, 128), (64, 64, 192), (65, 136, 256), (127, 128, 320), (129, 264, 384), (191, 40, 448), (255, 256, 512),
+                                                (257, 520, 576), (300, 200, 1024)])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4])
+@pytest.mark.parametrize("form", FORMS)
+def test_every_tile_at_its_edges(ops, form, tile, rows, columns, inner):
+    """A sum in 32 bits is off by at most (inner + 1) 2^-24 of the sum of its products' sizes, the activations' slopes are below 1.13 (the square's: twice the sum),
+    and the one rounding (bfloat16 has eight bits) takes up to 2^-8 of the result."""
+    if tile == 4 and form != "gated":
+        pytest.skip("tiles of 256 have the gated form only")
+    print(f"tiled product {form} {tile} {rows} {columns} {inner}", flush=True)
+    x, weight = drawn(rows, 2 * columns if form == "gated" else columns, inner, rows + inner)
+    exact, sizes = x.double() @ weight.double().T, x.double().abs() @ weight.double().abs().T
+    off = (inner + 1) * 2.0 ** -24 * sizes
+    lib = ops._product
+    for activation in range({"gated": 2, "activated": 3}.get(form, 1)):
+        for parts in (1, 2, 4, 8) if form == "sums" else (1,):
+            if parts > inner // 64:
+                continue
+            out = torch.full((parts, rows, columns), float("nan"), device="cuda", dtype=torch.float32 if form == "sums" else torch.bfloat16)
+            beyond = torch.full((1024,), 7.0, device="cuda")                     # (allocated behind it: nothing writes there)
+            assert lib.lsa_product(16 * parts + tile, FORMS.index(form), activation, x.data_ptr(), weight.data_ptr(), out.data_ptr(), rows, columns, inner,
+                                   torch.cuda.current_stream().cuda_stream) == 0
+            got = out.double().sum(0)
+            act = (silu, gelu, lambda z: z.clamp(min=0) ** 2)[activation]
+            if form == "gated":
+                gate, up = exact.split(columns, 1)
+                want = act(gate) * up
+                bound = 1.13 * off[:, :columns] * up.abs() + act(gate).abs() * off[:, columns:] + 2.0 ** -8 * want.abs() * (1 + 2.0 ** -8)
+            elif form == "activated":
+                want = act(exact)
+                bound = off * (1.13 if activation < 2 else 2 * exact.abs() + off) + 2.0 ** -8 * want.abs()
+            else:
+                want, bound = exact, off + (2.0 ** -8 * exact.abs() if form == "plain" else 0.0)
+            bound = bound * 1.01 + 2.0 ** -18 * want.abs().max()                 # (expf and tanhf: a few parts in 2^23)
+            assert torch.isfinite(got).all() and bool(((got - want).abs() <= bound).all()), float(((got - want).abs() - bound).max())
+            assert bool((beyond == 7.0).all())
+
+
+def test_what_does_not_fit_is_refused(ops):
+    x, weight = drawn(64, 64, 128, 1)
+    out = torch.empty(64, 64, device="cuda", dtype=torch.bfloat16)
+    call = lambda plan, form, activation, xp, rows, columns, inner: ops._product.lsa_product(plan, form, activation, xp, weight.data_ptr(), out.data_ptr(), rows, columns, inner,
+                                                                                            torch.cuda.current_stream().cuda_stream)
+    for plan, form, activation, shift, rows, columns, inner in ((16, 0, 0, 0, 64, 64, 128), (21, 0, 0, 0, 64, 64, 128), (20, 0, 0, 0, 64, 64, 128), (33, 0, 0, 0, 64, 64, 128), (17, 4, 0, 0, 64, 64, 128),
+                                                                (17, 0, 3, 0, 64, 64, 128), (17, 1, 2, 0, 64, 32, 128), (17, 0, 0, 2, 63, 64, 128), (17, 0, 0, 0, 64, 60, 128),
+                                                                (17, 0, 0, 0, 64, 64, 96), (16 * 9 + 1, 3, 0, 0, 64, 64, 128), (16 * 4 + 1, 3, 0, 0, 64, 64, 128)):
+        assert call(plan, form, activation, x.data_ptr() + shift, rows, columns, inner) == -1, (plan, form, activation, shift, rows, columns, inner)
+    assert call(17, 0, 0, x.data_ptr(), 0, 64, 128) == 0
+
+
+@pytest.mark.parametrize("rows", [130, 190, 333])
+def test_products_of_a_portion_go_to_the_tiles(ops, rows, monkeypatch):
+    """A layer's products at a few hundred rows, through the entry points that the parts call, against 64 bits; and what an entry point gives does not depend on
+    where the tensors lie, for other orders and places are the library's."""
+    taken = []
+    real = ops._tiled_product
+    monkeypatch.setattr(ops, "_tiled_product", lambda *a, **k: (lambda done: (taken.append(done is not None), done)[1])(real(*a, **k)))
+    x, weight = drawn(rows, 4096, 2048, rows)
+    want = x.double() @ weight.double().T
+
+    def close(got):
+        return float((got.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+    assert close(ops.linear(x, weight)) and taken == [True]
+    out = torch.empty(rows, 4096, device="cuda", dtype=torch.bfloat16)
+    assert ops.linear(x, weight, out=out) is out and close(out) and taken.pop()
+    exact32 = ops.linear(x, weight, out_float32=True)
+    assert exact32.dtype == torch.float32 and float((exact32.double() - want).norm() / want.norm()) < 2.0 ** -18 and taken.pop()
+    moved = torch.empty(rows * 2048 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(rows, 2048).copy_(x)          # (at an odd place)
+    wider = torch.zeros(rows, 2056, device="cuda", dtype=torch.bfloat16)
+    wider[:, :2048] = x
+    for other in (moved, wider[:, :2048], x.t().contiguous().t()):
+        assert close(ops.linear(other, weight)) and not taken.pop()
+    column_out = torch.empty(4096, rows, device="cuda", dtype=torch.bfloat16).t()
+    assert close(ops.linear(x, weight, out=column_out)) and not taken.pop()
+    followed = x.clone().requires_grad_()
+    with torch.enable_grad():
+        y = ops.linear(followed, weight)
+    assert y.requires_grad and close(y.detach()) and not taken.pop()
+    taken.clear()
+    hidden = ops.linear_gated(x, weight)
+    assert (hidden is None) == (not any(taken))
+    if hidden is not None:
+        gate, up = want.split(2048, 1)
+        assert float((hidden.double() - silu(gate) * up).norm() / (silu(gate) * up).norm()) < 2.0 ** -8
+
+
+def test_partial_sums_join_the_stream_as_the_product_would(ops):
+    """The sums of the parts are rounded to the stream's type as the whole product would be, then added: within one rounding of that."""
+    x, weight = drawn(190, 2048, 6144, 5)
+    sums = ops.linear_partial_sums(x, weight)
+    assert sums is not None and sums.dim() == 3 and sums.shape[0] > 1
+    want = x.double() @ weight.double().T
+    assert float((sums.double().sum(0) - want).norm() / want.norm()) < 2.0 ** -18
+    stream, normed, ones = torch.zeros(190, 2048, device="cuda", dtype=torch.bfloat16), torch.empty(190, 2048, device="cuda", dtype=torch.bfloat16), torch.ones(2048, device="cuda")
+    ops.add_rmsnorm(stream, sums, ones, 1e-6, normed)
+    assert float((stream.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
+def test_a_captured_step_replays_the_tiles(ops):
+    x, weight = drawn(190, 4096, 2048, 9)
+    ops.linear(x, weight), ops.linear_gated(x, weight)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        y, hidden = ops.linear(x, weight), ops.linear_gated(x, weight)
+    for seed in (10, 11, 12):
+        x.copy_(drawn(190, 8, 2048, seed)[0])
+        graph.replay()
+        torch.cuda.synchronize()
+        again = ops.linear_gated(x, weight)
+        assert torch.equal(y, ops.linear(x, weight)) and (hidden is None or torch.equal(hidden, again))

@@ -1,0 +1,44 @@
+"""Which products of many rows this package's own tiles take (host code of the kernel library: no GPU needed)."""
+import pytest
+
+PLAIN, GATED, ACTIVATED, SUMS = range(4)
+ROWS = {1: 64, 2: 128, 3: 128, 4: 256}
+COLUMNS = {1: 64, 2: 64, 3: 128, 4: 256}
+
+
+@pytest.fixture(scope="module")
+def plan():
+    from llmserver_amd.kernels import library
+    return library.load("product").lsa_product_plan
+
+
+def test_sizes_that_no_tile_takes_stay_the_librarys(plan):
+    for form in range(4):
+        assert not plan(form, 190, 4096, 2048 + 32) and not plan(form, 190, 4100, 2048) and not plan(form, 190, 0, 2048) and not plan(form, 0, 4096, 2048)
+        assert not plan(form, 190, 4096, 0)
+    assert not plan(-1, 190, 4096, 2048) and not plan(4, 190, 4096, 2048)
+    assert not plan(GATED, 4096, 2 ** 18, 4096 + 64)            # offsets into gate and up rows end at 4 GB
+
+
+def test_small_tiles_go_round_the_compute_units_once(plan):
+    seen = set()
+    for form in range(4):
+        for rows in (17, 33, 64, 100, 128, 190, 333, 500, 777, 1000, 2048, 5000):
+            for columns, inner in ((1024, 2048), (2048, 2048), (2048, 6144), (4096, 1024), (4096, 4096), (6144, 2560), (8192, 4096), (12288, 2048), (12288, 4096)):
+                tile, parts = plan(form, rows, columns, inner) % 16, plan(form, rows, columns, inner) // 16
+                seen.add((form, tile))
+                assert parts in ((1,) if form != SUMS else (1, 2, 4, 8)) or not tile
+                if tile in (1, 2, 3):
+                    width = COLUMNS[tile] // (2 if form == GATED else 1)
+                    assert -(-rows // ROWS[tile]) * -(-columns // width) * parts <= 256 and inner // 64 >= 4 * parts
+                assert tile != 4 or form == GATED
+    assert {tile for _, tile in seen} == {0, 1, 2, 3, 4} and {form for form, tile in seen if tile} == {PLAIN, GATED, ACTIVATED, SUMS}
+
+
+def test_products_that_were_measured_to_be_faster(plan):
+    for form, rows, columns, inner in ((PLAIN, 190, 4096, 2048), (PLAIN, 2048, 2048, 2048), (PLAIN, 150, 6144, 2560), (PLAIN, 333, 4096, 1024), (GATED, 190, 6144, 2048),
+                                       (GATED, 33, 8192, 4096), (GATED, 2048, 12288, 4096), (SUMS, 190, 2048, 6144), (SUMS, 333, 2560, 9728), (ACTIVATED, 333, 8448, 2048)):
+        assert plan(form, rows, columns, inner), (form, rows, columns, inner)
+    for form, rows, columns, inner in ((PLAIN, 2048, 6144, 4096), (PLAIN, 2048, 4096, 12288), (PLAIN, 640, 16384, 4096), (PLAIN, 33, 4096, 4096), (PLAIN, 60, 2048, 2048),
+                                       (GATED, 333, 6144, 2048), (GATED, 2048, 8448, 2048), (ACTIVATED, 2048, 8192, 4096), (SUMS, 2048, 4096, 12288)):
+        assert not plan(form, rows, columns, inner), (form, rows, columns, inner)
