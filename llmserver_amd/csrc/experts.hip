@@ -13,6 +13,8 @@
 #include "lds_loads.hpp"
 #include "wide_product.hpp"
 
+#include <math.h>
+
 using namespace lsa;
 
 constexpr float NEG_INF = -__builtin_huge_valf();
@@ -841,6 +843,117 @@ __global__ __launch_bounds__(256) void experts_tile_kernel(const bf16_t* __restr
         }
 }
 
+// ---- few pairs an expert ----------------------------------------------------------------------------------------------------
+// C = A . B^T as above for tiles of 64 sorted pairs and 128 rows of the expert's matrix (GATED: for each 32 of them sixteen gate rows and their up rows), where k
+// is a multiple of 64 and all rows begin at multiples of 16 bytes: eight wavefronts of 32 x 32, slabs of 64 of k through three buffers of LDS that loads fill
+// without registers, two workgroups a compute unit.  Rows and columns of padding are neither loaded nor multiplied.
+//   What bounds it is the experts' way from memory, which those loads keep fuller than the tiles above do with a slab in registers: 32 tokens, 6 of 64 experts of 1,408 at
+// width 2,048 (56 of them chosen), all launches 213 -> 193 us (5.3 TB/s in the two products); 330 tokens 268 -> 246; 8 experts, 100 tokens 87 -> 56; 16 of 768, 64 tokens
+// 77 -> 51; 32 of 2,048 at 4,096, 250 tokens 449 -> 360.  No faster: tiles of 64 or 256 rows of the matrix, four wavefronts, 32 rows of pairs, four to six buffers.
+constexpr int STREAM_ROWS = 128, STREAM_BUFFERS = 3, STREAM_THREADS = 512;
+template <int FORM, typename O>
+__global__ __launch_bounds__(STREAM_THREADS) void experts_stream_kernel(const bf16_t* __restrict__ a, int a_stride, int pair_div, const bf16_t* __restrict__ b,
+                                                                        long expert_stride, int b_up_offset, const int* __restrict__ sorted,
+                                                                        const Tile* __restrict__ tiles_of, int max_tiles, O* __restrict__ out, int out_stride, int n_out,
+                                                                        int k, float limit, int blocks) {
+    constexpr bool GATED = FORM == 1;
+    constexpr int COLUMNS = GATED ? STREAM_ROWS / 2 : STREAM_ROWS, SLAB = 64, BUFFER = (TILE_M + STREAM_ROWS) * SLAB * 2;
+    __shared__ __attribute__((aligned(1024))) unsigned char buffers[STREAM_BUFFERS * BUFFER];
+    __shared__ int rows_of[TILE_M];
+    // Workgroups go to the eight XCDs in turn by their number (there are a multiple of eight): an XCD has neighbours of an order that walks the list of tiles for one
+    // block of columns after the other, so that an expert's tiles run on one XCD at about the same time and its rows are fetched into one L2.
+    const int place = (int)(blockIdx.x % XCDS) * (int)(gridDim.x / XCDS) + (int)(blockIdx.x / XCDS), tile = place % max_tiles, block_n = place / max_tiles;
+    if (block_n >= blocks || tile >= tiles_of[max_tiles].expert) return;
+    const int expert = tiles_of[tile].expert;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), col = lane & 15, quad = lane >> 4;
+    const int wave_m = wave >> 2, wave_n = wave & 3, n0 = block_n * COLUMNS;
+    if (threadIdx.x < TILE_M) rows_of[threadIdx.x] = sorted[tile * TILE_M + threadIdx.x];
+    __syncthreads();
+    // A load of a wavefront is 8 rows: wavefront w's are rows 8 w on of A, 8 w and 64 + 8 w on of B.  The eight 16-byte pieces of row r stand at places
+    // piece ^ f(r), so that sixteen lanes whose reads are served together meet all 64 banks (wide_product.hpp).
+    const buffer_t a_buffer = buffer_at(a), b_buffer = buffer_at(b + (size_t)expert * expert_stride);
+    const int line = 8 * wave + (lane >> 3), pair = rows_of[line];
+    const unsigned a_at = pair < 0 ? NOWHERE : 2u * ((unsigned)(pair / pair_div) * (unsigned)a_stride) + 16 * ((lane & 7) ^ (line >> 1 & 7));
+    unsigned b_at[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int r = 64 * u + line, c = n0 + (GATED ? 16 * (r >> 5) + (r & 15) : r);
+        b_at[u] = c >= n_out ? NOWHERE : 2u * ((unsigned)(c + (GATED && (r & 16) ? b_up_offset : 0)) * (unsigned)k)
+                                             + 16 * ((lane & 7) ^ (GATED ? r >> 1 & 7 : (r >> 1 & 1) | (r >> 3 & 3) << 1));
+    }
+    const int slabs = k / SLAB;
+    unsigned landing = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(lds_ptr_t)buffers) + 1024 * wave;
+    int asked = 0;
+    auto ask = [&]() __attribute__((always_inline)) {
+        const unsigned from = min(asked, slabs - 1) * (2 * SLAB);  // (behind the last slab: that once more, into a buffer that nobody reads again)
+        load_16_bytes_a_lane_to_lds(a_buffer, a_at, from, landing);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) load_16_bytes_a_lane_to_lds(b_buffer, b_at[u], from, landing + 8192 * (1 + u));
+        ++asked;
+        landing += asked % STREAM_BUFFERS == 0 ? -(STREAM_BUFFERS - 1) * BUFFER : BUFFER;
+    };
+    f32x4 sums[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) sums[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int pieces[2] = {16 * (quad ^ (col >> 1)), 16 * ((quad + 4) ^ (col >> 1))};
+    const unsigned char* a_rows = buffers + (32 * wave_m + col) * 128;
+    const unsigned char* b_rows = buffers + (TILE_M + 32 * wave_n + (GATED ? col : 8 * (col >> 2) + (col & 3))) * 128;
+    constexpr int B_STEP = (GATED ? 16 : 4) * 128;                 // (not GATED: a lane has eight neighbouring columns of the result)
+    const int used = __builtin_amdgcn_readfirstlane((rows_of[32 * wave_m] >= 0) + (rows_of[32 * wave_m + 16] >= 0));      // rows of MFMA tiles that hold pairs
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // (the count below starts from nothing under way)
+#pragma unroll
+    for (int i = 0; i < STREAM_BUFFERS - 1; ++i) ask();
+    int buffer = 0;
+    for (int slab = 0; slab < slabs; ++slab) {
+        loads_landed_then_barrier<3 * (STREAM_BUFFERS - 2)>();     // and everybody is through with the slab before this one, whose buffer is asked for
+        bf16x8 av[2][2], bv[2][2];
+        if (used)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    if (i < used) av[s][i] = *reinterpret_cast<const bf16x8*>(a_rows + buffer + 2048 * i + pieces[s]);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) bv[s][j] = *reinterpret_cast<const bf16x8*>(b_rows + buffer + B_STEP * j + pieces[s]);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        ask();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (i < used)
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv[s][j], av[s][i], sums[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        buffer = buffer == (STREAM_BUFFERS - 1) * BUFFER ? 0 : buffer + BUFFER;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // (no load may land when this LDS is somebody else's)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int of = rows_of[32 * wave_m + 16 * i + col], n = n0 + (GATED ? 16 * wave_n + 4 * quad : 32 * wave_n + 8 * quad);
+        if (of < 0 || n >= n_out) continue;                        // (n_out is a multiple of 32)
+        O* o = out + (size_t)of * out_stride + n;
+        if (GATED) {
+            struct alignas(4 * sizeof(O)) Four { O v[4]; } four;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) four.v[r] = (O)gated_activation(sums[i][0][r], sums[i][1][r], limit);
+            *reinterpret_cast<Four*>(o) = four;
+        } else {
+            struct alignas(16) Eight { O v[8]; } eight;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const float z = sums[i][r >> 2][r & 3];
+                eight.v[r] = (O)(FORM == 2 ? rectified_square(z) : z);
+            }
+            *reinterpret_cast<Eight*>(o) = eight;
+        }
+    }
+}
+
 // ---- many pairs an expert ---------------------------------------------------------------------------------------------------
 // C = A . B^T as above for tiles of 256 sorted pairs and 256 rows of the expert's matrix (GATED: 128 gate rows and their up rows, 128 columns of the result).
 //   What bounds it is what passes between the XCDs' L2 and the memory side: a workgroup's share of an expert's matrix is read once for each 256 of its pairs and
@@ -952,7 +1065,7 @@ __global__ __launch_bounds__(256) void experts_combine_kernel(const float* __res
     *reinterpret_cast<Floats*>(out + (size_t)t * width + c) = result;
 }
 
-// Whether the wide kernel can multiply such a step: its loads straight into LDS are of 16 bytes at multiples of 16 (`aligned`: x, gate_up and down
+// Whether loads straight into LDS can multiply such a step (the wide kernel's and those of few pairs an expert): they are of 16 bytes at multiples of 16 (`aligned`: x, gate_up and down
 // begin at such), from offsets of 32 bits.
 static bool wide_fits(int pairs, int inter, int width, bool aligned) {
     return aligned && (size_t)pairs * (size_t)(inter > width ? inter : width) * 2 < BUFFER_BYTES && (size_t)2 * inter * width * 2 < BUFFER_BYTES;
@@ -971,6 +1084,15 @@ LSA_EXPORT int lsa_experts_tile_rows(int pairs, int experts, int inter, int widt
     return tiles * ((inter + columns - 1) / columns) + tiles * ((width + WIDE_TILE - 1) / WIDE_TILE) >= 224 ? WIDE_M : TILE_M;
 }
 
+// Whether the product of few pairs an expert goes to experts_stream_kernel.  Two of its workgroups a compute unit are 512, and where the experts that so many pairs can be
+// expected to choose make little more than that, the second round is nearly empty; the tiles above, five a compute unit, are then as fast or faster: 32 experts of
+// 2,048 at 4,096, first product, at 12, 16, 24 and 32 tokens (21, 25, 27 and 29 chosen, 32 blocks each) 152, 169, 183, 192 us and 169, 178, 189, 190; 96 of 512 at 1,024, 32
+// tokens (69 chosen, 8 blocks) 31.2 and 32.9.  With shorter rows it pays earlier (64 of 1,408 at 2,048, 36 chosen, 22 blocks: 145, 135 for all launches).
+static bool stream_pays(int pairs, int experts, int blocks, int k) {
+    const double chosen = experts * (1.0 - exp(-(double)pairs / experts)), rounds = chosen * blocks / 512;
+    return rounds <= 1.0 || rounds >= (k > 3072 ? 1.85 : 1.3);
+}
+
 // Ints of scratch memory that lsa_experts_tiled wants: the sorted pairs, then the tiles and their number.
 LSA_EXPORT int lsa_experts_tiled_ints(int pairs, int experts, int tile_rows) { return ((pairs + tile_rows - 1) / tile_rows + experts) * (tile_rows + 3) + 3; }
 
@@ -986,7 +1108,8 @@ LSA_EXPORT int lsa_experts_tiled(const void* x, const void* gate_up, const void*
     if (width % 32 || inter % 32 || (size_t)experts * 8 > 60000) return -1;
     const bool wide = tile_rows == WIDE_M;
     if (!wide && tile_rows != TILE_M) return -1;
-    if (wide && !wide_fits(pairs, inter, width, ((size_t)x | (size_t)gate_up | (size_t)down | (size_t)hidden) % 16 == 0)) return -1;
+    const bool whole_pieces = wide_fits(pairs, inter, width, ((size_t)x | (size_t)gate_up | (size_t)down | (size_t)hidden) % 16 == 0);
+    if (wide && !whole_pieces) return -1;
     const int max_tiles = (pairs + tile_rows - 1) / tile_rows + experts;
     int* sorted = scratch;
     Tile* tiles_of = reinterpret_cast<Tile*>(scratch + (size_t)max_tiles * tile_rows);
@@ -1017,6 +1140,14 @@ LSA_EXPORT int lsa_experts_tiled(const void* x, const void* gate_up, const void*
         for (int pass = 0; pass < 2; ++pass) {
             const bool second = pass == 1;
             const bool wide_slab = (second ? inter : width) % 64 == 0;
+            const int k = second ? inter : width, columns = second ? width : inter, block = second || plain ? STREAM_ROWS : STREAM_ROWS / 2;
+            const int blocks = (columns + block - 1) / block;
+            const long grid = ((long)max_tiles * blocks + XCDS - 1) / XCDS * XCDS;
+            if (whole_pieces && wide_slab && grid < (1 << 23) && stream_pays(pairs, experts, blocks, k)) {
+                if (second) experts_stream_kernel<0, float><<<(int)grid, STREAM_THREADS, 0, stream>>>(hb, inter, 1, dn, (long)width * inter, 0, sorted, tiles_of, max_tiles, y, width, width, inter, 0.f, blocks);
+                else if (plain) experts_stream_kernel<2, bf16_t><<<(int)grid, STREAM_THREADS, 0, stream>>>(xb, width, top, gu, (long)inter * width, 0, sorted, tiles_of, max_tiles, hb, inter, inter, width, 0.f, blocks);
+                else experts_stream_kernel<1, bf16_t><<<(int)grid, STREAM_THREADS, 0, stream>>>(xb, width, top, gu, (long)2 * inter * width, inter, sorted, tiles_of, max_tiles, hb, inter, inter, width, limit, blocks);
+            } else
             if (wide_slab && many) LSA_TILES(64, 8);
             else if (wide_slab) LSA_TILES(64, 4);
             else if (many) LSA_TILES(32, 8);
