@@ -473,7 +473,10 @@ template <typename T> struct BesideExperts {
     int inter;
 };
 
-template <typename T>
+// AHEAD: how many pieces of 16 bytes of the matrix a lane asks for before it uses the first.  With all conditions between them (a division, the expert and a wait a
+// piece) a launch took, us, before and now: 6 of 64 experts of 1,408 at 2,048, 1 token 12.2, 8.9, 4 tokens 27.6, 21.7, 8 tokens 45.9, 39.6; 4 of 32 of 2,048 at 4,096, 2 tokens
+// 25.7, 20.7, 8 tokens 78, 69.5; 8 of 128 of 768 at 2,048, 1 token 9.3, 7.2.  (Eight ahead leave too few wavefronts: 8 tokens 50.)
+template <typename T, int AHEAD>
 __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__ hidden, const T* __restrict__ down,
                                                            const int* __restrict__ chosen, const float* __restrict__ weights,
                                                            float* __restrict__ out, int top, int inter, int width, int experts,
@@ -514,19 +517,30 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__
     const int c0 = block * columns_per_block, c1 = min(width, c0 + columns_per_block);
     for (int c = c0 + wave; c < c1; c += waves) {
         float acc = 0.f;
-        if (vectors && top <= MOST) {
+        if (vectors && top <= MOST && (size_t)top * (inter / V) * (inter / V) < 0xFFFFFFFFu) {
             // The pairs' rows end to end are one long vector of top * inter / V pieces, spread over the lanes: every
             // lane is busy whatever the experts' size, and its loads do not wait for one another.
             const int pieces = inter / V, all = top * pieces;
-            for (int p = lane; p < all; p += 64) {
-                const int s = p / pieces, i = (p - s * pieces) * V;
-                if (expert_of[s] < 0) continue;          // (an identity expert)
-                const Vec16<T> a = load_vec16(down + ((size_t)expert_of[s] * width + c) * inter + i);
-                const Vec16<T> b = *reinterpret_cast<const Vec16<T>*>(h_lds + (size_t)s * inter + i);
-                float part = 0.f;
+            const unsigned inverse = 0xFFFFFFFFu / (unsigned)pieces + 1;      // p / pieces = p * inverse >> 32 while p * pieces < 2^32
+            for (int p0 = lane; p0 < all; p0 += 64 * AHEAD) {
+                Vec16<T> a[AHEAD], b[AHEAD];
+                float weight[AHEAD];
+                bool counts[AHEAD];
 #pragma unroll
-                for (int k = 0; k < V; ++k) part += (float)a.v[k] * (float)b.v[k];
-                acc += weight_of[s] * part;
+                for (int u = 0; u < AHEAD; ++u) {                // (no load under a condition: the compiler would wait for each)
+                    const int p = min(p0 + 64 * u, all - 1), s = (int)__umulhi((unsigned)p, inverse), i = (p - s * pieces) * V, expert = expert_of[s];
+                    weight[u] = weight_of[s];
+                    counts[u] = p0 + 64 * u < all && expert >= 0;    // (not behind the last piece, no identity expert)
+                    a[u] = load_vec16(down + ((size_t)max(expert, 0) * width + c) * inter + i);
+                    b[u] = *reinterpret_cast<const Vec16<T>*>(h_lds + (size_t)s * inter + i);
+                }
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u) {
+                    float part = 0.f;
+#pragma unroll
+                    for (int k = 0; k < V; ++k) part += (float)a[u].v[k] * (float)b[u].v[k];
+                    acc = counts[u] ? acc + weight[u] * part : acc;
+                }
             }
         } else {
             for (int s = 0; s < top; ++s) {
@@ -644,8 +658,16 @@ LSA_EXPORT int lsa_experts_down(int code, const void* hidden, const void* down, 
     dim3 grid;
     if (!shared_grid(n > 1, n, (width + columns - 1) / columns, grid)) return -1;
 #define LSA_BESIDE(T) BesideExperts<T>{(const T*)x, shared_gate, (const T*)shared_y, (const T*)shared_down, (const T*)shared_hidden, shared_inter}
-    if (code) experts_down_kernel<bf16_t><<<grid, 256, lds, stream>>>((const bf16_t*)hidden, (const bf16_t*)down, chosen, weights, out, top, inter, width, experts, columns, in_lds, LSA_BESIDE(bf16_t), n > 1);
-    else experts_down_kernel<float><<<grid, 256, lds, stream>>>((const float*)hidden, (const float*)down, chosen, weights, out, top, inter, width, experts, columns, in_lds, LSA_BESIDE(float), n > 1);
+    // (trips of a lane: in fours or threes, whichever leaves fewer behind the last piece; a handful one by one)
+    const int trips = (int)(((size_t)top * inter / (code ? 8 : 4) + 63) / 64), ahead = trips < 3 ? 1 : trips % 4 == 0 ? 4 : 3;
+#define LSA_DOWN(T, AHEAD) experts_down_kernel<T, AHEAD><<<grid, 256, lds, stream>>>((const T*)hidden, (const T*)down, chosen, weights, out, top, inter, width, experts, columns, in_lds, LSA_BESIDE(T), n > 1)
+    if (code && ahead == 4) LSA_DOWN(bf16_t, 4);
+    else if (code && ahead == 3) LSA_DOWN(bf16_t, 3);
+    else if (code) LSA_DOWN(bf16_t, 1);
+    else if (ahead == 4) LSA_DOWN(float, 4);
+    else if (ahead == 3) LSA_DOWN(float, 3);
+    else LSA_DOWN(float, 1);
+#undef LSA_DOWN
 #undef LSA_BESIDE
     LSA_LAUNCH_CHECK();
 }
