@@ -191,22 +191,26 @@ __global__ __launch_bounds__(WIDE_THREADS) void wide_gated_kernel(const bf16_t* 
         }
 }
 
-// What lsa_product can be asked for: a tile, and for SUMS the parts of K, as 16 parts + tile.
+// What lsa_product can be asked for: a tile, and for SUMS the parts of K, as 16 parts + tile.  ADDED in a plan for PLAIN or GATED: the sums, and a kernel behind
+// them that adds the parts up (lsa_sum_parts, lsa_gated_parts).
 enum Tile { NONE, SMALL, TALL, LARGE, WIDE };
 struct TileShape { int rows, columns; double start, slab; };       // columns of W; us of a launch with a tile a compute unit, and a slab's
 static const TileShape SHAPES[] = {{0, 0, 0, 0}, {64, 64, 3.0, 0.31}, {128, 64, 3.6, 0.31}, {128, 128, 4.2, 0.50}, {256, 256, 4.5, 0}};
 constexpr int UNITS = 256;                                         // compute units
-constexpr int MOST_PARTS = 8;
+constexpr int MOST_PARTS = 8, ADDED = 1 << 12;
 
+constexpr int FEW_ROWS = 128;
 static bool fits(int form, long M, long N, long K) {
     return M >= 1 && N >= 8 && K >= SLAB && K % SLAB == 0 && N % 8 == 0 && (form == GATED ? 2 * N : 256) * K * 2 + K * 2 < (long)BUFFER_BYTES && 256 * K * 2 < (long)BUFFER_BYTES;
 }
 
 // The tile (and parts) for a product of these sizes, or 0 where the library's product is expected to be as fast (with the kernel of the activation behind it).  Both
 // times are lines through what was measured at 17 to 3,000 rows of 31 products of this package's models: a launch's start and a slab's time for the tiles here,
-// for the library (whose own choice of tiles nobody can foretell) a start, K and the operations.  Over 186 of them at random rows, the way taken against the library: gated 1.12
-// times as fast, plain 1.06, activated 1.12, sums with the norm behind them 1.15, the worst 0.94.  A product whose tiles do not go round the compute units in one
-// round stays the library's unless it is gated and large.
+// for the library (whose own choice of tiles nobody can foretell) a start, K and the operations.  Over 31 products and 17 to 900 rows, the way taken against the one
+// before, up to 128 rows and beyond: gated 1.17 and 1.12 times as fast, plain 1.10 and 1.09, activated 1.07 and 1.13, sums with the norm behind them 1.12 and 1.06, heads
+// 1.04 and 1.00, the worst 0.98 and 0.95.  A product whose tiles do not go round the compute units in one round stays the library's unless it is gated and large.  Up to 128
+// rows the parts may be added up by a launch of their own (64 rows, 2,816 x 2,048 library 12.1, one launch 12.2, so 9.7; 32 rows of 4,096 x 4,096 13.9, 17.9, 12.0; gated
+// 2,816 x 4,096 15.4, 18.4, 12.2).
 LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     if (form < PLAIN || form > SUMS || !fits(form, M, N, K)) return NONE;
     const double slabs = K / SLAB, weights = (form == GATED ? 2.0 : 1.0) * N, megabytes = weights * K * 2e-6, gigaflops = 2e-9 * M * weights * K;
@@ -216,14 +220,20 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
         const TileShape& shape = SHAPES[tile];
         const int columns = form == GATED ? shape.columns / 2 : shape.columns;
         const long tiles = (long)((M + shape.rows - 1) / shape.rows) * ((N + columns - 1) / columns);
-        for (int parts = 1; parts <= (form == SUMS ? MOST_PARTS : 1); parts *= 2) {
-            if (tiles * parts > UNITS || slabs < 4 * parts) continue;
-            double us = shape.start + shape.slab * ((K / SLAB + parts - 1) / parts) * (tiles * parts > 7 * UNITS / 8 ? 1.15 : 1.0);
-            us = us > megabytes / 5.2 + 3.0 ? us : megabytes / 5.2 + 3.0;
+        const bool added = (form == PLAIN || form == GATED) && M <= FEW_ROWS;
+        for (int parts = 1; parts <= (form == SUMS || added ? MOST_PARTS : 1); parts *= 2) {
+            // (the sums take the tile's 64 or 128 rows of W whatever they are: gated, half as many tiles)
+            // (two of the small tiles' workgroups fit a compute unit: where the weights' way bounds them, 33 rows of 32,768 x 4,096 63 us for the library, 55)
+            if (tiles * parts > (tile == SMALL && parts == 1 ? 2 : 1) * UNITS || slabs < 4 * parts) continue;
+            // (the fewer tiles share W's lines, the longer a tall one waits for them: 0.41 us a slab where it has them alone, 0.33 with three)
+            const double slab = shape.slab + (tile == TALL ? 0.1 / ((M + 127) / 128) : 0.0), rate = tile == LARGE ? 4.1 : 5.2;
+            double us = shape.start + slab * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.7 : tiles * parts > 7 * UNITS / 8 ? 1.2 : 1.0);
+            us = us > megabytes / rate + 3.0 ? us : megabytes / rate + 3.0;
             if (form == SUMS) us += parts * 8e-6 * M * N / 4.0;    // written and read
+            else if (parts > 1) us += 3.4 + parts * 8e-6 * M * weights / 3.0;      // and a launch
             if (us < best) {
                 best = us;
-                plan = 16 * parts + tile;
+                plan = 16 * parts + tile + (form != SUMS && parts > 1 ? ADDED : 0);
             }
         }
     }
@@ -238,7 +248,10 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
         const double us = 3.0 + tiles / UNITS * (4.5 + 1.5 * slabs) + (last ? 4.5 + (1.05 + 0.45 * last / UNITS) * slabs : 0.0);
         if (us < best && us < 0.97 * library) return 16 + WIDE;
     }
-    return best < (form == SUMS ? 0.9 : 0.95) * library ? plan : NONE;
+    // (up to 128 rows the sums were faster than the few-row kernels' throughout: 33 rows, with the norm, 2,048 x 6,144 13.7, 12.3; 4,096 x 4,096 15.3, 14.1; 100 rows 18.8, 15.2 and
+    // 21.3, 17.9; but for 24 rows and fewer of a large weight: 17 rows, 4,096 x 8,192 19.6, 20.9)
+    if (form == SUMS && M <= FEW_ROWS) return M <= 24 && weights * K > 3e7 ? NONE : plan;
+    return best < 0.9 * library ? plan : NONE;
 }
 
 template <int FORM>

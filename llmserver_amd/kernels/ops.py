@@ -416,12 +416,16 @@ class HipOps(KernelNamespace):
             return self._linear_few_rows_float32(x, weight, out, bias)
         if not out_float32 and bias is None and not rows_per_workgroup and (out is None or (out.dtype == torch.bfloat16 and out.is_contiguous() and
                 out.device == x.device and tuple(out.shape) == (x.shape[0], weight.shape[0]) and not out.requires_grad and out.data_ptr() % 8 == 0)):
+            if not self._split_first(x):
+                done = self._tiled_product("plain", x, weight, out=out)
+                if done is not None:
+                    return done
             sums = self._partial_sums_to_add(x, weight)
             if sums is not None:
                 out = torch.empty((x.shape[0], weight.shape[0]), device=x.device, dtype=torch.bfloat16) if out is None else out
                 _launched(self._elementwise.lsa_sum_parts(_ptr(sums), sums.shape[0], _ptr(out), x.shape[0], weight.shape[0], _stream()), "sum_parts")
                 return out
-        if bias is None and not rows_per_workgroup and (out is None or not out_float32):
+        if bias is None and not rows_per_workgroup and (out is None or not out_float32) and (out_float32 or self._split_first(x)):
             done = self._tiled_product("plain", x, weight, out=out, out_float32=out_float32)
             if done is not None:
                 return done
@@ -441,7 +445,7 @@ class HipOps(KernelNamespace):
         rounding), behind the library's product otherwise."""
         if self._few_rows(x, weight) and not self.library_is_faster("plain", x, weight, False, False):
             return self.linear_few_rows(x, weight, activation=activation)
-        done = self._tiled_product("activated", x, weight, activation) if activation in self.PLAIN_ACTIVATIONS else None
+        done = self._tiled_product("activated", x, weight, activation) if activation in self.PLAIN_ACTIVATIONS and not self._split_first(x) else None
         if done is not None:
             return done
         y = self.linear(x, weight)
@@ -483,6 +487,13 @@ class HipOps(KernelNamespace):
         return out
 
     PRODUCT_FORMS = ("plain", "gated", "activated", "sums")           # what lsa_product computes (its codes)
+    PRODUCT_ADDED = 1 << 12                                            # in a plan: partial sums, which a kernel behind them adds up
+
+    @staticmethod
+    def _split_first(x) -> bool:
+        """Whether partial sums of the few-row kernel, added up, go before the tiles: few rows whose inner dimension is long enough for many parts (us at 17, 25 and 32
+        rows, those and the tiles: 2,112 x 2,048 7.3, 7.7, 8.0 and 7.7, 8.2, 8.0; 4,096 x 2,048 9.0, 9.7, 10.4 and 9.0, 9.0, 9.7; 4,096 x 1,024 7.2, 7.4, 7.7 and 6.0, 6.0, 6.2)."""
+        return x.shape[0] <= 28 and x.shape[1] >= 2048
 
     def _tiled_product(self, form, x, weight, activation="silu", out=None, out_float32=False):
         """The product of many rows by this package's own tiles where they are expected to be faster than the library's (the rule stands in ``csrc/product.hip``,
@@ -497,6 +508,8 @@ class HipOps(KernelNamespace):
         if form == "gated" and weight.shape[0] % 2:
             return None
         plan = self._product.lsa_product_plan(code, rows, columns, width)
+        if out_float32 and plan & self.PRODUCT_ADDED:
+            return None
         if not plan or (form == "sums" and plan < 32) or _followed(x, weight, out) or not _on_current_gpu(x) or (x.data_ptr() | weight.data_ptr()) % 16:
             return None
         if out is not None:
@@ -506,6 +519,15 @@ class HipOps(KernelNamespace):
             out = torch.empty((plan // 16, rows, columns), device=x.device, dtype=torch.float32)
         else:
             out = torch.empty((rows, columns), device=x.device, dtype=torch.float32 if out_float32 else torch.bfloat16)
+        if plan & self.PRODUCT_ADDED:                                 # in parts, which a kernel behind it adds up
+            parts, sums_code = (plan - self.PRODUCT_ADDED) // 16, self.PRODUCT_FORMS.index("sums")
+            sums = torch.empty((parts, rows, weight.shape[0]), device=x.device, dtype=torch.float32)
+            _launched(self._product.lsa_product(plan - self.PRODUCT_ADDED, sums_code, 0, _ptr(x), _ptr(weight), _ptr(sums), rows, weight.shape[0], width, _stream()), "product")
+            if form == "gated":
+                _launched(self._elementwise.lsa_gated_parts(_ptr(sums), parts, _ptr(out), rows, columns, self.ACTIVATIONS.index(activation), _stream()), "gated_parts")
+            else:
+                _launched(self._elementwise.lsa_sum_parts(_ptr(sums), parts, _ptr(out), rows, columns, _stream()), "sum_parts")
+            return out
         if out_float32:
             code = self.PRODUCT_FORMS.index("sums")                   # of one part
         activations = self.ACTIVATIONS if form == "gated" else self.PLAIN_ACTIVATIONS
@@ -590,8 +612,12 @@ class HipOps(KernelNamespace):
         if not ((0 if few_rows_too else self.skinny_rows) < rows <= self.SPLIT_ROWS) or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 \
                 or x.shape[1] != weight.shape[1] or not self.split_products:
             return None
-        if not few_rows_too and self.library_is_faster("partial", x, weight):
-            return None
+        if not few_rows_too:
+            sums = self._tiled_product("sums", x, weight)
+            if sums is not None:
+                return sums
+            if self.library_is_faster("partial", x, weight):
+                return None
         size = (rows, weight.shape[0], width)
         parts = self._split_parts.get(size)
         if parts is None:
@@ -668,6 +694,9 @@ class HipOps(KernelNamespace):
         if rows > self.skinny_rows:
             if row_scale is not None or pairs_per_workgroup:
                 return None
+            done = None if self._split_first(x) else self._tiled_product("gated", x, gate_up_weight, activation)
+            if done is not None:
+                return done
             sums = self._partial_sums_to_add(x, gate_up_weight, gated=True)
             if sums is None:
                 done = self._linear_gated_beyond_few_rows(x, gate_up_weight)

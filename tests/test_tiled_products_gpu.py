@@ -87,28 +87,32 @@ def test_products_of_a_portion_go_to_the_tiles(ops, rows, monkeypatch):
     x, weight = drawn(rows, 4096, 2048, rows)
     want = x.double() @ weight.double().T
 
+    def tiled():
+        got = any(taken)
+        taken.clear()
+        return got
+
     def close(got):
         return float((got.double() - want).norm() / want.norm()) < 2.0 ** -8
 
-    assert close(ops.linear(x, weight)) and taken == [True]
+    assert close(ops.linear(x, weight)) and tiled()
     out = torch.empty(rows, 4096, device="cuda", dtype=torch.bfloat16)
-    assert ops.linear(x, weight, out=out) is out and close(out) and taken.pop()
+    assert ops.linear(x, weight, out=out) is out and close(out) and tiled()
     exact32 = ops.linear(x, weight, out_float32=True)
-    assert exact32.dtype == torch.float32 and float((exact32.double() - want).norm() / want.norm()) < 2.0 ** -18 and taken.pop()
+    assert exact32.dtype == torch.float32 and float((exact32.double() - want).norm() / want.norm()) < 2.0 ** -18 and tiled()
     moved = torch.empty(rows * 2048 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(rows, 2048).copy_(x)          # (at an odd place)
     wider = torch.zeros(rows, 2056, device="cuda", dtype=torch.bfloat16)
     wider[:, :2048] = x
     for other in (moved, wider[:, :2048], x.t().contiguous().t()):
-        assert close(ops.linear(other, weight)) and not taken.pop()
+        assert close(ops.linear(other, weight)) and not tiled()
     column_out = torch.empty(4096, rows, device="cuda", dtype=torch.bfloat16).t()
-    assert close(ops.linear(x, weight, out=column_out)) and not taken.pop()
+    assert close(ops.linear(x, weight, out=column_out)) and not tiled()
     followed = x.clone().requires_grad_()
     with torch.enable_grad():
         y = ops.linear(followed, weight)
-    assert y.requires_grad and close(y.detach()) and not taken.pop()
-    taken.clear()
+    assert y.requires_grad and close(y.detach()) and not tiled()
     hidden = ops.linear_gated(x, weight)
-    assert (hidden is None) == (not any(taken))
+    assert (hidden is None) == (not tiled())
     if hidden is not None:
         gate, up = want.split(2048, 1)
         assert float((hidden.double() - silu(gate) * up).norm() / (silu(gate) * up).norm()) < 2.0 ** -8
@@ -124,6 +128,26 @@ def test_partial_sums_join_the_stream_as_the_product_would(ops):
     stream, normed, ones = torch.zeros(190, 2048, device="cuda", dtype=torch.bfloat16), torch.empty(190, 2048, device="cuda", dtype=torch.bfloat16), torch.ones(2048, device="cuda")
     ops.add_rmsnorm(stream, sums, ones, 1e-6, normed)
     assert float((stream.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("rows", [29, 33, 64, 65, 100, 128])
+def test_parts_that_another_launch_adds_up(ops, rows):
+    """Plain and gated products of up to 128 rows: the parts' sums are of 32 bits, so that the one rounding is the result's."""
+    x, weight = drawn(rows, 4096, 4096, rows)
+    plain, gated = (ops._product.lsa_product_plan(form, rows, columns, 4096) for form, columns in ((0, 4096), (1, 2048)))
+    print(f"parts added {rows}: plans {plain:#x} {gated:#x}", flush=True)
+    assert gated & ops.PRODUCT_ADDED and (plain & ops.PRODUCT_ADDED or rows > 64)
+    exact, sizes = x.double() @ weight.double().T, x.double().abs() @ weight.double().abs().T
+    off = 4100 * 2.0 ** -24 * sizes
+    assert bool(((ops.linear(x, weight).double() - exact).abs() <= (off + 2.0 ** -8 * exact.abs()) * 1.01).all())
+    for activation, act in (("silu", silu), ("gelu_tanh", gelu)):
+        got = ops.linear_gated(x, weight, activation=activation).double()
+        gate, up = exact.split(2048, 1)
+        want = act(gate) * up
+        bound = 1.13 * off[:, :2048] * up.abs() + act(gate).abs() * off[:, 2048:] + 2.0 ** -8 * want.abs()
+        assert bool(((got - want).abs() <= bound * 1.01 + 2.0 ** -18 * want.abs().max()).all())
+    sums = ops.linear_partial_sums(x, weight)
+    assert sums is not None and bool(((sums.double().sum(0) - exact).abs() <= off * 1.01).all())
 
 
 def test_a_captured_step_replays_the_tiles(ops):

@@ -4,6 +4,7 @@ import pytest
 PLAIN, GATED, ACTIVATED, SUMS = range(4)
 ROWS = {1: 64, 2: 128, 3: 128, 4: 256}
 COLUMNS = {1: 64, 2: 64, 3: 128, 4: 256}
+ADDED = 1 << 12
 
 
 @pytest.fixture(scope="module")
@@ -21,24 +22,30 @@ def test_sizes_that_no_tile_takes_stay_the_librarys(plan):
 
 
 def test_small_tiles_go_round_the_compute_units_once(plan):
-    seen = set()
+    """But for those of 64 x 64, two of whose workgroups fit a unit; and only plain and gated products of up to 128 rows have parts that another launch adds up."""
+    seen, added = set(), set()
     for form in range(4):
         for rows in (17, 33, 64, 100, 128, 190, 333, 500, 777, 1000, 2048, 5000):
             for columns, inner in ((1024, 2048), (2048, 2048), (2048, 6144), (4096, 1024), (4096, 4096), (6144, 2560), (8192, 4096), (12288, 2048), (12288, 4096)):
-                tile, parts = plan(form, rows, columns, inner) % 16, plan(form, rows, columns, inner) // 16
+                whole = plan(form, rows, columns, inner)
+                tile, parts = whole % 16, whole % ADDED // 16
                 seen.add((form, tile))
-                assert parts in ((1,) if form != SUMS else (1, 2, 4, 8)) or not tile
+                if whole >= ADDED:
+                    added.add(form)
+                    assert form in (PLAIN, GATED) and rows <= 128 and parts > 1
+                assert parts in ((1,) if form != SUMS and whole < ADDED else (1, 2, 4, 8)) or not tile
                 if tile in (1, 2, 3):
                     width = COLUMNS[tile] // (2 if form == GATED else 1)
-                    assert -(-rows // ROWS[tile]) * -(-columns // width) * parts <= 256 and inner // 64 >= 4 * parts
+                    assert -(-rows // ROWS[tile]) * -(-columns // width) * parts <= (512 if tile == 1 and parts == 1 else 256) and inner // 64 >= 4 * parts
                 assert tile != 4 or form == GATED
     assert {tile for _, tile in seen} == {0, 1, 2, 3, 4} and {form for form, tile in seen if tile} == {PLAIN, GATED, ACTIVATED, SUMS}
+    assert added == {PLAIN, GATED}
 
 
 def test_products_that_were_measured_to_be_faster(plan):
-    for form, rows, columns, inner in ((PLAIN, 190, 4096, 2048), (PLAIN, 2048, 2048, 2048), (PLAIN, 150, 6144, 2560), (PLAIN, 333, 4096, 1024), (GATED, 190, 6144, 2048),
-                                       (GATED, 33, 8192, 4096), (GATED, 2048, 12288, 4096), (SUMS, 190, 2048, 6144), (SUMS, 333, 2560, 9728), (ACTIVATED, 333, 8448, 2048)):
+    for form, rows, columns, inner in ((PLAIN, 190, 4096, 2048), (PLAIN, 2048, 2048, 2048), (PLAIN, 33, 4096, 4096), (PLAIN, 33, 32768, 4096), (PLAIN, 333, 4096, 1024), (GATED, 190, 6144, 2048),
+                                       (GATED, 33, 8192, 4096), (GATED, 64, 2816, 4096), (GATED, 2048, 12288, 4096), (SUMS, 33, 2048, 2048), (SUMS, 190, 2048, 6144), (SUMS, 333, 2560, 9728), (ACTIVATED, 333, 8448, 2048)):
         assert plan(form, rows, columns, inner), (form, rows, columns, inner)
-    for form, rows, columns, inner in ((PLAIN, 2048, 6144, 4096), (PLAIN, 2048, 4096, 12288), (PLAIN, 640, 16384, 4096), (PLAIN, 33, 4096, 4096), (PLAIN, 60, 2048, 2048),
-                                       (GATED, 333, 6144, 2048), (GATED, 2048, 8448, 2048), (ACTIVATED, 2048, 8192, 4096), (SUMS, 2048, 4096, 12288)):
+    for form, rows, columns, inner in ((PLAIN, 2048, 6144, 4096), (PLAIN, 2048, 4096, 12288), (PLAIN, 640, 16384, 4096), (PLAIN, 60, 2048, 2048),
+                                       (GATED, 333, 6144, 2048), (GATED, 2048, 8448, 2048), (ACTIVATED, 2048, 8192, 4096), (SUMS, 20, 4096, 8192), (SUMS, 2048, 4096, 12288)):
         assert not plan(form, rows, columns, inner), (form, rows, columns, inner)
