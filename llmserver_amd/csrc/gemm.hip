@@ -823,36 +823,47 @@ LSA_EXPORT int lsa_gemm_split_gated(const void* x, const void* w, void* hidden, 
 // up of 8 gate rows and their 8 up rows), for up to 8 rows (each wavefront finds the scale of one): every norm, activation and sum that is a kernel of its
 // own costs such a step 2 to 3 us (two rows of a 0.6B-sized model: 24 launches fewer a step, a prompt of 333 tokens and 8 steps 6.22 -> 5.85 ms).
 // In 32 bits the stream update has no roundings of its own: s' = resid + y, and the next product takes s' * weight with 1 / rms(s') on its sums.
-constexpr int F32_STEPS = 8, F32_FUSED_ROWS = GEMM_WAVES;
-template <bool GATED>
-__global__ __launch_bounds__(GEMM_WAVES * 64, 4) void gemm_few_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y,
+//
+// FOLDED: up to 8 rows of W a workgroup and of X would leave three quarters of the products' 16 x 16 places empty: the second eight rows of both operands are the same
+// rows' next 16 inner indices, so that a step is 32 of them (of the four quarters of a product two count), a trip to memory brings twice as much of what is needed, and
+// the trips, one behind the other for a wavefront and about 1.3 us each, are half as many.  Weights become lighter for a workgroup too (4,096 rows and more had to share a
+// unit's way to memory by 16): us before and now at 2 rows, 1,024 x 1,024 4.2, 3.6; 1,024 x 2,048 6.4, 5.0; 2,048 x 2,048 7.9, 6.0; 1,024 x 3,072 8.7, 6.1; 2,048 x 6,144
+// 17.6, 12.9; 3,072 x 1,024 6.9, 5.7; 6,144 x 1,024 9.1, 7.6, gated 9.0, 7.8; 8 rows 1,024 x 2,048 7.6, 6.1, 1,024 x 3,072 10.3, 7.6.
+//   STEPS are a trip's: 4, 6 or 8, whichever a wavefront's share needs fewest trips of with the least beside it (what lies behind its share is read for nothing: 1,024 x 1,024
+// in one trip of 8 5.0, of 4 3.7).  One trip of 12 or 16 is no faster than two (1,024 x 4,096 8.7 in one, 8.5).
+constexpr int F32_FUSED_ROWS = GEMM_WAVES;
+template <bool GATED, bool FOLDED, int STEPS>
+__global__ __launch_bounds__(GEMM_WAVES * 64, STEPS > 8 ? 2 : 4) void gemm_few_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y,
                                                                           int M, int N, int K, int R, Fusion fusion) {
     __shared__ float partial[GEMM_WAVES][256];
     __shared__ float row_scale[F32_FUSED_ROWS];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), col = lane & 15, quad = lane >> 4;
-    const int n0 = blockIdx.x * R;                                 // GATED: R <= 8 pairs, the up rows in the tile's second half
-    const int steps = (K + 15) / 16, share = (steps + GEMM_WAVES - 1) / GEMM_WAVES;
+    const int n0 = blockIdx.x * R;                                 // GATED: R <= 8 pairs (FOLDED: 4), the up rows in the tile's second half (FOLDED: in each half's)
+    constexpr int STEP = FOLDED ? 32 : 16;
+    const int steps = (K + STEP - 1) / STEP, share = (steps + GEMM_WAVES - 1) / GEMM_WAVES;
     const int begin = min(steps, wave * share), end = min(steps, begin + share);
-    const int w_row = GATED ? (col < 8 ? 0 : N / 2) + min(n0 + min(col & 7, R - 1), N / 2 - 1) : min(n0 + min(col, R - 1), N - 1);
+    constexpr int UP = FOLDED ? 4 : 8;
+    const int w_row = GATED ? (col & UP ? N / 2 : 0) + min(n0 + min(col & (UP - 1), R - 1), N / 2 - 1) : min(n0 + min(FOLDED ? col & 7 : col, R - 1), N - 1);
     const float* wp = w + (size_t)w_row * K;
-    const float* xp = x + (size_t)min(col, M - 1) * K;
+    const float* xp = x + (size_t)min(FOLDED ? col & 7 : col, M - 1) * K;
+    const int inner = 4 * quad + (FOLDED ? 16 * (col >> 3) : 0);
     RowScaleLoads scale_loads;
     f32x4 acc[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] = (f32x4){0.f, 0.f, 0.f, 0.f};
     if (fusion.square_sums) row_scale_issue(scale_loads, fusion, x, M, wave, lane);        // (there by the time the last products are through)
-    for (int step = begin; step < end; step += F32_STEPS) {
-        f32x4 ws[F32_STEPS], xs[F32_STEPS];
+    for (int step = begin; step < end; step += STEPS) {
+        f32x4 ws[STEPS], xs[STEPS];
 #pragma unroll
-        for (int u = 0; u < F32_STEPS; ++u) {                      // (places behind the row's end: its last four numbers, which count as zeros)
-            const int k = min(16 * (step + u) + 4 * quad, K - 4);
+        for (int u = 0; u < STEPS; ++u) {                      // (places behind the row's end: its last four numbers, which count as zeros)
+            const int k = min(STEP * (step + u) + inner, K - 4);
             xs[u] = *reinterpret_cast<const f32x4*>(xp + k);
             ws[u] = *reinterpret_cast<const f32x4*>(wp + k);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < F32_STEPS; ++u) {
-            const bool there = step + u < end && 16 * (step + u) + 4 * quad < K;
+        for (int u = 0; u < STEPS; ++u) {
+            const bool there = step + u < end && STEP * (step + u) + inner < K;
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(there ? ws[u][e] : 0.f, there ? xs[u][e] : 0.f, acc[e], 0, 0, 0);
         }
@@ -868,13 +879,13 @@ __global__ __launch_bounds__(GEMM_WAVES * 64, 4) void gemm_few_f32_kernel(const 
     auto total_of = [&](int at) {
         float p[GEMM_WAVES];
 #pragma unroll
-        for (int v = 0; v < GEMM_WAVES; ++v) p[v] = partial[v][at];
+        for (int v = 0; v < GEMM_WAVES; ++v) p[v] = FOLDED ? partial[v][at & 127] + partial[v][(at & 119) + 136] : partial[v][at];       // (row 8 of X, row 8 of W: 136)
         const float total = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         return fusion.square_sums ? total * row_scale[min(m, F32_FUSED_ROWS - 1)] : total;
     };
     const float total = total_of(threadIdx.x);
     if (GATED) {
-        if (j < R && m < M && n < N / 2) y[(size_t)m * (N / 2) + n] = total / (1.f + expf(-total)) * total_of(threadIdx.x + 8);
+        if (j < R && m < M && n < N / 2) y[(size_t)m * (N / 2) + n] = total / (1.f + expf(-total)) * total_of(threadIdx.x + UP);
         return;
     }
     const bool own = m < M && j < R && n < N;
@@ -899,28 +910,50 @@ __global__ __launch_bounds__(GEMM_WAVES * 64, 4) void gemm_few_f32_kernel(const 
 // rows and at rows of 1,024 and 2,048 numbers, and good between and behind those.  Here eight wavefronts want four steps of 16 each to have anything
 // under way together, a workgroup more than a compute unit's share waits for a second round, and from 5 rows on X takes a noticeable part of
 // the way into a compute unit.  us against the library's, N x K, replayed from a graph with cold weights, at 2 rows unless stated:
-//   up to 2,048 rows of W: 1,024 x 512 4.0, 4.5; 1,024 x 1,024 4.3, 8.0; 2,048 x 2,048 6.2, 8.7 (8 rows 7.4, 8.8); 1,024 x 3,072 8.5, 8.7 (8 rows 9.8,
-// 8.7); 1,024 x 6,144 1.07 times the library's time, 1,024 x 8,192 1.07.
-//   up to 8,192: 4,096 x 1,024 5.7, 8.6; 6,144 x 1,024 8.1, 9.1 (8 rows 8.9, 9.1); 4,096 x 768 0.73 times the library's time (8 rows 0.77, 6,144 x
-// 768 1.07); 6,144 x 512 1.16; 6,144 x 1,536 1.33; 4,096 x 2,048 8.8, 11.1; 2,560 x 2,048 (a round and a quarter) 1.14; 2,560 x 9,728 43, 32.
+//   up to 2,048 rows of W: 1,024 x 1,024 3.6, 8.0; 2,048 x 2,048 6.0, 12.0; 1,024 x 3,072 6.1, 10.9; 4 rows of 1,024 x 6,144 11.4, 17.4, of 2,048 x 6,144 14.3, 18.0 (8 rows
+// 16.5, 18.1).
+//   up to 8,192: 4,096 x 1,024 6.2, 11.7; 6,144 x 1,024 7.6, 12.7 (8 rows 8.7, 12.5); 6,144 x 768 7.6, 10.5; 6,144 x 1,536 at 8 rows 13.7, 12.0; 4,096 x 2,048 8.7, 12.4; 2,560 x 4,096
+// 13.9, 14.2 (8 rows 18.2, 13.8); 2,560 x 9,728 30, 32 (8 rows 41, 28).
 //   a vocabulary: 151,936 x 1,024 111, 209 (8 rows 138, 212; 16 rows 163, 210), x 2,048 218, 256 (8 rows 270, 262); x 512 1.77 times the library's time, x 2,560
 // 1.11; 65,536 x 1,024 1.07 (16 rows 1.40), x 2,560 1.27 (16 rows 232, 120); 16,384 x 1,024 at 16 rows 22, 19.
 LSA_EXPORT int lsa_gemm_few_f32_fits(int M, int N, int K) {
     if (M < 1 || M > 16 || N < 1 || K < 512 || K % 4 != 0) return 0;
     if (N >= 100000) return K >= 768 && K <= (M <= 6 ? 2048 : M <= 8 ? 1536 : 1024) ? 1 : 0;
     if (M > 8) return 0;
-    if (N <= 2048) return K <= (M <= 2 ? 3072 : 2048) ? 1 : 0;
+    if (N <= 2048) return K <= (M <= 4 ? 6144 : 2048) ? 1 : 0;
     if (N > 8192) return 0;
     if (K <= 1024) return K >= 768 + 64 * (M > 4 ? M - 4 : 0) ? 1 : 0;
     const int workgroups = (N + 15) / 16, rounds = (workgroups + 255) / 256;
     return K == 2048 && M <= 4 && N >= 4096 && 10 * workgroups >= 9 * 256 * rounds ? 1 : 0;
 }
 
-// rows of W a workgroup: 16 where every compute unit gets them, else 8 or 4 (1,024 x 2,048: 7.3, 5.9 and 5.7 us; 4,096 x 1,024: 5.5, 5.9, 9.2)
-static int few_f32_rows(int N) { return N >= 4096 ? 16 : N >= 1024 ? 8 : 4; }
+// Rows of W a workgroup: 4 while that is a workgroup a compute unit (2 rows of 1,024 x 3,072: 8 rows 7.1 us, 4 6.1; of 1,536 x 4,096 9.4, 12.1), 16 from where 8 would be four
+// rounds of workgroups, and between them 16 for as many rows of X as make their way into the units the longer one (4,096 x 1,024 at 2 rows: 16 6.5, 8 6.2; at 8 rows 6.8, 7.4;
+// 6,144 x 1,024 9.1, 7.6 and 9.8, 8.7).
+static int few_f32_rows(int M, int N) {
+    if (N <= 1024) return 4;
+    return N >= 8192 || (N >= 4096 && M > (N >= 6144 ? 8 : 4)) ? 16 : 8;
+}
+// ... where a workgroup leaves a sum of squares a row behind
+static int few_f32_stream_rows(int N) { return N >= 4096 ? 16 : N > 1024 ? 8 : 4; }
 static bool few_f32_takes(const float* x, const float* w, int M, int K, const float* square_sums, int n_parts, const void* resid) {
     if (M > 16 || K < 4 || K % 4 != 0 || ((reinterpret_cast<size_t>(x) | reinterpret_cast<size_t>(w)) & 15)) return false;
     return M <= F32_FUSED_ROWS ? fusion_fits(M, square_sums, n_parts, resid) : !square_sums && !resid;
+}
+template <bool GATED, bool FOLDED>
+static void launch_few_f32_of(int rows, int blocks, const float* x, const float* w, float* y, int M, int N, int K, const Fusion& fusion, hipStream_t stream) {
+    const int steps = (K + (FOLDED ? 31 : 15)) / (FOLDED ? 32 : 16), share = (steps + GEMM_WAVES - 1) / GEMM_WAVES;
+#define LSA_FEW(S) gemm_few_f32_kernel<GATED, FOLDED, S><<<blocks, GEMM_WAVES * 64, 0, stream>>>(x, w, y, M, N, K, rows, fusion)
+    if (share <= 4) LSA_FEW(4);
+    else if (share <= 6) LSA_FEW(6);
+    else if (share <= 8 || share > 12) LSA_FEW(8);
+    else LSA_FEW(6);
+#undef LSA_FEW
+}
+static void launch_few_f32(int rows, const float* x, const float* w, float* y, int M, int N, int K, const Fusion& fusion, hipStream_t stream) {
+    const int blocks = (N + rows - 1) / rows;
+    if (rows <= 8 && M <= 8) launch_few_f32_of<false, true>(rows, blocks, x, w, y, M, N, K, fusion, stream);
+    else launch_few_f32_of<false, false>(rows, blocks, x, w, y, M, N, K, fusion, stream);
 }
 
 // x [M, K], w [N, K], y [M, N], bias [N] or nullptr, all float32; M <= 16, K a multiple of 4, x and w at multiples of 16 bytes.  square_sums [M, n_parts]
@@ -930,8 +963,7 @@ LSA_EXPORT int lsa_gemm_few_f32(const float* x, const float* w, float* y, int M,
     if (M <= 0 || N <= 0) return 0;
     if (!few_f32_takes(x, w, M, K, square_sums, n_parts, nullptr)) return -1;
     const Fusion fusion = {square_sums, n_parts, eps, nullptr, nullptr, nullptr, nullptr, nullptr, bias, 0};
-    const int rows = few_f32_rows(N);
-    gemm_few_f32_kernel<false><<<(N + rows - 1) / rows, GEMM_WAVES * 64, 0, stream>>>(x, w, y, M, N, K, rows, fusion);
+    launch_few_f32(few_f32_rows(M, N), x, w, y, M, N, K, fusion, stream);
     LSA_LAUNCH_CHECK();
 }
 
@@ -941,13 +973,14 @@ LSA_EXPORT int lsa_gemm_few_f32_gated(const float* x, const float* w, float* hid
     if (M <= 0 || I <= 0) return 0;
     if (M > F32_FUSED_ROWS || !few_f32_takes(x, w, M, K, square_sums, n_parts, nullptr)) return -1;
     const Fusion fusion = {square_sums, n_parts, eps, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-    const int pairs = few_f32_rows(2 * I) / 2;
-    gemm_few_f32_kernel<true><<<(I + pairs - 1) / pairs, GEMM_WAVES * 64, 0, stream>>>(x, w, hidden, M, 2 * I, K, pairs, fusion);
+    const int pairs = few_f32_rows(M, 2 * I) / 2, blocks = (I + pairs - 1) / pairs;
+    if (pairs <= 4) launch_few_f32_of<true, true>(pairs, blocks, x, w, hidden, M, 2 * I, K, fusion, stream);
+    else launch_few_f32_of<true, false>(pairs, blocks, x, w, hidden, M, 2 * I, K, fusion, stream);
     LSA_LAUNCH_CHECK();
 }
 
 // Partial sums per row that lsa_gemm_few_f32_stream writes (the second dimension of square_sums_out).
-LSA_EXPORT int lsa_gemm_few_f32_parts(int N) { return N <= 0 ? -1 : (N + few_f32_rows(N) - 1) / few_f32_rows(N); }
+LSA_EXPORT int lsa_gemm_few_f32_parts(int N) { return N <= 0 ? -1 : (N + few_f32_stream_rows(N) - 1) / few_f32_stream_rows(N); }
 
 // resid_out = resid + x . w^T [/ rms, if square_sums], weighted_out = resid_out * norm_weight, square_sums_out [M, lsa_gemm_few_f32_parts(N)] = sums of
 // resid_out^2 over the columns of each workgroup; M <= 8.  resid_out may be resid itself.
@@ -958,7 +991,6 @@ LSA_EXPORT int lsa_gemm_few_f32_stream(const float* x, const float* w, int M, in
     if (M > F32_FUSED_ROWS || !resid || !norm_weight || !resid_out || !weighted_out || !square_sums_out
         || !few_f32_takes(x, w, M, K, square_sums, n_parts, resid)) return -1;
     const Fusion fusion = {square_sums, n_parts, eps, (const bf16_t*)resid, norm_weight, (bf16_t*)resid_out, (bf16_t*)weighted_out, square_sums_out, nullptr, 0};
-    const int rows = few_f32_rows(N);
-    gemm_few_f32_kernel<false><<<(N + rows - 1) / rows, GEMM_WAVES * 64, 0, stream>>>(x, w, nullptr, M, N, K, rows, fusion);
+    launch_few_f32(few_f32_stream_rows(N), x, w, nullptr, M, N, K, fusion, stream);
     LSA_LAUNCH_CHECK();
 }
