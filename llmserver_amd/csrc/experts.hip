@@ -521,14 +521,14 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__
             // The pairs' rows end to end are one long vector of top * inter / V pieces, spread over the lanes: every
             // lane is busy whatever the experts' size, and its loads do not wait for one another.
             const int pieces = inter / V, all = top * pieces;
-            const unsigned inverse = 0xFFFFFFFFu / (unsigned)pieces + 1;      // p / pieces = p * inverse >> 32 while p * pieces < 2^32
+            const unsigned inverse = 0xFFFFFFFFu / (unsigned)pieces + 1;      // p / pieces = p * inverse >> 32 while p * pieces < 2^32 and pieces > 1 (2^32 has no place here)
             for (int p0 = lane; p0 < all; p0 += 64 * AHEAD) {
                 Vec16<T> a[AHEAD], b[AHEAD];
                 float weight[AHEAD];
                 bool counts[AHEAD];
 #pragma unroll
                 for (int u = 0; u < AHEAD; ++u) {                // (no load under a condition: the compiler would wait for each)
-                    const int p = min(p0 + 64 * u, all - 1), s = (int)__umulhi((unsigned)p, inverse), i = (p - s * pieces) * V, expert = expert_of[s];
+                    const int p = min(p0 + 64 * u, all - 1), s = pieces == 1 ? p : (int)__umulhi((unsigned)p, inverse), i = (p - s * pieces) * V, expert = expert_of[s];
                     weight[u] = weight_of[s];
                     counts[u] = p0 + 64 * u < all && expert >= 0;    // (not behind the last piece, no identity expert)
                     a[u] = load_vec16(down + ((size_t)max(expert, 0) * width + c) * inter + i);

@@ -5,8 +5,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# (choices, numbers of a hidden row): one to nine trips of 64 pieces of 16 bytes, whole and not, in ones, threes and fours
-@pytest.mark.parametrize("top,inter", [(1, 8), (1, 504), (2, 256), (3, 344), (2, 768), (4, 512), (5, 408), (3, 1408), (8, 72), (6, 704), (2, 2304), (9, 512)])
+# (choices, numbers of a hidden row): one to nine trips of 64 pieces of 16 bytes, whole and not, in ones, threes and fours; rows of one piece (of 4 or 8 numbers)
+@pytest.mark.parametrize("top,inter", [(1, 8), (2, 8), (7, 8), (3, 4), (1, 504), (2, 256), (3, 344), (2, 768), (4, 512), (5, 408), (3, 1408), (8, 72), (6, 704), (2, 2304), (9, 512)])
 @pytest.mark.parametrize("tokens", [1, 3])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_rows_that_end_between_pieces(dtype, tokens, top, inter):
