@@ -213,6 +213,7 @@ static bool fits(int form, long M, long N, long K) {
 // 2,816 x 4,096 15.4, 18.4, 12.2).
 LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     if (form < PLAIN || form > SUMS || !fits(form, M, N, K)) return NONE;
+    if (form == SUMS && M > FEW_ROWS && N < 1024) return NONE;     // (measured from 1,024 columns on: fewer go the library's way, whole or in ranges)
     const double slabs = K / SLAB, weights = (form == GATED ? 2.0 : 1.0) * N, megabytes = weights * K * 2e-6, gigaflops = 2e-9 * M * weights * K;
     double best = 1e30;
     int plan = NONE;
@@ -223,8 +224,9 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
         const bool added = (form == PLAIN || form == GATED) && M <= FEW_ROWS;
         for (int parts = 1; parts <= (form == SUMS || added ? MOST_PARTS : 1); parts *= 2) {
             // (the sums take the tile's 64 or 128 rows of W whatever they are: gated, half as many tiles)
-            // (two of the small tiles' workgroups fit a compute unit: where the weights' way bounds them, 33 rows of 32,768 x 4,096 63 us for the library, 55)
-            if (tiles * parts > (tile == SMALL && parts == 1 ? 2 : 1) * UNITS || slabs < 4 * parts) continue;
+            // (two of the small tiles' workgroups fit a compute unit: where the weights' way bounds them, 33 rows of 32,768 x 4,096 63 us for the library, 55; gated products
+            // beyond one round, and with less than 1,024 of K, stay with the kernel that shares the activations, or the library)
+            if (tiles * parts > (tile == SMALL && parts == 1 && form != GATED ? 2 : 1) * UNITS || slabs < 4 * parts || (form == GATED && slabs < 16)) continue;
             // (the fewer tiles share W's lines, the longer a tall one waits for them: 0.41 us a slab where it has them alone, 0.33 with three)
             const double slab = shape.slab + (tile == TALL ? 0.1 / ((M + 127) / 128) : 0.0), rate = tile == LARGE ? 4.1 : 5.2;
             double us = shape.start + slab * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.7 : tiles * parts > 7 * UNITS / 8 ? 1.2 : 1.0);
