@@ -244,9 +244,9 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     library = library > megabytes / 4.3 ? library : megabytes / 4.3;
     if (form == GATED) library += 3.5 + 6e-6 * M * N / 5.0;
     if (form == ACTIVATED) library += 3.5 + 4e-6 * M * N / 5.0;
-    if (form == GATED) {
+    if (form == GATED && slabs >= 16) {
         const long tiles = (long)((M + WIDE_TILE - 1) / WIDE_TILE) * ((N + WIDE_TILE / 2 - 1) / (WIDE_TILE / 2)), last = tiles % UNITS;
-        // (a slab takes 1.05 us where few compute units work, 1.5 where all do: power)
+        // (a slab takes 1.05 us where few compute units work, 1.5 where all do: power; shorter inner dimensions as above)
         const double us = 3.0 + tiles / UNITS * (4.5 + 1.5 * slabs) + (last ? 4.5 + (1.05 + 0.45 * last / UNITS) * slabs : 0.0);
         if (us < best && us < 0.97 * library) return 16 + WIDE;
     }

@@ -49,3 +49,8 @@ def test_products_that_were_measured_to_be_faster(plan):
     for form, rows, columns, inner in ((PLAIN, 2048, 6144, 4096), (PLAIN, 2048, 4096, 12288), (PLAIN, 640, 16384, 4096), (PLAIN, 60, 2048, 2048),
                                        (GATED, 333, 6144, 2048), (GATED, 2048, 8448, 2048), (ACTIVATED, 2048, 8192, 4096), (SUMS, 20, 4096, 8192), (SUMS, 2048, 4096, 12288)):
         assert not plan(form, rows, columns, inner), (form, rows, columns, inner)
+
+
+def test_gated_products_of_short_inner_dimensions_stay_where_they_were(plan):
+    """Neither small tiles nor large ones: the kernel that shares the activations, or the library, has them."""
+    assert not any(plan(GATED, rows, columns, inner) for rows in (17, 33, 70, 206, 777, 2048, 9000) for columns in (32, 64, 96, 768, 3072, 12288) for inner in (64, 128, 512, 960))
