@@ -1460,6 +1460,10 @@ LSA_EXPORT int lsa_attention_single_fits(int page_size, int fused) {
     return page_size > 0 && page_size % 16 == 0 && (!LSA_BF16 || D % 32 == 0) && (!fused || D % (LSA_BF16 ? 64 : 32) == 0) ? 1 : 0;
 }
 
+// Workgroups that share a row's keys of a KV head (a quarter of the value's dimensions each, in sixteens), and the compute units: more rows than give each of them one
+// keep a workgroup to themselves, for what the scores cost is paid in each (attention_single.hpp has both sides).
+constexpr int SINGLE_PARTS = 4, SINGLE_UNITS = 256;
+
 // A step of `rows` rows of one token each, row i's at place i, in one launch (see attention_single.hpp).
 LSA_EXPORT int lsa_attention_single(
     const void* q, long q_token_stride, void* out, const void* keys, const void* values, const int* table, int table_stride, const int* row_ctx,
@@ -1477,10 +1481,11 @@ LSA_EXPORT int lsa_attention_single(
     if (decode_fusion && (q_weight == nullptr || k_weight == nullptr || cos_sin == nullptr)) return -1;
     const Geometry g = geometry_of(n_q, n_kv, gheads, 1, gtiles, page_size, window, scale, sinks, softcap, chunk, slopes, gates, gate_stride);
     const DecodeFusion fusion = {q_weight, k_weight, cos_sin, norm_eps, decode_fusion};
-    constexpr int CHUNK = ND < 8 ? ND : 8;
-    const dim3 grid(rows, n_kv * gtiles);
-#define LSA_SINGLE(MODE, WAVES, HEADS) attention_single_kernel<MODE, WAVES, HEADS><<<grid, 64 * WAVES, \
-        (size_t)WAVES * CHUNK * (HEADS ? 16 * HEADS : 4 * gheads) * 16, stream>>>( \
+    const bool shared = ND % SINGLE_PARTS == 0 && (long)rows * n_kv * gtiles * SINGLE_PARTS <= SINGLE_UNITS;
+    const dim3 grid(rows, n_kv * gtiles, shared ? SINGLE_PARTS : 1);
+#define LSA_SINGLE(MODE, WAVES, HEADS) do { if (shared) LSA_SINGLE_OF(MODE, WAVES, HEADS, (ND % SINGLE_PARTS ? 1 : SINGLE_PARTS)); else LSA_SINGLE_OF(MODE, WAVES, HEADS, 1); } while (0)
+#define LSA_SINGLE_OF(MODE, WAVES, HEADS, PARTS) attention_single_kernel<MODE, WAVES, HEADS, PARTS><<<grid, 64 * WAVES, \
+        (size_t)WAVES * (ND / PARTS < 8 ? ND / PARTS : 8) * (HEADS ? 16 * HEADS : 4 * gheads) * 16, stream>>>( \
         (const elem_t*)q, q_token_stride, (elem_t*)out, (const elem_t*)keys, (const elem_t*)values, table, table_stride, row_ctx, g, fusion)
 #if LSA_BF16 ? LSA_ND % 4 == 0 : LSA_ND % 2 == 0
 #define LSA_SINGLE_MODES(WAVES, HEADS) do { if (decode_fusion == 3) LSA_SINGLE(3, WAVES, HEADS); else if (decode_fusion == 1) LSA_SINGLE(1, WAVES, HEADS); \
@@ -1501,6 +1506,7 @@ LSA_EXPORT int lsa_attention_single(
     LSA_SINGLE_MODES(4, 0);
 #undef LSA_SINGLE_MODES
 #undef LSA_SINGLE
+#undef LSA_SINGLE_OF
     LSA_LAUNCH_CHECK();
 #endif
 }

@@ -15,6 +15,13 @@
 //   float32, 16 heads on 8 of 128, 1 row 9.6, 12.1, 21.9 against 6.4, 9.5, 19.8; 32 rows 10.4, 14.5, 30.0 against 6.9, 11.1, 26.1
 // (The host takes this kernel as long as every workgroup has a compute unit of its own, and beyond that where it stays the faster one.  float32, 16 heads
 // on 1 of 256, 16, 128, 256 and 512 keys: 11.7, 18.3, 27.2, 43.9 against 9.8, 17.0, 27.2, 48.4: the last of these contexts are a little slower.)
+// (Figures of one workgroup to a row's keys of a KV head.)  Where there are few rows, four workgroups share them (PARTS): what one compute unit pulls is the bound, so each
+// reads all keys, forms all scores and takes a quarter of the value's dimensions, five eighths of the bytes, and nothing has to meet afterwards; the sums, and so the
+// bits, are the same.  us, one workgroup and four, norm and rotation folded in, at contexts of 16, 128, 333 and 512 keys:
+//   float32, 16 heads on 8 of 128, 1 row 7.5, 11.4, 17.5, 23.4 and 7.2, 9.8, 14.0, 17.8; 4 rows 7.6, 11.9, 18.6, 25.2 and 7.3, 10.1, 14.7, 19.0; 16 on 1 of 256, 4 rows 11.3, 20.4,
+//   38.0, 51.5 and 9.0, 14.3, 22.6, 28.4
+//   bfloat16, 16 heads on 8 of 128, 1 row 7.0, 8.7, 11.5, 14.5 and 6.8, 8.1, 10.3, 12.6; 8 rows (256 workgroups) 7.4, 9.5, 12.9, 16.4 and 7.2, 8.9, 11.9, 14.4; 16 on 1 of 256,
+//   16 rows 9.5, 13.4, 19.2, 25.1 and 8.0, 10.2, 13.8, 17.1
 // Eight wavefronts where registers and LDS allow it (up to 256 keys in one round), else four.  A thread computes one head's outputs at the end, so
 // that few of them work out the wavefronts' weights (all of them doing so: 6.9 us instead of 6.2 at 40 keys).
 #pragma once
@@ -45,7 +52,7 @@ template <typename F> __device__ __forceinline__ float over_columns(float x, F f
 __device__ __forceinline__ float larger(float a, float b) { return fmaxf(a, b); }
 __device__ __forceinline__ float added(float a, float b) { return a + b; }
 
-template <int MODE, int WAVES, int HEADS>
+template <int MODE, int WAVES, int HEADS, int PARTS>
 __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel(
     const elem_t* __restrict__ q, long q_token_stride, elem_t* __restrict__ out, const elem_t* keys, const elem_t* values,
     const int* __restrict__ table, int table_stride, const int* __restrict__ row_ctx, Geometry g, DecodeFusion fusion) {
@@ -53,6 +60,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
     // HEADS > 0 (float32 only): that many query heads share the KV head, and the products are plain multiply-adds of a lane's own
     // numbers: the 32-bit matrix products would do sixteen columns' work for one or two of them (1,024 cycles against 128 a step and head).
     constexpr bool VECTOR = HEADS > 0;
+    // PARTS workgroups share a row's keys of a KV head: each forms all scores and takes a part of the value's dimensions, first_value on.
+    constexpr int NV = ND / PARTS;
+    const int first_value = PARTS == 1 ? 0 : (int)blockIdx.z * 16 * NV;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int col = lane & 15, quad = lane >> 4;
     const int row = blockIdx.x, kv_head = blockIdx.y / g.gtiles, gtile = blockIdx.y % g.gtiles;
@@ -84,9 +94,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
     struct Step {
         piece_t k[KEY_STEP / 16][NS];
 #if LSA_BF16
-        bf16x4 v[ND][2];
+        bf16x4 v[NV][2];
 #else
-        f32x4 v[ND];
+        f32x4 v[NV];
 #endif
     };
     auto load_step = [&](Step& f, int kt) {
@@ -98,9 +108,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
             const elem_t* kp = keys + page + ((size_t)kv_head * ps + slot + col) * D + PIECE * quad;
 #pragma unroll
             for (int s = 0; s < NS; ++s) f.k[t][s] = *reinterpret_cast<const piece_t*>(kp + 4 * PIECE * s);
-            const elem_t* vp = values + page + ((size_t)kv_head * D + col) * ps + slot + 4 * quad;
+            const elem_t* vp = values + page + ((size_t)kv_head * D + first_value + col) * ps + slot + 4 * quad;
 #pragma unroll
-            for (int c = 0; c < ND; ++c) {
+            for (int c = 0; c < NV; ++c) {
 #if LSA_BF16
                 f.v[c][t] = *reinterpret_cast<const bf16x4*>(vp + (size_t)(16 * c) * ps);
 #else
@@ -129,10 +139,10 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
                 }
             }
     }
-    // Which outputs a thread writes at the very end, always of one head (VECTOR: one of its 16 * ND; else four neighbouring ones, every `places`th of
+    // Which outputs a thread writes at the very end, always of one head (VECTOR: one of its 16 * NV; else four neighbouring ones, every `places`th of
     // them), and that head's sink and gate (where there is none, any number will do).
-    const int places = VECTOR ? 1 : 64 * WAVES / heads, my_head = VECTOR ? (int)threadIdx.x / (16 * ND) : (int)threadIdx.x % heads;
-    const int my_place = VECTOR ? (int)threadIdx.x % (16 * ND) : (int)threadIdx.x / heads;
+    const int places = VECTOR ? 1 : 64 * WAVES / heads, my_head = VECTOR ? (int)threadIdx.x / (16 * NV) : (int)threadIdx.x % heads;
+    const int my_place = VECTOR ? (int)threadIdx.x % (16 * NV) : (int)threadIdx.x / heads;
     const int last_head = first_head + min(my_head, heads - 1);
     const float sink = *(g.sinks != nullptr ? g.sinks + last_head : reinterpret_cast<const float*>(row_ctx));
     const float gate = (float)*(g.gates != nullptr ? g.gates + (size_t)row * g.gate_stride + last_head : token);
@@ -199,7 +209,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
     // (VECTOR) The heads' queries, in LDS for the whole step (a lane reads its quad's numbers of a head, the same for all columns: in
     // registers they would leave no room for the next step's keys), and a lane's share of the output: dimension 16 c + col, keys of its quad.
     __shared__ f32x4 queries[VECTOR ? WAVES : 1][VECTOR ? HEADS : 1][VECTOR ? NS * 4 : 1];
-    float share[VECTOR ? HEADS : 1][VECTOR ? ND : 1];
+    float share[VECTOR ? HEADS : 1][VECTOR ? NV : 1];
     auto query = [&](int h, int s) { return queries[VECTOR ? wave : 0][h][VECTOR ? 4 * s + quad : 0]; };
     if constexpr (VECTOR) {
         if (col < HEADS) {
@@ -210,28 +220,28 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
 #pragma unroll
         for (int h = 0; h < HEADS; ++h)
 #pragma unroll
-            for (int c = 0; c < ND; ++c) share[h][c] = 0.f;
+            for (int c = 0; c < NV; ++c) share[h][c] = 0.f;
     }
 #endif
-    f32x4 acc[VECTOR ? 1 : ND];
+    f32x4 acc[VECTOR ? 1 : NV];
     if constexpr (!VECTOR) {
 #pragma unroll
-        for (int c = 0; c < ND; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < NV; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
 
     if constexpr (NEW_TOKEN) if (takes_new_token) {
         // The softmax starts from the new token's key (maximum = its score, sum = 1, output = its value); its key and value go into the cache.
         const int slot = q_pos - (int)__umulhi((unsigned)q_pos, g.page_magic) * ps;
         const int entry = row_table[min((int)__umulhi((unsigned)q_pos, g.page_magic), table_stride - 1)];
-        const elem_t* vh = token + (size_t)(g.n_q + g.n_kv + kv_head) * D;
+        const elem_t* vh = token + (size_t)(g.n_q + g.n_kv + kv_head) * D + first_value;
 #if LSA_BF16
-        bf16x4 vnew[ND];
+        bf16x4 vnew[NV];
 #pragma unroll
-        for (int c = 0; c < ND; ++c) vnew[c] = *reinterpret_cast<const bf16x4*>(vh + 16 * c + 4 * quad);
+        for (int c = 0; c < NV; ++c) vnew[c] = *reinterpret_cast<const bf16x4*>(vh + 16 * c + 4 * quad);
 #else
-        f32x4 vnew[ND];
+        f32x4 vnew[NV];
 #pragma unroll
-        for (int c = 0; c < ND; ++c) vnew[c] = *reinterpret_cast<const f32x4*>(vh + 16 * c + 4 * quad);
+        for (int c = 0; c < NV; ++c) vnew[c] = *reinterpret_cast<const f32x4*>(vh + 16 * c + 4 * quad);
 #endif
         if constexpr (FUSED) {
 #pragma unroll
@@ -257,7 +267,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
                 run_sum[h] = 1.f / 16.f;                           // (of the column's sixteenth: the sums of the columns are added up)
                 // the value's dimension 16 c + col, in quad 0 alone
 #pragma unroll
-                for (int c = 0; c < ND; ++c) share[h][c] = quad == 0 ? vh[16 * c + col] : 0.f;
+                for (int c = 0; c < NV; ++c) share[h][c] = quad == 0 ? vh[16 * c + col] : 0.f;
             }
 #endif
         } else {
@@ -270,17 +280,19 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
             run_max[0] = capped(dot * g.scale, g);
             run_sum[0] = quad == 0 ? 1.f : 0.f;
 #pragma unroll
-            for (int c = 0; c < ND; ++c)
+            for (int c = 0; c < NV; ++c)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[c][r] = (float)vnew[c][r];
         }
         if (col == 0 && entry >= 0 && gtile == 0) {
             elem_t* kp = const_cast<elem_t*>(keys) + (size_t)entry * page_elems + ((size_t)kv_head * ps + slot) * D + PIECE * quad;
+            if (first_value == 0) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) *reinterpret_cast<piece_t*>(kp + 4 * PIECE * s) = kh[s];
-            elem_t* vp = const_cast<elem_t*>(values) + (size_t)entry * page_elems + ((size_t)kv_head * D + 4 * quad) * ps + slot;
+                for (int s = 0; s < NS; ++s) *reinterpret_cast<piece_t*>(kp + 4 * PIECE * s) = kh[s];
+            }
+            elem_t* vp = const_cast<elem_t*>(values) + (size_t)entry * page_elems + ((size_t)kv_head * D + first_value + 4 * quad) * ps + slot;
 #pragma unroll
-            for (int c = 0; c < ND; ++c)
+            for (int c = 0; c < NV; ++c)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) vp[(size_t)(16 * c + r) * ps] = vnew[c][r];
         }
@@ -300,7 +312,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
             for (int r = 0; r < 4; ++r) {                          // values of keys outside may hold anything: keep them out of the sum
                 const bool there = kt + 4 * quad + r >= lo && kt + 4 * quad + r < hi;
 #pragma unroll
-                for (int c = 0; c < ND; ++c) now.v[c][r] = there ? now.v[c][r] : 0.f;
+                for (int c = 0; c < NV; ++c) now.v[c][r] = there ? now.v[c][r] : 0.f;
             }
 #pragma unroll
             for (int h = 0; h < HEADS; ++h) {
@@ -321,7 +333,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
 #pragma unroll
                 for (int r = 0; r < 4; ++r) weight[r] = __shfl(p, 16 * quad + 4 * quad + r, 64);
 #pragma unroll
-                for (int c = 0; c < ND; ++c) {
+                for (int c = 0; c < NV; ++c) {
                     float sum = share[h][c] * alpha;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) sum += weight[r] * now.v[c][r];
@@ -375,7 +387,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
                     keep[t][r / 2] = r & 1 ? keep[t][r / 2] | there : there;
                 }
 #pragma unroll
-            for (int c = 0; c < ND; ++c) {
+            for (int c = 0; c < NV; ++c) {
                 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
                 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
                 const u32x2 a = __builtin_bit_cast(u32x2, now.v[c][0]), b = __builtin_bit_cast(u32x2, now.v[c][1]);
@@ -392,7 +404,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
                 there[r] = kt + 4 * quad + r >= lo && kt + 4 * quad + r < hi;
             }
 #pragma unroll
-            for (int c = 0; c < ND; ++c) {
+            for (int c = 0; c < NV; ++c) {
                 acc[c] *= alpha;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(there[r] ? now.v[c][r] : 0.f, weight[r], acc[c], 0, 0, 0);
@@ -404,7 +416,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
     }
 
     // The wavefronts' sums meet in LDS, CHUNK times 16 dimensions a round; every wavefront gets here, and the loop's trips are the workgroup's.
-    constexpr int CHUNK = ND < 8 ? ND : 8;
+    constexpr int CHUNK = NV < 8 ? NV : 8;
     extern __shared__ f32x4 partial[];                             // [WAVES][CHUNK][4][heads], VECTOR: [WAVES][HEADS][CHUNK][16] of four quads' shares
     __shared__ float wave_max_of[WAVES][16], wave_sum_of[WAVES][16];
     if constexpr (VECTOR) {
@@ -447,20 +459,20 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) scale_of[w] *= inv;
     };
-    elem_t* row_out = out + ((size_t)row * g.n_q + first_head) * D;
+    elem_t* row_out = out + ((size_t)row * g.n_q + first_head) * D + first_value;
 #pragma unroll
-    for (int c0 = 0; c0 < ND; c0 += CHUNK) {
+    for (int c0 = 0; c0 < NV; c0 += CHUNK) {
         if (c0) __syncthreads();                                   // (the round before has been read)
-        const int chunk = min(CHUNK, ND - c0);
+        const int chunk = min(CHUNK, NV - c0);
         if constexpr (VECTOR) {
 #if !LSA_BF16
 #pragma unroll
             for (int h = 0; h < R; ++h)
 #pragma unroll
                 for (int c = 0; c < CHUNK; ++c)
-                    if (c0 + c < ND) reinterpret_cast<float*>(partial)[(((wave * HEADS + h) * CHUNK + c) * 16 + col) * 4 + quad] = share[h][c0 + c];
+                    if (c0 + c < NV) reinterpret_cast<float*>(partial)[(((wave * HEADS + h) * CHUNK + c) * 16 + col) * 4 + quad] = share[h][c0 + c];
             __syncthreads();
-            static_assert(CHUNK == ND && CHUNK * 16 * HEADS <= 64 * WAVES, "an output a thread");
+            static_assert(CHUNK == NV && CHUNK * 16 * HEADS <= 64 * WAVES, "an output a thread");
             if (my_head < HEADS) {
                 find_scales(my_head);
                 f32x4 sum = {0.f, 0.f, 0.f, 0.f};
@@ -472,7 +484,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void attention_single_kernel
         } else {
 #pragma unroll
             for (int c = 0; c < CHUNK; ++c)
-                if (c0 + c < ND && col < heads) partial[((wave * CHUNK + c) * 4 + quad) * heads + col] = acc[c0 + c];
+                if (c0 + c < NV && col < heads) partial[((wave * CHUNK + c) * 4 + quad) * heads + col] = acc[c0 + c];
             __syncthreads();
             if (my_place < chunk * 4 && my_place < places) {
                 if (c0 == 0) find_scales(my_head);
