@@ -230,7 +230,9 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
             // (the fewer tiles share W's lines, the longer a tall one waits for them: 0.41 us a slab where it has them alone, 0.33 with three)
             const double slab = shape.slab + (tile == TALL ? 0.1 / ((M + 127) / 128) : 0.0), rate = tile == LARGE ? 4.1 : 5.2;
             double us = shape.start + slab * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.7 : tiles * parts > 7 * UNITS / 8 ? 1.2 : 1.0);
-            us = us > megabytes / rate + 3.0 ? us : megabytes / rate + 3.0;
+            // (the weights come as fast as many workgroups pull: with 160 of them 33 rows of 5,120 x 25,600 took 71 us, with 320 67)
+            const double load = tiles * parts < UNITS ? (double)(tiles * parts) / UNITS : 1.0, way = megabytes / (rate * (0.5 + 0.5 * load)) + 3.0;
+            us = us > way ? us : way;
             if (form == SUMS) us += parts * 8e-6 * M * N / 4.0;    // written and read
             else if (parts > 1) us += 3.4 + parts * 8e-6 * M * weights / 3.0;      // and a launch
             if (us < best) {
@@ -250,9 +252,12 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
         const double us = 3.0 + tiles / UNITS * (4.5 + 1.5 * slabs) + (last ? 4.5 + (1.05 + 0.45 * last / UNITS) * slabs : 0.0);
         if (us < best && us < 0.97 * library) return 16 + WIDE;
     }
-    // (up to 128 rows the sums were faster than the few-row kernels' throughout: 33 rows, with the norm, 2,048 x 6,144 13.7, 12.3; 4,096 x 4,096 15.3, 14.1; 100 rows 18.8, 15.2 and
-    // 21.3, 17.9; but for 24 rows and fewer of a large weight: 17 rows, 4,096 x 8,192 19.6, 20.9)
-    if (form == SUMS && M <= FEW_ROWS) return M <= 24 && weights * K > 3e7 ? NONE : plan;
+    // Up to 128 rows the other way for sums is the kernel that shares the rows in LDS (lsa_gemm_split): slower for weights of up to 50 MB throughout (33 rows, with the norm,
+    // 2,048 x 6,144 13.7, 12.3; 4,096 x 4,096 15.3, 14.1; 100 rows 18.8, 15.2 and 21.3, 17.9); beyond that its time, again with the norm, is a line in the weights and the rows, and
+    // where tiles leave compute units idle it is the faster one: 48 rows of 5,120 x 25,600 62.8, 79.0, of 5,120 x 17,408 49.6, 52.5, 29 rows of 5,120 x 5,120 20.6, 24.5, of
+    // 4,096 x 8,192 21.5, 23.3; 128 rows of 4,096 x 12,288 41.4, 35.6.
+    if (form == SUMS && M <= FEW_ROWS)
+        return weights * K <= 2.6e7 || best + 4.0 < 0.86 * (7.1 + megabytes / 4.9 + 0.05 * M + 0.00066 * M * megabytes) ? plan : NONE;
     return best < 0.9 * library ? plan : NONE;
 }
 

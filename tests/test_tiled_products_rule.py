@@ -54,3 +54,14 @@ def test_products_that_were_measured_to_be_faster(plan):
 def test_gated_products_of_short_inner_dimensions_stay_where_they_were(plan):
     """Neither small tiles nor large ones: the kernel that shares the activations, or the library, has them."""
     assert not any(plan(GATED, rows, columns, inner) for rows in (17, 33, 70, 206, 777, 2048, 9000) for columns in (32, 64, 96, 768, 3072, 12288) for inner in (64, 128, 512, 960))
+
+
+def test_sums_of_large_weights_on_few_tiles_stay_with_the_few_row_kernel(plan):
+    """Output and down projections whose tiles leave compute units idle, at a batch's 17 to 128 rows; where they do not, or the weight is small, the tiles keep them."""
+    for rows in (17, 28, 29, 33, 48, 64):
+        for columns, inner in ((5120, 5120), (5120, 8192), (5120, 17408), (5120, 25600)):
+            assert plan(SUMS, rows, columns, inner) < 32, (rows, columns, inner)
+    assert all(plan(SUMS, rows, 4096, 8192) < 32 for rows in (17, 24, 28, 29, 32))
+    assert all(plan(SUMS, rows, 5120, 25600) < 32 for rows in (65, 96, 128))
+    assert all(plan(SUMS, rows, columns, inner) >= 32 for rows in (17, 33, 64, 128) for columns, inner in ((2048, 6144), (4096, 4096), (2560, 9728)))
+    assert all(plan(SUMS, rows, 4096, 12288) >= 32 for rows in (48, 64, 112, 128))
