@@ -248,8 +248,12 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     if (form == ACTIVATED) library += 3.5 + 4e-6 * M * N / 5.0;
     if (form == GATED && slabs >= 16) {
         const long tiles = (long)((M + WIDE_TILE - 1) / WIDE_TILE) * ((N + WIDE_TILE / 2 - 1) / (WIDE_TILE / 2)), last = tiles % UNITS;
-        // (a slab takes 1.05 us where few compute units work, 1.5 where all do: power; shorter inner dimensions as above)
-        const double us = 3.0 + tiles / UNITS * (4.5 + 1.5 * slabs) + (last ? 4.5 + (1.05 + 0.45 * last / UNITS) * slabs : 0.0);
+        // A launch takes 13 us around the slabs of its last round and 6 around those of a full one (1,024 rows of 3,072 x 1,024, 16 slabs on 96 compute units, 33 us, 26.6 for the
+        // library's product and the activation), a slab 1.0 us where few compute units work, 1.5 where all do: power.  A tile of 64 rows and fewer leaves three tenths of that out,
+        // and there the weights' way is what counts (17 rows, 25,600 x 5,120 on 200 compute units 101 us, 17,408 x 5,120 on 136 84).
+        const double load = (double)last / UNITS, blocks = M > 192 ? 4 : (M + 63) / 64, pulled = tiles < UNITS ? load : 1.0;
+        const double products = 7.0 + tiles / UNITS * (6.0 + 1.5 * slabs) + (last ? 6.0 + (1.0 + 0.5 * load) * (0.6 + 0.1 * blocks) * slabs : 0.0);
+        const double way = megabytes / (5.4 * (0.5 + 0.5 * pulled)) + 3.0, us = products > way ? products : way;
         if (us < best && us < 0.97 * library) return 16 + WIDE;
     }
     // Up to 128 rows the other way for sums is the kernel that shares the rows in LDS (lsa_gemm_split): slower for weights of up to 50 MB throughout (33 rows, with the norm,

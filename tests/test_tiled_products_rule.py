@@ -65,3 +65,11 @@ def test_sums_of_large_weights_on_few_tiles_stay_with_the_few_row_kernel(plan):
     assert all(plan(SUMS, rows, 5120, 25600) < 32 for rows in (65, 96, 128))
     assert all(plan(SUMS, rows, columns, inner) >= 32 for rows in (17, 33, 64, 128) for columns, inner in ((2048, 6144), (4096, 4096), (2560, 9728)))
     assert all(plan(SUMS, rows, 4096, 12288) >= 32 for rows in (48, 64, 112, 128))
+
+
+def test_large_gated_tiles_are_not_taken_for_a_few_slabs(plan):
+    """A launch of 256 x 256 tiles costs some 13 us beside its slabs: 16 or 32 of them on a part of the compute units are the library's."""
+    assert not any(plan(GATED, rows, 3072, 1024) % 16 == 4 for rows in (17, 256, 641, 820, 1000, 1024, 1100, 1200, 1280, 1400))
+    assert all(plan(GATED, rows, 3072, 1024) % 16 == 4 for rows in (2001, 2048, 2300, 2560))
+    assert not any(plan(GATED, rows, 6144, 2048) % 16 == 4 for rows in (257, 512, 700, 768, 820)) and plan(GATED, 1200, 6144, 2048) % 16 == 4
+    assert not any(plan(GATED, rows, 17408, 5120) for rows in (17, 24, 29, 48, 64))          # (136 compute units pull its weights)
