@@ -194,8 +194,8 @@ __global__ __launch_bounds__(WIDE_THREADS) void wide_gated_kernel(const bf16_t* 
 // What lsa_product can be asked for: a tile, and for SUMS the parts of K, as 16 parts + tile.  ADDED in a plan for PLAIN or GATED: the sums, and a kernel behind
 // them that adds the parts up (lsa_sum_parts, lsa_gated_parts).
 enum Tile { NONE, SMALL, TALL, LARGE, WIDE };
-struct TileShape { int rows, columns; double start, slab; };       // columns of W; us of a launch with a tile a compute unit, and a slab's
-static const TileShape SHAPES[] = {{0, 0, 0, 0}, {64, 64, 3.0, 0.31}, {128, 64, 3.6, 0.31}, {128, 128, 4.2, 0.50}, {256, 256, 4.5, 0}};
+struct TileShape { int rows, columns; double start, slab, full; };     // columns of W; us of a launch with a tile a compute unit, of a slab, and what full rows add to that
+static const TileShape SHAPES[] = {{0, 0, 0, 0, 0}, {64, 64, 3.4, 0.21, 0.10}, {128, 64, 4.0, 0.25, 0.18}, {128, 128, 4.6, 0.38, 0.18}, {256, 256, 0, 0, 0}};
 constexpr int UNITS = 256;                                         // compute units
 constexpr int MOST_PARTS = 8, ADDED = 1 << 12;
 
@@ -204,13 +204,15 @@ static bool fits(int form, long M, long N, long K) {
     return M >= 1 && N >= 8 && K >= SLAB && K % SLAB == 0 && N % 8 == 0 && (form == GATED ? 2 * N : 256) * K * 2 + K * 2 < (long)BUFFER_BYTES && 256 * K * 2 < (long)BUFFER_BYTES;
 }
 
-// The tile (and parts) for a product of these sizes, or 0 where the library's product is expected to be as fast (with the kernel of the activation behind it).  Both
-// times are lines through what was measured at 17 to 3,000 rows of 31 products of this package's models: a launch's start and a slab's time for the tiles here,
-// for the library (whose own choice of tiles nobody can foretell) a start, K and the operations.  Over 31 products and 17 to 900 rows, the way taken against the one
-// before, up to 128 rows and beyond: gated 1.17 and 1.12 times as fast, plain 1.10 and 1.09, activated 1.07 and 1.13, sums with the norm behind them 1.12 and 1.06, heads
-// 1.04 and 1.00, the worst 0.98 and 0.95.  A product whose tiles do not go round the compute units in one round stays the library's unless it is gated and large.  Up to 128
-// rows the parts may be added up by a launch of their own (64 rows, 2,816 x 2,048 library 12.1, one launch 12.2, so 9.7; 32 rows of 4,096 x 4,096 13.9, 17.9, 12.0; gated
-// 2,816 x 4,096 15.4, 18.4, 12.2).
+// The tile (and parts) for a product of these sizes, or 0 where the other way is expected to be as fast: the library's product, with the kernel of the activation behind
+// it, or up to 128 rows the few-row kernels.  Both times are lines through what was measured at 50 numbers of rows from 17 to 4,096 of 48 products of this package's
+// models: a launch's start and a slab's time for the tiles here, for the library (whose own choice of tiles nobody can foretell: with its tiles' rounds in the line its
+// times are met no better, within an eighth) a start, K and the operations.  So where the library has just begun a round its price is too low, and sizes that the tiles would
+// make faster stay with it.  At 48 other numbers of rows, 18 to 4,000, of 52 products 709 of 2,433 are taken, up to 128 rows and beyond: gated 1.18 and 1.22 times as fast as the other
+// way, plain 1.19 and 1.22, activated 1.19 and 1.23, sums with the norm behind them 1.12 and 1.15, heads 1.11 and none.  The worst: 0.94 (240 rows, sums of 2,560 x 9,728 33.4, 35.4), 0.96
+// (sums of 2,048 x 1,408 at 400 rows; gated 3,072 x 1,024 at 1,600); all others 0.97 and more.  A product whose tiles do not go round the compute units in one round stays the
+// library's unless it is gated and large.  Up to 128 rows the parts may be added up by a launch of their own (64 rows, 2,816 x 2,048 library 12.1, one launch 12.2, so 9.7; 32
+// rows of 4,096 x 4,096 13.9, 17.9, 12.0; gated 2,816 x 4,096 15.4, 18.4, 12.2).
 LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     if (form < PLAIN || form > SUMS || !fits(form, M, N, K)) return NONE;
     if (form == SUMS && M > FEW_ROWS && N < 1024) return NONE;     // (measured from 1,024 columns on: fewer go the library's way, whole or in ranges)
@@ -227,9 +229,10 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
             // (two of the small tiles' workgroups fit a compute unit: where the weights' way bounds them, 33 rows of 32,768 x 4,096 63 us for the library, 55; gated products
             // beyond one round, and with less than 1,024 of K, stay with the kernel that shares the activations, or the library)
             if (tiles * parts > (tile == SMALL && parts == 1 && form != GATED ? 2 : 1) * UNITS || slabs < 4 * parts || (form == GATED && slabs < 16)) continue;
-            // (the fewer tiles share W's lines, the longer a tall one waits for them: 0.41 us a slab where it has them alone, 0.33 with three)
-            const double slab = shape.slab + (tile == TALL ? 0.1 / ((M + 127) / 128) : 0.0), rate = tile == LARGE ? 4.1 : 5.2;
-            double us = shape.start + slab * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.7 : tiles * parts > 7 * UNITS / 8 ? 1.2 : 1.0);
+            // (rows behind the last one repeat it and cost no way of their own: 257 and 384 rows of 2,048 x 2,048 on tiles of 128 x 64 13.9 and 16.7 us, 513 and 512 14.2 and 16.8,
+            // where tiles of 64 x 64 take 12.0 for 512, one a compute unit)
+            const double filled = (double)M / ((M + shape.rows - 1) / shape.rows * shape.rows), rate = tile == LARGE ? 4.1 : 5.2;
+            double us = shape.start + (shape.slab + shape.full * filled) * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.8 : 1.0);
             // (the weights come as fast as many workgroups pull: with 160 of them 33 rows of 5,120 x 25,600 took 71 us, with 320 67)
             const double load = tiles * parts < UNITS ? (double)(tiles * parts) / UNITS : 1.0, way = megabytes / (rate * (0.5 + 0.5 * load)) + 3.0;
             us = us > way ? us : way;
@@ -261,8 +264,8 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     // where tiles leave compute units idle it is the faster one: 48 rows of 5,120 x 25,600 62.8, 79.0, of 5,120 x 17,408 49.6, 52.5, 29 rows of 5,120 x 5,120 20.6, 24.5, of
     // 4,096 x 8,192 21.5, 23.3; 128 rows of 4,096 x 12,288 41.4, 35.6.
     if (form == SUMS && M <= FEW_ROWS)
-        return weights * K <= 2.6e7 || best + 4.0 < 0.86 * (7.1 + megabytes / 4.9 + 0.05 * M + 0.00066 * M * megabytes) ? plan : NONE;
-    return best < 0.9 * library ? plan : NONE;
+        return weights * K <= 2.6e7 || best + 4.0 < 0.85 * (7.1 + megabytes / 4.9 + 0.05 * M + 0.00066 * M * megabytes) ? plan : NONE;
+    return best < (M > FEW_ROWS ? 0.95 : 0.88) * library ? plan : NONE;
 }
 
 template <int FORM>

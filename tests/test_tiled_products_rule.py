@@ -73,3 +73,14 @@ def test_large_gated_tiles_are_not_taken_for_a_few_slabs(plan):
     assert all(plan(GATED, rows, 3072, 1024) % 16 == 4 for rows in (2001, 2048, 2300, 2560))
     assert not any(plan(GATED, rows, 6144, 2048) % 16 == 4 for rows in (257, 512, 700, 768, 820)) and plan(GATED, 1200, 6144, 2048) % 16 == 4
     assert not any(plan(GATED, rows, 17408, 5120) for rows in (17, 24, 29, 48, 64))          # (136 compute units pull its weights)
+
+
+def test_tiles_whose_rows_are_full_are_priced_so(plan):
+    """A slab of a tile with all its rows takes longer than one whose last rows repeat: whole multiples of 128 rows do not go to tiles of 128 x 64 for one row more to a launch."""
+    assert plan(PLAIN, 512, 2048, 2048) == 16 + 1
+    for form, rows, columns, inner in ((PLAIN, 768, 2048, 2048), (PLAIN, 384, 4096, 2048), (SUMS, 384, 2048, 1408), (SUMS, 512, 2048, 1408), (ACTIVATED, 384, 8192, 4096)):
+        assert plan(form, rows, columns, inner) < (32 if form == SUMS else 1), (form, rows, columns, inner)
+    for rows in (1792, 1900, 2001, 2047, 2048):                  # one round of tiles of 128 x 128, whatever the last one holds
+        assert plan(PLAIN, rows, 2048, 2048) == 16 + 3, rows
+    for form, rows, columns, inner in ((PLAIN, 820, 2048, 2048), (PLAIN, 448, 4096, 2048), (ACTIVATED, 257, 8448, 2048)):
+        assert plan(form, rows, columns, inner), (form, rows, columns, inner)
