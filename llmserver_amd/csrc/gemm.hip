@@ -833,7 +833,7 @@ LSA_EXPORT int lsa_gemm_split_gated(const void* x, const void* w, void* hidden, 
 // in one trip of 8 5.0, of 4 3.7).  One trip of 12 or 16 is no faster than two (1,024 x 4,096 8.7 in one, 8.5).
 constexpr int F32_FUSED_ROWS = GEMM_WAVES;
 template <bool GATED, bool FOLDED, int STEPS>
-__global__ __launch_bounds__(GEMM_WAVES * 64, STEPS > 8 ? 2 : 4) void gemm_few_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y,
+__global__ __launch_bounds__(GEMM_WAVES * 64, 4) void gemm_few_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y,
                                                                           int M, int N, int K, int R, Fusion fusion) {
     __shared__ float partial[GEMM_WAVES][256];
     __shared__ float row_scale[F32_FUSED_ROWS];
@@ -907,13 +907,15 @@ __global__ __launch_bounds__(GEMM_WAVES * 64, STEPS > 8 ? 2 : 4) void gemm_few_f
 }
 
 // Whether the sizes go this way (K a multiple of 4): where this stream was measured to be no slower than the library's product, which is poor at short
-// rows and at rows of 1,024 and 2,048 numbers, and good between and behind those.  Here eight wavefronts want four steps of 16 each to have anything
-// under way together, a workgroup more than a compute unit's share waits for a second round, and from 5 rows on X takes a noticeable part of
+// rows and at rows of 1,024 and 2,048 numbers, and good between and behind those.  Here eight wavefronts want four steps each to have anything
+// under way together, and from 5 rows on X takes a noticeable part of
 // the way into a compute unit.  us against the library's, N x K, replayed from a graph with cold weights, at 2 rows unless stated:
 //   up to 2,048 rows of W: 1,024 x 1,024 3.6, 8.0; 2,048 x 2,048 6.0, 12.0; 1,024 x 3,072 6.1, 10.9; 4 rows of 1,024 x 6,144 11.4, 17.4, of 2,048 x 6,144 14.3, 18.0 (8 rows
 // 16.5, 18.1).
 //   up to 8,192: 4,096 x 1,024 6.2, 11.7; 6,144 x 1,024 7.6, 12.7 (8 rows 8.7, 12.5); 6,144 x 768 7.6, 10.5; 6,144 x 1,536 at 8 rows 13.7, 12.0; 4,096 x 2,048 8.7, 12.4; 2,560 x 4,096
-// 13.9, 14.2 (8 rows 18.2, 13.8); 2,560 x 9,728 30, 32 (8 rows 41, 28).
+// 13.9, 14.2 (8 rows 18.2, 13.8); 2,560 x 9,728 30, 32 (8 rows 41, 28).  x 2,048 at 1 and 4 rows, eight rows of W a workgroup and two workgroups a compute unit: 4,104 rows (one
+// workgroup more than a round) 10.6, 14.9 and 12.2, 14.9; 5,120 11.6, 16.2 and 12.9, 16.2; 6,144 12.3, 16.4 and 14.1, 16.4; 7,168 14.1, 16.9 and 16.3, 17.0; 8,192 (sixteen a
+// workgroup) 16.4, 17.8 and 18.0, 17.9; with the sum and the norm behind it, 5,120 15.2, 21.8 and 16.7, 22.1; gated 13.0, 18.2 and 14.6, 18.4.  (2,304 to 4,000 rows were faster here as well, 2,560 8.6, 13.0; they have stayed the library's.)
 //   a vocabulary: 151,936 x 1,024 111, 209 (8 rows 138, 212; 16 rows 163, 210), x 2,048 218, 256 (8 rows 270, 262); x 512 1.77 times the library's time, x 2,560
 // 1.11; 65,536 x 1,024 1.07 (16 rows 1.40), x 2,560 1.27 (16 rows 232, 120); 16,384 x 1,024 at 16 rows 22, 19.
 LSA_EXPORT int lsa_gemm_few_f32_fits(int M, int N, int K) {
@@ -923,8 +925,7 @@ LSA_EXPORT int lsa_gemm_few_f32_fits(int M, int N, int K) {
     if (N <= 2048) return K <= (M <= 4 ? 6144 : 2048) ? 1 : 0;
     if (N > 8192) return 0;
     if (K <= 1024) return K >= 768 + 64 * (M > 4 ? M - 4 : 0) ? 1 : 0;
-    const int workgroups = (N + 15) / 16, rounds = (workgroups + 255) / 256;
-    return K == 2048 && M <= 4 && N >= 4096 && 10 * workgroups >= 9 * 256 * rounds ? 1 : 0;
+    return K == 2048 && M <= 4 && N >= 4096 ? 1 : 0;
 }
 
 // Rows of W a workgroup: 4 while that is a workgroup a compute unit (2 rows of 1,024 x 3,072: 8 rows 7.1 us, 4 6.1; of 1,536 x 4,096 9.4, 12.1), 16 from where 8 would be four
