@@ -416,7 +416,7 @@ class HipOps(KernelNamespace):
             return self._linear_few_rows_float32(x, weight, out, bias)
         if not out_float32 and bias is None and not rows_per_workgroup and (out is None or (out.dtype == torch.bfloat16 and out.is_contiguous() and
                 out.device == x.device and tuple(out.shape) == (x.shape[0], weight.shape[0]) and not out.requires_grad and out.data_ptr() % 8 == 0)):
-            if not self._split_first(x):
+            if not self._sums_first(x, weight):
                 done = self._tiled_product("plain", x, weight, out=out)
                 if done is not None:
                     return done
@@ -425,7 +425,7 @@ class HipOps(KernelNamespace):
                 out = torch.empty((x.shape[0], weight.shape[0]), device=x.device, dtype=torch.bfloat16) if out is None else out
                 _launched(self._elementwise.lsa_sum_parts(_ptr(sums), sums.shape[0], _ptr(out), x.shape[0], weight.shape[0], _stream()), "sum_parts")
                 return out
-        if bias is None and not rows_per_workgroup and (out is None or not out_float32) and (out_float32 or self._split_first(x)):
+        if bias is None and not rows_per_workgroup and (out is None or not out_float32) and (out_float32 or self._sums_first(x, weight)):
             done = self._tiled_product("plain", x, weight, out=out, out_float32=out_float32)
             if done is not None:
                 return done
@@ -445,7 +445,7 @@ class HipOps(KernelNamespace):
         rounding), behind the library's product otherwise."""
         if self._few_rows(x, weight) and not self.library_is_faster("plain", x, weight, False, False):
             return self.linear_few_rows(x, weight, activation=activation)
-        done = self._tiled_product("activated", x, weight, activation) if activation in self.PLAIN_ACTIVATIONS and not self._split_first(x) else None
+        done = self._tiled_product("activated", x, weight, activation) if activation in self.PLAIN_ACTIVATIONS and not self._sums_first(x, weight) else None
         if done is not None:
             return done
         y = self.linear(x, weight)
@@ -489,11 +489,13 @@ class HipOps(KernelNamespace):
     PRODUCT_FORMS = ("plain", "gated", "activated", "sums")           # what lsa_product computes (its codes)
     PRODUCT_ADDED = 1 << 12                                            # in a plan: partial sums, which a kernel behind them adds up
 
-    @staticmethod
-    def _split_first(x) -> bool:
+    def _sums_first(self, x, weight, gated=False) -> bool:
         """Whether partial sums of the few-row kernel, added up, go before the tiles: few rows whose inner dimension is long enough for many parts (us at 17, 25 and 32
-        rows, those and the tiles: 2,112 x 2,048 7.3, 7.7, 8.0 and 7.7, 8.2, 8.0; 4,096 x 2,048 9.0, 9.7, 10.4 and 9.0, 9.0, 9.7; 4,096 x 1,024 7.2, 7.4, 7.7 and 6.0, 6.0, 6.2)."""
-        return x.shape[0] <= 28 and x.shape[1] >= 2048
+        rows, those and the tiles: 2,112 x 2,048 7.3, 7.7, 8.0 and 7.7, 8.2, 8.0; 4,096 x 2,048 9.0, 9.7, 10.4 and 9.0, 9.0, 9.7; 4,096 x 1,024 7.2, 7.4, 7.7 and 6.0, 6.0, 6.2), and a
+        weight of the size that those sums take (:meth:`_partial_sums_to_add`): of any other the tiles are asked at once (17 and 28 rows of 8,448 x 2,048, activated: 13.5 and 13.2,
+        library and activation 17.4 and 17.2)."""
+        low, high = self.SUMMED_GATED_WEIGHT if gated else self.SUMMED_WEIGHT
+        return x.shape[0] <= 28 and x.shape[1] >= 2048 and low <= weight.numel() <= high
 
     def _tiled_product(self, form, x, weight, activation="silu", out=None, out_float32=False):
         """The product of many rows by this package's own tiles where they are expected to be faster than the library's (the rule stands in ``csrc/product.hip``,
@@ -694,13 +696,14 @@ class HipOps(KernelNamespace):
         if rows > self.skinny_rows:
             if row_scale is not None or pairs_per_workgroup:
                 return None
-            done = None if self._split_first(x) else self._tiled_product("gated", x, gate_up_weight, activation)
+            sums_first = self._sums_first(x, gate_up_weight, gated=True)
+            done = None if sums_first else self._tiled_product("gated", x, gate_up_weight, activation)
             if done is not None:
                 return done
             sums = self._partial_sums_to_add(x, gate_up_weight, gated=True)
             if sums is None:
                 done = self._linear_gated_beyond_few_rows(x, gate_up_weight)
-                return done if done is not None else self._tiled_product("gated", x, gate_up_weight, activation)
+                return self._tiled_product("gated", x, gate_up_weight, activation) if done is None and sums_first else done
             out = torch.empty((rows, inter), device=x.device, dtype=torch.bfloat16)
             _launched(self._elementwise.lsa_gated_parts(_ptr(sums), sums.shape[0], _ptr(out), rows, inter, self.ACTIVATIONS.index(activation), _stream()),
                       "gated_parts")

@@ -164,3 +164,24 @@ def test_a_captured_step_replays_the_tiles(ops):
         torch.cuda.synchronize()
         again = ops.linear_gated(x, weight)
         assert torch.equal(y, ops.linear(x, weight)) and (hidden is None or torch.equal(hidden, again))
+
+
+@pytest.mark.parametrize("rows", [17, 28, 29])
+@pytest.mark.parametrize("columns", [2112, 8448])
+def test_activated_products_of_few_rows_are_asked_for_by_the_weights_size(ops, rows, columns, monkeypatch):
+    """Up to 28 rows a weight that partial sums take goes there; one that they refuse goes to the tiles, where the activation is formed on the 32-bit sums and the result rounded
+    once.  Of a product that stays the library's the plan is asked once."""
+    print(f"activated products of few rows {rows} {columns}", flush=True)
+    asked = []
+    real = ops._tiled_product
+    monkeypatch.setattr(ops, "_tiled_product", lambda *a, **k: (lambda done: (asked.append((a[0], done is not None)), done)[1])(real(*a, **k)))
+    x, weight = drawn(rows, columns, 2048, rows)
+    got = ops.linear_activated(x, weight, "relu2").double()
+    assert (("activated", True) in asked) == (rows > 28 or columns == 8448)
+    exact, off = x.double() @ weight.double().T, 2049 * 2.0 ** -24 * (x.double().abs() @ weight.double().abs().T)
+    want = exact.clamp(min=0) ** 2
+    roundings = 1 if rows > 28 or columns == 8448 else 3         # (of the result; behind a rounded product twice that rounding more, for the square)
+    assert bool(((got - want).abs() <= off * (2 * exact.abs() + off) + roundings * 2.0 ** -8 * want * 1.01).all())
+    asked.clear()
+    x, weight = drawn(333, 12288, 2048, rows)
+    assert ops.linear_gated(x, weight) is None and asked == [("gated", False)]
