@@ -195,7 +195,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void wide_gated_kernel(const bf16_t* 
 // them that adds the parts up (lsa_sum_parts, lsa_gated_parts).
 enum Tile { NONE, SMALL, TALL, LARGE, WIDE };
 struct TileShape { int rows, columns; double start, slab, full; };     // columns of W; us of a launch with a tile a compute unit, of a slab, and what full rows add to that
-static const TileShape SHAPES[] = {{0, 0, 0, 0, 0}, {64, 64, 3.4, 0.21, 0.10}, {128, 64, 4.0, 0.25, 0.18}, {128, 128, 4.6, 0.38, 0.18}, {256, 256, 0, 0, 0}};
+static const TileShape SHAPES[] = {{0, 0, 0, 0, 0}, {64, 64, 3.4, 0.25, 0.06}, {128, 64, 3.8, 0.31, 0.11}, {128, 128, 4.6, 0.46, 0.10}, {256, 256, 0, 0, 0}};
 constexpr int UNITS = 256;                                         // compute units
 constexpr int MOST_PARTS = 8, ADDED = 1 << 12;
 
@@ -215,7 +215,9 @@ static bool fits(int form, long M, long N, long K) {
 // rows of 4,096 x 4,096 13.9, 17.9, 12.0; gated 2,816 x 4,096 15.4, 18.4, 12.2).
 LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     if (form < PLAIN || form > SUMS || !fits(form, M, N, K)) return NONE;
-    if (form == SUMS && M > FEW_ROWS && N < 1024) return NONE;     // (measured from 1,024 columns on: fewer go the library's way, whole or in ranges)
+    // (sums beyond 128 rows were measured from 1,024 columns on: fewer go the library's way, whole or in ranges; and in parts of few slabs they are slower from 257 rows on: 384 and 512 rows
+    // of 2,048 x 1,408 with the norm 15.8 and 17.1, the library 14.8 and 15.3)
+    if (form == SUMS && M > FEW_ROWS && (N < 1024 || (M > 2 * FEW_ROWS && K < 2048))) return NONE;
     const double slabs = K / SLAB, weights = (form == GATED ? 2.0 : 1.0) * N, megabytes = weights * K * 2e-6, gigaflops = 2e-9 * M * weights * K;
     double best = 1e30;
     int plan = NONE;
@@ -229,10 +231,10 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
             // (two of the small tiles' workgroups fit a compute unit: where the weights' way bounds them, 33 rows of 32,768 x 4,096 63 us for the library, 55; gated products
             // beyond one round, and with less than 1,024 of K, stay with the kernel that shares the activations, or the library)
             if (tiles * parts > (tile == SMALL && parts == 1 && form != GATED ? 2 : 1) * UNITS || slabs < 4 * parts || (form == GATED && slabs < 16)) continue;
-            // (rows behind the last one repeat it and cost no way of their own: 257 and 384 rows of 2,048 x 2,048 on tiles of 128 x 64 13.9 and 16.7 us, 513 and 512 14.2 and 16.8,
-            // where tiles of 64 x 64 take 12.0 for 512, one a compute unit)
+            // (rows behind the last one repeat it and cost no way of their own; it is the last eighth that costs: tiles of 128 x 64, us for 2,048 x 2,048 at 257, 320, 448 and 384 rows,
+            // 0.67, 0.83, 0.88 and all of them full, 13.9, 14.4, 14.7 and 16.7; 513 and 512 rows 14.2 and 16.8, where tiles of 64 x 64 take 12.0 for 512, one a compute unit)
             const double filled = (double)M / ((M + shape.rows - 1) / shape.rows * shape.rows), rate = tile == LARGE ? 4.1 : 5.2;
-            double us = shape.start + (shape.slab + shape.full * filled) * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.8 : 1.0);
+            double us = shape.start + (shape.slab + shape.full * filled * filled * filled * filled) * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.8 : 1.0);
             // (the weights come as fast as many workgroups pull: with 160 of them 33 rows of 5,120 x 25,600 took 71 us, with 320 67)
             const double load = tiles * parts < UNITS ? (double)(tiles * parts) / UNITS : 1.0, way = megabytes / (rate * (0.5 + 0.5 * load)) + 3.0;
             us = us > way ? us : way;

@@ -82,5 +82,5 @@ def test_tiles_whose_rows_are_full_are_priced_so(plan):
         assert plan(form, rows, columns, inner) < (32 if form == SUMS else 1), (form, rows, columns, inner)
     for rows in (1792, 1900, 2001, 2047, 2048):                  # one round of tiles of 128 x 128, whatever the last one holds
         assert plan(PLAIN, rows, 2048, 2048) == 16 + 3, rows
-    for form, rows, columns, inner in ((PLAIN, 820, 2048, 2048), (PLAIN, 448, 4096, 2048), (ACTIVATED, 257, 8448, 2048)):
+    for form, rows, columns, inner in ((PLAIN, 820, 2048, 2048), (PLAIN, 320, 4096, 2048), (PLAIN, 333, 4096, 2048), (PLAIN, 448, 4096, 2048), (ACTIVATED, 257, 8448, 2048)):
         assert plan(form, rows, columns, inner), (form, rows, columns, inner)
