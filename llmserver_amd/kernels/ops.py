@@ -269,7 +269,8 @@ class HipOps(KernelNamespace):
         """Whether, for these sizes, the library's product (with a norm kernel before it if ``scaled``, and the
         activation kernel after it if ``kind`` is "gated") beats the kernel of this repository that does it all;
         ``kind`` "partial": the product in partial sums and the norm kernel that adds them up, against the library's
-        product and the plain norm kernel.  Looked up in the table of choices; measured only inside ``measuring()``."""
+        product, whole or in ranges, and the norm kernel.  Looked up in the table of choices, before any rule by sizes is; measured only inside
+        ``measuring()``, this repository's side in whatever form would run."""
         if not self.consult_choices or x.dtype == torch.float32:      # (the table speaks of bfloat16)
             return False
         rows, width = x.shape
@@ -281,6 +282,7 @@ class HipOps(KernelNamespace):
             return known
         if not self._measuring or torch.cuda.is_current_stream_capturing():
             return False                                  # unknown shape: this repository's kernel
+        ranges = self.library_parts(x, weight) if kind == "partial" else 0
         sums = torch.ones((rows, 16), device=x.device, dtype=torch.float32) if scaled else None
         row_scale = (sums, 1e-6) if scaled else None
         stream = torch.zeros_like(x) if scaled else None
@@ -294,13 +296,13 @@ class HipOps(KernelNamespace):
                 normed = torch.empty_like(stream)
 
                 def few():
-                    sums = self.linear_partial_sums(x, weight, few_rows_too=True)
+                    sums = self.linear_partial_sums(x, weight)
                     if sums is not None:
                         self.add_rmsnorm(stream, sums, norm_weight, 1e-6, normed)
                     return sums
 
                 def library():
-                    self.add_rmsnorm(stream, torch.mm(x, weight.t()), norm_weight, 1e-6, normed)
+                    self.add_rmsnorm(stream, self._in_parts(x, weight, ranges) if ranges else torch.mm(x, weight.t()), norm_weight, 1e-6, normed)
             elif kind == "gated":
                 hidden = torch.empty((rows, weight.shape[0] // 2), device=x.device, dtype=x.dtype)
 
@@ -603,23 +605,25 @@ class HipOps(KernelNamespace):
         over ranges of the inner dimension (their sum is the product), or None if this is no case for it.  Whoever
         adds the result to the residual stream adds the parts up (:meth:`add_rmsnorm` takes them).  Beyond 128 rows
         this package's tiles multiply where they leave several parts (190 rows, 2,048 x 6,144: 12 us against 19 for the library's product in
-        ranges), else the library, in ranges where the table of choices says that this is faster (see :meth:`library_parts`)."""
+        ranges), else the library, in ranges where the table of choices says that this is faster (see :meth:`library_parts`).  A size
+        that the table gives to the library (:meth:`library_is_faster`) goes there at any number of rows."""
         rows, width = x.shape
         if rows > self.SPLIT_ROWS and x.shape[1] == weight.shape[1]:
-            sums = self._tiled_product("sums", x, weight) if self.split_products else None
-            if sums is not None:
-                return sums
+            if self.split_products and not self.library_is_faster("partial", x, weight):
+                sums = self._tiled_product("sums", x, weight)
+                if sums is not None:
+                    return sums
             parts = self.library_parts(x, weight)      # beyond this repository's products: the library's, whole or in ranges
             return self._in_parts(x, weight, parts) if parts else None
         if not ((0 if few_rows_too else self.skinny_rows) < rows <= self.SPLIT_ROWS) or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 \
                 or x.shape[1] != weight.shape[1] or not self.split_products:
             return None
         if not few_rows_too:
+            if self.library_is_faster("partial", x, weight):
+                return None
             sums = self._tiled_product("sums", x, weight)
             if sums is not None:
                 return sums
-            if self.library_is_faster("partial", x, weight):
-                return None
         size = (rows, weight.shape[0], width)
         parts = self._split_parts.get(size)
         if parts is None:
@@ -684,7 +688,9 @@ class HipOps(KernelNamespace):
         rows, width = x.shape
         inter = gate_up_weight.shape[0] // 2
         if activation not in self.FUSED_ACTIVATIONS:
-            return None if row_scale is not None or pairs_per_workgroup or activation not in self.ACTIVATIONS else self._tiled_product("gated", x, gate_up_weight, activation)
+            if rows <= self.skinny_rows or row_scale is not None or pairs_per_workgroup or activation not in self.ACTIVATIONS or self.library_is_faster("gated", x, gate_up_weight):
+                return None
+            return self._tiled_product("gated", x, gate_up_weight, activation)
         if x.dtype == torch.float32:
             if pairs_per_workgroup or gate_up_weight.shape[1] != width or gate_up_weight.shape[0] % 2 or not self._fuses_float32(x, gate_up_weight, row_scale):
                 return None
@@ -694,7 +700,7 @@ class HipOps(KernelNamespace):
                       "gemm_few_f32_gated")
             return out
         if rows > self.skinny_rows:
-            if row_scale is not None or pairs_per_workgroup:
+            if row_scale is not None or pairs_per_workgroup or self.library_is_faster("gated", x, gate_up_weight):
                 return None
             sums_first = self._sums_first(x, gate_up_weight, gated=True)
             done = None if sums_first else self._tiled_product("gated", x, gate_up_weight, activation)
@@ -757,7 +763,7 @@ class HipOps(KernelNamespace):
         fits = self._split_parts.get(size)
         if fits is None:
             fits = self._split_parts[size] = self._gemm.lsa_gemm_split_gated_fits(rows, inter, width)
-        if not fits or self.library_is_faster("gated", x, gate_up_weight):
+        if not fits:
             return None
         _check(x, "x", torch.bfloat16)
         _check(gate_up_weight, "gate_up_weight", torch.bfloat16)

@@ -185,3 +185,35 @@ def test_activated_products_of_few_rows_are_asked_for_by_the_weights_size(ops, r
     asked.clear()
     x, weight = drawn(333, 12288, 2048, rows)
     assert ops.linear_gated(x, weight) is None and asked == [("gated", False)]
+
+
+@pytest.mark.parametrize("rows", [40, 190])
+def test_the_table_of_choices_goes_before_the_plan(ops, rows, monkeypatch):
+    """A size that the table gives to the library goes there whatever the plan says of it, an unknown one as the plan says; and what is timed when somebody measures is the way that runs."""
+    from llmserver_amd.kernels.choices import ChoiceTable, choice_key
+    print(f"table before plan {rows}", flush=True)
+    bucket = -(-rows // 8) * 8
+    gated, wide = drawn(rows, 12288, 2048, rows)
+    down_x, down = drawn(rows, 2048, 6144, rows)
+    stream = ops._tiled_product("sums", down_x, down)
+    assert ops._tiled_product("gated", gated, wide) is not None and stream is not None
+    gated_key, partial_key = choice_key("gated", bucket, 12288, 2048, False, False), choice_key("partial", bucket, 2048, 6144, False, False)
+    monkeypatch.setattr(ops, "choices", ChoiceTable(ops.choices.device_name))
+    monkeypatch.setattr(ops, "consult_choices", True)
+    for library in (False, None, True):
+        ops.choices.entries.update({gated_key: library, partial_key: library}) if library is not None else ops.choices.entries.clear()
+        for activation in ops.ACTIVATIONS:
+            assert (ops.linear_gated(gated, wide, activation=activation) is None) == bool(library)
+        sums = ops.linear_partial_sums(down_x, down)
+        assert sums is None if library else torch.equal(sums, stream)
+    if rows > ops.SPLIT_ROWS:                                     # ... and in ranges there, if the table says so
+        ops.choices.entries.update({choice_key(f"parts{parts}", ops._parts_bucket(rows), 2048, 6144, False, False): parts == 4 for parts in (2, 4)})
+        assert ops.linear_partial_sums(down_x, down).shape[0] == 4
+    ops.choices.entries.clear()
+    taken, real = [], ops._tiled_product
+    monkeypatch.setattr(ops, "_tiled_product", lambda *a, **k: (lambda done: (taken.append(a[0]) if done is not None else None, done)[1])(real(*a, **k)))
+    timed = []
+    monkeypatch.setattr(ops, "_second_is_faster", lambda first, second: (taken.clear(), first(), timed.append(list(taken)), second(), True)[-1])
+    with ops.measuring():
+        assert ops.linear_gated(gated, wide) is None and ops.linear_partial_sums(down_x, down) is None or rows > ops.SPLIT_ROWS
+    assert timed == [["gated"], ["sums"]] and ops.choices.entries[gated_key] and ops.choices.entries[partial_key]
