@@ -45,8 +45,9 @@ def test_every_tile_at_its_edges(ops, form, tile, rows, columns, inner):
         for parts in (1, 2, 4, 8) if form == "sums" else (1,):
             if parts > inner // 64:
                 continue
-            out = torch.full((parts, rows, columns), float("nan"), device="cuda", dtype=torch.float32 if form == "sums" else torch.bfloat16)
-            beyond = torch.full((1024,), 7.0, device="cuda")                     # (allocated behind it: nothing writes there)
+            margin = 256 * columns                                               # a tile's rows on both sides, in one tensor with the result: nothing writes there
+            whole = torch.full((2 * margin + parts * rows * columns,), 7.0, device="cuda", dtype=torch.float32 if form == "sums" else torch.bfloat16)
+            out = whole[margin:-margin].view(parts, rows, columns).fill_(float("nan"))
             assert lib.lsa_product(16 * parts + tile, FORMS.index(form), activation, x.data_ptr(), weight.data_ptr(), out.data_ptr(), rows, columns, inner,
                                    torch.cuda.current_stream().cuda_stream) == 0
             got = out.double().sum(0)
@@ -62,7 +63,7 @@ def test_every_tile_at_its_edges(ops, form, tile, rows, columns, inner):
                 want, bound = exact, off + (2.0 ** -8 * exact.abs() if form == "plain" else 0.0)
             bound = bound * 1.01 + 2.0 ** -18 * want.abs().max()                 # (expf and tanhf: a few parts in 2^23)
             assert torch.isfinite(got).all() and bool(((got - want).abs() <= bound).all()), float(((got - want).abs() - bound).max())
-            assert bool((beyond == 7.0).all())
+            assert bool((whole[:margin] == 7.0).all()) and bool((whole[-margin:] == 7.0).all())
 
 
 def test_what_does_not_fit_is_refused(ops):
@@ -112,10 +113,9 @@ def test_products_of_a_portion_go_to_the_tiles(ops, rows, monkeypatch):
         y = ops.linear(followed, weight)
     assert y.requires_grad and close(y.detach()) and not tiled()
     hidden = ops.linear_gated(x, weight)
-    assert (hidden is None) == (not tiled())
-    if hidden is not None:
-        gate, up = want.split(2048, 1)
-        assert float((hidden.double() - silu(gate) * up).norm() / (silu(gate) * up).norm()) < 2.0 ** -8
+    assert hidden is not None and tiled()
+    gate, up = want.split(2048, 1)
+    assert float((hidden.double() - silu(gate) * up).norm() / (silu(gate) * up).norm()) < 2.0 ** -8
 
 
 def test_partial_sums_join_the_stream_as_the_product_would(ops):
@@ -162,8 +162,7 @@ def test_a_captured_step_replays_the_tiles(ops):
         x.copy_(drawn(190, 8, 2048, seed)[0])
         graph.replay()
         torch.cuda.synchronize()
-        again = ops.linear_gated(x, weight)
-        assert torch.equal(y, ops.linear(x, weight)) and (hidden is None or torch.equal(hidden, again))
+        assert torch.equal(y, ops.linear(x, weight)) and torch.equal(hidden, ops.linear_gated(x, weight))
 
 
 @pytest.mark.parametrize("rows", [17, 28, 29])
