@@ -1,8 +1,8 @@
 """The tiles of 256 x 256 whose wavefronts take turns (``csrc/wide_product.hpp``) at the edges of what they leave out: blocks of 64 rows that are padding, columns from
 128 on that the matrix does not have, slabs of 64 and a half one, from a single half slab on.
 
-The narrow tiles add a sum's products in the same order, so the two agree bit by bit; both lie within 2^-9 of the products in 64 bits (a hidden row is rounded to
-bfloat16 once, 2^-9 of its numbers, and no other rounding comes near that)."""
+The narrow tiles add a sum's products in the same order, so the two agree bit by bit.  Against the products in 64 bits, whose hidden rows are rounded to bfloat16 as well: where sums in 32
+and in 64 bits lie on two sides of a rounding's edge a hidden number is off by up to 2^-8 of it; few are, and the limit for the norm, 2^-9, is what was observed with room, not a bound."""
 import pytest
 import torch
 
