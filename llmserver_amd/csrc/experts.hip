@@ -981,7 +981,8 @@ __global__ __launch_bounds__(STREAM_THREADS) void experts_stream_kernel(const bf
 //   What bounds it is what passes between the XCDs' L2 and the memory side: a workgroup's share of an expert's matrix is read once for each 256 of its pairs and
 // half of that comes from the neighbour's read.  12,288 pairs of 64 gated experts of 1,408 at width 2,048, chosen unevenly, us a launch, first and second product, with sixteen
 // wavefronts of 64 x 64 in step and now: 251 + 143, 224 + 138 (191 of them the matrices' loads alone); 32,760 pairs of 2,112 without gates, all launches 808, 710; with the same
-// number of pairs everywhere and experts of 2,048 230 for the first product (1.19 PFLOP/s).  No faster: one workgroup a compute unit that goes from tile to tile with its loads running on;
+// number of pairs everywhere and experts of 2,048 230 for the first product (1.19 PFLOP/s).  (Of few slabs it is the slower one, by its start: 16 experts of 352 at 512, 4,096 tokens, all
+// launches 65.9, 68.1.)  No faster: one workgroup a compute unit that goes from tile to tile with its loads running on;
 // shares of the XCDs by work; slabs in another order for each block of columns; the experts' pairs shared evenly by its tiles; three slabs of the matrix in LDS.
 template <int FORM, typename O>
 __global__ __launch_bounds__(WIDE_THREADS) void experts_wide_kernel(const bf16_t* __restrict__ a, int a_stride, int pair_div,
@@ -1093,15 +1094,16 @@ static bool wide_fits(int pairs, int inter, int width, bool aligned) {
     return aligned && (size_t)pairs * (size_t)(inter > width ? inter : width) * 2 < BUFFER_BYTES && (size_t)2 * inter * width * 2 < BUFFER_BYTES;
 }
 
-// Pairs a tile that lsa_experts_tiled should take for a step with so many pairs: 256 (the wide kernel) or 64.  Wide tiles pay from some 40 pairs
-// an expert on, and where the two products make 224 workgroups or more together, not quite one a compute unit for each: with fewer,
-// tiles of 64 pairs spread the same work over units that would stand idle.  All launches of a step, us, narrow and wide: 64 experts of 1,408 at
-// width 2,048, 40 pairs an expert 270, 259; 64: 316, 278; 128: 404, 327; 192: 502, 383; 16 experts of 2,048 at 4,096 (512 workgroups), 128 pairs
-// 354, 246; 8 of them (256) 183, 159; 16 of 768 at 2,048 (224) 90, 76; 4 of 2,048 at 4,096 (128) 111, 129, with 192 pairs 115, 158; 8 of 1,408
-// at 2,048 (152) with 192 pairs 92, 99; 4 (76) 71, 97; 1 of 512 at 1,024 (8) with 256 pairs 40, 55.  Without gates, 16 of 1,024 at 4,096 (320),
-// 96 pairs 133, 128; 8 of 1,408 at 2,048 (112) with 192 pairs 75, 95.
+// Pairs a tile that lsa_experts_tiled should take for a step with so many pairs: 256 (the wide kernel) or 64.  The line: some 40 pairs an
+// expert, and the two products make 224 workgroups or more together, not quite one a compute unit for each: with fewer, tiles of 64 pairs spread the same work over units that
+// would stand idle.  All launches of a step, us, narrow and wide, pairs chosen unevenly: 64 experts of 1,408 at width 2,048, 40 pairs an expert 254, 247; 64: 277, 280; 96: 323, 307;
+// 128: 377, 343; 192: 477, 400; 128 of 768 at 2,048, 40 pairs 274, 267; 32 of 2,048 at 4,096 (1,024 workgroups) 356, 336; 16 of them (512) 196, 203, 128 pairs 285, 298, 192: 361, 320;
+// 8 (256), 128 pairs 157, 154; 4 (128) 79, 131, with 192 pairs 93, 138; 8 of 1,408 at 2,048 (152) with 192 pairs 75, 97; 4 (76) 47, 90; 1 of 512 at 1,024 (8) with 256 pairs 26,
+// 58.  (Behind the line there are steps that the narrow tiles, since their matrices go through LDS without registers, would make faster: 16 of 768 at 2,048 (224) with 128 pairs
+// 64, 87; without gates, 16 of 1,024 at 4,096 (320) with 128 pairs 125, 155.)
+//   Inner dimensions below 512 are so few slabs that a wide launch is mostly its start: 64 of 256 at 1,024, 40 pairs 43, 59; 128: 67, 76; 200: 87, 89; 256: 101, 95.
 LSA_EXPORT int lsa_experts_tile_rows(int pairs, int experts, int inter, int width, int plain, int aligned) {
-    if (pairs < 40 * experts || !wide_fits(pairs, inter, width, aligned != 0)) return TILE_M;
+    if (pairs < (inter < 512 || width < 512 ? 200 : 40) * experts || !wide_fits(pairs, inter, width, aligned != 0)) return TILE_M;
     const long tiles = (long)experts * ((pairs / experts + WIDE_M - 1) / WIDE_M), columns = plain ? WIDE_TILE : WIDE_TILE / 2;
     return tiles * ((inter + columns - 1) / columns) + tiles * ((width + WIDE_TILE - 1) / WIDE_TILE) >= 224 ? WIDE_M : TILE_M;
 }

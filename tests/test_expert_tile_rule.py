@@ -37,6 +37,13 @@ def test_wide_tiles_where_they_were_measured_to_be_faster(tile_rows):
     assert tile_rows(16 * 100, 16, 1024, 2048) == 256 and tile_rows(16 * 100, 16, 1024, 2048, plain=True) == 64
 
 
+def test_short_inner_dimensions_want_more_pairs_for_wide_tiles(tile_rows):
+    """A wide launch of a few slabs is mostly its start."""
+    for each in (40, 64, 100, 128, 199):
+        assert tile_rows(64 * each, 64, 256, 1024) == 64 and tile_rows(64 * each, 64, 1024, 256) == 64, each
+    assert tile_rows(64 * 200, 64, 256, 1024) == 256 and tile_rows(64 * 40, 64, 512, 1024) == 256
+
+
 def test_sorted_products_where_they_were_measured_to_be_faster():
     """(Tensors without storage: what is not refused by its sizes is refused for where it lives.)"""
     def taken(pairs, experts, width, inter, plain=False):
