@@ -46,8 +46,9 @@ template <int N> struct WideLeft { static constexpr int value = N; };
 // k: a multiple of 32.  row_blocks: how many of the four blocks of 64 rows of A are wanted (1 to 4), second_half: whether columns from 128 on are;
 // sums of others are left undefined.  `buffers`: 2 * WIDE_BUFFER bytes at a multiple of 1,024.  All 512 threads come here; nothing is under way afterwards.
 //
-//   What bounds it is power: 4,096 cubed runs 2,190 cycles a slab, of which the matrix cores are busy 2,048, at 1.73 GHz (2.4 with half the compute
-// units).  So what counts beside full matrix cores is what else takes energy: products of 16 x 16 x 32 and not of 32 x 32 x 16 (1.49 against 1.33 PFLOP/s: the
+//   What bounds it is power: by counters a tile takes 2,290 cycles a slab, of which the matrix cores are busy 2,048, and 32,000 around its slabs, with half the compute units
+// as with all of them; but the clock is 2.5 GHz with half, 2.0 with all and falls on in launches one behind the other (256 tiles of 128 slabs: 185 and 206 us, 128 tiles 140).  So
+// what counts beside full matrix cores is what else takes energy: products of 16 x 16 x 32 and not of 32 x 32 x 16 (1.49 against 1.33 PFLOP/s: the
 // clock falls to 1.52 GHz), and products of padding are left out.
 //   A slab is four regions, the halves of A and of B (128 rows of 128 bytes, 16 KB), and four phases, of which each multiplies one half of A with
 // one half of B, reads one region's operands from LDS for the phases behind it, and asks for one region of the slab after the next:
