@@ -208,9 +208,10 @@ static bool fits(int form, long M, long N, long K) {
 // it, or up to 128 rows the few-row kernels.  Both times are lines through what was measured at 50 numbers of rows from 17 to 4,096 of 48 products of this package's
 // models: a launch's start and a slab's time for the tiles here, for the library (whose own choice of tiles nobody can foretell: with its tiles' rounds in the line its
 // times are met no better, within an eighth) a start, K and the operations.  So where the library has just begun a round its price is too low, and sizes that the tiles would
-// make faster stay with it.  At 48 other numbers of rows, 18 to 4,000, of 52 products 709 of 2,433 are taken, up to 128 rows and beyond: gated 1.18 and 1.22 times as fast as the other
-// way, plain 1.19 and 1.22, activated 1.19 and 1.23, sums with the norm behind them 1.12 and 1.15, heads 1.11 and none.  The worst: 0.94 (240 rows, sums of 2,560 x 9,728 33.4, 35.4), 0.96
-// (sums of 2,048 x 1,408 at 400 rows; gated 3,072 x 1,024 at 1,600); all others 0.97 and more.  A product whose tiles do not go round the compute units in one round stays the
+// make faster stay with it.  At 64 other numbers of rows, 19 to 3,900, of 52 products 1,037 of 3,233 sizes are taken, up to 128 rows and beyond: gated 1.19 and 1.22 times as fast as the
+// other way, plain 1.19 and 1.18, activated 1.21 and 1.24, sums with the norm behind them 1.13 and 1.14, heads 1.11 and none.  The worst: 0.94 (380 rows of 4,096 x 2,048 15.9, 17.0; 250 rows, sums
+// of 2,560 x 9,728 33.6, 35.6), 0.95 (230 rows of 5,376 x 2,048), 0.96 (750 rows of 2,048 x 2,048; gated 3,072 x 1,024 at 1,550; activated 2,112 x 2,048 at 30); all others 0.96 and
+// more, all but three 0.97.  A product whose tiles do not go round the compute units in one round stays the
 // library's unless it is gated and large.  Up to 128 rows the parts may be added up by a launch of their own (64 rows, 2,816 x 2,048 library 12.1, one launch 12.2, so 9.7; 32
 // rows of 4,096 x 4,096 13.9, 17.9, 12.0; gated 2,816 x 4,096 15.4, 18.4, 12.2).
 LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {

@@ -681,10 +681,11 @@ class HipOps(KernelNamespace):
     FUSED_ACTIVATIONS = ("silu",)             # ... and what the gated products' epilogues compute
 
     def linear_gated(self, x, gate_up_weight, pairs_per_workgroup=0, row_scale=None, activation="silu"):
-        """``silu(x @ gate^T) * (x @ up^T)`` with ``gate_up_weight [2I, K]`` in one launch for few rows (the
-        activation sits in the product's epilogue), or None if this is not such a case (another activation is none).  ``pairs_per_workgroup``:
+        """``act(x @ gate^T) * (x @ up^T)`` with ``gate_up_weight [2I, K]``, the activation in the product's epilogue or in the kernel that adds its parts up, or None
+        where the library's product and the activation's kernel are to be used.  Up to 16 rows (float32: 8) in one launch, with SiLU only; beyond, the tiles of
+        :meth:`_tiled_product` with either of ``ACTIVATIONS`` and, for SiLU and up to 64 rows, the kernels that share the rows in LDS.  ``pairs_per_workgroup``:
         1 to 16 pairs of a gate and an up row in two tiles, -1 for 8 pairs in one tile, 0 lets the size decide.
-        ``row_scale`` as in :meth:`linear_few_rows`."""
+        ``row_scale`` as in :meth:`linear_few_rows` (up to 16 rows)."""
         rows, width = x.shape
         inter = gate_up_weight.shape[0] // 2
         if activation not in self.FUSED_ACTIVATIONS:
