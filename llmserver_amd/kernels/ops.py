@@ -689,7 +689,7 @@ class HipOps(KernelNamespace):
         rows, width = x.shape
         inter = gate_up_weight.shape[0] // 2
         if activation not in self.FUSED_ACTIVATIONS:
-            if rows <= self.skinny_rows or row_scale is not None or pairs_per_workgroup or activation not in self.ACTIVATIONS or self.library_is_faster("gated", x, gate_up_weight):
+            if activation not in self.ACTIVATIONS or row_scale is not None or pairs_per_workgroup or rows <= self.skinny_rows or self.library_is_faster("gated", x, gate_up_weight):
                 return None
             return self._tiled_product("gated", x, gate_up_weight, activation)
         if x.dtype == torch.float32:
