@@ -268,6 +268,9 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     // 4,096 x 8,192 21.5, 23.3; 128 rows of 4,096 x 12,288 41.4, 35.6.
     if (form == SUMS && M <= FEW_ROWS)
         return weights * K <= 2.6e7 || best + 4.0 < 0.85 * (7.1 + megabytes / 4.9 + 0.05 * M + 0.00066 * M * megabytes) ? plan : NONE;
+    // (a weight of more than 50 MB in parts: the library cuts K up to 32 rows and not beyond: 18, 28, 34 and 44 rows of 4,096 x 8,192 17.6, 18.6, 22.9 and 23.0, here 19.9, 20.1, 20.2
+    // and 20.6; 2,048 x 8,448, at 18 rows 27.2, here 11.5, and 4,096 x 4,096, 13.3 and 11.1, lie before that)
+    if (form == PLAIN && (plan & ADDED) && M <= 32 && weights * K > 2.6e7) return NONE;
     return best < (M > FEW_ROWS ? 0.95 : 0.88) * library ? plan : NONE;
 }
 

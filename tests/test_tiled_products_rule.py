@@ -84,3 +84,10 @@ def test_tiles_whose_rows_are_full_are_priced_so(plan):
         assert plan(PLAIN, rows, 2048, 2048) == 16 + 3, rows
     for form, rows, columns, inner in ((PLAIN, 820, 2048, 2048), (PLAIN, 320, 4096, 2048), (PLAIN, 333, 4096, 2048), (PLAIN, 448, 4096, 2048), (ACTIVATED, 257, 8448, 2048)):
         assert plan(form, rows, columns, inner), (form, rows, columns, inner)
+
+
+def test_a_large_weight_in_parts_stays_with_the_library_up_to_32_rows(plan):
+    """The library cuts the inner dimension there itself; from 33 rows on it does not, and weights of up to 50 MB are faster in parts before that too."""
+    assert not any(plan(PLAIN, rows, 4096, 8192) for rows in range(17, 33))
+    assert all(plan(PLAIN, rows, 4096, 8192) for rows in (33, 44, 64, 100))
+    assert all(plan(PLAIN, rows, columns, inner) for rows in (17, 28, 32) for columns, inner in ((2048, 8448), (4096, 4096)))
