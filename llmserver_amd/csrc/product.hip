@@ -194,8 +194,11 @@ __global__ __launch_bounds__(WIDE_THREADS) void wide_gated_kernel(const bf16_t* 
 // What lsa_product can be asked for: a tile, and for SUMS the parts of K, as 16 parts + tile.  ADDED in a plan for PLAIN or GATED: the sums, and a kernel behind
 // them that adds the parts up (lsa_sum_parts, lsa_gated_parts).
 enum Tile { NONE, SMALL, TALL, LARGE, WIDE };
-struct TileShape { int rows, columns; double start, slab, full; };     // columns of W; us of a launch with a tile a compute unit, of a slab, and what full rows add to that
-static const TileShape SHAPES[] = {{0, 0, 0, 0, 0}, {64, 64, 3.4, 0.25, 0.06}, {128, 64, 3.8, 0.31, 0.11}, {128, 128, 4.6, 0.46, 0.10}, {256, 256, 0, 0, 0}};
+struct TileShape { int rows, columns; double start, slab, alone, among, last, rate; };
+// Columns of W; us of a launch, of a slab, and what a slab takes more for each compute unit in use (its share of all) where one workgroup alone reads its lines of W and where many read
+// them, and for a last block of rows that is full (times its share squared); TB/s of W's way.  Fitted to 1,000 to 2,000 sizes each, within 4 to 6 %.
+static const TileShape SHAPES[] = {{0, 0, 0, 0, 0, 0, 0, 0}, {64, 64, 3.94, 0.2, 0.12, 0.02, 0.04, 4.7}, {128, 64, 4.22, 0.25, 0.13, 0.06, 0.105, 4.7},
+                                   {128, 128, 4.41, 0.375, 0.28, 0.08, 0.06, 4.5}, {256, 256, 0, 0, 0, 0, 0, 0}};
 constexpr int UNITS = 256;                                         // compute units
 constexpr int MOST_PARTS = 8, ADDED = 1 << 12;
 
@@ -205,13 +208,14 @@ static bool fits(int form, long M, long N, long K) {
 }
 
 // The tile (and parts) for a product of these sizes, or 0 where the other way is expected to be as fast: the library's product, with the kernel of the activation behind
-// it, or up to 128 rows the few-row kernels.  Both times are lines through what was measured at 50 numbers of rows from 17 to 4,096 of 48 products of this package's
-// models: a launch's start and a slab's time for the tiles here, for the library (whose own choice of tiles nobody can foretell: with its tiles' rounds in the line its
-// times are met no better, within an eighth) a start, K and the operations.  So where the library has just begun a round its price is too low, and sizes that the tiles would
-// make faster stay with it.  At 64 other numbers of rows, 19 to 3,900, of 52 products 1,037 of 3,233 sizes are taken, up to 128 rows and beyond: gated 1.19 and 1.22 times as fast as the
-// other way, plain 1.19 and 1.18, activated 1.21 and 1.24, sums with the norm behind them 1.13 and 1.14, heads 1.11 and none.  The worst: 0.94 (380 rows of 4,096 x 2,048 15.9, 17.0; 250 rows, sums
-// of 2,560 x 9,728 33.6, 35.6), 0.95 (230 rows of 5,376 x 2,048), 0.96 (750 rows of 2,048 x 2,048; gated 3,072 x 1,024 at 1,550; activated 2,112 x 2,048 at 30); all others 0.96 and
-// more, all but three 0.97.  A product whose tiles do not go round the compute units in one round stays the
+// it, or up to 128 rows the few-row kernels.  Both times are lines through what was measured, every tile beside the other way, at 70 numbers of rows from 17 to 4,096 of 73 products of this
+// package's models: for the tiles a launch's start and a slab's time, for the library (whose own choice of tiles nobody can foretell: with its tiles' rounds in the line its
+// times are met no better, within an eighth) a start, K and the operations.  So where the library has just begun a round, or has one of its slow sizes (many whole multiples of 64 rows: 256
+// rows of 6,144 x 2,048 24.8, 17.4 here), its price is too low, and sizes that the tiles would make faster stay with it.  At 70 other numbers of rows 1,949 of 4,094 sizes are taken, up to
+// 128 rows and beyond: gated 1.16 and 1.20 times as fast as the other way, plain 1.24 and 1.20, activated 1.25 and 1.23, sums with the norm behind them 1.13 and 1.16, heads 1.08 and none.
+// Eighteen of them are slower than 0.97 of it: 95 rows of 2,560 x 4,096 0.93, 63 of 4,096 x 3,072 0.94, 320 to 448 of 64 x 2,048 0.95, 30 of 2,112 x 2,048 activated 0.97; sums at 531
+// and 545 rows of 2,048 x 2,048 0.93 and 0.95, 232 of 2,560 x 9,728 0.94, 127 of 5,120 x 17,408 0.96, 35 of 4,096 x 8,192 and 255 of 4,096 x 12,288 0.97.  A product whose tiles
+// do not go round the compute units in one round stays the
 // library's unless it is gated and large.  Up to 128 rows the parts may be added up by a launch of their own (64 rows, 2,816 x 2,048 library 12.1, one launch 12.2, so 9.7; 32
 // rows of 4,096 x 4,096 13.9, 17.9, 12.0; gated 2,816 x 4,096 15.4, 18.4, 12.2).
 LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
@@ -232,24 +236,27 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
             // (two of the small tiles' workgroups fit a compute unit: where the weights' way bounds them, 33 rows of 32,768 x 4,096 63 us for the library, 55; gated products
             // beyond one round, and with less than 1,024 of K, stay with the kernel that shares the activations, or the library)
             if (tiles * parts > (tile == SMALL && parts == 1 && form != GATED ? 2 : 1) * UNITS || slabs < 4 * parts || (form == GATED && slabs < 16)) continue;
-            // (rows behind the last one repeat it and cost no way of their own; it is the last eighth that costs: tiles of 128 x 64, us for 2,048 x 2,048 at 257, 320, 448 and 384 rows,
-            // 0.67, 0.83, 0.88 and all of them full, 13.9, 14.4, 14.7 and 16.7; 513 and 512 rows 14.2 and 16.8, where tiles of 64 x 64 take 12.0 for 512, one a compute unit)
-            const double filled = (double)M / ((M + shape.rows - 1) / shape.rows * shape.rows), rate = tile == LARGE ? 4.1 : 5.2;
-            double us = shape.start + (shape.slab + shape.full * filled * filled * filled * filled) * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.8 : 1.0);
+            // (rows behind the last one repeat it and cost no way of their own: tiles of 128 x 64, us for 2,048 x 2,048 at 257, 320 and 384 rows 13.9, 14.4 and 16.7; 513 and 512 rows 14.2
+            // and 16.8, where tiles of 64 x 64 take 12.0 for 512, one a compute unit)
+            const double load = tiles * parts < UNITS ? (double)(tiles * parts) / UNITS : 1.0, blocks = (M + shape.rows - 1) / shape.rows, last = (double)((M - 1) % shape.rows + 1) / shape.rows;
+            const double slab = shape.slab + load * (shape.among + (shape.alone - shape.among) / blocks) + shape.last * last * last;
+            double us = shape.start + slab * ((K / SLAB + parts - 1) / parts) * (tiles * parts > UNITS ? 1.9 : 1.0);
             // (the weights come as fast as many workgroups pull: with 160 of them 33 rows of 5,120 x 25,600 took 71 us, with 320 67)
-            const double load = tiles * parts < UNITS ? (double)(tiles * parts) / UNITS : 1.0, way = megabytes / (rate * (0.5 + 0.5 * load)) + 3.0;
+            const double way = megabytes / (shape.rate * (0.5 + 0.5 * load)) + 3.0;
             us = us > way ? us : way;
-            if (form == SUMS) us += parts * 8e-6 * M * N / 4.0;    // written and read
-            else if (parts > 1) us += 3.4 + parts * 8e-6 * M * weights / 3.0;      // and a launch
+            if (form == SUMS) us += parts * 1.7e-6 * M * N;        // written and read
+            else if (parts > 1) us += 2.2 + parts * 2.0e-6 * M * weights;      // and a launch
             if (us < best) {
                 best = us;
                 plan = 16 * parts + tile + (form != SUMS && parts > 1 ? ADDED : 0);
             }
         }
     }
-    double library = 10.0 + 0.0016 * K + (gigaflops < 40 ? 0.75 * gigaflops : 30 + 0.69 * (gigaflops - 40));
+    double library = 9.9 + 0.0016 * K + (gigaflops < 40 ? 0.77 * gigaflops : 30.8 + 0.69 * (gigaflops - 40));
+    // (it cuts K where few rows meet few columns: from 129 rows on, us at 156 and 191 rows of 2,048 x 4,096 16.1 and 16.4, in whole tiles here 17.7 and 19.8)
+    if (form != GATED && M > FEW_ROWS && K >= 4096 && (double)M * N < 4.5e5 && library > 3.7 + 0.0033 * K + 0.77 * gigaflops) library = 3.7 + 0.0033 * K + 0.77 * gigaflops;
     if (M <= 64 && N <= 2048 && form != GATED) library = 4.0 + 0.0022 * K;        // (it cuts K there)
-    library = library > megabytes / 4.3 ? library : megabytes / 4.3;
+    library = library > megabytes / 4.5 ? library : megabytes / 4.5;
     if (form == GATED) library += 3.5 + 6e-6 * M * N / 5.0;
     if (form == ACTIVATED) library += 3.5 + 4e-6 * M * N / 5.0;
     if (form == GATED && slabs >= 16) {
@@ -260,18 +267,20 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
         const double load = (double)last / UNITS, blocks = M > 192 ? 4 : (M + 63) / 64, pulled = tiles < UNITS ? load : 1.0;
         const double products = 7.0 + tiles / UNITS * (6.0 + 1.5 * slabs) + (last ? 6.0 + (1.0 + 0.5 * load) * (0.6 + 0.1 * blocks) * slabs : 0.0);
         const double way = megabytes / (5.4 * (0.5 + 0.5 * pulled)) + 3.0, us = products > way ? products : way;
-        if (us < best && us < 0.97 * library) return 16 + WIDE;
+        if (us < best && us < 0.99 * library) return 16 + WIDE;
     }
     // Up to 128 rows the other way for sums is the kernel that shares the rows in LDS (lsa_gemm_split): slower for weights of up to 50 MB throughout (33 rows, with the norm,
     // 2,048 x 6,144 13.7, 12.3; 4,096 x 4,096 15.3, 14.1; 100 rows 18.8, 15.2 and 21.3, 17.9); beyond that its time, again with the norm, is a line in the weights and the rows, and
     // where tiles leave compute units idle it is the faster one: 48 rows of 5,120 x 25,600 62.8, 79.0, of 5,120 x 17,408 49.6, 52.5, 29 rows of 5,120 x 5,120 20.6, 24.5, of
     // 4,096 x 8,192 21.5, 23.3; 128 rows of 4,096 x 12,288 41.4, 35.6.
     if (form == SUMS && M <= FEW_ROWS)
-        return weights * K <= 2.6e7 || best + 4.0 < 0.85 * (7.1 + megabytes / 4.9 + 0.05 * M + 0.00066 * M * megabytes) ? plan : NONE;
+        return weights * K <= 2.6e7 || best + 4.0 < 0.93 * (7.1 + megabytes / 4.9 + 0.05 * M + 0.00066 * M * megabytes) ? plan : NONE;
     // (a weight of more than 50 MB in parts: the library cuts K up to 32 rows and not beyond: 18, 28, 34 and 44 rows of 4,096 x 8,192 17.6, 18.6, 22.9 and 23.0, here 19.9, 20.1, 20.2
     // and 20.6; 2,048 x 8,448, at 18 rows 27.2, here 11.5, and 4,096 x 4,096, 13.3 and 11.1, lie before that)
     if (form == PLAIN && (plan & ADDED) && M <= 32 && weights * K > 2.6e7) return NONE;
-    return best < (M > FEW_ROWS ? 0.95 : 0.88) * library ? plan : NONE;
+    // How far the lines are trusted: up to 128 rows the library takes longer than its line nearly everywhere, and a gated product's (with the activation) at any number of rows.
+    static const double MARGINS[4][2] = {{1.22, 0.95}, {1.16, 1.16}, {0.87, 0.92}, {0, 0.94}};
+    return best < (plan & ADDED ? 0.92 : MARGINS[form][M > FEW_ROWS]) * library ? plan : NONE;
 }
 
 template <int FORM>

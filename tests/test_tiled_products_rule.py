@@ -91,3 +91,10 @@ def test_a_large_weight_in_parts_stays_with_the_library_up_to_32_rows(plan):
     assert not any(plan(PLAIN, rows, 4096, 8192) for rows in range(17, 33))
     assert all(plan(PLAIN, rows, 4096, 8192) for rows in (33, 44, 64, 100))
     assert all(plan(PLAIN, rows, columns, inner) for rows in (17, 28, 32) for columns, inner in ((2048, 8448), (4096, 4096)))
+
+
+def test_tiles_are_priced_by_their_last_block_of_rows_and_by_who_else_reads_the_weight(plan):
+    """Sizes where the tiles were measured to be 1.15 times as fast as the other way and more, and which a price by how full all rows are together had refused."""
+    for form, rows, columns, inner in ((GATED, 100, 8448, 2048), (GATED, 128, 8448, 2048), (PLAIN, 38, 10304, 2048), (PLAIN, 45, 10304, 2048), (PLAIN, 128, 3328, 2048), (PLAIN, 126, 4240, 2048),
+                                       (PLAIN, 46, 2048, 4096), (PLAIN, 592, 2048, 2112)):
+        assert plan(form, rows, columns, inner), (form, rows, columns, inner)
