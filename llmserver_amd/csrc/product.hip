@@ -221,8 +221,9 @@ static bool fits(int form, long M, long N, long K) {
 LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     if (form < PLAIN || form > SUMS || !fits(form, M, N, K)) return NONE;
     // (sums beyond 128 rows were measured from 1,024 columns on: fewer go the library's way, whole or in ranges; and in parts of few slabs they are slower from 257 rows on: 384 and 512 rows
-    // of 2,048 x 1,408 with the norm 15.8 and 17.1, the library 14.8 and 15.3)
-    if (form == SUMS && M > FEW_ROWS && (N < 1024 || (M > 2 * FEW_ROWS && K < 2048))) return NONE;
+    // of 2,048 x 1,408 with the norm 15.8 and 17.1, the library 14.8 and 15.3; and beyond 1,100 rows: 1,121, 1,223 and 1,338 of 1,024 x 2,048 19.3, 19.6 and 21.2, the library 19.1, 19.6 and
+    // 19.2, 1,330 and 1,980 of 1,024 x 3,072 25.1 and 27.9, 24.0 and 28.3)
+    if (form == SUMS && M > FEW_ROWS && (N < 1024 || M > 1100 || (M > 2 * FEW_ROWS && K < 2048))) return NONE;
     const double slabs = K / SLAB, weights = (form == GATED ? 2.0 : 1.0) * N, megabytes = weights * K * 2e-6, gigaflops = 2e-9 * M * weights * K;
     double best = 1e30;
     int plan = NONE;

@@ -98,3 +98,7 @@ def test_tiles_are_priced_by_their_last_block_of_rows_and_by_who_else_reads_the_
     for form, rows, columns, inner in ((GATED, 100, 8448, 2048), (GATED, 128, 8448, 2048), (PLAIN, 38, 10304, 2048), (PLAIN, 45, 10304, 2048), (PLAIN, 128, 3328, 2048), (PLAIN, 126, 4240, 2048),
                                        (PLAIN, 46, 2048, 4096), (PLAIN, 592, 2048, 2112)):
         assert plan(form, rows, columns, inner), (form, rows, columns, inner)
+
+
+def test_sums_of_more_than_1100_rows_are_the_librarys(plan):
+    assert not any(plan(SUMS, rows, 1024, inner) for rows in (1101, 1121, 1338, 1980) for inner in (2048, 3072)) and plan(SUMS, 900, 1024, 3072) >= 32
