@@ -211,9 +211,9 @@ static bool fits(int form, long M, long N, long K) {
 // it, or up to 128 rows the few-row kernels.  Both times are lines through what was measured, every tile beside the other way, at 70 numbers of rows from 17 to 4,096 of 73 products of this
 // package's models: for the tiles a launch's start and a slab's time, for the library (whose own choice of tiles nobody can foretell: with its tiles' rounds in the line its
 // times are met no better, within an eighth) a start, K and the operations.  So where the library has just begun a round, or has one of its slow sizes (many whole multiples of 64 rows: 256
-// rows of 6,144 x 2,048 24.8, 17.4 here), its price is too low, and sizes that the tiles would make faster stay with it.  At 70 other numbers of rows 1,949 of 4,094 sizes are taken, up to
-// 128 rows and beyond: gated 1.16 and 1.20 times as fast as the other way, plain 1.24 and 1.20, activated 1.25 and 1.23, sums with the norm behind them 1.13 and 1.16, heads 1.08 and none.
-// Eighteen of them are slower than 0.97 of it: 95 rows of 2,560 x 4,096 0.93, 63 of 4,096 x 3,072 0.94, 320 to 448 of 64 x 2,048 0.95, 30 of 2,112 x 2,048 activated 0.97; sums at 531
+// rows of 6,144 x 2,048 24.8, 17.4 here), its price is too low, and sizes that the tiles would make faster stay with it.  At 70 other numbers of rows 1,923 of 4,094 sizes are taken, up to
+// 128 rows and beyond: gated 1.18 and 1.20 times as fast as the other way, plain 1.24 and 1.20, activated 1.25 and 1.23, sums with the norm behind them 1.13 and 1.16, heads 1.08 and none.
+// Seventeen of them are slower than 0.97 of it: 95 rows of 2,560 x 4,096 0.93, 63 of 4,096 x 3,072 0.94, 320 to 448 of 64 x 2,048 0.95, 30 of 2,112 x 2,048 activated 0.97; sums at 531
 // and 545 rows of 2,048 x 2,048 0.93 and 0.95, 232 of 2,560 x 9,728 0.94, 127 of 5,120 x 17,408 0.96, 35 of 4,096 x 8,192 and 255 of 4,096 x 12,288 0.97.  A product whose tiles
 // do not go round the compute units in one round stays the
 // library's unless it is gated and large.  Up to 128 rows the parts may be added up by a launch of their own (64 rows, 2,816 x 2,048 library 12.1, one launch 12.2, so 9.7; 32
@@ -280,7 +280,7 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     // and 20.6; 2,048 x 8,448, at 18 rows 27.2, here 11.5, and 4,096 x 4,096, 13.3 and 11.1, lie before that)
     if (form == PLAIN && (plan & ADDED) && M <= 32 && weights * K > 2.6e7) return NONE;
     // How far the lines are trusted: up to 128 rows the library takes longer than its line nearly everywhere, and a gated product's (with the activation) at any number of rows.
-    static const double MARGINS[4][2] = {{1.22, 0.95}, {1.16, 1.16}, {0.87, 0.92}, {0, 0.94}};
+    static const double MARGINS[4][2] = {{1.22, 0.95}, {1.1, 1.1}, {0.87, 0.92}, {0, 0.94}};
     return best < (plan & ADDED ? 0.92 : MARGINS[form][M > FEW_ROWS]) * library ? plan : NONE;
 }
 
