@@ -125,9 +125,12 @@ class HipOps(KernelNamespace):
     # key they load but start later, two halves shorten the longest workgroup's walk but make every step dearer).  A GPU
     # that is not listed plans with the attention part's neutral costs; other head sizes scale the trips and steps by
     # head size / 128 (loads and products of a step grow with the head; untuned beyond that).
-    TILE_COSTS = {"gfx950-256cu": (((False, 1), TileLaunchCost(3.2, 0.89, 1.55)), ((True, 1), TileLaunchCost(8.7, 0.94, 2.45)),
-                                   ((False, 2), TileLaunchCost(3.3, 1.11, 2.08)), ((True, 2), TileLaunchCost(8.8, 1.44, 2.84)))}
+    TILE_COSTS = {"gfx950-256cu": (((False, 1), TileLaunchCost(3.2, 0.89, 1.55)), ((True, 1), TileLaunchCost(7.5, 0.645, 1.93)),
+                                   ((False, 2), TileLaunchCost(3.3, 1.11, 2.08)), ((True, 2), TileLaunchCost(10.0, 0.92, 2.10)))}
     TILE_COSTS_HEAD_DIM = 128
+    # Eight tiles to a workgroup of heads beyond 128 dimensions: one workgroup fills a compute unit's registers, and a step of all of them costs accordingly
+    # (us, four and eight tiles: 16 heads on 4 of 256, 2,048 tokens 124 and 105; 32 of 192, windows of 1,024, 334 to 1,000 tokens 62 and 73).
+    WIDE_TILE_COSTS = {"gfx950-256cu": {(True, 1): TileLaunchCost(9.0, 0.85, 3.9)}}
 
     @property
     def attention_tuning(self) -> AttentionTuning:
@@ -146,8 +149,10 @@ class HipOps(KernelNamespace):
             costs = self.TILE_COSTS.get(self.device_kind)
             if costs is not None:
                 scale = head_dim / self.TILE_COSTS_HEAD_DIM
+                if scale > 1:
+                    costs = tuple({**dict(costs), **self.WIDE_TILE_COSTS.get(self.device_kind, {})}.items())
                 costs = tuple((form, TileLaunchCost(cost.start_us, cost.trip_us * scale, cost.step_ns * scale)) for form, cost in costs)
-                tuning = dataclasses.replace(tuning, tile_costs=costs)
+                tuning = dataclasses.replace(tuning, tile_costs=costs, slot_ns=4.0)
             self._tunings[key] = tuning
         return self._tunings[key]
 
