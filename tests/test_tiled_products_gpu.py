@@ -66,6 +66,14 @@ def test_every_tile_at_its_edges(ops, form, tile, rows, columns, inner):
             assert bool((whole[:margin] == 7.0).all()) and bool((whole[-margin:] == 7.0).all())
 
 
+# On both sides of the line between tiles of 64 x 32 (up to 256 of them, parts of the sums included: 4,096 columns of gated products, 8,192 of the others for one block of rows) and of 64 x 64, from
+# one slab to more than either has buffers for.
+@pytest.mark.parametrize("rows,columns,inner", [(1, 8200, 64), (33, 4096, 640), (33, 4104, 704), (64, 8192, 704), (64, 8200, 576), (65, 2056, 768), (127, 4160, 384), (250, 1032, 832), (250, 2112, 320)])
+@pytest.mark.parametrize("form", FORMS)
+def test_small_tiles_on_both_sides_of_their_line(ops, form, rows, columns, inner):
+    test_every_tile_at_its_edges(ops, form, 1, rows, columns, inner)
+
+
 def test_what_does_not_fit_is_refused(ops):
     x, weight = drawn(64, 64, 128, 1)
     out = torch.empty(64, 64, device="cuda", dtype=torch.bfloat16)
