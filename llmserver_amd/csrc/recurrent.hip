@@ -1139,10 +1139,17 @@ __global__ __launch_bounds__(256, 3) void memory_chunk_read16_kernel(const bf16_
 //
 // What bounds the scan is the chain of a row's tokens (0.45 us a token, on rows * heads * value_dim / 64 workgroups: 918 us for
 // one row of 2,048 tokens, 16 heads of 128 x 128, 1,171 us for 8 heads of 128 x 256, most of the chip idle); here all chunks
-// run at once and only the walk over the chunks (2) is serial.  A workgroup of eight wavefronts has one (chunk, head, 128 value
-// columns): scores are formed once for all of them, operands stay in LDS (129 KB at 128 channels), products run on 32-bit MFMA but where said.
+// run at once and only the walk over the chunks (2) is serial.  A workgroup has one (chunk, head, 128 value columns): scores are formed once
+// for all of them, operands stay in LDS (158 KB at 128 channels, so one workgroup a compute unit), products run on 32-bit MFMA but where said.
+//   What bounds the first launch is what one compute unit gets through between its barriers, operands from memory and their decays, diagonals, 64-bit products, one
+// after another; sixteen wavefronts hide more of it than eight did: a workgroup takes 25 us instead of 45, of which 5 (9 with sigmoids' roots) the operands, 6 the
+// diagonals, 4 what lies between, 2 what leaves and 7.5 the values' products, both halves of the columns at once.  us with the walk and the read-out, before and now:
+// 2,048 tokens of 16 heads of 128 x 128 132, 119; of 8 heads of 128 x 256 139, 124; 1,024 tokens 106, 92 and 113, 98; 2,048 of 16 heads of 64 x 64 70, 65; six rows of 510
+// tokens together 65, 57.  (3) is no faster with its loads a slab ahead, and with registers for four workgroups a compute unit faster behind 768 of them only (120, 114; 92, 96).
 constexpr int CHANNEL_MOST = 128;        // widest head that fits LDS so
 constexpr int CHANNEL_COLUMNS = 128;     // value columns a workgroup
+constexpr int CHANNEL_THREADS = 1024;    // of a workgroup: sixteen wavefronts
+constexpr int CHANNEL_QUARTERS = 4;      // ... of which four share the channels of a block of tokens
 
 template <int DP>
 struct ChannelChunkLds {                 // DP: key channels filled up to 64 or 128
@@ -1150,15 +1157,20 @@ struct ChannelChunkLds {                 // DP: key channels filled up to 64 or 
     static constexpr int B = DP + 16;    // ... read along its rows
     float q[MC * B];                     // queries; then (row length B) the keys as the chunk's sum wants them
     float k[MC * B];                     // (row length A) keys; then (row length B) what rounding took from the keys as the sum wants them
-    float d[MC * (A > MC_B ? A : MC_B)]; // decays; then (row length A) what rounding took from the keys; then the values of 64 columns (row length MC_B)
+    float d[MC * (A > MC_B ? A : MC_B)]; // decays; then (row length A) what rounding took from the keys; then the values of the first 64 columns (row length MC_B)
     float score[MC * MC_A];
     double total[MC / BC][DP];
+    union {
+        double diagonal[CHANNEL_QUARTERS][BC][MC];                                 // sums of a quarter of the channels: [tokens back][token]
+        double between[6][64][4];                                                  // ... of half of them, as a wavefront's lanes hold a tile
+        float v[MC * MC_B];                                                        // the values of the second 64 columns
+    };
 };
 
 // (1) out = the chunks' own read-outs, sums [item][head][dim][value_dim] and totals [item][head][dim] as the walk wants them,
 // and queries [T][heads][dim] as they read the state in front of their chunk.  grid (items, heads, blocks of 128 value columns).
 template <typename T, int DP>
-__global__ __launch_bounds__(512) void channel_chunk_kernel(const T* __restrict__ q, long q_stride, const T* __restrict__ k, long k_stride,
+__global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunk_kernel(const T* __restrict__ q, long q_stride, const T* __restrict__ k, long k_stride,
                                                             const T* __restrict__ v, long v_stride, const float* __restrict__ decay,
                                                             const float* __restrict__ decay_bias, int mode, float inv_tau,
                                                             const float* __restrict__ bonus, float q_scale, const int* __restrict__ row_start,
@@ -1180,12 +1192,12 @@ __global__ __launch_bounds__(512) void channel_chunk_kernel(const T* __restrict_
     // Queries, keys and decays into LDS; tokens behind the chunk's last one and channels behind the head's last one read and write
     // nothing and keep everything.  (Every load is of a place that is there: none stands under a condition.)
     {
-        constexpr int PER = MC * DP / 512;
+        constexpr int PER = MC * DP / CHANNEL_THREADS;
         T raw_q[PER], raw_k[PER];
         float raw_z[PER];
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            const int i = tid + 512 * e, t = min(i / DP, n - 1), c = min(i % DP, dim - 1);
+            const int i = tid + CHANNEL_THREADS * e, t = min(i / DP, n - 1), c = min(i % DP, dim - 1);
             const size_t token = token0 + t;
             raw_q[e] = q[token * q_stride + key_column + c];
             raw_k[e] = k[token * k_stride + key_column + c];
@@ -1193,21 +1205,21 @@ __global__ __launch_bounds__(512) void channel_chunk_kernel(const T* __restrict_
         }
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            const int i = tid + 512 * e, t = i / DP, c = i % DP;
+            const int i = tid + CHANNEL_THREADS * e, t = i / DP, c = i % DP;
             const bool there = t < n && c < dim;
             s.q[t * A + c] = there ? (float)raw_q[e] * q_scale : 0.f;
             s.k[t * A + c] = there ? (float)raw_k[e] : 0.f;
             s.d[t * A + c] = there ? decay_of(raw_z[e], mode, inv_tau) : 1.f;
         }
-        for (int i = tid; i < MC * MC_A; i += 512) s.score[i] = 0.f;
+        for (int i = tid; i < MC * MC_A; i += CHANNEL_THREADS) s.score[i] = 0.f;
     }
     __syncthreads();
 
-    // Inside the blocks: wavefront = (block, half of the channels), lane = (token t of the block, a quarter of every 16 channels).  The
+    // Inside the blocks: wavefront = (block, quarter of the channels), lane = (token t of the block, a quarter of every 16 channels).  The
     // diagonals j = t - back one after another, the query times its decays so far in registers.
     {
-        const int block = wave >> 1, half = wave & 1, t = lane & 15, c0 = half * (DP / 2) + 4 * (lane >> 4);
-        constexpr int U = DP / 32;
+        const int block = wave / CHANNEL_QUARTERS, quarter = wave % CHANNEL_QUARTERS, t = lane & 15, c0 = quarter * (DP / CHANNEL_QUARTERS) + 4 * (lane >> 4);
+        constexpr int U = DP / (16 * CHANNEL_QUARTERS);
         float weighted[U][4];
         double sum[BC];                                                            // (their last additions would be the score's largest roundings)
 #pragma unroll
@@ -1237,83 +1249,99 @@ __global__ __launch_bounds__(512) void channel_chunk_kernel(const T* __restrict_
             }
             sum[back] = ((double)part[0] + (double)part[1]) + ((double)part[2] + (double)part[3]);
         }
+        // (added up over the four lanes of a token, each of which ends with four of the diagonals)
+        const bool upper = lane & 32, odd = lane & 16;
 #pragma unroll
-        for (int back = 0; back < BC; ++back) {
-            sum[back] += __shfl_xor(sum[back], 16, 64);
-            sum[back] += __shfl_xor(sum[back], 32, 64);
+        for (int back = 0; back < BC / 2; ++back) {
+            const double other = __shfl_xor(upper ? sum[back] : sum[BC / 2 + back], 32, 64);
+            sum[back] = (upper ? sum[BC / 2 + back] : sum[back]) + other;
         }
-        float* mine = &s.score[(block * BC + t) * MC_A + block * BC + t];
-        for (int turn = 0; turn < 2; ++turn) {                                     // one half of the channels after the other
-            if (half == turn && lane < 16) {
 #pragma unroll
-                for (int back = 0; back < BC; ++back)
-                    if (back <= t) mine[-back] = (float)((double)mine[-back] + sum[back]);
-            }
-            __syncthreads();
+        for (int back = 0; back < BC / 4; ++back) {
+            const double other = __shfl_xor(odd ? sum[back] : sum[BC / 4 + back], 16, 64);
+            s.diagonal[quarter][(upper ? BC / 2 : 0) + (odd ? BC / 4 : 0) + back][block * BC + t] = (odd ? sum[BC / 4 + back] : sum[back]) + other;
         }
     }
+    __syncthreads();
+    {                                                                              // (a thread one score: BC diagonals of MC tokens)
+        const int t = tid % MC, back = tid / MC;
+        if (back <= t % BC)
+            s.score[t * MC_A + t - back] = (float)((s.diagonal[0][back][t] + s.diagonal[1][back][t]) + (s.diagonal[2][back][t] + s.diagonal[3][back][t]));
+    }
 
-    // Queries times the decays from their block's first token, keys times those up to its last one; a thread a (block, channel).  The
-    // products are formed in 64-bit: sixteen factors then cost a weight one rounding, as they do the scan's state.
-    for (int i = tid; i < (MC / BC) * DP; i += 512) {
-        const int block = i / DP, c = i % DP;
-        float* qs = &s.q[block * BC * A + c];
-        float* ks = &s.k[block * BC * A + c];
+    // Queries times the decays from their block's first token (one half of the threads), keys times those up to its last one (the other); a thread a (block, channel).
+    // The products are formed in 64-bit: sixteen factors then cost a weight one rounding, as they do the scan's state.
+    {
+        const bool keys = tid >= (MC / BC) * DP;
+        const int i = keys ? tid - (MC / BC) * DP : tid, block = i / DP, c = i % DP;
+        const bool some = i < (MC / BC) * DP;
         float d[BC];
 #pragma unroll
-        for (int t = 0; t < BC; ++t) d[t] = s.d[(block * BC + t) * A + c];
+        for (int t = 0; t < BC; ++t) d[t] = some ? s.d[(block * BC + t) * A + c] : 1.f;
+        __syncthreads();                                                           // (what the keys lose in rounding takes the decays' place)
         double product = 1.0;
+        if (some && !keys) {
+            float* qs = &s.q[block * BC * A + c];
 #pragma unroll
-        for (int t = 0; t < BC; ++t) {
-            if (bonus == nullptr) product *= (double)d[t];
-            qs[t * A] = (float)((double)qs[t * A] * product);
-            if (bonus != nullptr) product *= (double)d[t];
-        }
-        s.total[block][c] = product;
-        product = 1.0;
+            for (int t = 0; t < BC; ++t) {
+                if (bonus == nullptr) product *= (double)d[t];
+                qs[t * A] = (float)((double)qs[t * A] * product);
+                if (bonus != nullptr) product *= (double)d[t];
+            }
+            s.total[block][c] = product;
+        } else if (some) {
+            float* ks = &s.k[block * BC * A + c];
 #pragma unroll
-        for (int t = BC - 1; t >= 0; --t) {
-            const double key = (double)ks[t * A] * product;
-            ks[t * A] = (float)key;
-            s.d[(block * BC + t) * A + c] = (float)(key - (double)(float)key);
-            product *= (double)d[t];
+            for (int t = BC - 1; t >= 0; --t) {
+                const double key = (double)ks[t * A] * product;
+                ks[t * A] = (float)key;
+                s.d[(block * BC + t) * A + c] = (float)(key - (double)(float)key);
+                product *= (double)d[t];
+            }
         }
     }
     __syncthreads();
 
-    // Between blocks: six tiles of 16 x 16 scores on six wavefronts.
-    if (wave < 6) {
-        const int block = wave < 3 ? 3 : wave < 5 ? 2 : 1, other = wave < 3 ? wave : wave < 5 ? wave - 3 : 0;
+    // Between blocks: six tiles of 16 x 16 scores, two wavefronts a tile, each with half of the channels.
+    {
+        const int tile = wave >> 1, half = wave & 1, block = tile < 3 ? 3 : tile < 5 ? 2 : 1, other = tile < 3 ? tile : tile < 5 ? tile - 3 : 0;
         const int r = lane & 15, g = lane >> 4;
-        const float* a = &s.q[(block * BC + r) * A + g];
-        const float* b = &s.k[(other * BC + r) * A + g];
-        mc_f4 part[4] = {};
-        for (int i = 0; i < DP; i += 16) {
-            float x[4], y[4];
+        double sum[4] = {};
+        if (tile < 6) {
+            const float* a = &s.q[(block * BC + r) * A + g];
+            const float* b = &s.k[(other * BC + r) * A + g];
+            mc_f4 part[4] = {};
+            for (int i = half * (DP / 2); i < (half + 1) * (DP / 2); i += 16) {
+                float x[4], y[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                x[u] = a[i + 4 * u];
-                y[u] = b[i + 4 * u];
-                double skipped = 1.0;
-                for (int between = other + 1; between < block; ++between) skipped *= s.total[between][i + 4 * u + g];
-                x[u] = (float)((double)x[u] * skipped);
+                for (int u = 0; u < 4; ++u) {
+                    y[u] = b[i + 4 * u];
+                    const double next = s.total[other + 1][i + 4 * u + g], after = s.total[min(other + 2, MC / BC - 1)][i + 4 * u + g];
+                    const double skipped = (block > other + 1 ? next : 1.0) * (block > other + 2 ? after : 1.0);
+                    x[u] = (float)((double)a[i + 4 * u] * skipped);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) part[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[u], part[u], 0, 0, 0);
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) part[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[u], part[u], 0, 0, 0);
+            for (int e = 0; e < 4; ++e) {
+                sum[e] = ((double)part[0][e] + (double)part[1][e]) + ((double)part[2][e] + (double)part[3][e]);
+                if (half == 1) s.between[tile][lane][e] = sum[e];
+            }
         }
-        const mc_f4 acc = together(part);
+        __syncthreads();
+        if (tile < 6 && half == 0)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s.score[(block * BC + 4 * g + e) * MC_A + other * BC + r] = acc[e];
+            for (int e = 0; e < 4; ++e) s.score[(block * BC + 4 * g + e) * MC_A + other * BC + r] = (float)(sum[e] + s.between[tile][lane][e]);
     }
-    __syncthreads();
 
     // The queries and the totals leave (whatever lies in front of or behind a block in one product, 64-bit as above); the keys are brought up to the chunk's end, into the queries' place behind them.
     {
-        constexpr int PER = MC * DP / 512;
+        constexpr int PER = MC * DP / CHANNEL_THREADS;
         float kept[PER], rest[PER];
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            const int i = tid + 512 * e, t = i / DP, c = i % DP, block = t / BC;
+            const int i = tid + CHANNEL_THREADS * e, t = i / DP, c = i % DP, block = t / BC;
             double before = 1.0, behind = 1.0;
 #pragma unroll
             for (int o = 0; o < MC / BC; ++o) {
@@ -1331,34 +1359,36 @@ __global__ __launch_bounds__(512) void channel_chunk_kernel(const T* __restrict_
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            const int i = tid + 512 * e;
+            const int i = tid + CHANNEL_THREADS * e;
             s.q[(i / DP) * B + i % DP] = kept[e];
             s.k[(i / DP) * B + i % DP] = rest[e];
         }
     }
 
-    // 64 value columns at a time: scores x values, and the keys' sum with the values.
-    float* s_v = s.d;
-    for (int column0 = blockIdx.z * CHANNEL_COLUMNS; column0 < min(value_dim, (int)(blockIdx.z + 1) * CHANNEL_COLUMNS); column0 += 64) {
-        T values[MC * 64 / 512];
+    // Scores x values, and the keys' sum with the values: 64 columns for each eight wavefronts.
+    const int of = wave / 8, column0 = blockIdx.z * CHANNEL_COLUMNS + 64 * of;
+    float* s_v = of ? s.v : s.d;
+    constexpr int VALUES = MC * 64 / 512;
+    T values[VALUES];
 #pragma unroll
-        for (int e = 0; e < MC * 64 / 512; ++e) {
-            const int t = min(8 * e + (tid >> 6), n - 1), c = min(column0 + (tid & 63), value_dim - 1);
-            values[e] = v[(token0 + t) * v_stride + (size_t)head * value_dim + c];
-        }
-        __syncthreads();                                 // the keys are in place; the columns before have been read
-        float no_number = 0.f;                           // NaN once a value is no number
+    for (int e = 0; e < VALUES; ++e) {
+        const int t = min(8 * e + (wave & 7), n - 1), c = min(column0 + lane, value_dim - 1);
+        values[e] = v[(token0 + t) * v_stride + (size_t)head * value_dim + c];
+    }
+    __syncthreads();                                     // the keys are in place, and nobody reads what the values replace
+    float no_number = 0.f;                               // NaN once a value is no number
 #pragma unroll
-        for (int e = 0; e < MC * 64 / 512; ++e) {
-            const int t = 8 * e + (tid >> 6);
-            const float value = t < n && column0 + (tid & 63) < value_dim ? (float)values[e] : 0.f;
-            s_v[t * MC_B + (tid & 63)] = value;
-            no_number = __builtin_fmaf(value, 0.f, no_number);
-        }
-        const bool all_finite = !__syncthreads_or(no_number != 0.f);
+    for (int e = 0; e < VALUES; ++e) {
+        const int t = 8 * e + (wave & 7);
+        const float value = t < n && column0 + lane < value_dim ? (float)values[e] : 0.f;
+        s_v[t * MC_B + lane] = value;
+        no_number = __builtin_fmaf(value, 0.f, no_number);
+    }
+    const bool all_finite = !__syncthreads_or(no_number != 0.f);
+    if (column0 < value_dim) {
         const int r = lane & 15, g = lane >> 4, half = wave & 1;
         {
-            const int block = wave >> 1;
+            const int block = (wave & 7) >> 1;
             mc_f4 acc[2] = {};
             if (all_finite) {
                 channel_product<2>(acc, &s.score[block * BC * MC_A], MC_A, 1, s_v + 32 * half, MC_B, 1, (block + 1) * BC, lane);
@@ -1388,7 +1418,7 @@ __global__ __launch_bounds__(512) void channel_chunk_kernel(const T* __restrict_
         // touched.  With 32-bit ones the state behind a short memory (decays around 0.6 a token) was off by 1.32 times what the walk's
         // is (bfloat16; 1.15 in float32); it is 1.06 and 0.90, 0.76 of it where memories are long.  11 us of 133 for 2,048 tokens of 16 heads.
         const int exact_from = BC * max(0, (n + BC - 1) / BC - 2);
-        for (int tile = wave >> 1; tile < DP / 16; tile += 4) {
+        for (int tile = (wave & 7) >> 1; tile < DP / 16; tile += 4) {
             mc_f4 part[2][4] = {};
             const int turned = 4 * (r & 3) + (r >> 2);   // (in this order of rows the 32-bit instruction's results lie where the 64-bit one's do)
             for (int i = 0; i < exact_from; i += 16) {
@@ -1613,7 +1643,7 @@ LSA_EXPORT int lsa_linear_recurrence_chunked(int code, const void* q, long q_str
     if (items <= 0 || sums == nullptr || totals == nullptr || queries == nullptr) return -1;
     const dim3 grid(items, heads, (value_dim + CHANNEL_COLUMNS - 1) / CHANNEL_COLUMNS);
 #define LSA_LAUNCH(T, DP) \
-        channel_chunk_kernel<T, DP><<<grid, 512, sizeof(ChannelChunkLds<DP>), stream>>>((const T*)q, q_stride, (const T*)k, k_stride, (const T*)v, v_stride, \
+        channel_chunk_kernel<T, DP><<<grid, CHANNEL_THREADS, sizeof(ChannelChunkLds<DP>), stream>>>((const T*)q, q_stride, (const T*)k, k_stride, (const T*)v, v_stride, \
             decay, decay_bias, mode, 1.f / tau, bonus, q_scale, row_start, row_len, rows, sums, totals, queries, out, heads, dim, value_dim)
     if (code) { if (dim <= 64) LSA_LAUNCH(bf16_t, 64); else LSA_LAUNCH(bf16_t, 128); }
     else { if (dim <= 64) LSA_LAUNCH(float, 64); else LSA_LAUNCH(float, 128); }

@@ -110,6 +110,13 @@ def plain_delta(q, k, v, decay, beta, state):
     return torch.stack(out), state
 
 
+# Value columns that end inside the second 64 of a workgroup's 128, in its first number, and inside a third.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 96, 100), (1, 128, 65), (2, 33, 150)])
+def test_linear_recurrence_in_chunks_at_the_edges_of_value_columns(ops, dtype, heads, dim, vdim):
+    test_linear_recurrence_in_chunks(ops, dtype, heads, dim, vdim, "double_exp" if vdim == 100 else "sigmoid_root", 1.0)
+
+
 @pytest.mark.parametrize("per_channel", [False, True])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,spread", [(2, 2, 128, 128, 1.0), (3, 3, 24, 40, 2.0), (4, 2, 64, 130, 3.0), (2, 1, 65, 256, 0.5),
                                                             (1, 1, 5, 1, 6.0)])
