@@ -325,7 +325,9 @@ def _single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, 
 
 FIXED_WORKGROUP_TILES = 4          # tiles a workgroup of the prompt-portion kernel takes in captured steps
 FIXED_WORKGROUPS = 1024            # workgroups that such a launch's key ranges aim at
-FIXED_LARGE_WORKGROUPS = 256       # ... if they take more tiles than that, in two halves of their keys: one on every compute unit
+# ... if they take more tiles than that, in two halves of their keys: one on every compute unit.  us a launch with its merge, four tiles at their best and eight in two halves: 16 heads on 8 of 128, 190 tokens behind
+# 8,064 keys 38 to 51 by their ranges, 34, 400 behind 8,600 70, 53; 32 on 8, 250 behind 3,750 48, 39, 64 behind 7,936 36, 34.
+FIXED_LARGE_WORKGROUPS = 256
 FIXED_KEYS_A_RANGE = 256           # fewest keys of a range at the longest context that the captured step serves
 
 
@@ -335,7 +337,7 @@ def fixed_workgroup_shape(n_tokens: int, n_rows: int, group_size: int, n_kv_head
     keys, runs the prompt-portion kernel with, or None where the wavefront-per-tile kernel is the better one.  Its items read the
     keys once for every tile of 16 (token, head) pairs, these workgroups once for four tiles: from 16 tiles behind 2,048 keys on that is
     what counts (eight layers, 16 heads over 8 of 128, a step of 190 tokens behind 8,064: 1,804 us as items, 1,388 so; behind 2,000: 1,256
-    and 1,141; 60 tokens behind 4,000, 8 tiles, which stay items: 925)."""
+    and 1,141; 60 tokens behind 4,000, 8 tiles, which stay items: 925).  ``per_workgroup``: tiles a workgroup takes, four or, where the kernel has them in two halves, eight."""
     _, tokens_per_tile, group_tiles = group_tiling(group_size, tuning.tile_rows)
     if n_tokens // tokens_per_tile < MIN_TILES_FOR_WORKGROUPS or max_keys < 2048:
         return None
