@@ -277,3 +277,20 @@ def test_short_rows_behind_long_contexts_share_their_keys_between_workgroups():
     # and a handful of tiles stays beside them: no launch of its own, and no merge, for two tiles
     plan = plan_of([1] * 8 + [8], [4096] * 9)
     assert len(plan.tiles) == 0 and {int(r) for r in plan.items[:, 0]} == set(range(9))
+
+
+@pytest.mark.parametrize("lengths,contexts,group_size", [([400], [9000], 2), ([200] * 3, [5200] * 3, 2), ([200] * 3, [5200] * 3, 4), ([500], [9500], 2), ([333] * 2, [6333] * 2, 4)])
+def test_cut_walks_fill_their_rounds(lengths, contexts, group_size):
+    """Ranges of long walks are about as long as each other: a launch has no last round that is nearly empty (one workgroup in ten more than the compute units hold), and meets every key once."""
+    from llmserver_amd.kernels.ops import HipOps
+    from llmserver_amd.parts import AttentionTuning
+    tuning = AttentionTuning(1024, HipOps.TILE_COSTS["gfx950-256cu"], slot_ns=4.0)
+    plan = build_attention_plan(lengths, contexts, group_size, 8, None, workgroup_tiles=8, tuning=tuning, tile_halves=2, tile_key_ranges=128)
+    workgroups = 8 * len(plan.tiles)
+    assert workgroups and (workgroups <= 256 or workgroups > 0.9 * 256 * -(-workgroups // 256)), workgroups
+    for (row, token), ranges in covered_tokens(plan, lengths, contexts, group_size, None).items():
+        at = 0
+        for begin, end in sorted(ranges):
+            assert begin == at
+            at = end
+        assert at >= contexts[row] - lengths[row] + token + 1
