@@ -152,8 +152,9 @@ class HipOps(KernelNamespace):
                 if scale > 1:
                     costs = tuple({**dict(costs), **self.WIDE_TILE_COSTS.get(self.device_kind, {})}.items())
                 costs = tuple((form, TileLaunchCost(cost.start_us, cost.trip_us * scale, cost.step_ns * scale)) for form, cost in costs)
-                # (a partial result's way is half as dear as the neutral costs have it: four rows of 256 tokens behind 3,840, 16 heads on 8 of 128, 71 us by 8 ns, 57 by 4; 99 portions and prompts
-                # together 1.24 and 1.26 times as fast as with the kernel before)
+                # (a partial result's way is half as dear as the neutral costs have it: four rows of 256 tokens behind 3,840, 16 heads on 8 of 128, 71 us by 8 ns, 58 by 4; two of 333 behind 6,000,
+                # 32 on 8, 99 and 113; 99 portions and prompts together are 1.22 times as fast as with the kernel before, by 6 ns as by 4, two of them slower: 400 tokens behind 8,600, 16 on 8, 78, 81;
+                # three rows of 200 behind 5,000 67, 69)
                 tuning = dataclasses.replace(tuning, tile_costs=costs, slot_ns=4.0)
             self._tunings[key] = tuning
         return self._tunings[key]

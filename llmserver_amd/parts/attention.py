@@ -207,15 +207,9 @@ def _workgroup_tiles_that_pay(row_len, row_ctx, tiles_per_row, tokens_per_tile, 
     when every compute unit is busy.  Ranges shorten the longest walk as far as one likes, for the price of a
     second launch and the partial results' way through memory.  Each way is priced with the tuning's costs: start,
     then the longest workgroup's trips and all workgroups' steps, whichever is more (blended, since both slow each
-    other down), then the merge.  Shorter and shorter walks are priced until one costs more than the one before.
-
-    Walks that are cut are about as long as each other, so the compute units are done in rounds: with 280 workgroups on 256 of them some get two while the others wait, which their
-    steps together do not show.  us without and with that in the price, bfloat16 heads of 128: 400 tokens behind 8,600, 16 heads on 8, 81, 62 (a plan of 280 workgroups and one of 256 or
-    fewer); three rows of 200 behind 5,000 69, 58, 32 on 8 96, 79; 500 behind 9,000 76, 66; 700 behind 7,000, 32 on 8, 132, 118; the other way rows of 333, 130 and 77 behind 4,000 49, 51, 600
-    behind 1,500, 16 on 16, 0.96; 99 portions and prompts together 1.03."""
+    other down), then the merge.  Shorter and shorter walks are priced until one costs more than the one before."""
     rows = np.flatnonzero(np.asarray(tiles_per_row) >= min_tiles)
     row_len, row_ctx = np.asarray(row_len, dtype=np.int64), np.asarray(row_ctx, dtype=np.int64)
-    units = max(1, tuning.target_waves // 4)
     best, best_key = None, None
     for per_workgroup in sorted({min(4, most), most}):
         of_rows = _workgroups_of_rows(rows, row_len, row_ctx, tokens_per_tile, window, per_workgroup, chunk)
@@ -237,10 +231,6 @@ def _workgroup_tiles_that_pay(row_len, row_ctx, tiles_per_row, tokens_per_tile, 
                     longest = int(per_range.max(initial=0))
                     slots = int((ranges * tiles_of_group)[ranges > 1].sum())
                 path, work = -(-longest // halves) * cost.trip_us, total * heads * cost.step_ns * 1e-3
-                if walk is not None:                             # (walks cut to one length end in rounds)
-                    started = int(ranges.sum()) * heads
-                    if started > units:
-                        work *= -(-started // units) * units / started
                 merge = tuning.merge_us + slots * heads * tuning.slot_ns * 1e-3 if slots else 0.0
                 estimate = cost.start_us + (path ** 4 + work ** 4) ** 0.25 + merge
                 key = (estimate, walk is not None, halves, per_workgroup)

@@ -279,18 +279,27 @@ def test_short_rows_behind_long_contexts_share_their_keys_between_workgroups():
     assert len(plan.tiles) == 0 and {int(r) for r in plan.items[:, 0]} == set(range(9))
 
 
-@pytest.mark.parametrize("lengths,contexts,group_size", [([400], [9000], 2), ([200] * 3, [5200] * 3, 2), ([200] * 3, [5200] * 3, 4), ([500], [9500], 2), ([333] * 2, [6333] * 2, 4)])
-def test_cut_walks_fill_their_rounds(lengths, contexts, group_size):
-    """Ranges of long walks are about as long as each other: a launch has no last round that is nearly empty (one workgroup in ten more than the compute units hold), and meets every key once."""
+@pytest.mark.parametrize("slot_ns", [4.0, 8.0])
+def test_search_over_walks_stops_behind_its_cheapest(slot_ns):
+    """Walks are priced from long to short until one costs more than the one before: no other walk may be cheaper than the one that was chosen (a search over that one and
+    any single other walk, which prices both, chooses it again)."""
+    import dataclasses
+
     from llmserver_amd.kernels.ops import HipOps
     from llmserver_amd.parts import AttentionTuning
-    tuning = AttentionTuning(1024, HipOps.TILE_COSTS["gfx950-256cu"], slot_ns=4.0)
-    plan = build_attention_plan(lengths, contexts, group_size, 8, None, workgroup_tiles=8, tuning=tuning, tile_halves=2, tile_key_ranges=128)
-    workgroups = 8 * len(plan.tiles)
-    assert workgroups and (workgroups <= 256 or workgroups > 0.9 * 256 * -(-workgroups // 256)), workgroups
-    for (row, token), ranges in covered_tokens(plan, lengths, contexts, group_size, None).items():
-        at = 0
-        for begin, end in sorted(ranges):
-            assert begin == at
-            at = end
-        assert at >= contexts[row] - lengths[row] + token + 1
+    from llmserver_amd.parts.attention import _workgroup_tiles_that_pay, group_tiling
+    tuning = AttentionTuning(1024, HipOps.TILE_COSTS["gfx950-256cu"], slot_ns=slot_ns)
+    draw = random.Random(5)
+    portions = [(1, 8, [604, 1190], [2164, 10887]), (1, 8, [180, 678], [3431, 10439]), (2, 4, [1430], [10084])]
+    for _ in range(300):
+        lens = [int(64 * 23 ** draw.random()) for _ in range(draw.choice((1, 1, 2, 3)))]
+        portions.append((draw.choice((1, 2, 4)), draw.choice((4, 8)), lens, [n + int(500 * 32 ** draw.random()) for n in lens]))
+    for group, heads, lens, ctxs in portions:
+        _, per_tile, _ = group_tiling(group, tuning.tile_rows)
+
+        def chosen(walks):
+            return _workgroup_tiles_that_pay(lens, ctxs, [-(-n // per_tile) for n in lens], per_tile, heads, None, 8, dataclasses.replace(tuning, tile_walks=walks), 2, 128, 1)
+        choice = chosen(tuning.tile_walks)
+        for walk in tuning.tile_walks:
+            pair = tuple(w for w in tuning.tile_walks if w in (walk, choice[2]))
+            assert chosen(pair) == choice, (group, heads, lens, ctxs, choice, walk)
