@@ -51,9 +51,6 @@ typedef float elem_t;
 
 struct Item { int row, q0, k_begin, k_end; };
 
-struct Merge { int row, q0, first_slot, n_slots; };
-constexpr int MERGE_MOST_SLOTS = 128;  // key ranges one tile may be split into (two slots' weights per lane of a wavefront)
-
 struct Geometry {
     int n_q, n_kv, group, gheads, tokens_per_tile, gtiles, page_size, window;
     unsigned page_magic;      // ceil(2^32 / page_size): key / page_size == mulhi(key, page_magic) for key < 2^32 / page_size
@@ -128,108 +125,6 @@ constexpr int KEY_STEP = 16;
 constexpr int NS = D / 16;                   // 16-dim steps (four 16x16x4 MFMAs each)
 #endif
 
-// How many of the workgroups that share a tile's key ranges have left their results: a counter per tile and KV head, zero before the launch and zero again
-// behind it (the last workgroup of a tile puts it back).
-struct Arrivals { int* counts; int workgroups_a_tile; };
-constexpr int MOST_ARRIVALS = 32;      // workgroups a tile
-
-// Two numbers that workgroups on other XCDs read in the same launch, past the caches that those do not share.
-__device__ __forceinline__ void store_for_all(float* to, float a, float b) {
-    const float2 both = make_float2(a, b);
-    __hip_atomic_store(reinterpret_cast<unsigned long long*>(to), __builtin_bit_cast(unsigned long long, both), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float2 load_for_all(const float* from) {
-    return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(from), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-
-// The end of a workgroup whose first wavefront has stored its part of a tile's result: counts it in, and if it is the tile's last one, merges all parts by
-// log-sum-exp into `o` (the token's heads).  Nobody waits for anybody: a workgroup that is not the last one ends.  All four wavefronts get here.
-// Order between workgroups: the stores have reached memory (the wait) before the count does, and the last one's loads, which go past its own caches, follow its count.
-// Bound by three trips to memory one behind the other (stores, count, loads: 2 us) where a launch of its own cost its start, its list, and two.
-template <int OTHERS>
-__device__ __forceinline__ void merge_arrived(elem_t* o, f32x4 (*scratch)[ND][64], const float* part_acc, const float* part_ml, const Geometry& g, const Arrivals& arrivals,
-                                              int kv_head, int gtile, size_t token) {
-    __shared__ int arrived_before;
-    __shared__ float slot_weight[16][MOST_ARRIVALS], inverse[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, parts = arrivals.workgroups_a_tile;
-    int* count = arrivals.counts + (size_t)(blockIdx.x / parts) * gridDim.y + blockIdx.y;
-    if (wave == 0) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (lane == 0) arrived_before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (arrived_before != parts - 1) return;
-    asm volatile("" ::: "memory");
-    if (threadIdx.x == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int heads = min(g.gheads, g.group - gtile * g.gheads);                   // of the tile: its pairs 0 .. heads - 1 are the token's
-    const size_t stride = (size_t)gridDim.y * 16, first = ((size_t)(blockIdx.x / parts) * parts * gridDim.y + blockIdx.y) * 16;
-    // The slots' weights: 32 neighbouring lanes are a pair's slots.
-    for (int p = threadIdx.x >> 5; p < heads; p += 8) {
-        const int s = threadIdx.x & 31;
-        float2 ml = make_float2(NEG_INF, 0.f);
-        if (s < parts) ml = load_for_all(part_ml + (first + s * stride + p) * 2);
-        float top = ml.x;
-#pragma unroll
-        for (int offset = 1; offset < 32; offset *= 2) top = fmaxf(top, __shfl_xor(top, offset, 64));
-        const float w = ml.x == NEG_INF ? 0.f : expf(ml.x - top);
-        float total = w * ml.y;
-#pragma unroll
-        for (int offset = 1; offset < 32; offset *= 2) total += __shfl_xor(total, offset, 64);
-        slot_weight[p][s] = w;
-        const int head = kv_head * g.group + gtile * g.gheads + p;
-        if (s == 0) inverse[p] = inverse_of_sum(total, top, g.sinks, head) * gate_of(g, token, head);
-    }
-    // Their sums: a lane four neighbouring dimensions of a pair, a wavefront every fourth slot; loads go out ahead of the weights.
-    // (two groups of 64 lanes at a time: all loads of two heads of 128, or four, are one trip)
-    constexpr int AT_ONCE = MOST_ARRIVALS / 4, GROUPS = 2;
-    const int vectors = heads * (D / 4);
-    for (int group = 0; 64 * group < vectors; group += GROUPS) {
-        float2 low[GROUPS][AT_ONCE], high[GROUPS][AT_ONCE];
-#pragma unroll
-        for (int u = 0; u < GROUPS; ++u) {
-            const int at = min(64 * (group + u) + lane, vectors - 1), p = at / (D / 4), dim = 4 * (at % (D / 4));
-            if (64 * (group + u) >= vectors) continue;
-#pragma unroll
-            for (int i = 0; i < AT_ONCE; ++i) {
-                if (4 * i >= parts) continue;
-                const float* from = part_acc + (first + (size_t)min(wave + 4 * i, parts - 1) * stride + p) * D + dim;
-                low[u][i] = load_for_all(from);
-                high[u][i] = load_for_all(from + 2);
-            }
-        }
-        if (group == 0) __syncthreads();                                           // (the weights are there)
-        f32x4 sum[GROUPS];
-#pragma unroll
-        for (int u = 0; u < GROUPS; ++u) {
-            const int p = min(64 * (group + u) + lane, vectors - 1) / (D / 4);
-            sum[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int i = 0; i < AT_ONCE; ++i)
-                if (wave + 4 * i < parts && 64 * (group + u) < vectors)
-                    sum[u] += (f32x4){low[u][i].x, low[u][i].y, high[u][i].x, high[u][i].y} * slot_weight[p][wave + 4 * i];
-            if (wave && 64 * (group + u) < vectors) scratch[wave - 1][group + u][lane] = sum[u];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < GROUPS; ++u) {
-            const int at = 64 * (group + u) + lane, p = at / (D / 4), dim = 4 * (at % (D / 4));
-            if (wave || at >= vectors) continue;
-#pragma unroll
-            for (int w = 0; w < OTHERS; ++w) sum[u] += scratch[w][group + u][lane];
-            sum[u] *= inverse[p];
-            elem_t* to = o + (size_t)(kv_head * g.group + gtile * g.gheads + p) * D + dim;
-#if LSA_BF16
-            bf16x4 r4;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) r4[e] = (bf16_t)sum[u][e];
-            *reinterpret_cast<bf16x4*>(to) = r4;
-#else
-            *reinterpret_cast<f32x4*>(to) = sum[u];
-#endif
-        }
-    }
-}
-
 // MODE is DecodeFusion::mode, known when the kernel is compiled: what a mode does not need is not in its code, and
 // no branch stands between the loads of the item's start (a load inside a branch makes every later wait a wait
 // for everything).
@@ -239,17 +134,14 @@ __device__ __forceinline__ void merge_arrived(elem_t* o, f32x4 (*scratch)[ND][64
 // results in memory, no merge launch.  For steps whose contexts are short, where that launch costs as much as the
 // attention, and for steps of many rows, whose tiles get no more ranges than that anyway.
 // BIAS: scores fall with the distance between query and key (Geometry::slopes); without it nothing of that is in the code.
-// ARRIVALS (steps of one token a row, four ranges a workgroup): a row has the ranges of `workgroups_a_tile` workgroups, one behind the other.  Each merges its four,
-// leaves the result in the slot of its number and counts itself in; whoever comes last finds the others' there and merges them, so that
-// long contexts need no second launch either (merge_arrived).
-template <int MODE, bool PLAIN, int WG_RANGES, bool BIAS, bool ARRIVALS = false>
+template <int MODE, bool PLAIN, int WG_RANGES, bool BIAS>
 __global__ __launch_bounds__(256, LSA_MIN_WAVES) void paged_attention_kernel(
     const elem_t* __restrict__ q, long q_token_stride, elem_t* __restrict__ out,
     const elem_t* keys, const elem_t* values,
     const int* __restrict__ table, int table_stride,
     const int* __restrict__ row_start, const int* __restrict__ row_len, const int* __restrict__ row_ctx,
     const Item* __restrict__ items, const int* __restrict__ item_slot, int n_items,
-    float* part_acc, float* part_ml, Geometry g, DecodeFusion fusion, Arrivals arrivals) {
+    float* __restrict__ part_acc, float* __restrict__ part_ml, Geometry g, DecodeFusion fusion) {
     const int lane = threadIdx.x & 63;
     // The wavefront's number, told to the compiler to be the same in all lanes: the item, its row and the key loop's bounds
     // then live in scalar registers and the loop's branches are scalar ones (a hundred branches on the execution mask
@@ -727,7 +619,7 @@ __global__ __launch_bounds__(256, LSA_MIN_WAVES) void paged_attention_kernel(
             for (int c = 0; c < ND; ++c) others_acc[first_wave / R * (R - 1) + member - 1][c][lane] = acc[c];
         }
         __syncthreads();
-        if (!ARRIVALS && (member > 0 || !pair_valid)) return;
+        if (member > 0 || !pair_valid) return;
         float top = NEG_INF;
 #pragma unroll
         for (int w = 0; w < R; ++w) top = fmaxf(top, ranges_max[first_wave + w][col]);
@@ -737,23 +629,6 @@ __global__ __launch_bounds__(256, LSA_MIN_WAVES) void paged_attention_kernel(
             const float m = ranges_max[first_wave + w][col];
             weight[w] = m == NEG_INF ? 0.f : expf(m - top);
             total += weight[w] * ranges_sum[first_wave + w][col];
-        }
-        if constexpr (ARRIVALS) {
-            if (member == 0 && pair_valid) {
-                const size_t base = ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * 16 + col;
-                float* pa = part_acc + base * D + 4 * quad;
-#pragma unroll
-                for (int c = 0; c < ND; ++c) {
-                    f32x4 sum = acc[c] * weight[0];
-#pragma unroll
-                    for (int w = 1; w < R; ++w) sum += others_acc[w - 1][c][lane] * weight[w];
-                    store_for_all(pa + 16 * c, sum[0], sum[1]);
-                    store_for_all(pa + 16 * c + 2, sum[2], sum[3]);
-                }
-                if (quad == 0) store_for_all(part_ml + base * 2, top, total);
-            }
-            merge_arrived<4 - TILES>(out + (size_t)token0 * g.n_q * D, &others_acc[0], part_acc, part_ml, g, arrivals, kv_head, gtile, (size_t)token0);
-            return;
         }
         const float inv = inverse_of_sum(total, top, g.sinks, head) * gate_of(g, token0 + pair_token, head);
         elem_t* o = out + ((size_t)(token0 + pair_token) * g.n_q + head) * D + 4 * quad;
@@ -1397,7 +1272,10 @@ __global__ __launch_bounds__(256) void paged_attention_tile_kernel_f32(
 #endif  // LSA_BF16
 
 // Merge the partial slots of a tile: out = sum_s w_s acc_s / sum_s w_s l_s, w_s = exp(m_s - max m).
+struct Merge { int row, q0, first_slot, n_slots; };
+
 constexpr int MERGE_WAVES = 4;         // at most; the launch brings as many as the merges' slots can use
+constexpr int MERGE_MOST_SLOTS = 128;  // key ranges one tile may be split into (two slots' weights per lane of a wavefront)
 
 __global__ __launch_bounds__(MERGE_WAVES * 64) void merge_kernel(
     elem_t* __restrict__ out, const int* __restrict__ row_start, const int* __restrict__ row_len,
@@ -1583,8 +1461,8 @@ LSA_EXPORT int lsa_paged_attention(
     float scale,
     int window, int page_size, int n_q, int n_kv, int gheads, int tokens_per_tile, int gtiles,
     int decode_fusion, const float* q_weight, const float* k_weight, float norm_eps, const float* cos_sin, int tiles_per_workgroup,
-    int merge_in_workgroup, int tile_halves, int* arrivals, int workgroups_a_tile, const float* sinks, float softcap, int chunk, const float* slopes,
-    const void* gates, long gate_stride, hipStream_t stream) {
+    int merge_in_workgroup, int tile_halves, const float* sinks, float softcap, int chunk, const float* slopes, const void* gates, long gate_stride,
+    hipStream_t stream) {
     if (n_items <= 0 && n_tiles <= 0) return 0;
     if (softcap < 0.f || chunk < 0 || (gates != nullptr && gate_stride < n_q)) return -1;
     if (slopes != nullptr && (decode_fusion || !(scale > 0.f))) return -1;      // (the fused start takes scores without a bias only)
@@ -1636,30 +1514,15 @@ LSA_EXPORT int lsa_paged_attention(
         // ranges of each of two tiles (some may be empty), no item has a slot, nothing is left to merge.
         if (merge_in_workgroup && ((merge_in_workgroup != 2 && merge_in_workgroup != 4) || n_items % 4 != 0 || n_merges != 0)) return -1;
         dim3 grid((n_items + 3) / 4, n_kv * gtiles);
-        // arrivals (counters, [rows, KV heads x tiles of a group], zero): the caller promises one token a row and the row's ranges, four times workgroups_a_tile of them,
-        // one behind the other.  Scores with a bias and half a fused start go the other way.
-        const bool whole_fusion = !decode_fusion || (q_weight != nullptr && cos_sin != nullptr);
-        const bool arriving = arrivals != nullptr && n_merges > 0 && !merge_in_workgroup && n_tiles == 0 && slopes == nullptr && whole_fusion;
-        if (arriving && (workgroups_a_tile < 1 || workgroups_a_tile > MOST_ARRIVALS || n_items != 4 * workgroups_a_tile * n_merges || part_acc == nullptr || part_ml == nullptr)) return -1;
-        const Arrivals counters = {arrivals, workgroups_a_tile};
 #define LSA_LAUNCH_ITEMS(MODE, PLAIN) LSA_LAUNCH_ITEMS_MERGE(MODE, PLAIN, 0)
-#define LSA_LAUNCH_ITEMS_MERGE(MODE, PLAIN, RANGES) LSA_LAUNCH_ITEMS_OF(MODE, PLAIN, RANGES, false, false)
-#define LSA_LAUNCH_ITEMS_OF(MODE, PLAIN, RANGES, BIAS, ARRIVE) paged_attention_kernel<MODE, PLAIN, RANGES, BIAS, ARRIVE><<<grid, 256, 0, stream>>>( \
+#define LSA_LAUNCH_ITEMS_MERGE(MODE, PLAIN, RANGES) LSA_LAUNCH_ITEMS_OF(MODE, PLAIN, RANGES, false)
+#define LSA_LAUNCH_ITEMS_OF(MODE, PLAIN, RANGES, BIAS) paged_attention_kernel<MODE, PLAIN, RANGES, BIAS><<<grid, 256, 0, stream>>>( \
             (const elem_t*)q, q_token_stride, (elem_t*)out, (const elem_t*)keys, (const elem_t*)values, table, table_stride, \
-            row_start, row_len, row_ctx, (const Item*)items, item_slot, n_items, part_acc, part_ml, g, fusion, counters)
-        if (arriving) {
-#if LSA_BF16
-            if (decode_fusion == 3) LSA_LAUNCH_ITEMS_OF(3, true, 4, false, true);
-            else if (decode_fusion == 1) LSA_LAUNCH_ITEMS_OF(1, true, 4, false, true);
-            else
-#endif
-            LSA_LAUNCH_ITEMS_OF(0, false, 4, false, true);
-            LSA_LAUNCH_CHECK();
-        }
+            row_start, row_len, row_ctx, (const Item*)items, item_slot, n_items, part_acc, part_ml, g, fusion)
         if (slopes != nullptr) {
-            if (merge_in_workgroup == 4) LSA_LAUNCH_ITEMS_OF(0, false, 4, true, false);
-            else if (merge_in_workgroup == 2) LSA_LAUNCH_ITEMS_OF(0, false, 2, true, false);
-            else LSA_LAUNCH_ITEMS_OF(0, false, 0, true, false);
+            if (merge_in_workgroup == 4) LSA_LAUNCH_ITEMS_OF(0, false, 4, true);
+            else if (merge_in_workgroup == 2) LSA_LAUNCH_ITEMS_OF(0, false, 2, true);
+            else LSA_LAUNCH_ITEMS_OF(0, false, 0, true);
         } else {
 #if LSA_BF16
             const bool plain = q_weight != nullptr && cos_sin != nullptr;

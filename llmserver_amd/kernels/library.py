@@ -26,8 +26,7 @@ _SIGNATURES = {
     "lsa_sample_static_max_rows": [],
     "lsa_sample_static_error": [c_int],
     "lsa_paged_attention": [_P, c_long, _P, _P, _P, _P, c_int, _P, _P, _P, _P, _P, c_int, _P, c_int, c_int, _P, _P, _P, _P, c_int,
-                            c_float, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P, _P, c_float, _P, c_int, c_int, c_int, _P, c_int, _P, c_float, c_int,
-                            _P, _P, c_long, _P],
+                            c_float, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P, _P, c_float, _P, c_int, c_int, c_int, _P, c_float, c_int, _P, _P, c_long, _P],
     "lsa_embedding_wide": [c_int, _P, _P, _P, c_int, c_int, c_int, c_float, c_int, _P],
     "lsa_stream_inject": [_P, c_int, _P, _P, c_float, _P, _P, c_float, _P, c_int, c_int, c_int, c_int, _P],
     "lsa_most_streams": [],

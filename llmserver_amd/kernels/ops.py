@@ -892,8 +892,6 @@ class HipOps(KernelNamespace):
         """Halves that a workgroup of the prompt-portion kernel can split its tiles' keys between (1: it cannot)."""
         return int(self._attention_library(dtype, head_dim).lsa_attention_tile_halves())
 
-    attention_counts_arrivals = True        # a plan may bring counters with which the last range of a row merges them all
-
     def attention_tile_key_ranges(self, dtype, head_dim) -> int:
         """Most ranges that the keys of a workgroup's tiles may be cut into, each range another workgroup's (their
         partial results are merged afterwards); 1: the kernel does not offer that."""
@@ -1020,11 +1018,6 @@ class HipOps(KernelNamespace):
                                    or (decode_fusion is not None and (q_weight is None or cos_sin is None))):
             raise ValueError("merging in the workgroup takes a plan that gives every tile four key ranges (or, in steps of one token "
                              "per row, two, with tiles in pairs) and no slots, and, with decode fusion, both norm weights and a rotation")
-        arrivals = plan.get("arrivals")
-        if arrivals is not None:
-            _check(arrivals, "plan arrivals", torch.int32, (rows, n_kv * gtiles))
-            if n != rows or n_merges != rows or n_slots != n_items:
-                raise ValueError("workgroups that count themselves in take a step of one token a row, a merge a row and a slot for every range")
         lib = self._attention_library(qkv.dtype, head_dim)
         if plan.get("rows_in_order") and merge_in_workgroup and n == rows and lib.lsa_attention_single_fits(page_size, int(fusion_mode > 0)) \
                 and (self.single_tokens_pay(qkv.dtype, head_dim, rows, n_q, n_kv, not softcap and slopes is None)
@@ -1045,8 +1038,7 @@ class HipOps(KernelNamespace):
             _ptr(row_len), _ptr(row_ctx), _ptr(plan["items"]), _ptr(plan["item_slot"]), n_items, _ptr(plan["merges"]),
             n_merges, n_slots, _ptr(part_acc), _ptr(part_ml), _ptr(tiles), _ptr(tile_slots), n_tiles, float(scale), int(window) if window else 0,
             page_size, n_q, n_kv, gheads, tokens_per_tile, gtiles, fusion_mode, _ptr(q_weight), _ptr(k_weight), float(norm_eps),
-            _ptr(cos_sin), int(plan.get("tiles_per_workgroup", 0)), merge_in_workgroup, int(plan.get("tile_halves", 1)), _ptr(arrivals),
-            int(plan.get("workgroups_a_tile", 0)), _ptr(sinks),
+            _ptr(cos_sin), int(plan.get("tiles_per_workgroup", 0)), merge_in_workgroup, int(plan.get("tile_halves", 1)), _ptr(sinks),
             float(softcap) if softcap else 0.0, int(chunk) if chunk else 0, _ptr(slopes), _ptr(gates), gates.stride(0) if gates is not None else 0,
             _stream()), "paged_attention")
 

@@ -242,7 +242,6 @@ def _workgroup_tiles_that_pay(row_len, row_ctx, tiles_per_row, tokens_per_tile, 
     return best
 
 
-ARRIVING_NUMBERS = 512  # most numbers of a KV head's heads whose merge the last workgroup of a row takes on itself
 WORKGROUP_RANGES = 4    # key ranges of a tile that one workgroup (four wavefronts) walks and merges itself
 SHORT_CONTEXT = 512     # captured steps whose contexts all stay within this are a shape of their own: a workgroup merges
                         # a tile's four key ranges itself (no partial results in memory, no launch that merges them)
@@ -540,16 +539,6 @@ def build_attention_plan(row_len, row_ctx, group_size: int, n_kv_heads: int, win
     return plan
 
 
-def arriving_workgroups(n_rows: int, ranges: int, numbers: int) -> Optional[int]:
-    """Workgroups that the key ranges of a step of one token make, four to each, if whoever of them ends last is to merge them, in place of a launch; None where
-    that launch is the better way: several rows (they share ranges by their lengths, and one wavefront for a row's few ranges takes longer than the launch: 8 rows of
-    1,500 keys 15.2 us, 17.6 so), and heads of a KV head with more than ``ARRIVING_NUMBERS`` ``numbers`` together, which one workgroup no longer adds up in one
-    trip to memory.  us with the launch and without, heads on KV heads of 128: 16 on 8, 600 keys 11.3, 10.9, 1,000 12.4, 11.5, 8,100 17.8, 15.5; 16 on 16, 3,000
-    15.5, 14.2; 32 on 8, 4,000 13.8, 13.6, 16,000 24.6, 22.1; 16 on 8 of 64, 1,900 10.7, 9.9; float32, 16 on 8, 3,000 17.0, 16.2.  Not so: 40 on 8, 3,000 14.9,
-    14.9; 64 on 8, 9,000 19.1, 19.8; 8 on 1 of 256, 3,000 20.5, 24.7."""
-    return ranges // WORKGROUP_RANGES if n_rows == 1 and numbers <= ARRIVING_NUMBERS and ranges % WORKGROUP_RANGES == 0 and ranges > WORKGROUP_RANGES else None
-
-
 def stage_attention_plan(ctx, key, group_size: int, n_kv_heads: int, head_dim: int, window: Optional[int], graph_shape,
                          chunk: Optional[int] = None, fused: bool = False) -> None:
     """Make the step's attention work list for a mixer of this geometry and put it among the step's staged arrays under
@@ -600,13 +589,7 @@ def stage_attention_plan(ctx, key, group_size: int, n_kv_heads: int, head_dim: i
                                     target_waves=tuning.target_waves, fixed_splits=fixed, workgroup_tiles=per_workgroup,
                                     merge_in_workgroup=in_workgroup, tuning=tuning, tile_halves=halves, tile_min_workgroups=fewest,
                                     tile_key_ranges=key_ranges, fixed_tiles=fixed_tiles, chunk=chunk, share_ranges=True, fused=fused)
-    arrivals, (heads, _, group_tiles) = {}, group_tiling(group_size, tuning.tile_rows)
-    if single_tokens and ctx.ops.attention_counts_arrivals and fixed is not None and not in_workgroup and bool((ctx.h_row_len == 1).all()):
-        workgroups = arriving_workgroups(ctx.n_rows, fixed, heads * head_dim)
-        if workgroups is not None:          # (staged with the step: zero before every run, whatever became of the one before)
-            arrivals = {"arrivals": np.zeros((ctx.n_rows, n_kv_heads * group_tiles), np.int32), "workgroups_a_tile": workgroups}
     ctx.set_plan(key, {
-        **arrivals,
         **({"tile_slots": plan.tile_slots} if plan.tile_slots is not None else {}),
         "items": plan.items, "item_slot": plan.item_slot, "merges": plan.merges, "tiles": plan.tiles,
         "n_tiles": len(plan.tiles), "n_items": len(plan.items), "n_merges": len(plan.merges),

@@ -399,9 +399,6 @@ class KernelNamespace:
     def attention_tile_halves(self, dtype, head_dim) -> int:
         return 1
 
-    # Whether plans of single-token steps may bring ``arrivals`` (counters, zeros), with which whoever of a row's key ranges ends last merges them.
-    attention_counts_arrivals = False
-
     def attention_tile_key_ranges(self, dtype, head_dim) -> int:
         """Most ranges the keys of a workgroup's tiles may be cut into for workgroups of their own (1: not offered)."""
         return 1
