@@ -681,8 +681,8 @@ __global__ __launch_bounds__(256, LSA_MIN_WAVES) void paged_attention_kernel(
 
 #if LSA_BF16
 // ------------------------------------------------------------------------------------------------
-// Portions of prompts: the four wavefronts of a workgroup take four consecutive tiles of 16 pairs
-// of one request.  They see (almost) the same keys, so each step's 32 keys and values are fetched
+// Portions of prompts: the four wavefronts of a workgroup take 4 * SUB consecutive tiles of 16 pairs
+// of one request (SUB tiles each).  They see (almost) the same keys, so each step's 32 keys and values are fetched
 // from the pages once per workgroup, straight into LDS (global_load_lds, 16 bytes a lane: no registers and no LDS
 // stores on the way), into a ring of STAGES buffers: the loads of step i + STAGES - 1 are issued before the products
 // of step i, one barrier a step, and every wavefront reads its MFMA operands from LDS, 16 bytes per lane and read
@@ -727,10 +727,16 @@ constexpr int STEP_LOADS = K_BLOCK_CHUNKS > V_BLOCK_CHUNKS ? K_BLOCK_CHUNKS : V_
 #define LSA_TILE_STAGES 2
 #endif
 constexpr int STAGES = LSA_TILE_STAGES;
+// Tiles of 16 pairs per wavefront (SUB): with two, every key and value operand read from LDS feeds two products, which
+// halves the LDS traffic per flop; the accumulators of two tiles fit the registers up to a head size of 128.
+// The host picks one or two per launch: two pay when the rows are long (the longest workgroup then does not
+// decide the time), one when they are short and there are few workgroups.
+constexpr int MAX_SUB = LSA_ND <= 8 ? 2 : 1;
 // Halves of a workgroup that split the keys between them (see the kernel): two where their buffers fit into LDS.
 constexpr int MAX_HALVES = LSA_ND <= 8 ? 2 : 1;
-// Wavefronts per SIMD wanted (they hide the latency of a step's dependent chain: LDS read, MFMA, softmax, MFMA), as far as the registers allow.
-#define LSA_TILE_MIN_WAVES (LSA_ND <= 8 ? 3 : 1)
+// Wavefronts per SIMD wanted (they hide the latency of a step's dependent chain: LDS read, MFMA, softmax, MFMA),
+// as far as the registers of SUB tiles allow.
+#define LSA_TILE_MIN_WAVES(SUB) ((SUB) == 1 ? (LSA_ND <= 8 ? 3 : 1) : (LSA_ND <= 4 ? 3 : 2))
 struct FullStep { static constexpr bool value = true; };        // every key of the step is seen by every pair
 struct MaskedStep { static constexpr bool value = false; };
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -749,8 +755,8 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // combines a tile's slots.  first < 0 (or no `tile_slots` at all): the entry holds all keys and writes the output.
 struct TileSlots { int first, stride; };
 
-template <int HALVES, bool BIAS>
-__global__ __launch_bounds__(256 * HALVES, LSA_TILE_MIN_WAVES) void paged_attention_tile_kernel(
+template <int SUB, int HALVES, bool BIAS>
+__global__ __launch_bounds__(256 * HALVES, LSA_TILE_MIN_WAVES(SUB)) void paged_attention_tile_kernel(
     const elem_t* __restrict__ q, long q_token_stride, elem_t* __restrict__ out,
     const elem_t* __restrict__ keys, const elem_t* __restrict__ values,
     const int* __restrict__ table, int table_stride,
@@ -772,11 +778,18 @@ __global__ __launch_bounds__(256 * HALVES, LSA_TILE_MIN_WAVES) void paged_attent
     const int col = lane & 15, quad = lane >> 4;
     const int row = tile.row;
     const int n = row_len[row], first_pos = row_ctx[row] - n;
-    const int q0 = tile.q0 + wave * g.tokens_per_tile;    // first token of this wavefront's tile
+    const int q0 = tile.q0 + wave * SUB * g.tokens_per_tile;    // first token of this wavefront's SUB consecutive tiles
     const int pair_token = col / g.gheads, pair_head_in_group = gtile * g.gheads + col % g.gheads;
     const int head = kv_head * g.group + pair_head_in_group;
-    const bool pair_valid = pair_token < g.tokens_per_tile && q0 + pair_token < n && pair_head_in_group < g.group;
-    const int q_pos = pair_valid ? first_pos + q0 + pair_token : -1, first_seen = first_key_of(q_pos, g);
+    bool pair_valid[SUB];
+    int q_pos[SUB], first_seen[SUB];
+#pragma unroll
+    for (int u = 0; u < SUB; ++u) {
+        const int token = q0 + u * g.tokens_per_tile + pair_token;
+        pair_valid[u] = pair_token < g.tokens_per_tile && token < n && pair_head_in_group < g.group;
+        q_pos[u] = pair_valid[u] ? first_pos + token : -1;
+        first_seen[u] = first_key_of(q_pos[u], g);
+    }
     // (scores stay in units of 1 / scale here, and so does what they lose per position)
     float slope = 0.f;
     if constexpr (BIAS) slope = g.slopes[min(head, g.n_q - 1)] * g.scale_inverse;
@@ -785,25 +798,31 @@ __global__ __launch_bounds__(256 * HALVES, LSA_TILE_MIN_WAVES) void paged_attent
     const size_t kv_head_keys = (size_t)kv_head * ps * D, kv_head_values = (size_t)kv_head * D * ps;
     const size_t page_elems = (size_t)g.n_kv * ps * D;
     // Keys this wavefront's pairs can see at all: [wave_lo, wave_hi).
-    const int wave_tokens = max(0, min(g.tokens_per_tile, n - q0));
+    const int wave_tokens = max(0, min(SUB * g.tokens_per_tile, n - q0));
     const int wave_hi = wave_tokens > 0 ? first_pos + q0 + wave_tokens : 0;
     const int wave_lo = max(0, first_key_of(first_pos + q0, g));
     const int q_pos_min = first_pos + q0;                       // smallest position among the wavefront's valid pairs
     const float scale_log2 = g.scale * 1.44269504088896340736f;
 
-    bf16x8 qf[NS];
-    f32x4 acc[ND];
-    float run_max = NEG_INF, run_sum = 0.f;
+    bf16x8 qf[SUB][NS];
+    f32x4 acc[SUB][ND];
+    float run_max[SUB], run_sum[SUB];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        const int dim = 32 * s + 8 * quad;
-        bf16x8 x = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (pair_valid && dim < D)
-            x = *reinterpret_cast<const bf16x8*>(q + (size_t)(row_start[row] + q0 + pair_token) * q_token_stride + (size_t)head * D + dim);
-        qf[s] = x;
+    for (int u = 0; u < SUB; ++u) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const int dim = 32 * s + 8 * quad;
+            bf16x8 x = {0, 0, 0, 0, 0, 0, 0, 0};
+            if (pair_valid[u] && dim < D)
+                x = *reinterpret_cast<const bf16x8*>(q + (size_t)(row_start[row] + q0 + u * g.tokens_per_tile + pair_token) * q_token_stride +
+                                                     (size_t)head * D + dim);
+            qf[u][s] = x;
+        }
+#pragma unroll
+        for (int c = 0; c < ND; ++c) acc[u][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        run_max[u] = NEG_INF;
+        run_sum[u] = 0.f;
     }
-#pragma unroll
-    for (int c = 0; c < ND; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
     // The steps of 32 keys that cover the tile's keys, and this half's share of them: [k_begin, k_end).
     const int first_step = (tile.k_begin / 32) * 32;
@@ -897,7 +916,7 @@ __global__ __launch_bounds__(256 * HALVES, LSA_TILE_MIN_WAVES) void paged_attent
     const int value_at = K_TILE_BYTES + (quad >> 1) * V_BLOCK_BYTES + col * V_ROW + 16 * (quad & 1);
     // The steps that every pair of the wavefront sees completely (they need no mask) lie in [full_from, full_to]; the
     // steps that have anything for its pairs in (active_from, active_to).
-    const bool whole_tiles = wave_tokens == g.tokens_per_tile && g.gheads * g.tokens_per_tile == 16 && (gtile + 1) * g.gheads <= g.group;
+    const bool whole_tiles = wave_tokens == SUB * g.tokens_per_tile && g.gheads * g.tokens_per_tile == 16 && (gtile + 1) * g.gheads <= g.group;
     const int full_from = !whole_tiles ? 0x7fffffff : max(k_begin, first_key_of(first_pos + q0 + wave_tokens - 1, g));
     const int full_to = min(k_end - 32, q_pos_min - 31);
     // Scores stay as the products left them; the scale (in units of ln 2, so that the exponential is one
@@ -906,33 +925,41 @@ __global__ __launch_bounds__(256 * HALVES, LSA_TILE_MIN_WAVES) void paged_attent
     auto compute_step = [&](auto full_tag, int stage, int kt) __attribute__((always_inline)) {
         constexpr bool FULL = decltype(full_tag)::value;
         const unsigned char* buffer = lds_all + lds_base + stage * STEP_BYTES;
-        float sv[8];
-        float tile_max = NEG_INF;
+        float sv[SUB][8];
+        float tile_max[SUB];
+#pragma unroll
+        for (int u = 0; u < SUB; ++u) tile_max[u] = NEG_INF;
 #pragma unroll
         for (int t2 = 0; t2 < 2; ++t2) {
-            f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
+            f32x4 s4[SUB];
+#pragma unroll
+            for (int u = 0; u < SUB; ++u) s4[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 bf16x8 kf = {0, 0, 0, 0, 0, 0, 0, 0};
                 if (32 * s + 32 <= D || quad < 2) kf = *reinterpret_cast<const bf16x8*>(buffer + key_row_at[t2] + 64 * s);
-                s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[s], s4, 0, 0, 0);
+#pragma unroll
+                for (int u = 0; u < SUB; ++u) s4[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[u][s], s4[u], 0, 0, 0);
             }
-            float nearest = 0.f;
+            float nearest[SUB];
             if constexpr (BIAS) {
-                nearest = -slope * (float)(q_pos - (kt + 8 * quad + 4 * t2));      // what the first of the four loses
+#pragma unroll
+                for (int u = 0; u < SUB; ++u) nearest[u] = -slope * (float)(q_pos[u] - (kt + 8 * quad + 4 * t2));      // what the first of the four loses
             }
 #pragma unroll
+            for (int u = 0; u < SUB; ++u)
+#pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = s4[r];
+                    float v = s4[u][r];
                     if (g.cap > 0.f) v = capped(v * g.scale, g) * g.scale_inverse;       // (scores stay in units of 1 / scale here)
-                    if constexpr (BIAS) v += __builtin_fmaf(slope, (float)r, nearest);
+                    if constexpr (BIAS) v += __builtin_fmaf(slope, (float)r, nearest[u]);
                     if (!FULL) {
                         const int kpos = kt + 8 * quad + 4 * t2 + r;
-                        const bool seen = kpos >= k_begin && kpos < k_end && kpos <= q_pos && kpos >= first_seen;
+                        const bool seen = kpos >= k_begin && kpos < k_end && kpos <= q_pos[u] && kpos >= first_seen[u];
                         v = seen ? v : NEG_INF;
                     }
-                    sv[4 * t2 + r] = v;
-                    tile_max = fmaxf(tile_max, v);
+                    sv[u][4 * t2 + r] = v;
+                    tile_max[u] = fmaxf(tile_max[u], v);
                 }
         }
         // Values of keys outside the range may be anything (a page's places behind the context were never written):
@@ -949,29 +976,43 @@ __global__ __launch_bounds__(256 * HALVES, LSA_TILE_MIN_WAVES) void paged_attent
             const u32x4 raw = *reinterpret_cast<const u32x4*>(buffer + value_at + 16 * c * V_ROW);
             return __builtin_bit_cast(bf16x8, FULL ? raw : (raw & keep));
         };
+        // The value operands are asked for now, so that they arrive while the softmax runs, and the output products
+        // of the first tile are issued before the softmax of the second: the MFMA pipe works on them meanwhile.
+        // (With one tile per wavefront there is nothing to overlap them with; they are read where they are used.)
+        bf16x8 vf[SUB > 1 ? ND : 1];
+        if (SUB > 1) {
+#pragma unroll
+            for (int c = 0; c < ND; ++c) vf[c] = value_operand(c);
+        }
         // The running maximum of a pair only moves when some key of this step beats it, which
         // soon becomes rare: then the exchange between the lanes of a pair and the rescaling of
         // the accumulators are skipped (the result is the same, the maximum being unchanged).
-        if (__any(tile_max > run_max)) {
-            float top = fmaxf(tile_max, __shfl_xor(tile_max, 16, 64));
-            top = fmaxf(top, __shfl_xor(top, 32, 64));
-            const float new_max = fmaxf(run_max, top);
-            const float alpha = __builtin_amdgcn_exp2f((run_max - (new_max == NEG_INF ? 0.f : new_max)) * scale_log2);
-            run_max = new_max;
-            run_sum *= alpha;
 #pragma unroll
-            for (int c = 0; c < ND; ++c) acc[c] *= alpha;
+        for (int u = 0; u < SUB; ++u) {
+            if (__any(tile_max[u] > run_max[u])) {
+                float top = fmaxf(tile_max[u], __shfl_xor(tile_max[u], 16, 64));
+                top = fmaxf(top, __shfl_xor(top, 32, 64));
+                const float new_max = fmaxf(run_max[u], top);
+                const float alpha = __builtin_amdgcn_exp2f((run_max[u] - (new_max == NEG_INF ? 0.f : new_max)) * scale_log2);
+                run_max[u] = new_max;
+                run_sum[u] *= alpha;
+#pragma unroll
+                for (int c = 0; c < ND; ++c) acc[u][c] *= alpha;
+            }
+            const float shift = run_max[u] == NEG_INF ? 0.f : -run_max[u] * scale_log2;
+            bf16x8 pf;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[u][e], scale_log2, shift));
+                run_sum[u] += p;
+                pf[e] = (bf16_t)p;
+            }
+#pragma unroll
+            for (int c = 0; c < ND; ++c) {
+                const bf16x8 value = SUB > 1 ? vf[SUB > 1 ? c : 0] : value_operand(c);
+                acc[u][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(value, pf, acc[u][c], 0, 0, 0);
+            }
         }
-        const float shift = run_max == NEG_INF ? 0.f : -run_max * scale_log2;
-        bf16x8 pf;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[e], scale_log2, shift));
-            run_sum += p;
-            pf[e] = (bf16_t)p;
-        }
-#pragma unroll
-        for (int c = 0; c < ND; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(value_operand(c), pf, acc[c], 0, 0, 0);
     };
     auto compute = [&](int stage, int kt) __attribute__((always_inline)) {
         if (kt >= wave_hi || kt + 32 <= wave_lo) return;          // nothing for this wavefront's pairs in this step
@@ -1010,82 +1051,98 @@ __global__ __launch_bounds__(256 * HALVES, LSA_TILE_MIN_WAVES) void paged_attent
         // of keys and values are free once every load has landed and everybody has passed the barrier.
         loads_landed_then_barrier<0>();
         float* handed = reinterpret_cast<float*>(lds_all);
-        constexpr int PER_WAVE = ND * 256 + 32;               // floats: accumulators (ND x 64 lanes x 4), then max and sum of 16 pairs
+        constexpr int PER_WAVE = SUB * (ND * 256 + 32);               // floats: accumulators (ND x 64 lanes x 4), then max and sum of 16 pairs
         static_assert(4 * PER_WAVE * sizeof(float) <= sizeof(lds_all), "the buffers of keys and values hold what the second half hands over");
         float* mine = handed + (size_t)wave * PER_WAVE;
-        run_sum += __shfl_xor(run_sum, 16, 64);
-        run_sum += __shfl_xor(run_sum, 32, 64);                // the pair's whole sum, in every lane of the pair
+#pragma unroll
+        for (int u = 0; u < SUB; ++u) {
+            float total = run_sum[u];
+            total += __shfl_xor(total, 16, 64);
+            total += __shfl_xor(total, 32, 64);
+            run_sum[u] = total;                                       // the pair's whole sum, in every lane of the pair
+        }
         if (half) {
 #pragma unroll
-            for (int c = 0; c < ND; ++c) *reinterpret_cast<f32x4*>(mine + (c * 64 + lane) * 4) = acc[c];
-            if (quad == 0) {
-                mine[ND * 256 + col] = run_max;
-                mine[ND * 256 + 16 + col] = run_sum;
+            for (int u = 0; u < SUB; ++u) {
+                float* block = mine + u * (ND * 256 + 32);
+#pragma unroll
+                for (int c = 0; c < ND; ++c) *reinterpret_cast<f32x4*>(block + (c * 64 + lane) * 4) = acc[u][c];
+                if (quad == 0) {
+                    block[ND * 256 + col] = run_max[u];
+                    block[ND * 256 + 16 + col] = run_sum[u];
+                }
             }
         }
         __syncthreads();
         if (half) return;
-        const float other_max = mine[ND * 256 + col], other_sum = mine[ND * 256 + 16 + col];
-        const float top = fmaxf(run_max, other_max);
-        const float w0 = run_max == NEG_INF ? 0.f : __builtin_amdgcn_exp2f((run_max - top) * scale_log2);
-        const float w1 = other_max == NEG_INF ? 0.f : __builtin_amdgcn_exp2f((other_max - top) * scale_log2);
-        const float total = w0 * run_sum + w1 * other_sum;
-        if (!pair_valid) return;
-        if (slots.first >= 0) {
-            const size_t base = ((size_t)(slots.first + wave * slots.stride) * heads + head_index) * 16 + col;
-            float* pa = part_acc + base * D + 4 * quad;
+#pragma unroll
+        for (int u = 0; u < SUB; ++u) {
+            const float* block = mine + u * (ND * 256 + 32);
+            const float other_max = block[ND * 256 + col], other_sum = block[ND * 256 + 16 + col];
+            const float top = fmaxf(run_max[u], other_max);
+            const float w0 = run_max[u] == NEG_INF ? 0.f : __builtin_amdgcn_exp2f((run_max[u] - top) * scale_log2);
+            const float w1 = other_max == NEG_INF ? 0.f : __builtin_amdgcn_exp2f((other_max - top) * scale_log2);
+            const float total = w0 * run_sum[u] + w1 * other_sum;
+            if (!pair_valid[u]) continue;
+            if (slots.first >= 0) {
+                const size_t base = ((size_t)(slots.first + (wave * SUB + u) * slots.stride) * heads + head_index) * 16 + col;
+                float* pa = part_acc + base * D + 4 * quad;
+#pragma unroll
+                for (int c = 0; c < ND; ++c) {
+                    const f32x4 other = *reinterpret_cast<const f32x4*>(block + (c * 64 + lane) * 4);
+                    *reinterpret_cast<f32x4*>(pa + 16 * c) = acc[u][c] * w0 + other * w1;
+                }
+                if (quad == 0) {
+                    part_ml[base * 2] = top == NEG_INF ? NEG_INF : top * g.scale;
+                    part_ml[base * 2 + 1] = total;
+                }
+                continue;
+            }
+            const size_t token = (size_t)(row_start[row] + q0 + u * g.tokens_per_tile + pair_token);
+            const float inv = inverse_of_sum(total, top == NEG_INF ? NEG_INF : top * g.scale, g.sinks, head) * gate_of(g, token, head);
+            elem_t* o = out + (token * g.n_q + head) * D + 4 * quad;
 #pragma unroll
             for (int c = 0; c < ND; ++c) {
-                const f32x4 other = *reinterpret_cast<const f32x4*>(mine + (c * 64 + lane) * 4);
-                *reinterpret_cast<f32x4*>(pa + 16 * c) = acc[c] * w0 + other * w1;
-            }
-            if (quad == 0) {
-                part_ml[base * 2] = top == NEG_INF ? NEG_INF : top * g.scale;
-                part_ml[base * 2 + 1] = total;
-            }
-            return;
-        }
-        const size_t token = (size_t)(row_start[row] + q0 + pair_token);
-        const float inv = inverse_of_sum(total, top == NEG_INF ? NEG_INF : top * g.scale, g.sinks, head) * gate_of(g, token, head);
-        elem_t* o = out + (token * g.n_q + head) * D + 4 * quad;
+                const f32x4 other = *reinterpret_cast<const f32x4*>(block + (c * 64 + lane) * 4);
+                bf16x4 r4;
 #pragma unroll
-        for (int c = 0; c < ND; ++c) {
-            const f32x4 other = *reinterpret_cast<const f32x4*>(mine + (c * 64 + lane) * 4);
-            bf16x4 r4;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) r4[r] = (bf16_t)((acc[c][r] * w0 + other[r] * w1) * inv);
-            *reinterpret_cast<bf16x4*>(o + 16 * c) = r4;
+                for (int r = 0; r < 4; ++r) r4[r] = (bf16_t)((acc[u][c][r] * w0 + other[r] * w1) * inv);
+                *reinterpret_cast<bf16x4*>(o + 16 * c) = r4;
+            }
         }
         return;
     }
     // (the loads issued past the end still write LDS: a wavefront ends only when they have landed)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    run_sum += __shfl_xor(run_sum, 16, 64);
-    run_sum += __shfl_xor(run_sum, 32, 64);
-    if (!pair_valid) return;
-    if (slots.first >= 0) {
-        const size_t base = ((size_t)(slots.first + wave * slots.stride) * heads + head_index) * 16 + col;
-        float* pa = part_acc + base * D + 4 * quad;
 #pragma unroll
-        for (int c = 0; c < ND; ++c) *reinterpret_cast<f32x4*>(pa + 16 * c) = acc[c];
-        if (quad == 0) {
-            part_ml[base * 2] = run_max == NEG_INF ? NEG_INF : run_max * g.scale;
-            part_ml[base * 2 + 1] = run_sum;
+    for (int u = 0; u < SUB; ++u) {
+        float total = run_sum[u];
+        total += __shfl_xor(total, 16, 64);
+        total += __shfl_xor(total, 32, 64);
+        if (!pair_valid[u]) continue;
+        if (slots.first >= 0) {
+            const size_t base = ((size_t)(slots.first + (wave * SUB + u) * slots.stride) * heads + head_index) * 16 + col;
+            float* pa = part_acc + base * D + 4 * quad;
+#pragma unroll
+            for (int c = 0; c < ND; ++c) *reinterpret_cast<f32x4*>(pa + 16 * c) = acc[u][c];
+            if (quad == 0) {
+                part_ml[base * 2] = run_max[u] == NEG_INF ? NEG_INF : run_max[u] * g.scale;
+                part_ml[base * 2 + 1] = total;
+            }
+            continue;
         }
-        return;
-    }
-    const size_t token = (size_t)(row_start[row] + q0 + pair_token);
-    const float inv = inverse_of_sum(run_sum, run_max == NEG_INF ? NEG_INF : run_max * g.scale, g.sinks, head) * gate_of(g, token, head);
-    elem_t* o = out + (token * g.n_q + head) * D + 4 * quad;
+        const size_t token = (size_t)(row_start[row] + q0 + u * g.tokens_per_tile + pair_token);
+        const float inv = inverse_of_sum(total, run_max[u] == NEG_INF ? NEG_INF : run_max[u] * g.scale, g.sinks, head) * gate_of(g, token, head);
+        elem_t* o = out + (token * g.n_q + head) * D + 4 * quad;
 #pragma unroll
-    for (int c = 0; c < ND; ++c) {
-        bf16x4 r4;
+        for (int c = 0; c < ND; ++c) {
+            bf16x4 r4;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) r4[r] = (bf16_t)(acc[c][r] * inv);
-        *reinterpret_cast<bf16x4*>(o + 16 * c) = r4;
+            for (int r = 0; r < 4; ++r) r4[r] = (bf16_t)(acc[u][c][r] * inv);
+            *reinterpret_cast<bf16x4*>(o + 16 * c) = r4;
+        }
     }
 }
-#include "attention_portions.hpp"
 #else  // float32
 // ------------------------------------------------------------------------------------------------
 // Portions of prompts in float32: the same arrangement as the bfloat16 kernel above in its plainest form.  The four
@@ -1474,27 +1531,19 @@ LSA_EXPORT int lsa_paged_attention(
     if (n_tiles > 0) {
 #if LSA_BF16
         // The plan's entries of `tiles` span what a workgroup takes: 4 or 8 tiles.  A load brings 8 keys of a value row.
-        if (tiles_per_workgroup != 4 && tiles_per_workgroup != PORTION_TILES) return -1;
+        if (tiles_per_workgroup != 4 && tiles_per_workgroup != 4 * MAX_SUB) return -1;
         if (page_size % 8 != 0) return -1;
         dim3 tgrid(n_tiles * n_kv * gtiles);
         if (tile_halves != 1 && tile_halves != MAX_HALVES) return -1;
-#define LSA_LAUNCH_TILES(HALVES) do { if (slopes != nullptr) LSA_LAUNCH_TILES_OF(HALVES, true); else LSA_LAUNCH_TILES_OF(HALVES, false); } while (0)
-#define LSA_LAUNCH_TILES_OF(HALVES, BIAS) paged_attention_tile_kernel<HALVES, BIAS><<<tgrid, 256 * HALVES, 0, stream>>>( \
+#define LSA_LAUNCH_TILES(SUB, HALVES) do { if (slopes != nullptr) LSA_LAUNCH_TILES_OF(SUB, HALVES, true); else LSA_LAUNCH_TILES_OF(SUB, HALVES, false); } while (0)
+#define LSA_LAUNCH_TILES_OF(SUB, HALVES, BIAS) paged_attention_tile_kernel<SUB, HALVES, BIAS><<<tgrid, 256 * HALVES, 0, stream>>>( \
                 (const elem_t*)q, q_token_stride, (elem_t*)out, (const elem_t*)keys, (const elem_t*)values, table, table_stride, \
                 row_start, row_len, row_ctx, (const Item*)tiles, (const TileSlots*)tile_slots, part_acc, part_ml, g)
         if (tile_slots != nullptr && (part_acc == nullptr || part_ml == nullptr || n_merges <= 0)) return -1;
-        if (tiles_per_workgroup == 4 && tile_halves == 1) LSA_LAUNCH_TILES(1);
-        else if (tiles_per_workgroup == 4) LSA_LAUNCH_TILES(MAX_HALVES);
-#define LSA_LAUNCH_PORTIONS_OF(HALVES, BIAS, PAGES) paged_attention_portion_kernel<HALVES, BIAS, PAGES><<<tgrid, 256 * HALVES, 0, stream>>>( \
-                (const elem_t*)q, q_token_stride, (elem_t*)out, (const elem_t*)keys, (const elem_t*)values, table, table_stride, \
-                row_start, row_len, row_ctx, (const Item*)tiles, (const TileSlots*)tile_slots, part_acc, part_ml, g)
-#define LSA_LAUNCH_PORTIONS(HALVES, BIAS) do { if (page_size % 16 == 0) LSA_LAUNCH_PORTIONS_OF(HALVES, BIAS, true); else LSA_LAUNCH_PORTIONS_OF(HALVES, BIAS, false); } while (0)
-        else if (tile_halves == 1 && slopes != nullptr) LSA_LAUNCH_PORTIONS(1, true);
-        else if (tile_halves == 1) LSA_LAUNCH_PORTIONS(1, false);
-        else if (slopes != nullptr) LSA_LAUNCH_PORTIONS(MAX_HALVES, true);
-        else LSA_LAUNCH_PORTIONS(MAX_HALVES, false);
-#undef LSA_LAUNCH_PORTIONS_OF
-#undef LSA_LAUNCH_PORTIONS
+        if (tiles_per_workgroup == 4 && tile_halves == 1) LSA_LAUNCH_TILES(1, 1);
+        else if (tiles_per_workgroup == 4) LSA_LAUNCH_TILES(1, MAX_HALVES);
+        else if (tile_halves == 1) LSA_LAUNCH_TILES(MAX_SUB, 1);
+        else LSA_LAUNCH_TILES(MAX_SUB, MAX_HALVES);
 #undef LSA_LAUNCH_TILES
 #undef LSA_LAUNCH_TILES_OF
         const int terr = (int)hipGetLastError();
@@ -1563,7 +1612,7 @@ LSA_EXPORT int lsa_paged_attention(
 LSA_EXPORT int lsa_attention_tile_page_multiple() { return LSA_BF16 ? 8 : 4; }
 LSA_EXPORT int lsa_attention_workgroup_tiles() {
 #if LSA_BF16
-    return PORTION_TILES;
+    return 4 * MAX_SUB;
 #else
     return 4;
 #endif

@@ -18,6 +18,7 @@ __device__ __forceinline__ void load_16_bytes_a_lane_to_lds(const void* source, 
 __device__ __forceinline__ void load_16_bytes_a_lane_to_lds(const void* base, unsigned offset, unsigned lds_address) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_address) : "memory", "m0");
 }
+
 // Waits until at most PENDING of this wavefront's loads are still under way (they land in the order they were
 // issued), then for the workgroup.  Written out because __syncthreads() would wait for every load, also for those
 // of the steps ahead, which are meant to stay in flight across the barrier.

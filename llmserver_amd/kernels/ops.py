@@ -125,12 +125,9 @@ class HipOps(KernelNamespace):
     # key they load but start later, two halves shorten the longest workgroup's walk but make every step dearer).  A GPU
     # that is not listed plans with the attention part's neutral costs; other head sizes scale the trips and steps by
     # head size / 128 (loads and products of a step grow with the head; untuned beyond that).
-    TILE_COSTS = {"gfx950-256cu": (((False, 1), TileLaunchCost(3.2, 0.89, 1.55)), ((True, 1), TileLaunchCost(7.5, 0.645, 1.93)),
-                                   ((False, 2), TileLaunchCost(3.3, 1.11, 2.08)), ((True, 2), TileLaunchCost(10.0, 0.92, 2.10)))}
+    TILE_COSTS = {"gfx950-256cu": (((False, 1), TileLaunchCost(3.2, 0.89, 1.55)), ((True, 1), TileLaunchCost(8.7, 0.94, 2.45)),
+                                   ((False, 2), TileLaunchCost(3.3, 1.11, 2.08)), ((True, 2), TileLaunchCost(8.8, 1.44, 2.84)))}
     TILE_COSTS_HEAD_DIM = 128
-    # Eight tiles to a workgroup of heads beyond 128 dimensions: one workgroup fills a compute unit's registers, and a step of all of them costs accordingly
-    # (us, four and eight tiles: 16 heads on 4 of 256, 2,048 tokens 124 and 105; 32 of 192, windows of 1,024, 334 to 1,000 tokens 62 and 73).
-    WIDE_TILE_COSTS = {"gfx950-256cu": {(True, 1): TileLaunchCost(9.0, 0.85, 3.9)}}
 
     @property
     def attention_tuning(self) -> AttentionTuning:
@@ -149,13 +146,8 @@ class HipOps(KernelNamespace):
             costs = self.TILE_COSTS.get(self.device_kind)
             if costs is not None:
                 scale = head_dim / self.TILE_COSTS_HEAD_DIM
-                if scale > 1:
-                    costs = tuple({**dict(costs), **self.WIDE_TILE_COSTS.get(self.device_kind, {})}.items())
                 costs = tuple((form, TileLaunchCost(cost.start_us, cost.trip_us * scale, cost.step_ns * scale)) for form, cost in costs)
-                # (a partial result's way is half as dear as the neutral costs have it: four rows of 256 tokens behind 3,840, 16 heads on 8 of 128, 71 us by 8 ns, 58 by 4; two of 333 behind 6,000,
-                # 32 on 8, 99 and 113; 99 portions and prompts together are 1.22 times as fast as with the kernel before, by 6 ns as by 4, two of them slower: 400 tokens behind 8,600, 16 on 8, 78, 81;
-                # three rows of 200 behind 5,000 67, 69)
-                tuning = dataclasses.replace(tuning, tile_costs=costs, slot_ns=4.0)
+                tuning = dataclasses.replace(tuning, tile_costs=costs)
             self._tunings[key] = tuning
         return self._tunings[key]
 

@@ -324,43 +324,38 @@ def _single_token_plan(row_ctx: np.ndarray, window: Optional[int], splits: int, 
 
 FIXED_WORKGROUP_TILES = 4          # tiles a workgroup of the prompt-portion kernel takes in captured steps
 FIXED_WORKGROUPS = 1024            # workgroups that such a launch's key ranges aim at
-# ... if they take more tiles than that, in two halves of their keys: one on every compute unit.  us a launch with its merge, four tiles at their best and eight in two halves: 16 heads on 8 of 128, 190 tokens behind
-# 8,064 keys 38 to 51 by their ranges, 34, 400 behind 8,600 70, 53; 32 on 8, 250 behind 3,750 48, 39, 64 behind 7,936 36, 34.
-FIXED_LARGE_WORKGROUPS = 256
 FIXED_KEYS_A_RANGE = 256           # fewest keys of a range at the longest context that the captured step serves
 
 
-def fixed_workgroup_shape(n_tokens: int, n_rows: int, group_size: int, n_kv_heads: int, max_keys: int, tuning: AttentionTuning,
-                          per_workgroup: int = FIXED_WORKGROUP_TILES):
+def fixed_workgroup_shape(n_tokens: int, n_rows: int, group_size: int, n_kv_heads: int, max_keys: int, tuning: AttentionTuning):
     """(groups of tiles, key ranges each) that a captured step of ``n_tokens`` tokens in ``n_rows`` rows, a query of which sees up to ``max_keys``
     keys, runs the prompt-portion kernel with, or None where the wavefront-per-tile kernel is the better one.  Its items read the
     keys once for every tile of 16 (token, head) pairs, these workgroups once for four tiles: from 16 tiles behind 2,048 keys on that is
     what counts (eight layers, 16 heads over 8 of 128, a step of 190 tokens behind 8,064: 1,804 us as items, 1,388 so; behind 2,000: 1,256
-    and 1,141; 60 tokens behind 4,000, 8 tiles, which stay items: 925).  ``per_workgroup``: tiles a workgroup takes, four or, where the kernel has them in two halves, eight."""
+    and 1,141; 60 tokens behind 4,000, 8 tiles, which stay items: 925)."""
     _, tokens_per_tile, group_tiles = group_tiling(group_size, tuning.tile_rows)
     if n_tokens // tokens_per_tile < MIN_TILES_FOR_WORKGROUPS or max_keys < 2048:
         return None
-    groups = n_tokens // (per_workgroup * tokens_per_tile) + n_rows
-    workgroups = FIXED_WORKGROUPS if per_workgroup == FIXED_WORKGROUP_TILES else FIXED_LARGE_WORKGROUPS
-    return groups, max(1, min(tuning.most_splits, workgroups // (groups * n_kv_heads * group_tiles), max_keys // FIXED_KEYS_A_RANGE))
+    groups = n_tokens // (FIXED_WORKGROUP_TILES * tokens_per_tile) + n_rows
+    return groups, max(1, min(tuning.most_splits, FIXED_WORKGROUPS // (groups * n_kv_heads * group_tiles), max_keys // FIXED_KEYS_A_RANGE))
 
 
 def fixed_workgroup_plan(row_len, row_ctx, group_size: int, window: Optional[int], chunk: Optional[int], groups: int, ranges: int, n_tiles: int,
-                         tuning: AttentionTuning, per_workgroup: int = FIXED_WORKGROUP_TILES, halves: int = 1) -> AttentionPlan:
-    """All rows' tiles in workgroups of ``per_workgroup``, the keys of each cut into exactly ``ranges`` ranges (the last ones may be empty), filled up to
+                         tuning: AttentionTuning) -> AttentionPlan:
+    """All rows' tiles in workgroups of four, the keys of each cut into exactly ``ranges`` ranges (the last ones may be empty), filled up to
     ``groups`` workgroups' entries and ``n_tiles`` merges with repetitions of the first one's, which compute and write the same numbers
     once more: arrays of one shape whatever the rows' lengths and contexts are."""
     _, tokens_per_tile, _ = group_tiling(group_size, tuning.tile_rows)
     row_len, row_ctx = np.asarray(row_len, dtype=np.int64), np.asarray(row_ctx, dtype=np.int64)
     of_row, starts, k_begin, k_end, tiles_of_group = _workgroups_of_rows(np.flatnonzero(row_len > 0), row_len, row_ctx, tokens_per_tile, window,
-                                                                         per_workgroup, chunk)
+                                                                         FIXED_WORKGROUP_TILES, chunk)
     real = len(starts)
     if not 1 <= real <= groups or int(tiles_of_group.sum()) > n_tiles:
         raise ValueError(f"the step's rows make {real} groups of tiles, the shape they are filled up to holds {groups}")
     aligned = (k_begin // tuning.key_align) * tuning.key_align
     per = -(-(k_end - aligned) // ranges)
     per = np.maximum(-(-per // tuning.key_align) * tuning.key_align, 1)
-    first = np.arange(real) * per_workgroup * ranges          # a group's slots: range s of its tile j at first + j * ranges + s
+    first = np.arange(real) * FIXED_WORKGROUP_TILES * ranges          # a group's slots: range s of its tile j at first + j * ranges + s
     group, s = np.repeat(np.arange(real), ranges), np.tile(np.arange(ranges), real)
     begin = np.minimum(np.maximum(k_begin[group], aligned[group] + s * per[group]), k_end[group])
     end = np.maximum(begin, np.minimum(aligned[group] + (s + 1) * per[group], k_end[group]))
@@ -371,8 +366,8 @@ def fixed_workgroup_plan(row_len, row_ctx, group_size: int, window: Optional[int
     merges = np.stack([of_row[group], starts[group] + j * tokens_per_tile, first[group] + j * ranges, np.full(len(group), ranges)], axis=1)
     merges = np.concatenate([merges, np.tile(merges[:1], (n_tiles - len(group), 1))]).astype(np.int32)
     tiles = tiles[np.argsort(tiles[:, 2] - tiles[:, 3], kind="stable")].astype(np.int32)          # most keys first
-    plan = AttentionPlan(np.zeros((0, 4), np.int32), np.zeros((0,), np.int32), merges, groups * per_workgroup * ranges,
-                         np.ascontiguousarray(tiles[:, :4]), per_workgroup, halves, np.ascontiguousarray(tiles[:, 4:]))
+    plan = AttentionPlan(np.zeros((0, 4), np.int32), np.zeros((0,), np.int32), merges, groups * FIXED_WORKGROUP_TILES * ranges,
+                         np.ascontiguousarray(tiles[:, :4]), FIXED_WORKGROUP_TILES, 1, np.ascontiguousarray(tiles[:, 4:]))
     plan.merge_in_workgroup = 0
     return plan
 
@@ -580,10 +575,9 @@ def stage_attention_plan(ctx, key, group_size: int, n_kv_heads: int, head_dim: i
     shape = None
     if fixed_tiles is not None and not in_workgroup and per_workgroup and key_ranges > 1:
         seen = min([ctx.static_max_keys] + [limit for limit in (window, chunk) if limit is not None])
-        form = (per_workgroup, halves) if per_workgroup > FIXED_WORKGROUP_TILES and halves > 1 else (FIXED_WORKGROUP_TILES, 1)
-        shape = fixed_workgroup_shape(ctx.n_tokens, ctx.n_rows, group_size, n_kv_heads, seen, tuning, form[0])
+        shape = fixed_workgroup_shape(ctx.n_tokens, ctx.n_rows, group_size, n_kv_heads, seen, tuning)
     if shape is not None:
-        plan = fixed_workgroup_plan(ctx.h_row_len, ctx.h_row_ctx, group_size, window, chunk, *shape, fixed_tiles, tuning, *form)
+        plan = fixed_workgroup_plan(ctx.h_row_len, ctx.h_row_ctx, group_size, window, chunk, *shape, fixed_tiles, tuning)
     else:
         plan = build_attention_plan(ctx.h_row_len, ctx.h_row_ctx, group_size, n_kv_heads, window,
                                     target_waves=tuning.target_waves, fixed_splits=fixed, workgroup_tiles=per_workgroup,
