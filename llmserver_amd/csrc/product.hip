@@ -201,15 +201,15 @@ static const TileShape SHAPES[] = {{0, 0, 0, 0, 0, 0, 0, 0}, {64, 64, 3.94, 0.2,
                                    {128, 128, 4.41, 0.375, 0.28, 0.08, 0.06, 4.5}, {256, 256, 0, 0, 0, 0, 0, 0}};
 constexpr int UNITS = 256;                                         // compute units
 // SMALL's tiles are 64 x 32 where that many still go round the compute units once.  A slab takes as long as its bytes do on the way from L2 into a compute unit, some 30 a cycle, next to what
-// the weights' way takes: half the columns are a quarter less, and twice as many units pull the weights.  us, 64 x 64 and 64 x 32: 33 rows of 6,144 x 4,096 19.6, 15.3 (the library 17.9), of
-// 4,096 x 2,048 10.6, 8.7, of 3,072 x 1,024 6.7, 5.8; 17 rows of 8,192 x 4,096 (256 tiles) 19.1, 16.3; 128 rows of 4,096 x 2,048 12.0, 10.2; 48 rows of 5,120 x 2,560 16.6, 12.6; sums of 33 rows of
-// 4,096 x 8,192 in two parts 20.9, 16.9.  Beyond one round they lose: 33 rows of 10,240 x 5,120 (320) 31.0, 35.3; 96 rows of 6,144 x 2,048 (384) 11.4, 16.2.  Two or four slabs a barrier, fewer or
-// more buffers, or another first slab for each workgroup change nothing.  The prices are a fit to 292 sizes (within 6 %) and a tenth more, so that nothing goes from parts to one launch for the
-// fit's error (64 rows of 3,840 x 2,560 12.4 in two parts, 13.6 so).
-static const TileShape SLIM = {64, 32, 3.3, 0.125, 0.11, 0.022, 0.055, 4.5};
-static bool slim_tiles(int form, int M, int N, int parts) {
-    const int columns = form == GATED ? SLIM.columns / 2 : SLIM.columns;
-    return (long)((M + SLIM.rows - 1) / SLIM.rows) * ((N + columns - 1) / columns) * parts <= UNITS;
+// the weights' way takes: half the columns are a quarter less, and twice as many units pull the weights.  us, 64 x 64 and 64 x 32, the weights from memory: 33 rows of 3,840 x 2,560 activated
+// 16.2, 11.2, gated 15.9, 11.8; 128 of 4,096 x 2,048 activated 13.6, 10.8; 190 of 1,024 x 3,072 gated 16.5, 12.8; 190 of 1,408 x 2,048 9.5, 9.2; 17 of 2,048 x 1,024 in four parts 3.7, 3.8.  119 sizes
+// of 17 to 250 rows that the plan has them for are 1.20 times as fast.  Beyond one round they lose: 33 rows of 10,240 x 5,120 (320) 31.0, 35.3; 96 rows of 6,144 x 2,048 (384) 11.4, 16.2.
+//   Both add up the same products in the same order, so that their results are the same bits.  Those of parts and of the library need not be, and the plan, which decides between them, goes on
+// pricing 64 x 64: what it takes ends sooner than it says.  By a price of 64 x 32 it took more from both, a little faster each alone (gated 32 rows of 2,816 x 4,096 in parts 15.4, 14.3; 33 rows
+// of 6,144 x 4,096 within a step 17.2 by the library, 15.6) and not in a job: 33 requests decoding, eight layers and eight steps, 9,100 and 9,232.
+static int small_columns(int form, int M, int N, int parts) {
+    const int slim = form == GATED ? 16 : 32;
+    return (long)((M + 63) / 64) * ((N + slim - 1) / slim) * parts <= UNITS ? slim : 2 * slim;
 }
 constexpr int MOST_PARTS = 8, ADDED = 1 << 12;
 
@@ -225,7 +225,8 @@ static bool fits(int form, long M, long N, long K) {
 // rows of 6,144 x 2,048 24.8, 17.4 here), its price is too low, and sizes that the tiles would make faster stay with it.  At 70 other numbers of rows 1,923 of 4,094 sizes are taken, up to
 // 128 rows and beyond: gated 1.18 and 1.20 times as fast as the other way, plain 1.24 and 1.20, activated 1.25 and 1.23, sums with the norm behind them 1.13 and 1.16, heads 1.08 and none.
 // Seventeen of them are slower than 0.97 of it: 95 rows of 2,560 x 4,096 0.93, 63 of 4,096 x 3,072 0.94, 320 to 448 of 64 x 2,048 0.95, 30 of 2,112 x 2,048 activated 0.97; sums at 531
-// and 545 rows of 2,048 x 2,048 0.93 and 0.95, 232 of 2,560 x 9,728 0.94, 127 of 5,120 x 17,408 0.96, 35 of 4,096 x 8,192 and 255 of 4,096 x 12,288 0.97.  A product whose tiles
+// and 545 rows of 2,048 x 2,048 0.93 and 0.95, 232 of 2,560 x 9,728 0.94, 127 of 5,120 x 17,408 0.96, 35 of 4,096 x 8,192 and 255 of 4,096 x 12,288 0.97 (counted with tiles of 64 x 64
+// everywhere, before any of 64 x 32 ran).  A product whose tiles
 // do not go round the compute units in one round stays the
 // library's unless it is gated and large.  Up to 128 rows the parts may be added up by a launch of their own (64 rows, 2,816 x 2,048 library 12.1, one launch 12.2, so 9.7; 32
 // rows of 4,096 x 4,096 13.9, 17.9, 12.0; gated 2,816 x 4,096 15.4, 18.4, 12.2).
@@ -236,19 +237,14 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     // 19.2, 1,330 and 1,980 of 1,024 x 3,072 25.1 and 27.9, 24.0 and 28.3)
     if (form == SUMS && M > FEW_ROWS && (N < 1024 || M > 1100 || (M > 2 * FEW_ROWS && K < 2048))) return NONE;
     const double slabs = K / SLAB, weights = (form == GATED ? 2.0 : 1.0) * N, megabytes = weights * K * 2e-6, gigaflops = 2e-9 * M * weights * K;
-    // (Priced are tiles of 64 x 32 where they win.  Behind 64 rows and 2,048 of K parts or the library's ranges of K do as well: 128 rows of 2,048 x 4,096 15.7, the library 12.8, 192 of 1,024 x
-    // 3,072 9.8, 8.8, 128 of 2,560 x 4,096 16.3, in parts 15.7; so they do with weights of more than 50 MB up to 32 rows, 32 of 4,096 x 8,192 17.6 for the library and 25 so.  Sums keep the parts
-    // they had, and plain products of up to 64 rows and 2,048 columns who has them.)
-    const bool priced_slim = form != SUMS && !(form == PLAIN && M <= 64 && N <= 2048) && !(form == PLAIN && M <= 32 && weights * K > 2.6e7) && !(M > 64 && K > 2048);
-    double best = 1e30, parts_and_activation = 1e30;               // (activated: the plain product in parts, the kernel that adds them up and the activation's)
+    double best = 1e30;
     int plan = NONE;
     for (int tile = SMALL; tile <= LARGE; ++tile) {
-        const bool added = form != SUMS && M <= FEW_ROWS;
+        const TileShape& shape = SHAPES[tile];
+        const int columns = form == GATED ? shape.columns / 2 : shape.columns;
+        const long tiles = (long)((M + shape.rows - 1) / shape.rows) * ((N + columns - 1) / columns);
+        const bool added = (form == PLAIN || form == GATED) && M <= FEW_ROWS;
         for (int parts = 1; parts <= (form == SUMS || added ? MOST_PARTS : 1); parts *= 2) {
-            const bool slim = tile == SMALL && priced_slim && parts == 1 && slim_tiles(form, M, N, parts);
-            const TileShape& shape = slim ? SLIM : SHAPES[tile];
-            const int columns = form == GATED ? shape.columns / 2 : shape.columns;
-            const long tiles = (long)((M + shape.rows - 1) / shape.rows) * ((N + columns - 1) / columns);
             // (the sums take the tile's 64 or 128 rows of W whatever they are: gated, half as many tiles)
             // (two of the small tiles' workgroups fit a compute unit: where the weights' way bounds them, 33 rows of 32,768 x 4,096 63 us for the library, 55; gated products
             // beyond one round, and with less than 1,024 of K, stay with the kernel that shares the activations, or the library)
@@ -263,10 +259,6 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
             us = us > way ? us : way;
             if (form == SUMS) us += parts * 1.7e-6 * M * N;        // written and read
             else if (parts > 1) us += 2.2 + parts * 2.0e-6 * M * weights;      // and a launch
-            if (form == ACTIVATED && parts > 1) {                  // (there the other way is the plain product's parts and the activation's kernel: 40 rows of 2,560 x 4,096 13.0, 14.7 in one launch)
-                parts_and_activation = us + 2.0 < parts_and_activation ? us + 2.0 : parts_and_activation;
-                continue;
-            }
             if (us < best) {
                 best = us;
                 plan = 16 * parts + tile + (form != SUMS && parts > 1 ? ADDED : 0);
@@ -299,7 +291,6 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
     // (a weight of more than 50 MB in parts: the library cuts K up to 32 rows and not beyond: 18, 28, 34 and 44 rows of 4,096 x 8,192 17.6, 18.6, 22.9 and 23.0, here 19.9, 20.1, 20.2
     // and 20.6; 2,048 x 8,448, at 18 rows 27.2, here 11.5, and 4,096 x 4,096, 13.3 and 11.1, lie before that)
     if (form == PLAIN && (plan & ADDED) && M <= 32 && weights * K > 2.6e7) return NONE;
-    if (form == ACTIVATED && best > parts_and_activation) return NONE;
     // How far the lines are trusted: up to 128 rows the library takes longer than its line nearly everywhere, and a gated product's (with the activation) at any number of rows.
     static const double MARGINS[4][2] = {{1.22, 0.95}, {1.1, 1.1}, {0.87, 0.92}, {0, 0.94}};
     return best < (plan & ADDED ? 0.92 : MARGINS[form][M > FEW_ROWS]) * library ? plan : NONE;
@@ -307,13 +298,12 @@ LSA_EXPORT int lsa_product_plan(int form, int M, int N, int K) {
 
 template <int FORM>
 static int launch(int tile, int parts, const bf16_t* x, const bf16_t* w, void* out, int M, int N, int K, int activation, hipStream_t stream) {
-    const int columns = FORM == GATED ? SHAPES[tile].columns / 2 : SHAPES[tile].columns, blocks = workgroups(M, N, SHAPES[tile].rows, columns);
+    const int columns = tile == SMALL ? small_columns(FORM, M, N, parts) : FORM == GATED ? SHAPES[tile].columns / 2 : SHAPES[tile].columns;
+    const int blocks = workgroups(M, N, SHAPES[tile].rows, columns);
     if (blocks < 0) return -1;
     const dim3 grid(blocks, parts);
-    if (tile == SMALL && slim_tiles(FORM, M, N, parts)) {
-        const int slim_columns = FORM == GATED ? SLIM.columns / 2 : SLIM.columns;
-        product_kernel<4, 1, 1, 10, FORM><<<dim3(workgroups(M, N, SLIM.rows, slim_columns), parts), 256, 0, stream>>>(x, w, out, M, N, K, activation);
-    } else if (tile == SMALL) product_kernel<2, 2, 2, 5, FORM><<<grid, 256, 0, stream>>>(x, w, out, M, N, K, activation);
+    if (tile == SMALL && columns == (FORM == GATED ? 16 : 32)) product_kernel<4, 1, 1, 10, FORM><<<grid, 256, 0, stream>>>(x, w, out, M, N, K, activation);
+    else if (tile == SMALL) product_kernel<2, 2, 2, 5, FORM><<<grid, 256, 0, stream>>>(x, w, out, M, N, K, activation);
     else if (tile == TALL) product_kernel<4, 2, 2, 6, FORM><<<grid, 512, 0, stream>>>(x, w, out, M, N, K, activation);
     else product_kernel<2, 4, 4, 4, FORM><<<grid, 512, 0, stream>>>(x, w, out, M, N, K, activation);
     LSA_LAUNCH_CHECK();

@@ -74,6 +74,21 @@ def test_small_tiles_on_both_sides_of_their_line(ops, form, rows, columns, inner
     test_every_tile_at_its_edges(ops, form, 1, rows, columns, inner)
 
 
+@pytest.mark.parametrize("form,columns", [("plain", 8192), ("gated", 4096), ("activated", 8192), ("sums", 4096)])
+def test_both_small_tiles_give_the_same_bits(ops, form, columns):
+    """Sixty-four rows, the most columns that tiles of 64 x 32 take (sums: in two parts) and eight more, which tiles of 64 x 64 take: the columns of both are the same numbers."""
+    rows, inner, parts = 64, 704, 2 if form == "sums" else 1
+    x, weight = drawn(rows, (columns + 8) * (2 if form == "gated" else 1), inner, 11)
+    fewer = torch.cat([weight[:columns], weight[columns + 8:2 * columns + 8]]) if form == "gated" else weight[:columns].contiguous()
+    results = []
+    for count, w in ((columns + 8, weight), (columns, fewer)):
+        print(f"small tiles {form} {count}", flush=True)
+        out = torch.full((parts, rows, count), float("nan"), device="cuda", dtype=torch.float32 if form == "sums" else torch.bfloat16)
+        assert ops._product.lsa_product(16 * parts + 1, FORMS.index(form), 0, x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, count, inner, torch.cuda.current_stream().cuda_stream) == 0
+        results.append(out[:, :, :columns])
+    assert not bool(results[0].isnan().any()) and torch.equal(*results)
+
+
 def test_what_does_not_fit_is_refused(ops):
     x, weight = drawn(64, 64, 128, 1)
     out = torch.empty(64, 64, device="cuda", dtype=torch.bfloat16)
