@@ -1140,16 +1140,16 @@ __global__ __launch_bounds__(256, 3) void memory_chunk_read16_kernel(const bf16_
 // What bounds the scan is the chain of a row's tokens (0.45 us a token, on rows * heads * value_dim / 64 workgroups: 918 us for
 // one row of 2,048 tokens, 16 heads of 128 x 128, 1,171 us for 8 heads of 128 x 256, most of the chip idle); here all chunks
 // run at once and only the walk over the chunks (2) is serial.  A workgroup has one (chunk, head, 128 value columns): scores are formed once
-// for all of them, operands stay in LDS (158 KB at 128 channels, so one workgroup a compute unit), products run on 32-bit MFMA but where said.
+// for all of them, operands stay in LDS (146 KB at 128 channels, so one workgroup a compute unit), products run on 32-bit MFMA but where said.
 //   What bounds the first launch is what one compute unit gets through between its barriers, operands from memory and their decays, diagonals, 64-bit products, one
-// after another; sixteen wavefronts hide more of it than eight did: a workgroup takes 25 us instead of 45, of which 5 (9 with sigmoids' roots) the operands, 6 the
-// diagonals, 4 what lies between, 2 what leaves and 7.5 the values' products, both halves of the columns at once.  us with the walk and the read-out, before and now:
-// 2,048 tokens of 16 heads of 128 x 128 132, 119; of 8 heads of 128 x 256 139, 124; 1,024 tokens 106, 92 and 113, 98; 2,048 of 16 heads of 64 x 64 70, 65; six rows of 510
-// tokens together 65, 57.  (3) is no faster with its loads a slab ahead, and with registers for four workgroups a compute unit faster behind 768 of them only (120, 114; 92, 96).
+// after another; sixteen wavefronts hide more of it than eight did.  They share the work so that every sum is formed in the order that eight formed it in (diagonals between two wavefronts, not their
+// channels; a tile's four sums between two), and the results are the same bits.  us with the walk and the read-out, eight wavefronts and sixteen: 2,048 tokens of 16 heads of
+// 128 x 128 125, 110; of 8 heads of 128 x 256 123, 107; 1,024 tokens 102, 86 and 100, 85; 2,048 of 16 heads of 64 x 64 67, 60; six rows of 510 tokens of those 104, 91.  (3) is
+// no faster with its loads a slab ahead, and with registers for four workgroups a compute unit faster behind 768 of them only (120, 114; 92, 96).
 constexpr int CHANNEL_MOST = 128;        // widest head that fits LDS so
 constexpr int CHANNEL_COLUMNS = 128;     // value columns a workgroup
 constexpr int CHANNEL_THREADS = 1024;    // of a workgroup: sixteen wavefronts
-constexpr int CHANNEL_QUARTERS = 4;      // ... of which four share the channels of a block of tokens
+constexpr int CHANNEL_DIAGONALS = 8;     // that a wavefront forms of a block of tokens: two share its sixteen, for each half of the channels
 
 template <int DP>
 struct ChannelChunkLds {                 // DP: key channels filled up to 64 or 128
@@ -1161,10 +1161,11 @@ struct ChannelChunkLds {                 // DP: key channels filled up to 64 or 
     float score[MC * MC_A];
     double total[MC / BC][DP];
     union {
-        double diagonal[CHANNEL_QUARTERS][BC][MC];                                 // sums of a quarter of the channels: [tokens back][token]
-        double between[6][64][4];                                                  // ... of half of them, as a wavefront's lanes hold a tile
+        double diagonal[2][BC][MC];                                                // sums of a half of the channels: [tokens back][token]
+        double between[6][64][4];                                                  // ... of every second four of them, as a wavefront's lanes hold a tile
         float v[MC * MC_B];                                                        // the values of the second 64 columns
     };
+    int no_number[2];                                                              // one once a value of the first or the second 64 columns is none
 };
 
 // (1) out = the chunks' own read-outs, sums [item][head][dim][value_dim] and totals [item][head][dim] as the walk wants them,
@@ -1212,24 +1213,33 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunk_kernel(const T*
             s.d[t * A + c] = there ? decay_of(raw_z[e], mode, inv_tau) : 1.f;
         }
         for (int i = tid; i < MC * MC_A; i += CHANNEL_THREADS) s.score[i] = 0.f;
+        if (tid < 2) s.no_number[tid] = 0;
     }
     __syncthreads();
 
-    // Inside the blocks: wavefront = (block, quarter of the channels), lane = (token t of the block, a quarter of every 16 channels).  The
-    // diagonals j = t - back one after another, the query times its decays so far in registers.
+    // Inside the blocks: wavefront = (block, half of the channels, half of the diagonals), lane = (token t of the block, a quarter of every 16 channels).
+    // The diagonals j = t - back one after another, the query times its decays so far in registers (the later half of them begins behind the earlier one's decays).
     {
-        const int block = wave / CHANNEL_QUARTERS, quarter = wave % CHANNEL_QUARTERS, t = lane & 15, c0 = quarter * (DP / CHANNEL_QUARTERS) + 4 * (lane >> 4);
-        constexpr int U = DP / (16 * CHANNEL_QUARTERS);
+        const int block = wave >> 2, half = (wave >> 1) & 1, first = CHANNEL_DIAGONALS * (wave & 1), t = lane & 15, c0 = half * (DP / 2) + 4 * (lane >> 4);
+        constexpr int U = DP / 32;
         float weighted[U][4];
-        double sum[BC];                                                            // (their last additions would be the score's largest roundings)
+        double sum[CHANNEL_DIAGONALS];                                             // (their last additions would be the score's largest roundings)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const float4 x = *reinterpret_cast<const float4*>(&s.q[(block * BC + t) * A + c0 + 16 * u]);
             weighted[u][0] = x.x; weighted[u][1] = x.y; weighted[u][2] = x.z; weighted[u][3] = x.w;
         }
-#pragma unroll
-        for (int back = 0; back < BC; ++back) {
+        for (int back = bonus == nullptr ? 0 : 1; back < first; ++back) {
             const int j = block * BC + max(t - back, 0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float4 f = *reinterpret_cast<const float4*>(&s.d[j * A + c0 + 16 * u]);
+                weighted[u][0] *= f.x; weighted[u][1] *= f.y; weighted[u][2] *= f.z; weighted[u][3] *= f.w;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < CHANNEL_DIAGONALS; ++i) {
+            const int back = first + i, j = block * BC + max(t - back, 0);
             float part[4] = {};
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -1239,34 +1249,33 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunk_kernel(const T*
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     float own = weighted[u][e];
-                    if (bonus != nullptr && back == 0) {
+                    if (i == 0 && bonus != nullptr && back == 0) {
                         const int c = c0 + 16 * u + e;
                         own *= bonus[key_column + min(c, dim - 1)];               // (channels behind the head's last one: q is 0)
                     }
                     part[e] = __builtin_fmaf(own, ks[e], part[e]);
-                    if (bonus == nullptr || back > 0) weighted[u][e] *= ds[e];     // (the next diagonal lies behind token j's decay)
+                    if (i > 0 || bonus == nullptr || back > 0) weighted[u][e] *= ds[e];     // (the next diagonal lies behind token j's decay)
                 }
             }
-            sum[back] = ((double)part[0] + (double)part[1]) + ((double)part[2] + (double)part[3]);
+            sum[i] = ((double)part[0] + (double)part[1]) + ((double)part[2] + (double)part[3]);
         }
-        // (added up over the four lanes of a token, each of which ends with four of the diagonals)
+        // (added up over the four lanes of a token, neighbours first, each of which ends with two of the diagonals)
         const bool upper = lane & 32, odd = lane & 16;
 #pragma unroll
-        for (int back = 0; back < BC / 2; ++back) {
-            const double other = __shfl_xor(upper ? sum[back] : sum[BC / 2 + back], 32, 64);
-            sum[back] = (upper ? sum[BC / 2 + back] : sum[back]) + other;
+        for (int i = 0; i < CHANNEL_DIAGONALS / 2; ++i) {
+            const double other = __shfl_xor(odd ? sum[i] : sum[CHANNEL_DIAGONALS / 2 + i], 16, 64);
+            sum[i] = (odd ? sum[CHANNEL_DIAGONALS / 2 + i] : sum[i]) + other;
         }
 #pragma unroll
-        for (int back = 0; back < BC / 4; ++back) {
-            const double other = __shfl_xor(odd ? sum[back] : sum[BC / 4 + back], 16, 64);
-            s.diagonal[quarter][(upper ? BC / 2 : 0) + (odd ? BC / 4 : 0) + back][block * BC + t] = (odd ? sum[BC / 4 + back] : sum[back]) + other;
+        for (int i = 0; i < CHANNEL_DIAGONALS / 4; ++i) {
+            const double other = __shfl_xor(upper ? sum[i] : sum[CHANNEL_DIAGONALS / 4 + i], 32, 64);
+            s.diagonal[half][first + (odd ? CHANNEL_DIAGONALS / 2 : 0) + (upper ? CHANNEL_DIAGONALS / 4 : 0) + i][block * BC + t] = (upper ? sum[CHANNEL_DIAGONALS / 4 + i] : sum[i]) + other;
         }
     }
     __syncthreads();
     {                                                                              // (a thread one score: BC diagonals of MC tokens)
         const int t = tid % MC, back = tid / MC;
-        if (back <= t % BC)
-            s.score[t * MC_A + t - back] = (float)((s.diagonal[0][back][t] + s.diagonal[1][back][t]) + (s.diagonal[2][back][t] + s.diagonal[3][back][t]));
+        if (back <= t % BC) s.score[t * MC_A + t - back] = (float)((double)(float)(0.0 + s.diagonal[0][back][t]) + s.diagonal[1][back][t]);
     }
 
     // Queries times the decays from their block's first token (one half of the threads), keys times those up to its last one (the other); a thread a (block, channel).
@@ -1302,30 +1311,31 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunk_kernel(const T*
     }
     __syncthreads();
 
-    // Between blocks: six tiles of 16 x 16 scores, two wavefronts a tile, each with half of the channels.
+    // Between blocks: six tiles of 16 x 16 scores, two wavefronts a tile, each with two of the four sums of every fourth channel group that make one.
     {
         const int tile = wave >> 1, half = wave & 1, block = tile < 3 ? 3 : tile < 5 ? 2 : 1, other = tile < 3 ? tile : tile < 5 ? tile - 3 : 0;
         const int r = lane & 15, g = lane >> 4;
         double sum[4] = {};
         if (tile < 6) {
-            const float* a = &s.q[(block * BC + r) * A + g];
-            const float* b = &s.k[(other * BC + r) * A + g];
-            mc_f4 part[4] = {};
-            for (int i = half * (DP / 2); i < (half + 1) * (DP / 2); i += 16) {
-                float x[4], y[4];
+            const float* a = &s.q[(block * BC + r) * A + g + 8 * half];
+            const float* b = &s.k[(other * BC + r) * A + g + 8 * half];
+            mc_f4 part[2] = {};
+            for (int i = 0; i < DP; i += 16) {
+                float x[2], y[2];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
+                for (int u = 0; u < 2; ++u) {
+                    const int c = i + 8 * half + 4 * u + g;
                     y[u] = b[i + 4 * u];
-                    const double next = s.total[other + 1][i + 4 * u + g], after = s.total[min(other + 2, MC / BC - 1)][i + 4 * u + g];
+                    const double next = s.total[other + 1][c], after = s.total[min(other + 2, MC / BC - 1)][c];
                     const double skipped = (block > other + 1 ? next : 1.0) * (block > other + 2 ? after : 1.0);
                     x[u] = (float)((double)a[i + 4 * u] * skipped);
                 }
 #pragma unroll
-                for (int u = 0; u < 4; ++u) part[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[u], part[u], 0, 0, 0);
+                for (int u = 0; u < 2; ++u) part[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[u], part[u], 0, 0, 0);
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                sum[e] = ((double)part[0][e] + (double)part[1][e]) + ((double)part[2][e] + (double)part[3][e]);
+                sum[e] = (double)part[0][e] + (double)part[1][e];
                 if (half == 1) s.between[tile][lane][e] = sum[e];
             }
         }
@@ -1384,7 +1394,9 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunk_kernel(const T*
         s_v[t * MC_B + lane] = value;
         no_number = __builtin_fmaf(value, 0.f, no_number);
     }
-    const bool all_finite = !__syncthreads_or(no_number != 0.f);
+    if (no_number != 0.f) s.no_number[of] = 1;
+    __syncthreads();
+    const bool all_finite = s.no_number[of] == 0;        // (of these 64 columns: what lies in the others does not change how theirs are formed)
     if (column0 < value_dim) {
         const int r = lane & 15, g = lane >> 4, half = wave & 1;
         {

@@ -1749,8 +1749,8 @@ class HipOps(KernelNamespace):
         128 / 256 / 2,048 tokens 28, 51; 46, 51; 52, 52; 99, 54; 904, 129; 4 rows of 128 / 160 / 256 / 512 53, 62; 65, 64; 101, 109; 231, 124; 16 rows of
         64 / 256 / 512 66, 118; 239, 240; 462, 508; 8 rows of 2,048 1,039, 1,000; 512 tokens beside 16 single ones 207, 113; 16 heads of 64 x 64, 1 row of
         64 / 112 / 128 / 2,048 18, 30; 30, 30; 33, 31; 479, 68; 4 rows of 128 34, 33; 8 rows of 512 148, 111; 16 rows of 512 149, 211.
-        (With sixteen wavefronts a workgroup the chunks have become faster: 1 row of 112 / 128 / 256 / 2,048 of 128 x 128 49, 45; 55, 46; 103, 49; 924, 117; 4 rows of 256 105, 96; 16 rows
-        of 512 473, 448; 1 row of 112 of 64 x 64 33, 29.  The line has stayed where it was: steps beside it go as they went.)
+        (With sixteen wavefronts a workgroup, walk and chunks: 1 row of 112 / 128 / 256 / 2,048 of 128 x 128 46, 43; 53, 44; 101, 47; 918, 110; 4 rows of 256 102, 92; 16 rows of
+        512 468, 442; 1 row of 112 of 64 x 64 30, 26.  The line stays where it was: the two round otherwise, and a step that went the other way would give other bits than it did.)
 
         The walk: a row's tokens one after another, as many rounds of them as its workgroups (a head's 64 value columns each) go round 256
         compute units, a token slower where these share what leaves L2 and behind the first thousand.  The chunks: three launches, of which the

@@ -117,6 +117,57 @@ def test_linear_recurrence_in_chunks_at_the_edges_of_value_columns(ops, dtype, h
     test_linear_recurrence_in_chunks(ops, dtype, heads, dim, vdim, "double_exp" if vdim == 100 else "sigmoid_root", 1.0)
 
 
+def in_chunks(ops, q, k, v, decay, heads, dim, vdim):
+    """Read-outs of one row from an empty state, without a bonus and with queries as they are."""
+    n, ints = q.shape[0], lambda x: torch.tensor([x], dtype=torch.int32, device="cuda")
+    out = torch.full((n, heads * vdim), float("nan"), device="cuda")
+    state = torch.zeros(1, heads * dim * vdim, device="cuda")
+    scratch = {"sums": torch.full((n // 64 + 1, heads, dim, vdim), float("nan"), device="cuda"), "totals": torch.full((n // 64 + 1, heads, dim), float("nan"), device="cuda"),
+               "queries": torch.full((n, heads, dim), float("nan"), device="cuda")}
+    ops.linear_recurrence(q, k, v, decay, None, "double_exp", 1.0, None, 1.0, state, 0, ints(0), ints(0), ints(n), ints(n), out, heads, dim, vdim, **scratch)
+    return out, state
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("spoilt", [slice(64, 128), slice(0, 64), slice(128, 200)])
+def test_values_that_are_no_numbers_leave_other_columns_as_they_are(ops, dtype, spoilt):
+    """Whether products run on matrix cores or number by number is decided for 64 value columns, not for all that a workgroup has: the other columns' read-outs and states are the
+    same bits with and without infinities beside them."""
+    generator = torch.Generator("cuda").manual_seed(3)
+    draw = lambda *shape: torch.randn(*shape, device="cuda", generator=generator)
+    n, heads, dim, vdim = 150, 2, 128, 200
+    q, k, v = (0.5 * draw(n, heads * width) for width in (dim, dim, vdim))
+    q, k, v, decay = q.to(dtype), k.to(dtype), v.to(dtype), draw(n, heads * dim) - 1.0
+    print(f"no numbers in columns {spoilt} {dtype}", flush=True)
+    whole, state = in_chunks(ops, q, k, v, decay, heads, dim, vdim)
+    v.view(n, heads, vdim)[70, 1, spoilt] = float("inf")
+    beside, state_beside = in_chunks(ops, q, k, v, decay, heads, dim, vdim)
+    kept = torch.ones(heads, vdim, dtype=torch.bool, device="cuda")
+    kept[1, spoilt] = False
+    assert bool(whole.isfinite().all()) and not bool(beside.view(n, heads, vdim)[70:, 1, spoilt].isfinite().any())
+    assert torch.equal(whole.view(n, heads, vdim)[:, kept], beside.view(n, heads, vdim)[:, kept])
+    kept = kept[:, None].expand(heads, dim, vdim)
+    assert torch.equal(state.view(heads, dim, vdim)[kept], state_beside.view(heads, dim, vdim)[kept])
+
+
+@pytest.mark.parametrize("token", [0, 8, 15, 40])
+def test_scores_meet_in_the_order_of_the_halves_of_the_channels(ops, token):
+    """A score inside a block of tokens is the first half's sum, rounded, and the second half's: 2^24 + 1 and 1 are 2^24 then, however many wavefronts share the channels and the tokens
+    back.  The token at `token` reads the one at the start of its block, with nothing lost on the way."""
+    n, heads, dim, vdim = 64, 1, 128, 64
+    q, k, v = (torch.zeros(n, width, device="cuda") for width in (dim, dim, vdim))
+    source = token // 16 * 16
+    q[token, 0], k[source, 0] = 2.0 ** 12, 2.0 ** 12
+    q[token, 1], k[source, 1] = 1.0, 1.0
+    q[token, 64], k[source, 64] = 1.0, 1.0
+    v[source] = 1.0
+    print(f"order of halves, token {token}", flush=True)
+    out, _ = in_chunks(ops, q, k, v, torch.full((n, dim), -200.0, device="cuda"), heads, dim, vdim)
+    expected = torch.zeros(n, vdim, device="cuda")
+    expected[token] = 2.0 ** 24
+    assert torch.equal(out, expected)
+
+
 @pytest.mark.parametrize("per_channel", [False, True])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,spread", [(2, 2, 128, 128, 1.0), (3, 3, 24, 40, 2.0), (4, 2, 64, 130, 3.0), (2, 1, 65, 256, 0.5),
                                                             (1, 1, 5, 1, 6.0)])
