@@ -205,8 +205,8 @@ constexpr int UNITS = 256;                                         // compute un
 // 16.2, 11.2, gated 15.9, 11.8; 128 of 4,096 x 2,048 activated 13.6, 10.8; 190 of 1,024 x 3,072 gated 16.5, 12.8; 190 of 1,408 x 2,048 9.5, 9.2; 17 of 2,048 x 1,024 in four parts 3.7, 3.8.  119 sizes
 // of 17 to 250 rows that the plan has them for are 1.20 times as fast.  Beyond one round they lose: 33 rows of 10,240 x 5,120 (320) 31.0, 35.3; 96 rows of 6,144 x 2,048 (384) 11.4, 16.2.
 //   Both add up the same products in the same order, so that their results are the same bits.  Those of parts and of the library need not be, and the plan, which decides between them, goes on
-// pricing 64 x 64: what it takes ends sooner than it says.  By a price of 64 x 32 it took more from both, a little faster each alone (gated 32 rows of 2,816 x 4,096 in parts 15.4, 14.3; 33 rows
-// of 6,144 x 4,096 within a step 17.2 by the library, 15.6) and not in a job: 33 requests decoding, eight layers and eight steps, 9,100 and 9,232.
+// pricing 64 x 64: what it takes ends sooner than it says, and what goes another way keeps its bits.  By a price of 64 x 32 it would take more from both: gated 32 rows of 2,816 x 4,096 15.4 in
+// parts, 14.3 so; 33 rows of 6,144 x 4,096 within a step 17.2 by the library, 15.6 (33 requests decoding, eight steps: 9,050 to 9,230, by the library 9,090 to 9,150).
 static int small_columns(int form, int M, int N, int parts) {
     const int slim = form == GATED ? 16 : 32;
     return (long)((M + 63) / 64) * ((N + slim - 1) / slim) * parts <= UNITS ? slim : 2 * slim;
